@@ -259,6 +259,14 @@ int nq_pf_plan(const int32_t* counts, int E, int row_lo, int nrows, int32_t* til
 /* hits[e] += counts[e] (hits may be host-mapped). Replaces pf_hits (reference sm120/nqmoe.cu:1241-1245,1288-1293). */
 int nq_pf_hits(const int32_t* counts, int32_t* hits, int E, void* stream);
 
+/* Encoder: tail-biting trellis search of T rings of L <= 1024 targets w [T][L] through the 16-bit shift-register trellis with K = 1
+ * or 2 new bits per step and the values lut [65536]; states [T][L] = the states of the path of least squared error, ties to the
+ * smallest predecessor (reference threads/05-exl3-harness/harness.py:297-364). position_order = 0: w and states in step order; 1: in
+ * ring position order (step i <-> position (L - i) mod L). scratch: 4096 * L bytes for each ring searched at a time (one workgroup
+ * each; one per CU is the most that is of use). w must not hold NaN. */
+int nq_viterbi(const float* w, int T, int L, int K, const float* lut, int64_t* states, void* scratch, int64_t scratch_bytes,
+               int position_order, void* stream);
+
 /* ---- Refinement-record upgrade engine (host threads + one side stream; replaces the class Engine of the reference's
  * streaming/nqstream.cu:51-277 and its Python surface, :8-26). One engine per record file (one rank) and GPU. Unlike the
  * entry points above, an engine owns memory for its lifetime: n_host pinned host entries of rec_bytes each (bounce

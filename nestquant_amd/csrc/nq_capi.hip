@@ -277,3 +277,14 @@ extern "C" int nq_pf_hits(const int32_t* counts, int32_t* hits, int E, void* str
     if (!hits) return 0;
     return launch_pf_hits(counts, hits, E, (hipStream_t)stream);
 }
+
+extern "C" int nq_viterbi(const float* w, int T, int L, int K, const float* lut, int64_t* states, void* scratch, int64_t scratch_bytes, int position_order, void* stream)
+{
+    NQ_REQUIRE(T >= 0 && L >= 1 && L <= 1024 && (K == 1 || K == 2), "nq_viterbi: T=%d L=%d (1..1024) K=%d (1 or 2)", T, L, K);
+    if (T == 0) return 0;
+    NQ_REQUIRE(w && lut && states && scratch, "nq_viterbi: null pointer");
+    NQ_REQUIRE(aligned16(scratch) && aligned16(lut), "nq_viterbi: scratch and codebook must be 16-byte aligned");
+    const int64_t slots = scratch_bytes / ((int64_t)L * 4096);
+    NQ_REQUIRE(slots >= 1, "nq_viterbi: the scratch needs %d bytes for each ring searched at a time", L * 4096);
+    return launch_viterbi(w, T, L, K, lut, states, (uint32_t*)scratch, (int)(slots < T ? slots : T), position_order != 0, (hipStream_t)stream);
+}

@@ -64,5 +64,6 @@ int launch_pf_wdecode(const int64_t* table, const int32_t* hot, int E, int mode,
 int launch_pf_hits(const int32_t* counts, int32_t* hits, int E, hipStream_t st);
 int launch_pf_gemm(const int64_t* table, const int32_t* tiles, int ntiles, int bm, int mode, const void* A0, const void* A1, float* C,
                    int E, int H, int I, const void* Wop, hipStream_t st);
+int launch_viterbi(const float* w, int T, int L, int K, const float* lut, int64_t* st, uint32_t* back, int slots, int rev, hipStream_t s);
 
 }  // namespace nq
