@@ -8,9 +8,9 @@
 //   level 2  w = fp16(A * (1024 + S_b) + B)                                      A = 0x1eee, B = 0xc931
 //   level 3/4 F = (Mb S_b + N S_r + 128) >> 8 ; w = fp16(A' * (1024 + F) + C)   block word Mb | N << 8 per unit
 //
-// gfx950 instruction choices (every opcode of the chain issues at the same measured rate, so their count is what matters):
-//   * one v_alignbit_b32 yields the register that holds two windows 16 bits apart; v_and / v_lshrrev (or one v_bfe_u32 where
-//     the window lies inside a word) cuts the 16-bit state; the hash is ONE v_mul_lo_u32 by 0x83DCD12D;
+// gfx950 instruction choices (all of them but the v_add_u16 issue at the same measured rate, so their count is what matters):
+//   * one v_alignbit_b32 yields the register that holds two windows 16 bits apart; v_add_u16 0 / v_lshrrev cuts the 16-bit
+//     state (see state()); the hash is ONE v_mul_lo_u32 by 0x83DCD12D;
 //   * v_sad_u8 / v_sad_hi_u8 give the byte sums of two weights already packed as the fp16 pair (1024 + S);
 //   * v_dot4_u32_u8 folds Mb * S_b + N * S_r with the rounding constant in its accumulator; v_perm_b32 packs a pair;
 //   * v_pk_fma_f16 is the single-rounded fp16 FMA of the value map.
@@ -193,8 +193,7 @@ __device__ __forceinline__ void ext_words(uint32_t* w, uint32_t nb)
 
 // ---- hash -----------------------------------------------------------------------------------------------------------
 // x = st * 0x83DCD12D mod 2^32 for the 16-bit window st at bit offset O of the extended record w[]. Windows O and O + 16 share
-// one register (window_reg); state() takes the low or the high half of it (an and / a shift, which the compiler merges with
-// the funnel shift into one bit-field extract where the window lies inside a word), times_hash() is the 32-bit multiply
+// one register (window_reg); state() takes the low or the high half of it, times_hash() is the 32-bit multiply
 // (on gfx950 it issues at the rate of the 16-bit multiply-adds it replaces, two per weight before). The
 // multiply is volatile asm so that code which lays several weights side by side keeps that order (weight_pairs2).
 template <int O> __device__ __forceinline__ uint32_t window_reg(const uint32_t* w)
@@ -202,9 +201,19 @@ template <int O> __device__ __forceinline__ uint32_t window_reg(const uint32_t* 
     constexpr int o = (O & 31) >= 16 ? O - 16 : O, i = o >> 5, s = o & 31;
     if constexpr (s == 0) return w[i]; else return __builtin_amdgcn_alignbit(w[i + 1], w[i], s);
 }
+// The low half is cut out by a 16-bit add of 0 (it clears the upper half): of the instructions that do it, the 16-bit ones are the
+// only ones that pair with another wavefront's byte sum, funnel shift or 32-bit multiply. In a loop of one of those and one
+// cut the cut costs 0.9 ns per wavefront and SIMD as v_add_u16 and 1.85 ns as v_and_b32 or v_bfe_u32 (four wavefronts per SIMD);
+// decode layer of four tokens 246 -> 238 us, of one token 74.6 -> 72.9.
 template <int O> __device__ __forceinline__ uint32_t state(uint32_t r)
 {
-    if constexpr ((O & 31) < 16) return r & 0xFFFFu; else return r >> 16;
+    if constexpr ((O & 31) < 16)
+    {
+        uint32_t d;
+        asm("v_add_u16 %0, 0, %1" : "=v"(d) : "v"(r));
+        return d;
+    }
+    else return r >> 16;
 }
 __device__ __forceinline__ uint32_t times_hash(uint32_t st)
 {
