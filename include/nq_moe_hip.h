@@ -256,6 +256,35 @@ int nq_pf_post(const float* y, const int32_t* pos, const int64_t* sel, const voi
 int nq_pf_plan(const int32_t* counts, int E, int row_lo, int nrows, int32_t* tiles, int cap, int32_t* hot, int hot_min, int hot_cap,
                void* stream);
 
+/* A whole step of T tokens on device data, no host synchronisation: pairs sorted by expert, tile plan, rotation, gate|up, SwiGLU,
+ * down, combine -- the chain of the entry points above (reference moe.prefill, sm120/moe.py:282-326) with the casts of its caller
+ * (x.half(), ids.long(), w.half(), out.to(dtype), sm120/serve/nq_vllm.py:522,573) at the loads and the final store. Ids outside
+ * [0, E) contribute nothing. Steps with at most 32 pairs per expert on average run on `stream` alone, longer ones fork onto the side
+ * streams and join again. Calls that share scratch, side streams or events must be ordered on one stream. */
+typedef struct NqPfArgs
+{
+    const void* x;                 /* [T][H], type x_dtype */
+    const void* sel;               /* [T][topk], int64 or int32 (sel_dtype) */
+    const void* rw;                /* [T][topk], type rw_dtype */
+    const int64_t* table;          /* [E][NQ_TBL_W] */
+    void* out;                     /* [T][H], type out_dtype; written whole */
+    int32_t* hits;                 /* optional: hits[e] += picks of e with a weight other than 0 (may be host-mapped) */
+    void* meta; int64_t meta_bytes;   /* nq_pf_meta_bytes() */
+    void *xg, *xu, *h;             /* fp16 [rows][H], [rows][H], [rows][I] */
+    void *acc, *y;                 /* fp32 [rows][2I], [rows][H] */
+    float *zg, *zd;                /* fp32 [rows][4] each, or NULL when no expert has a low-rank plane */
+    void* wop; int64_t wop_bytes;  /* optional scratch of decoded weights (nq_pf_wdecode) with wop_slots slots for experts of >= hot_min rows */
+    void* side[3];                 /* streams of default priority */
+    void* events[4];               /* events without timing of the same device */
+    int32_t T, topk, E, H, I;
+    int32_t rows;                  /* pair rows the scratch holds; more pairs are worked through in chunks (out must then be fp32) */
+    int32_t x_dtype, sel_dtype, rw_dtype, out_dtype;   /* as in NqMoeArgs */
+    int32_t variants;              /* 1: every row has base code 0 and no mask-mode flags (others come out NaN); 3: unknown */
+    int32_t hot_min, wop_slots;
+} NqPfArgs;
+int nq_pf_step(const NqPfArgs* args, void* stream);
+int64_t nq_pf_meta_bytes(int T, int topk, int rows, int E);   /* -1: arguments out of range */
+
 /* hits[e] += counts[e] (hits may be host-mapped). Replaces pf_hits (reference sm120/nqmoe.cu:1241-1245,1288-1293). */
 int nq_pf_hits(const int32_t* counts, int32_t* hits, int E, void* stream);
 

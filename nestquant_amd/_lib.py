@@ -28,6 +28,15 @@ class NqMoeArgs(C.Structure):
                 ("mb_applied_host", C.c_void_p), ("hoist_value_map", C.c_int32), ("reserved_", C.c_int32)]
 
 
+class NqPfArgs(C.Structure):
+    """mirror of struct NqPfArgs in include/nq_moe_hip.h"""
+    _fields_ = [(n, C.c_void_p) for n in ("x", "sel", "rw", "table", "out", "hits", "meta")] + [("meta_bytes", C.c_int64)] + \
+               [(n, C.c_void_p) for n in ("xg", "xu", "h", "acc", "y", "zg", "zd", "wop")] + [("wop_bytes", C.c_int64)] + \
+               [("side", C.c_void_p * 3), ("events", C.c_void_p * 4)] + \
+               [(n, C.c_int32) for n in ("T", "topk", "E", "H", "I", "rows", "x_dtype", "sel_dtype", "rw_dtype", "out_dtype",
+                                         "variants", "hot_min", "wop_slots")]
+
+
 ROUTE_WS_BYTES = 32768          # NQ_ROUTE_WS_BYTES
 
 
@@ -52,6 +61,8 @@ SIGNATURES = {
     "nq_pf_mid_rows": (C.c_int, [_vp, _i32p, _i, _i64p, _vp, _vp, _vp, _i, _i, _i, _i32p, _i, _i, _vp]),
     "nq_pf_post": (C.c_int, [_vp, _i32p, _i64p, _vp, _i, _i, _i, _i, _i64p, _vp, _vp, _i, _i, _i, _vp]),
     "nq_pf_plan": (C.c_int, [_i32p, _i, _i, _i, _i32p, _i, _i32p, _i, _i, _vp]),
+    "nq_pf_step": (C.c_int, [C.POINTER(NqPfArgs), _vp]),
+    "nq_pf_meta_bytes": (C.c_int64, [_i, _i, _i, _i]),
     "nq_pf_hits": (C.c_int, [_i32p, _i32p, _i, _vp]),
     "nq_viterbi": (C.c_int, [_vp, _i, _i, _i, _vp, _vp, _vp, C.c_int64, _i, _vp]),
     # record upgrade engine (host threads; structures mirrored in stream_engine.py)

@@ -11,7 +11,8 @@ char* error_buffer()
     static thread_local char buf[512] = {0};
     return buf;
 }
-static bool shape_ok(int H, int I) { return H > 0 && I > 0 && H % 128 == 0 && I % 128 == 0; }
+// (the kernels address a plane by 32-bit byte offsets: its records, 16 bytes per 64 weights, stay below 4 GB)
+static bool shape_ok(int H, int I) { return H > 0 && I > 0 && H % 128 == 0 && I % 128 == 0 && 2 * (int64_t)H * I < ((int64_t)1 << 33); }
 // the kernels move 16 bytes per lane; rows are multiples of 256 bytes, so the base address decides
 static bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 }  // namespace nq
@@ -69,7 +70,7 @@ extern "C" int nq_dequant(const int64_t* row, int proj, int level, int H, int I,
     NQ_REQUIRE(level == 0 || level == 2 || level == 3 || level == 4, "nq_dequant: level %d not in {0,2,3,4}", level);
     {   // a single projection only needs whole units: N % 16 == 0 and K % 128 == 0
         const int N = proj == 0 ? 2 * I : H, K = proj == 0 ? H : I;
-        NQ_REQUIRE(H > 0 && I > 0 && N % 16 == 0 && K % 128 == 0, "nq_dequant: projection [%d][%d] is not whole 16x128 units", N, K);
+        NQ_REQUIRE(H > 0 && I > 0 && N % 16 == 0 && K % 128 == 0 && (int64_t)N * K < ((int64_t)1 << 33), "nq_dequant: projection [%d][%d] is not whole 16x128 units", N, K);
     }
     return launch_dequant(row, proj, level, H, I, out, (hipStream_t)stream);
 }
@@ -188,7 +189,7 @@ extern "C" int nq_pf_pre(const void* x, const int32_t* pt, const int32_t* pe, in
     NQ_REQUIRE(x && pt && pe && table && xg && xu, "nq_pf_pre: null pointer");
     NQ_REQUIRE(E >= 1 && shape_ok(H, I), "nq_pf_pre: E=%d H=%d I=%d (H, I positive multiples of 128)", E, H, I);
     NQ_REQUIRE(aligned16(x) && aligned16(xg) && aligned16(xu), "nq_pf_pre: x, xg and xu must be 16-byte aligned");
-    return launch_pf_pre(x, pt, pe, np, table, xg, xu, zg, E, H, I, nullptr, 0, 0, (hipStream_t)stream);
+    return launch_pf_pre(x, 0, pt, pe, np, table, xg, xu, zg, E, H, I, nullptr, 0, 0, (hipStream_t)stream);
 }
 
 extern "C" int nq_pf_pre_rows(const void* x, const int32_t* pt, const int32_t* pe, int np, const int64_t* table, void* xg, void* xu,
@@ -200,7 +201,7 @@ extern "C" int nq_pf_pre_rows(const void* x, const int32_t* pt, const int32_t* p
     NQ_REQUIRE(E >= 1 && shape_ok(H, I), "nq_pf_pre_rows: E=%d H=%d I=%d (H, I positive multiples of 128)", E, H, I);
     NQ_REQUIRE(aligned16(x) && aligned16(xg) && aligned16(xu) && aligned16(tiles), "nq_pf_pre_rows: x, xg, xu and tiles must be 16-byte aligned");
     NQ_REQUIRE(cap >= E, "nq_pf_pre_rows: cap=%d below E=%d", cap, E);
-    return launch_pf_pre(x, pt, pe, np, table, xg, xu, zg, E, H, I, tiles, cap, heights, (hipStream_t)stream);
+    return launch_pf_pre(x, 0, pt, pe, np, table, xg, xu, zg, E, H, I, tiles, cap, heights, (hipStream_t)stream);
 }
 
 extern "C" int nq_pf_gemm(const int64_t* table, const int32_t* tiles, int ntiles, int bm, int mode, const void* A0, const void* A1,
@@ -249,7 +250,7 @@ extern "C" int nq_pf_post(const float* y, const int32_t* pos, const int64_t* sel
     NQ_REQUIRE(y && pos && sel && rw && table && out, "nq_pf_post: null pointer");
     NQ_REQUIRE(E >= 1 && shape_ok(H, I), "nq_pf_post: E=%d H=%d I=%d (H, I positive multiples of 128)", E, H, I);
     NQ_REQUIRE(aligned16(y) && aligned16(out), "nq_pf_post: y and out must be 16-byte aligned");
-    return launch_pf_post(y, pos, sel, rw, T, topk, row_lo, nrows, table, out, zd, E, H, I, (hipStream_t)stream);
+    return launch_pf_post(y, pos, sel, 0, rw, 0, T, topk, row_lo, nrows, table, out, 0, 1, zd, E, H, I, (hipStream_t)stream);
 }
 
 extern "C" int nq_pf_wdecode(const int64_t* table, const int32_t* hot, int E, int mode, void* Wop, int64_t wop_bytes, int slots, int H, int I, void* stream)
@@ -287,4 +288,31 @@ extern "C" int nq_viterbi(const float* w, int T, int L, int K, const float* lut,
     const int64_t slots = scratch_bytes / ((int64_t)L * 4096);
     NQ_REQUIRE(slots >= 1, "nq_viterbi: the scratch needs %d bytes for each ring searched at a time", L * 4096);
     return launch_viterbi(w, T, L, K, lut, states, (uint32_t*)scratch, (int)(slots < T ? slots : T), position_order != 0, (hipStream_t)stream);
+}
+
+extern "C" int64_t nq_pf_meta_bytes(int T, int topk, int rows, int E)
+{
+    if (T < 0 || topk < 1 || topk > 64 || rows < 1 || E < 1 || E > 4096 || (int64_t)T * topk > INT32_MAX) return set_error("nq_pf_meta_bytes: T=%d topk=%d rows=%d E=%d", T, topk, rows, E), (int64_t)-1;
+    return pf_meta_bytes(T * topk, rows < T * topk ? rows : T * topk, E);
+}
+
+extern "C" int nq_pf_step(const NqPfArgs* p, void* stream)
+{
+    NQ_REQUIRE(p, "nq_pf_step: null args");
+    const NqPfArgs& a = *p;
+    NQ_REQUIRE(a.T >= 0 && a.topk >= 1 && a.topk <= 64 && (int64_t)a.T * a.topk <= INT32_MAX, "nq_pf_step: T=%d topk=%d (<= 64)", a.T, a.topk);
+    if (a.T == 0) return 0;
+    NQ_REQUIRE(a.x && a.sel && a.rw && a.table && a.out && a.meta && a.xg && a.xu && a.acc && a.h && a.y, "nq_pf_step: null pointer");
+    NQ_REQUIRE(a.E >= 1 && a.E <= 4096 && shape_ok(a.H, a.I), "nq_pf_step: E=%d (1..4096) H=%d I=%d (positive multiples of 128)", a.E, a.H, a.I);
+    NQ_REQUIRE(a.x_dtype >= 0 && a.x_dtype <= 2 && a.rw_dtype >= 0 && a.rw_dtype <= 2 && a.sel_dtype >= 0 && a.sel_dtype <= 1 && a.out_dtype >= 0 && a.out_dtype <= 2,
+               "nq_pf_step: dtype codes x=%d sel=%d rw=%d out=%d", a.x_dtype, a.sel_dtype, a.rw_dtype, a.out_dtype);
+    NQ_REQUIRE(a.variants >= 1 && a.variants <= 3, "nq_pf_step: variants=%d (1 common rows, 2 rare rows, 3 both)", a.variants);
+    NQ_REQUIRE(aligned16(a.x) && aligned16(a.out) && aligned16(a.meta) && aligned16(a.xg) && aligned16(a.xu) && aligned16(a.acc) && aligned16(a.h) && aligned16(a.y) && aligned16(a.wop),
+               "nq_pf_step: buffers must be 16-byte aligned");
+    NQ_REQUIRE(a.rows >= 1 && (a.out_dtype == 0 || a.rows >= (int64_t)a.T * a.topk), "nq_pf_step: rows=%d; a result of another type than fp32 needs all %d pairs in one chunk", a.rows, a.T * a.topk);
+    NQ_REQUIRE((int64_t)a.E + a.rows / 256 + 1 <= 65535, "nq_pf_step: rows=%d exceed one launch", a.rows);
+    NQ_REQUIRE(!a.wop || (a.hot_min >= 1 && a.wop_slots >= 1 && a.wop_bytes >= (int64_t)a.wop_slots * 3 * a.H * a.I * 2), "nq_pf_step: the decoded-weight scratch needs %d slots of 3 * H * I halfs", a.wop_slots);
+    for (int i = 0; i < 3; ++i) NQ_REQUIRE(a.side[i], "nq_pf_step: three side streams");
+    for (int i = 0; i < 4; ++i) NQ_REQUIRE(a.events[i], "nq_pf_step: four events");
+    return launch_pf_step(a, (hipStream_t)stream);
 }

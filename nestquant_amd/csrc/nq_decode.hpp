@@ -141,12 +141,15 @@ __device__ __forceinline__ void prepare_record(uint32_t* w)
 // records further on, the 64-bit record of plane P4: code 11's 128-bit record is the first followed by the second, code 12's
 // is the two interleaved bit by bit (stream bit 2 i = bit i of P3's record, bit 2 i + 1 = bit i of P4's), so that every
 // 16-bit window holds eight bits of each plane.
+// A record's place in its plane is a 32-bit byte offset from an address that is the same for the whole wavefront (planes stay below
+// 4 GB, which the entry points check), so a load takes a scalar base and one address register per lane.
+template <class T> __device__ __forceinline__ T at_offset(gp_u8 base, uint32_t off) { return *(const NQ_GLOBAL T*)(base + off); }
 template <int CODE>
-__device__ __forceinline__ void load_record(uint32_t* w, gp_u8 p, size_t rec, size_t nrec)
+__device__ __forceinline__ void load_record(uint32_t* w, gp_u8 p, uint32_t rec, size_t nrec)
 {
     if constexpr (Pat<CODE>::SPLIT)
     {
-        const u32x2 lo = ((gp_u2)p)[rec], hi = ((gp_u2)(p + nrec * 8))[rec];
+        const u32x2 lo = at_offset<u32x2>(p, rec * 8u), hi = at_offset<u32x2>(p + nrec * 8, rec * 8u);
         w[0] = lo.x; w[1] = lo.y; w[2] = hi.x; w[3] = hi.y;   // code 12: interleaved by prepare_record() where the record is used
     }
     else
@@ -154,20 +157,21 @@ __device__ __forceinline__ void load_record(uint32_t* w, gp_u8 p, size_t rec, si
         static constexpr SubArrays L = sub_arrays(Rec<CODE>::BITS);
         static_for<L.n>([&](auto tag) {
             constexpr int i = decltype(tag)::value, W = L.width[i], at = L.pos[i] >> 5;
-            const gp_u8 q = p + nrec * (size_t)L.before[i] + rec * (size_t)(W / 8);
-            if constexpr (W == 128) { const u32x4 v = *(gp_u4)q; w[at] = v.x; w[at + 1] = v.y; w[at + 2] = v.z; w[at + 3] = v.w; }
-            else if constexpr (W == 64) { const u32x2 v = *(gp_u2)q; w[at] = v.x; w[at + 1] = v.y; }
-            else if constexpr (W == 32) w[at] = *(gp_u32)q;
-            else w[at] = *(gp_u16)q;                              // a 16-bit piece always starts a word
+            const gp_u8 q = p + nrec * (size_t)L.before[i];
+            const uint32_t off = rec * (uint32_t)(W / 8);
+            if constexpr (W == 128) { const u32x4 v = at_offset<u32x4>(q, off); w[at] = v.x; w[at + 1] = v.y; w[at + 2] = v.z; w[at + 3] = v.w; }
+            else if constexpr (W == 64) { const u32x2 v = at_offset<u32x2>(q, off); w[at] = v.x; w[at + 1] = v.y; }
+            else if constexpr (W == 32) w[at] = at_offset<uint32_t>(q, off);
+            else w[at] = at_offset<uint16_t>(q, off);             // a 16-bit piece always starts a word
         });
         if constexpr (L.tail != 0)
         {
             // bits [rec * tail, + tail) of the bit-packed tail array; a field that can straddle two words (tail does not divide
             // 32) takes the second word too, which for the last record is the pad
-            const size_t bit = rec * (size_t)L.tail;
-            const gp_u32 q = (gp_u32)(p + nrec * (size_t)L.tail_before) + (bit >> 5);
+            const uint32_t bit = rec * (uint32_t)L.tail, off = (bit >> 5) * 4u;
+            const gp_u8 q = p + nrec * (size_t)L.tail_before;
             const int sh = (int)(bit & 31);
-            uint32_t v = (32 % L.tail) ? __builtin_amdgcn_alignbit(q[1], q[0], sh) : q[0] >> sh;
+            uint32_t v = (32 % L.tail) ? __builtin_amdgcn_alignbit(at_offset<uint32_t>(q, off + 4u), at_offset<uint32_t>(q, off), sh) : at_offset<uint32_t>(q, off) >> sh;
             v &= (1u << L.tail) - 1u;
             if constexpr ((L.tail_pos & 31) == 0) w[L.tail_pos >> 5] = v;       // the tail opens a word of its own,
             else w[L.tail_pos >> 5] |= v << (L.tail_pos & 31);                 // or sits above the 16-bit piece
@@ -334,9 +338,9 @@ struct Planes { gp_u4 base; gp_u8 res; gp_u32 dw; gp_u8 var; gp_u64 flags; int c
 // Base record of a lane: code 0 = one uint4 per record; other codes = the residual plane's sub-array layout at
 // Rec<BK>::BITS bits per record (reference sm120/NQ_RES_V2.md:38-46), at most 128 bits.
 template <int BK>
-__device__ __forceinline__ u32x4 load_base(const Planes& P, size_t rec, size_t nrec)
+__device__ __forceinline__ u32x4 load_base(const Planes& P, uint32_t rec, size_t nrec)
 {
-    if constexpr (BK == 0) return P.base[rec];
+    if constexpr (BK == 0) return at_offset<u32x4>((gp_u8)P.base, rec * 16u);
     else
     {
         static_assert(Rec<BK>::BITS <= 128, "base records are at most four words");
@@ -357,11 +361,11 @@ __device__ __forceinline__ void dispatch_base(int bcode, F&& f)
 // Mask mode (reference sm120/nqmoe.cu:22-24,202-206): flags = one uint64 per strip, bit c = chunk c is refined; the residual
 // plane and its block words are compact over the nm = popcount(flags) refined chunks of every strip, in chunk order, and
 // the other chunks decode at level 2. Flags are equal over the 8 strips of a 128-row group.
-struct MaskedUnit { bool on; size_t unit; size_t nrec; };     // refined?; residual unit index; residual records of the plane
-__device__ __forceinline__ MaskedUnit masked_unit(uint64_t f, size_t strip, int c, size_t nstrips)
+struct MaskedUnit { bool on; uint32_t unit; size_t nrec; };   // refined?; residual unit index; residual records of the plane
+__device__ __forceinline__ MaskedUnit masked_unit(uint64_t f, uint32_t strip, int c, size_t nstrips)
 {
     const int nm = __popcll(f);
-    return MaskedUnit{((f >> c) & 1ull) != 0, strip * nm + __popcll(f & ((1ull << c) - 1ull)), nstrips * nm * 32};
+    return MaskedUnit{((f >> c) & 1ull) != 0, strip * (uint32_t)nm + (uint32_t)__popcll(f & ((1ull << c) - 1ull)), nstrips * nm * 32};
 }
 __device__ __forceinline__ Planes planes_of(const int64_t* ent, int mode)
 {

@@ -49,7 +49,7 @@ __device__ __forceinline__ void decode_unit_bk(const Planes& P, int lv, size_t u
     const int src = (lane & ~3) | ((lane + 1) & 3);           // next lane of the ring
     uint32_t wb[6];
     {
-        const u32x4 v = load_base<BK>(P, unit * 32 + lane32, nrec);
+        const u32x4 v = load_base<BK>(P, (uint32_t)unit * 32 + lane32, nrec);
         wb[0] = v.x; wb[1] = v.y; wb[2] = v.z; wb[3] = v.w;
         ext_base<BK>(wb, __shfl(wb[0], src));
     }
@@ -60,7 +60,7 @@ __device__ __forceinline__ void decode_unit_bk(const Planes& P, int lv, size_t u
     {   // the two halves of a wavefront may sit in different strips or chunks: this branch may diverge between them, and the
         // ring neighbour of a lane is always in its own half
         const size_t strip = unit / C;
-        const MaskedUnit m = masked_unit(P.flags[strip], strip, (int)(unit - strip * C), nrec / 32 / C);
+        const MaskedUnit m = masked_unit(P.flags[strip], (uint32_t)strip, (int)(unit - strip * C), nrec / 32 / C);
         on = m.on; runit = m.unit; rnrec = m.nrec;
     }
     if (!on)
@@ -73,7 +73,7 @@ __device__ __forceinline__ void decode_unit_bk(const Planes& P, int lv, size_t u
     dispatch_code(P.code, [&](auto tag) {
         constexpr int CODE = decltype(tag)::value;
         uint32_t wr[Rec<CODE>::NW + 2];
-        load_record<CODE>(wr, P.res, runit * 32 + lane32, rnrec);
+        load_record<CODE>(wr, P.res, (uint32_t)runit * 32 + lane32, rnrec);
         prepare_record<CODE>(wr);
         ext_words<Rec<CODE>::BITS, Rec<CODE>::NW>(wr, __shfl(wr[0], src));
         decode_to_tile<true, CODE, BK>(wb, wr, k, tile, lane32);

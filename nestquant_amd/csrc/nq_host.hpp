@@ -5,6 +5,8 @@
 #include <stdio.h>
 #include <stdarg.h>
 
+struct NqPfArgs;                      // include/nq_moe_hip.h
+
 namespace nq {
 
 // last error text of the calling thread; every entry point returns 0 on success, non-zero after set_error()
@@ -51,12 +53,12 @@ int query_occ(int mode, int any_rows, int sb, int shm, int* out);
 int launch_mailbox(int64_t* table, const int64_t* stage, const int32_t* seq, int32_t* applied, int32_t* applied_host, int E, hipStream_t st);
 int launch_dequant(const int64_t* row, int proj, int level, int H, int I, void* out, hipStream_t st);
 int launch_pf_decode(const int64_t* table, const int32_t* experts, int G, void* Wgu, void* Wdn, int H, int I, hipStream_t st);
-int launch_pf_pre(const void* x, const int32_t* pt, const int32_t* pe, int np, const int64_t* table, void* xg, void* xu, float* zg, int E, int H, int I,
+int launch_pf_pre(const void* x, int xdt, const int32_t* pt, const int32_t* pe, int np, const int64_t* table, void* xg, void* xu, float* zg, int E, int H, int I,
                   const int32_t* tiles, int cap, int heights, hipStream_t st);
 int launch_pf_mid(const float* acc_gu, const int32_t* pe, int np, const int64_t* table, void* h, const float* zg, float* zd, int E, int H, int I,
                   const int32_t* tiles, int cap, int heights, hipStream_t st);
-int launch_pf_post(const float* y, const int32_t* pos, const int64_t* sel, const void* rw, int T, int topk, int row_lo, int nrows,
-                   const int64_t* table, float* out, const float* zd, int E, int H, int I, hipStream_t st);
+int launch_pf_post(const float* y, const int32_t* pos, const void* sel, int sdt, const void* rw, int wdt, int T, int topk, int row_lo, int nrows,
+                   const int64_t* table, void* out, int odt, int add, const float* zd, int E, int H, int I, hipStream_t st);
 int launch_sal(const void* x, int x_dtype, int64_t sx, const void* w, int w_dtype, const void* ids, int ids_dtype, int T, int H, int K,
                int E, float rsf, double* acc, double* host, hipStream_t st);
 int launch_pf_plan(const int32_t* counts, int E, int row_lo, int nrows, int32_t* tiles, int cap, int32_t* hot, int hot_min, int hot_cap, hipStream_t st);
@@ -64,6 +66,8 @@ int launch_pf_wdecode(const int64_t* table, const int32_t* hot, int E, int mode,
 int launch_pf_hits(const int32_t* counts, int32_t* hits, int E, hipStream_t st);
 int launch_pf_gemm(const int64_t* table, const int32_t* tiles, int ntiles, int bm, int mode, const void* A0, const void* A1, float* C,
                    int E, int H, int I, const void* Wop, hipStream_t st);
+int launch_pf_step(const ::NqPfArgs& a, hipStream_t st);
+int64_t pf_meta_bytes(int P, int R, int E);
 int launch_viterbi(const float* w, int T, int L, int K, const float* lut, int64_t* st, uint32_t* back, int slots, int rev, hipStream_t s);
 
 }  // namespace nq

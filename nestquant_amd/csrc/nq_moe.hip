@@ -78,44 +78,10 @@ __device__ __forceinline__ void sum_partials(const float* const* p, size_t strid
     }
 }
 
-// ---- caller dtypes: the casts a caller would otherwise launch as separate kernels (x.half(), ids.long(), w.half(),
-// out.to(x.dtype); reference sm120/serve/nq_vllm.py:522,560,573) happen at the loads and the final store, with the same
-// roundings: activations and routing weights pass through fp16, the fp32 result is rounded once to the output type.
-constexpr int DT_BF16 = 1, DT_F32 = 2, DT_I32 = 1, DT_OUT_F16 = 1, DT_OUT_BF16 = 2;   // 0 = the default type of each argument (fp16, int64, fp32 out)
-__device__ __forceinline__ float bf16_to_f(uint16_t v) { return __builtin_bit_cast(float, (uint32_t)v << 16); }
-__device__ __forceinline__ uint16_t f_to_bf16(float f)           // round to nearest even; NaN stays NaN
-{
-    uint32_t u = __builtin_bit_cast(uint32_t, f);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40u);
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return (uint16_t)(u >> 16);
-}
-__device__ __forceinline__ long long sel_at(const MoeArgs& a, int i)
-{
-    return a.sel_dtype == DT_I32 ? (long long)((const int32_t*)a.sel)[i] : (long long)((const int64_t*)a.sel)[i];
-}
-__device__ __forceinline__ float rw_at(const MoeArgs& a, int i)   // the weight as fp16 would hold it
-{
-    if (a.rw_dtype == DT_BF16) return (float)(_Float16)bf16_to_f(((const uint16_t*)a.rw)[i]);
-    if (a.rw_dtype == DT_F32) return (float)(_Float16)((const float*)a.rw)[i];
-    return (float)((const _Float16*)a.rw)[i];
-}
-__device__ __forceinline__ half2_t x2_at(const MoeArgs& a, size_t i)   // x[i], x[i + 1] (i even) as fp16
-{
-    if (a.x_dtype == DT_BF16)
-    {
-        const uint32_t v = *(const uint32_t*)((const uint16_t*)a.x + i);
-        return half2_t{(_Float16)bf16_to_f((uint16_t)v), (_Float16)bf16_to_f((uint16_t)(v >> 16))};
-    }
-    if (a.x_dtype == DT_F32) { const float2 v = *(const float2*)((const float*)a.x + i); return half2_t{(_Float16)v.x, (_Float16)v.y}; }
-    return *(const half2_t*)((const _Float16*)a.x + i);
-}
-__device__ __forceinline__ void out2_store(const MoeArgs& a, size_t i, float v0, float v1)   // out[i], out[i + 1] (i even)
-{
-    if (a.out_dtype == DT_OUT_F16) { half2_t h; h.x = (_Float16)v0; h.y = (_Float16)v1; *(half2_t*)((_Float16*)a.out + i) = h; }
-    else if (a.out_dtype == DT_OUT_BF16) *(uint32_t*)((uint16_t*)a.out + i) = (uint32_t)f_to_bf16(v0) | ((uint32_t)f_to_bf16(v1) << 16);
-    else *(float2*)((float*)a.out + i) = make_float2(v0, v1);
-}
+__device__ __forceinline__ long long sel_at(const MoeArgs& a, int i) { return id_at(a.sel, a.sel_dtype, i); }
+__device__ __forceinline__ float rw_at(const MoeArgs& a, int i) { return w_at(a.rw, a.rw_dtype, i); }
+__device__ __forceinline__ half2_t x2_at(const MoeArgs& a, size_t i) { return act2_at(a.x, a.x_dtype, i); }
+__device__ __forceinline__ void out2_store(const MoeArgs& a, size_t i, float v0, float v1) { res2_store(a.out, a.out_dtype, i, v0, v1); }
 
 constexpr int MAXTOK = 8;                      // tokens of one run = tokens of one call (the MFMA N dimension holds 16)
 // What the projection launches need to know about run r, written once per call by nq_prep_k (one per projection: the plane
@@ -503,15 +469,17 @@ __device__ __forceinline__ void finish_dn(const MoeArgs& a, const PickInfo& R, i
 // host says so, MoeArgs::common_rows). A run whose row is nevertheless of another kind is not decoded as if it were common:
 // its plane is not read and its partial sums are NaN, so every token that picked it comes out NaN. ANYROW = true also
 // carries the decode loops of the other base codes and of mask mode, which cost ~35 registers that the common kernel does
-// not have to pay for. Four wavefronts per SIMD is the measured optimum for the gate|up launch (three: +4 us per layer; five,
-// which the common kernel reaches at 92 registers: +1.5 us), so the register allocator is told to aim at exactly that. The
-// common down launch gains from five (96 registers, three of them spilled): its 1536 workgroups then need 1.2 rounds instead of
-// 1.5 (-0.4 us per layer at one token, -2.5 us at four); six spills sixteen registers and loses 0.9 us.
+// not have to pay for. Four wavefronts per SIMD is the measured optimum for the gate|up launch (three: +4 us per layer; five:
+// +1.5 us), so the register allocator is told to aim at exactly that. The common down launch gains from five (90 registers): its
+// 1536 workgroups then need 1.2 rounds instead of 1.5 (-0.4 us per layer at one token, -2.5 us at four).
 template <int MODE, bool ANYROW>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == 1 && !ANYROW ? 5 : 4, MODE == 1 && !ANYROW ? 5 : 4)))
 nq_gemv_k(MoeArgs a, int NC)
 {
     extern __shared__ __align__(16) char smem[];
+    // Exactly four gate|up workgroups per CU: at one token the launch has four for every CU, and with room for a fifth the
+    // dispatcher fills some CUs with five and leaves others with three. The body needs 90 registers; naming v100 claims 104.
+    if constexpr (MODE == 0 && !ANYROW) asm volatile("" ::: "v100");
     __builtin_amdgcn_s_setprio(3);                               // the head is a chain of latencies (see progress_priority)
     __shared__ float zl[MAXTOK][4];                              // gate|up finisher: x V_gu^T of the run's tokens (low-rank plane)
     __shared__ int last;
@@ -552,16 +520,16 @@ nq_gemv_k(MoeArgs a, int NC)
     const int strip = 2 * (blockIdx.x * SB + warp) + ss;
     const Planes P = R.P;                                        // block-uniform: the plane addresses stay in scalar registers
     LaneCtx L;
-    L.unit0 = (size_t)strip * C + chunk0; L.rec0 = L.unit0 * 32 + 4 * g + t4;
+    L.unit0 = (uint32_t)strip * C + chunk0; L.rec0 = L.unit0 * 32 + 4 * g + t4;
     L.nrec = (size_t)(N / 16) * C * 32;
     L.src = a.G == 2 ? lane ^ 16 : (lane + 16) & 63;             // next record of the ring: rings of four lanes, or of two
-    L.g = g; L.strip = (size_t)strip; L.nstrips = (size_t)(N / 16); L.chunk0 = chunk0;
+    L.g = g; L.strip = (uint32_t)strip; L.nstrips = (size_t)(N / 16); L.chunk0 = chunk0;
     L.xs = (n < ntok ? smem + n * rowstride : zero) + t4 * 16; L.xstep = n < ntok ? 256 : 0;
     // block-uniform: a row the common kernel has no loop for (its plane is not read: the records have another size or order)
     const bool foreign = !ANYROW && (P.bcode != 0 || (P.flags != nullptr && R.level != 2));
     u32x4 nb0 = {0u, 0u, 0u, 0u};
-    if constexpr (ANYROW) { if (P.bcode == 1) nb0 = load_base<1>(P, L.rec0, L.nrec); else nb0 = P.base[L.rec0]; }
-    else if (!foreign) nb0 = P.base[L.rec0];
+    if constexpr (ANYROW) { if (P.bcode == 1) nb0 = load_base<1>(P, L.rec0, L.nrec); else nb0 = load_base<0>(P, L.rec0, L.nrec); }
+    else if (!foreign) nb0 = load_base<0>(P, L.rec0, L.nrec);
 
     // ---- stage the run's tokens for this k-slice in B-operand order
     if constexpr (MODE == 0)

@@ -1,18 +1,21 @@
-// Prefill path (T > 8 tokens): every routed expert's weights are decoded once per 16..256-row tile of its tokens, inside
+// Prefill path (steps of more tokens than a decode call takes): every routed expert's weights are decoded once per 16..256-row tile of its tokens, inside
 // the grouped GEMM itself, never written to HBM (reference: pf_decode to fp16 in HBM + Triton/cuBLAS grouped GEMM,
 // sm120/nqmoe.cu:942-1240, sm120/pf_gemm.py:7-34, sm120/moe.py:282-326).
 //
+//   nq_pf_sort_k  pairs sorted by expert, per-expert counts, hits; the tile list of a step without tall tiles
 //   nq_pf_pre_k   per (token, expert) pair, sorted by expert: xg / xu = fp16(Hadamard-128(x * su_g / su_u)), written in
 //                 B-operand column order so the GEMM stages them with straight 16-byte copies      (reference nq_pf_pre)
 //   nq_pf_gemm_k  C[rows of expert j][N] = A[rows][K] @ W_j[N][K]^T: grid (N / 128, tiles); a tile = (expert, row0, rows
 //                 <= 16 TG). Per 128-column chunk the block stages the tile's activations in LDS while each wavefront
 //                 decodes two strips of the expert's records into MFMA A operands, then runs TG x 8 MFMAs
 //                 (v_mfma_f32_16x16x32_f16, fp32 accumulate) over the staged tokens. Level from the live table row.
+//   nq_pf_short_k the same for all tiles of up to 64 rows in one launch
 //   nq_pf_mid_k   Hadamard * sv, SwiGLU, * su_d, Hadamard -> h fp16 (B-operand order)               (reference nq_pf_mid)
 //   nq_pf_post_k  out[token] += sum over its picks of rw * sv_o (.) Hadamard(y): gathered per token, no atomics  (reference nq_pf_post)
 //   nq_pf_hits_k  hits[e] += counts[e]                                                            (reference nq_pf_hits)
 #include "nq_tile.hpp"
 #include "nq_host.hpp"
+#include "../../include/nq_moe_hip.h"
 
 namespace nq {
 
@@ -56,7 +59,7 @@ __device__ __forceinline__ bool row_in_heights(const int32_t* __restrict__ tiles
 
 // grid (npairs), block 256: wave w handles the 512-column segments w, w + 4, ... of the pair's row, gate and up together.
 // tiles (optional): work only on the rows of the tile heights in `heights`
-__global__ void __launch_bounds__(256) nq_pf_pre_k(const _Float16* __restrict__ x, const int32_t* __restrict__ pt, const int32_t* __restrict__ pe,
+__global__ void __launch_bounds__(256) nq_pf_pre_k(const void* __restrict__ x, int xdt, const int32_t* __restrict__ pt, const int32_t* __restrict__ pe,
                                                     const int64_t* __restrict__ table, _Float16* xg, _Float16* xu, float* zg, int E, int H, int I,
                                                     const int32_t* __restrict__ tiles, int cap, int heights)
 {
@@ -67,7 +70,7 @@ __global__ void __launch_bounds__(256) nq_pf_pre_k(const _Float16* __restrict__ 
     const int ng = H / 128;
     const bool live = e >= 0 && e < E && table[(size_t)e * TBL_W] > 0;
     const _Float16* signs = live ? (const _Float16*)table[(size_t)e * TBL_W + 9] : nullptr;
-    const _Float16* xr = x + (size_t)pt[p] * H;
+    const size_t xr = live ? (size_t)pt[p] * H : 0;             // first element of the token's row
     // low-rank plane (table words 14, 16): zg[p] = x V_gu^T over the raw activations, for the mid kernel
     const _Float16* lr = live ? (const _Float16*)table[(size_t)e * TBL_W + 14] : nullptr;
     const int rg = lr ? (int)table[(size_t)e * TBL_W + 16] : 0;
@@ -76,7 +79,7 @@ __global__ void __launch_bounds__(256) nq_pf_pre_k(const _Float16* __restrict__ 
         float zz[4] = {0.f, 0.f, 0.f, 0.f};
         for (int k = 2 * threadIdx.x; k < H; k += 512)
         {
-            const half2_t xv = *(const half2_t*)(xr + k);
+            const half2_t xv = act2_at(x, xdt, xr + k);
 #pragma unroll
             for (int r = 0; r < 4; ++r)
                 if (r < rg) { const half2_t vv = *(const half2_t*)(lr + (size_t)r * H + k); zz[r] += (float)xv.x * (float)vv.x + (float)xv.y * (float)vv.y; }
@@ -105,7 +108,7 @@ __global__ void __launch_bounds__(256) nq_pf_pre_k(const _Float16* __restrict__ 
         if (live)
         {
             const _Float16* sug = signs, *suu = signs + 2 * H + 3 * I;
-            const uint4 xi = *(const uint4*)(xr + k0 + 8 * lane), gi = *(const uint4*)(sug + k0 + 8 * lane), ui = *(const uint4*)(suu + k0 + 8 * lane);
+            const uint4 xi = act8_at(x, xdt, xr + k0 + 8 * lane), gi = *(const uint4*)(sug + k0 + 8 * lane), ui = *(const uint4*)(suu + k0 + 8 * lane);
             *(uint4*)(sb + 8 * lane) = xi; *(uint4*)(sb + 512 + 8 * lane) = gi; *(uint4*)(sb + 1024 + 8 * lane) = ui;
             wave_sync();
 #pragma unroll
@@ -146,7 +149,7 @@ __global__ void __launch_bounds__(256) nq_pf_pre_k(const _Float16* __restrict__ 
         if (live)
         {
             const _Float16* su = up ? signs + 2 * H + 3 * I : signs;
-            const half2_t xv = *(const half2_t*)(xr + k), sv = *(const half2_t*)(su + k);
+            const half2_t xv = act2_at(x, xdt, xr + k), sv = *(const half2_t*)(su + k);
             v0 = (float)xv.x * (float)sv.x; v1 = (float)xv.y * (float)sv.y;
             wht128(v0, v1, lane);
         }
@@ -239,12 +242,13 @@ __global__ void __launch_bounds__(256) nq_pf_mid_k(const float* __restrict__ acc
     }
 }
 
-// grid (T), block 256: out[t] += sum over the token's picks whose pair row lies in [row_lo, row_lo + nrows) of
-// rw * sv_o (.) Hadamard(y[row]); pos[t][k] = row of pair (t, k) in the expert-sorted order. One block owns a token, so
+// grid (T), block 256: out[t] (+)= sum over the token's picks whose pair row lies in [row_lo, row_lo + nrows) of
+// rw * sv_o (.) Hadamard(y[row]); pos[t][k] = row of pair (t, k) in the expert-sorted order; add: on top of what out holds (fp32),
+// else out is written whole, zeros included. One block owns a token, so
 // the sum needs no atomics and its order is fixed (the reference's pf_post adds with float atomics in arrival order).
-__global__ void __launch_bounds__(256) nq_pf_post_k(const float* __restrict__ y, const int32_t* __restrict__ pos, const int64_t* __restrict__ sel,
-                                                     const _Float16* __restrict__ rw, int topk, int row_lo, int nrows,
-                                                     const int64_t* __restrict__ table, float* out, const float* zd, int E, int H, int I)
+__global__ void __launch_bounds__(256) nq_pf_post_k(const float* __restrict__ y, const int32_t* __restrict__ pos, const void* __restrict__ sel, int sdt,
+                                                     const void* __restrict__ rw, int wdt, int topk, int row_lo, int nrows,
+                                                     const int64_t* __restrict__ table, void* out, int odt, int add, const float* zd, int E, int H, int I)
 {
     const int t = blockIdx.x, lane = threadIdx.x & 63, warp = threadIdx.x >> 6;
     // the token's live picks, gathered once: row, weight and sign vector (picks keep their order, so does the sum)
@@ -256,8 +260,8 @@ __global__ void __launch_bounds__(256) nq_pf_post_k(const float* __restrict__ y,
         if (lane < topk)
         {
             r = pos[(size_t)t * topk + lane] - row_lo;
-            const long long e = sel[(size_t)t * topk + lane];
-            w = (float)rw[(size_t)t * topk + lane];
+            const long long e = id_at(sel, sdt, (size_t)t * topk + lane);
+            w = w_at(rw, wdt, (size_t)t * topk + lane);
             if (r >= 0 && r < nrows && e >= 0 && e < E && w != 0.f && table[(size_t)e * TBL_W] > 0)
             {
                 ok = true; sv = (const _Float16*)table[(size_t)e * TBL_W + 9] + H + 3 * I;
@@ -277,7 +281,7 @@ __global__ void __launch_bounds__(256) nq_pf_post_k(const float* __restrict__ y,
     }
     __syncthreads();
     const int np = p_n;
-    if (np == 0) return;
+    if (np == 0 && add) return;
     for (int grp = warp; grp < H / 128; grp += 4)
     {
         const int col = grp * 128 + 2 * lane;
@@ -310,8 +314,8 @@ __global__ void __launch_bounds__(256) nq_pf_post_k(const float* __restrict__ y,
                 o0 += w * v0; o1 += w * v1;
             }
         }
-        float2* op = (float2*)(out + (size_t)t * H + col);
-        float2 cur = *op; cur.x += o0; cur.y += o1; *op = cur;
+        if (add) { const float2 cur = *(const float2*)((const float*)out + (size_t)t * H + col); o0 = cur.x + o0; o1 = cur.y + o1; }   // fp32 results only
+        res2_store(out, odt, (size_t)t * H + col, o0, o1);
     }
 }
 
@@ -420,10 +424,10 @@ template <bool RES, int CODE>
 __device__ __forceinline__ void wdecode_chunks(const Planes& P, const LaneCtx& L, int C, u32x4* dst, int lane)
 {
     constexpr int NW = RES ? Rec<CODE>::NW : 1;
-    u32x4 nb = P.base[L.rec0];
+    u32x4 nb = load_base<0>(P, L.rec0, L.nrec);
     uint32_t nr[NW + 2] = {0}, ndw = 0, nvar = 0;
-    if constexpr (RES) { load_record<CODE>(nr, P.res, L.rec0, L.nrec); ndw = P.dw[L.unit0]; }
-    if (P.var) nvar = P.var[L.unit0];
+    if constexpr (RES) { load_record<CODE>(nr, P.res, L.rec0, L.nrec); ndw = at_offset<uint32_t>((gp_u8)P.dw, L.unit0 * 4u); }
+    if (P.var) nvar = at_offset<uint8_t>(P.var, L.unit0);
     for (int c = 0; c < C; ++c)
     {
         uint32_t wb[6], wr[NW + 2];
@@ -433,9 +437,9 @@ __device__ __forceinline__ void wdecode_chunks(const Planes& P, const LaneCtx& L
         const uint32_t dw = ndw, var = nvar;
         if (c + 1 < C)
         {
-            nb = P.base[L.rec0 + (size_t)(c + 1) * 32];
-            if constexpr (RES) { load_record<CODE>(nr, P.res, L.rec0 + (size_t)(c + 1) * 32, L.nrec); ndw = P.dw[L.unit0 + c + 1]; }
-            if (P.var) nvar = P.var[L.unit0 + c + 1];
+            nb = load_base<0>(P, L.rec0 + (uint32_t)(c + 1) * 32, L.nrec);
+            if constexpr (RES) { load_record<CODE>(nr, P.res, L.rec0 + (uint32_t)(c + 1) * 32, L.nrec); ndw = at_offset<uint32_t>((gp_u8)P.dw, (L.unit0 + c + 1) * 4u); }
+            if (P.var) nvar = at_offset<uint8_t>(P.var, L.unit0 + c + 1);
         }
         ext_base<0>(wb, __shfl(wb[0], L.src));
         const uint32_t sgm = ((var >> L.g) & 1u) * 0x80008000u;
@@ -466,10 +470,10 @@ __global__ void __launch_bounds__(256) nq_pf_wdecode_k(const int64_t* table, con
     const int N = mode == 0 ? 2 * I : H, K = mode == 0 ? H : I, C = K / 128;
     const int sp = blockIdx.x * 4 + warp, t4 = lane >> 4, ss = (lane >> 3) & 1, g = lane & 7;
     LaneCtx L;
-    L.unit0 = (size_t)(2 * sp + ss) * C; L.rec0 = L.unit0 * 32 + 4 * g + t4;
+    L.unit0 = (uint32_t)(2 * sp + ss) * C; L.rec0 = L.unit0 * 32 + 4 * g + t4;
     L.nrec = (size_t)(N / 16) * C * 32;
     L.src = (lane + 16) & 63; L.g = g; L.xs = nullptr; L.xstep = 0;
-    L.strip = (size_t)(2 * sp + ss); L.nstrips = (size_t)(N / 16); L.chunk0 = 0;
+    L.strip = (uint32_t)(2 * sp + ss); L.nstrips = (size_t)(N / 16); L.chunk0 = 0;
     u32x4* dst = Wop + wop_base(slot, mode, H, I) + (size_t)sp * C * 8 * 64;
     if (lv == 2) wdecode_chunks<false, 0>(P, L, C, dst, lane);
     else dispatch_code(P.code, [&](auto tag) { wdecode_chunks<true, decltype(tag)::value>(P, L, C, dst, lane); });
@@ -591,8 +595,8 @@ __device__ __forceinline__ void pf_chunks(const Planes& P, const LaneCtx& L, int
     // an expert without flags that comes through this variant (base code other than 0) reads as "every chunk refined",
     // for which the compact residual indexing is the dense one
     const uint64_t mflags = masked ? (P.flags ? P.flags[L.strip] : (C >= 64 ? ~0ull : (1ull << C) - 1ull)) : 0ull;
-    if constexpr (RES && !masked) { load_record<CODE>(nr, P.res, L.rec0, L.nrec); ndw = P.dw[L.unit0]; }
-    if (P.var) nvar = P.var[L.unit0];
+    if constexpr (RES && !masked) { load_record<CODE>(nr, P.res, L.rec0, L.nrec); ndw = at_offset<uint32_t>((gp_u8)P.dw, L.unit0 * 4u); }
+    if (P.var) nvar = at_offset<uint8_t>(P.var, L.unit0);
     const int lane = threadIdx.x & 63, warp = threadIdx.x >> 6, t4 = lane >> 4, n = lane & 15;
     // Staging: wavefront w copies rows 16 u + 4 w + (lane >> 4), u = 0 .. TG - 1, of the tile, one 1 KB
     // global -> LDS load per u (64 lanes x 16 bytes land in LDS in lane order, so a load fills 4 rows x 256 bytes). The
@@ -623,9 +627,9 @@ __device__ __forceinline__ void pf_chunks(const Planes& P, const LaneCtx& L, int
             }
         if (c + 1 < C)
         {
-            nb = load_base<BK>(P, L.rec0 + (size_t)(c + 1) * 32, L.nrec);
-            if constexpr (RES && !masked) { load_record<CODE>(nr, P.res, L.rec0 + (size_t)(c + 1) * 32, L.nrec); ndw = P.dw[L.unit0 + c + 1]; }
-            if (P.var) nvar = P.var[L.unit0 + c + 1];
+            nb = load_base<BK>(P, L.rec0 + (uint32_t)(c + 1) * 32, L.nrec);
+            if constexpr (RES && !masked) { load_record<CODE>(nr, P.res, L.rec0 + (uint32_t)(c + 1) * 32, L.nrec); ndw = at_offset<uint32_t>((gp_u8)P.dw, (L.unit0 + c + 1) * 4u); }
+            if (P.var) nvar = at_offset<uint8_t>(P.var, L.unit0 + c + 1);
         }
         ext_base<BK>(wb, __shfl(wb[0], L.src));
         const uint32_t sgm = ((var >> L.g) & 1u) * 0x80008000u;
@@ -670,13 +674,9 @@ __device__ __forceinline__ void pf_chunks(const Planes& P, const LaneCtx& L, int
 // MASKED = false skips the tiles of experts in mask mode (table flags word set) or with a base window code other than 0,
 // MASKED = true takes only those: the rarely used paths keep their extra registers out of the common kernel
 template <int TG, bool MASKED>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) nq_pf_gemm_k(PfGemm a)
+__device__ __forceinline__ void pf_tile(const PfGemm& a, int e, int row0, int nrows, int slot, char* smem)
 {
-    extern __shared__ __align__(16) char smem[];
     const int lane = threadIdx.x & 63, warp = threadIdx.x >> 6;
-    const int32_t* tile = a.tiles + 4 * blockIdx.y;
-    const int e = tile[0], row0 = tile[1], nrows = tile[2], slot = tile[3] - 1;
-    if (e < 0 || e >= a.E || nrows <= 0) return;
     const int64_t* ent = a.table + (size_t)e * TBL_W;
     const int lv = (int)ent[0];
     if (lv <= 0) return;                                         // rows of a level-0 expert are skipped downstream
@@ -696,10 +696,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
         return;
     }
     LaneCtx L;
-    L.unit0 = (size_t)(2 * sp + ss) * C; L.rec0 = L.unit0 * 32 + 4 * g + t4;
+    L.unit0 = (uint32_t)(2 * sp + ss) * C; L.rec0 = L.unit0 * 32 + 4 * g + t4;
     L.nrec = (size_t)(N / 16) * C * 32;
     L.src = (lane + 16) & 63; L.g = g; L.xs = nullptr; L.xstep = 0;
-    L.strip = (size_t)(2 * sp + ss); L.nstrips = (size_t)(N / 16); L.chunk0 = 0;
+    L.strip = (uint32_t)(2 * sp + ss); L.nstrips = (size_t)(N / 16); L.chunk0 = 0;
     float4_t acc[TG][2];
 #pragma unroll
     for (int tg = 0; tg < TG; ++tg) { acc[tg][0] = float4_t{0.f, 0.f, 0.f, 0.f}; acc[tg][1] = float4_t{0.f, 0.f, 0.f, 0.f}; }
@@ -732,11 +732,133 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
     }
 }
 
-int launch_pf_pre(const void* x, const int32_t* pt, const int32_t* pe, int np, const int64_t* table, void* xg, void* xu, float* zg, int E, int H, int I,
+template <int TG, bool MASKED>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) nq_pf_gemm_k(PfGemm a)
+{
+    extern __shared__ __align__(16) char smem[];
+    const int32_t* tile = a.tiles + 4 * blockIdx.y;
+    const int e = tile[0], row0 = tile[1], nrows = tile[2], slot = tile[3] - 1;
+    if (e < 0 || e >= a.E || nrows <= 0) return;
+    pf_tile<TG, MASKED>(a, e, row0, nrows, slot, smem);
+}
+
+// Tiles of up to 64 rows of any height in one launch (the plan of nq_pf_sort_k). Steps of a few hundred tokens over many experts
+// have nothing taller, so a projection is one launch on the caller's stream instead of five on four; with at most 64 rows a tile
+// costs what decoding its expert costs, and the registers of the 64-row body (126) still let four wavefronts share a SIMD.
+template <bool MASKED>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MASKED ? 2 : 4))) nq_pf_short_k(PfGemm a)
+{
+    extern __shared__ __align__(16) char smem[];
+    const int32_t* tile = a.tiles + 4 * blockIdx.y;
+    const int e = tile[0], row0 = tile[1], nrows = tile[2];
+    if (e < 0 || e >= a.E || nrows <= 0) return;
+    if (nrows <= 16) pf_tile<1, MASKED>(a, e, row0, nrows, -1, smem);
+    else if (nrows <= 32) pf_tile<2, MASKED>(a, e, row0, nrows, -1, smem);
+    else pf_tile<4, MASKED>(a, e, row0, nrows, -1, smem);
+}
+
+// ---- pairs sorted by expert ----------------------------------------------------------------------------------------------
+// One launch in place of a library sort, its gathers and the counting scatter (a dozen launches, 150 us of them at 32768 pairs).
+// Every workgroup counts all picks in LDS, so that it knows where each expert's rows start without waiting for another one; its
+// eight wavefronts then gather the pairs of one expert each, in pair order, from the picks kept in LDS as 16-bit ids. Picks outside
+// [0, E) form a last group of rows of no expert (pe = -1), which every later kernel passes over. Workgroup 0 also writes the
+// tile list of nq_pf_short_k: at most 64 rows per tile, experts above level 2 first (their tiles take twice as long, so they
+// start first), unused entries -1.
+constexpr int SORT_TILE = 16384, SHORT_ROWS = 64;
+struct PfSort
+{
+    const void* sel; const void* rw; int sdt, wdt; int P, topk, E;
+    const int64_t* table; int32_t* cnt; int32_t* pe; int32_t* pt; int32_t* pos; int* hits; int32_t* tiles; int cap;
+};
+__global__ void __launch_bounds__(512) nq_pf_sort_k(PfSort a)
+{
+    extern __shared__ __align__(16) uint16_t ids[];              // [SORT_TILE], then hist | start | tmp, E + 1 each
+    int* hist = (int*)(ids + SORT_TILE); int* incl = hist + a.E + 1; int* tmp = incl + a.E + 1;
+    const int tid = threadIdx.x, lane = tid & 63, E1 = a.E + 1;
+    const bool one = a.P <= SORT_TILE;
+    auto load = [&](int t0, bool count) {
+        for (int i = tid; i < SORT_TILE; i += 512)
+        {
+            if (one && i >= ((a.P + 511) & ~511)) break;
+            int id = 0xFFFF;                                     // past the end: nobody's
+            if (t0 + i < a.P)
+            {
+                const long long e = id_at(a.sel, a.sdt, t0 + i);
+                id = e >= 0 && e < a.E ? (int)e : a.E;
+                if (count) atomicAdd(hist + id, 1);
+            }
+            ids[i] = (uint16_t)id;
+        }
+    };
+    for (int e = tid; e < E1; e += 512) hist[e] = 0;
+    __syncthreads();
+    for (int t0 = 0; t0 < a.P; t0 += SORT_TILE) { if (t0) __syncthreads(); load(t0, true); }
+    __syncthreads();
+    for (int e = tid; e < E1; e += 512) incl[e] = hist[e];
+    __syncthreads();
+    block_scan(incl, tmp, E1);
+    const int e = blockIdx.x * 8 + (tid >> 6);
+    int row = e < E1 ? incl[e] - hist[e] : 0, nz = 0;            // next row of this wavefront's expert
+    const int mine = e < E1 ? e : -1;
+    if (mine >= 0 && mine < a.E && lane == 0) a.cnt[mine] = hist[mine];
+    for (int t0 = 0; t0 < a.P; t0 += SORT_TILE)
+    {
+        if (!one) { __syncthreads(); load(t0, false); __syncthreads(); }
+        const int n = a.P - t0 < SORT_TILE ? a.P - t0 : SORT_TILE;
+        for (int i = 0; i < n; i += 512)
+        {
+            const uint4 v = *(const uint4*)(ids + i + 8 * lane);
+            const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int j = 0; j < 8; ++j)                          // rows of an expert: by blocks of 512 pairs, then by j, then by lane
+            {
+                const bool eq = (int)((w[j >> 1] >> (16 * (j & 1))) & 0xFFFFu) == mine;
+                const unsigned long long m = __ballot(eq);
+                if (!m) continue;
+                if (eq)
+                {
+                    const int pair = t0 + i + 8 * lane + j, r = row + __popcll(m & ((1ull << lane) - 1ull));
+                    a.pos[pair] = r; a.pt[r] = pair / a.topk; a.pe[r] = mine < a.E ? mine : -1;
+                }
+                if (a.hits) nz += __popcll(__ballot(eq && w_at(a.rw, a.wdt, t0 + i + 8 * lane + j) != 0.f));
+                row += __popcll(m);
+            }
+        }
+    }
+    if (a.hits && nz && mine >= 0 && mine < a.E && lane == 0) __hip_atomic_fetch_add(a.hits + mine, nz, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (blockIdx.x != 0 || !a.tiles) return;
+    __syncthreads();
+    // start rows into incl, then per class (0: above level 2, 1: level 2) a scan of the tile counts
+    int4* T4 = (int4*)a.tiles;
+    int base = 0;
+    for (int x = tid; x < a.E; x += 512) incl[x] -= hist[x];
+    int* nt = (int*)ids;                                         // E <= 4096 ints fit the id buffer
+    for (int cls = 0; cls < 2; ++cls)
+    {
+        __syncthreads();
+        for (int x = tid; x < a.E; x += 512)
+        {
+            const int lv = (int)a.table[(size_t)x * TBL_W];
+            nt[x] = lv > 0 && (lv > 2) == (cls == 0) ? (hist[x] + SHORT_ROWS - 1) / SHORT_ROWS : 0;
+        }
+        __syncthreads();
+        block_scan(nt, tmp, a.E);
+        for (int x = tid; x < a.E; x += 512)
+        {
+            const int k = nt[x] - (x ? nt[x - 1] : 0), at = base + nt[x] - k;
+            for (int q = 0; q < k; ++q)
+                T4[at + q] = make_int4(x, incl[x] + SHORT_ROWS * q, hist[x] - SHORT_ROWS * q < SHORT_ROWS ? hist[x] - SHORT_ROWS * q : SHORT_ROWS, 0);
+        }
+        base += nt[a.E - 1];
+    }
+    for (int i = base + tid; i < a.cap; i += 512) T4[i] = make_int4(-1, 0, 0, 0);
+}
+
+int launch_pf_pre(const void* x, int xdt, const int32_t* pt, const int32_t* pe, int np, const int64_t* table, void* xg, void* xu, float* zg, int E, int H, int I,
                   const int32_t* tiles, int cap, int heights, hipStream_t st)
 {
     if (!np) return 0;
-    nq_pf_pre_k<<<np, 256, 0, st>>>((const _Float16*)x, pt, pe, table, (_Float16*)xg, (_Float16*)xu, zg, E, H, I, tiles, cap, heights);
+    nq_pf_pre_k<<<np, 256, 0, st>>>(x, xdt, pt, pe, table, (_Float16*)xg, (_Float16*)xu, zg, E, H, I, tiles, cap, heights);
     NQ_LAUNCH_CHECK("nq_pf_pre");
     return 0;
 }
@@ -748,11 +870,11 @@ int launch_pf_mid(const float* acc_gu, const int32_t* pe, int np, const int64_t*
     NQ_LAUNCH_CHECK("nq_pf_mid");
     return 0;
 }
-int launch_pf_post(const float* y, const int32_t* pos, const int64_t* sel, const void* rw, int T, int topk, int row_lo, int nrows,
-                   const int64_t* table, float* out, const float* zd, int E, int H, int I, hipStream_t st)
+int launch_pf_post(const float* y, const int32_t* pos, const void* sel, int sdt, const void* rw, int wdt, int T, int topk, int row_lo, int nrows,
+                   const int64_t* table, void* out, int odt, int add, const float* zd, int E, int H, int I, hipStream_t st)
 {
-    if (!T || !nrows) return 0;
-    nq_pf_post_k<<<T, 256, 0, st>>>(y, pos, sel, (const _Float16*)rw, topk, row_lo, nrows, table, out, zd, E, H, I);
+    if (!T || (!nrows && add)) return 0;
+    nq_pf_post_k<<<T, 256, 0, st>>>(y, pos, sel, sdt, rw, wdt, topk, row_lo, nrows, table, out, odt, add, zd, E, H, I);
     NQ_LAUNCH_CHECK("nq_pf_post");
     return 0;
 }
@@ -794,5 +916,104 @@ int launch_pf_gemm(const int64_t* table, const int32_t* tiles, int ntiles, int b
     }
     return set_error("nq_pf_gemm: tile height %d not in {16, 32, 64, 128, 256}", bm);
 }
+
+// ---- a whole step --------------------------------------------------------------------------------------------------------
+// Bytes of the int32 scratch of a step: cnt [E] | pe [P] | pt [P] | pos [P] | hot [E] | tile lists, each on 16 bytes.
+struct PfMeta { int32_t *cnt, *pe, *pt, *pos, *hot, *tiles; int cap, scap; size_t bytes; };
+static PfMeta pf_meta(void* ws, int P, int R, int E)
+{
+    PfMeta m;
+    size_t off = 0;
+    auto take = [&](size_t n) { int32_t* p = (int32_t*)((char*)ws + off); off += (n * 4 + 15) & ~(size_t)15; return p; };
+    m.cap = E + R / 256 + 1; m.scap = E + P / SHORT_ROWS + 1;
+    m.cnt = take(E); m.pe = take(P); m.pt = take(P); m.pos = take(P); m.hot = take(E);
+    m.tiles = take(4 * (size_t)(5 * m.cap > m.scap ? 5 * m.cap : m.scap));
+    m.bytes = off;
+    return m;
+}
+
+// Steps whose experts hold few rows each take the one-launch plan of short tiles. The line: at 32 pair rows per expert on average
+// hardly an expert of an even routing exceeds one 64-row tile, and what a skewed routing's few popular ones decode twice costs
+// less than the side streams' extra launches and the taller bodies' lower occupancy; above it the tall tiles save decodes.
+static bool pf_is_short(int64_t P, int E) { return P <= 32 * (int64_t)E; }
+
+template <bool MASKED>
+static int launch_short(const PfGemm& a, int ntiles, int N, hipStream_t st)
+{
+    nq_pf_short_k<MASKED><<<dim3(N / 128, ntiles), 256, SHORT_ROWS * PF_ROW, st>>>(a);
+    NQ_LAUNCH_CHECK("nq_pf_short");
+    return 0;
+}
+
+int launch_pf_step(const NqPfArgs& a, hipStream_t st)
+{
+    const int P = a.T * a.topk, R = a.rows < P ? a.rows : P, E = a.E, H = a.H, I = a.I;
+    const PfMeta m = pf_meta(a.meta, P, R, E);
+    if (m.bytes > (size_t)a.meta_bytes) return set_error("nq_pf_step: meta needs %zu bytes, has %lld", m.bytes, (long long)a.meta_bytes);
+    const bool brief = R == P && !a.wop && pf_is_short(P, E);
+    {
+        const PfSort s{a.sel, a.rw, a.sel_dtype, a.rw_dtype, P, a.topk, E, a.table, m.cnt, m.pe, m.pt, m.pos, a.hits, brief ? m.tiles : nullptr, m.scap};
+        const int shm = SORT_TILE * 2 + 3 * (E + 1) * 4;
+        const hipError_t e = hipFuncSetAttribute((const void*)nq_pf_sort_k, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
+        if (e != hipSuccess) return set_error("nq_pf_sort: LDS %d bytes: %s", shm, hipGetErrorString(e));
+        nq_pf_sort_k<<<(E + 8) / 8, 512, shm, st>>>(s);
+        NQ_LAUNCH_CHECK("nq_pf_sort");
+    }
+    float *acc = (float*)a.acc, *y = (float*)a.y;
+    if (brief)
+    {
+        if (int rc = launch_pf_pre(a.x, a.x_dtype, m.pt, m.pe, P, a.table, a.xg, a.xu, a.zg, E, H, I, nullptr, 0, 0, st)) return rc;
+        for (int mode = 0; mode < 2; ++mode)
+        {
+            const PfGemm g{a.table, m.tiles, (const _Float16*)(mode ? a.h : a.xg), (const _Float16*)(mode ? nullptr : a.xu), mode ? y : acc, mode, E, H, I, a.variants == 1, nullptr};
+            const int N = mode ? H : 2 * I;
+            if (a.variants & 1) if (int rc = launch_short<false>(g, m.scap, N, st)) return rc;
+            if (a.variants & 2) if (int rc = launch_short<true>(g, m.scap, N, st)) return rc;
+            if (mode == 0) if (int rc = launch_pf_mid(acc, m.pe, P, a.table, a.h, a.zg, a.zd, E, H, I, nullptr, 0, 0, st)) return rc;
+        }
+        return launch_pf_post(y, m.pos, a.sel, a.sel_dtype, a.rw, a.rw_dtype, a.T, a.topk, 0, P, a.table, a.out, a.out_dtype, 0, a.zd, E, H, I, st);
+    }
+    // Tile heights 256 | 128 | 64, 32, 16 as four chains: the tallest on the caller's stream, the others on side streams between two
+    // events. A GEMM launch ends with the GPU partly idle while its last workgroups drain; the chains fill each other's tails, and
+    // the memory-bound kernels of one height run under the GEMMs of another.
+    hipStream_t streams[4] = {st, (hipStream_t)a.side[0], (hipStream_t)a.side[1], (hipStream_t)a.side[2]};
+    static const int stream_of[5] = {3, 3, 2, 1, 0};             // by height 16 << k
+    auto hip_ok = [](hipError_t e) { return e == hipSuccess ? 0 : set_error("nq_pf_step: %s", hipGetErrorString(e)); };
+    for (int c = 0; c < P; c += R)
+    {
+        const int n = P - c < R ? P - c : R;
+        const bool wop = a.wop && n >= a.hot_min;
+        if (int rc = launch_pf_plan(m.cnt, E, c, n, m.tiles, m.cap, wop ? m.hot : nullptr, a.hot_min, a.wop_slots, st)) return rc;
+        for (int mode = 0; wop && mode < 2; ++mode)
+            if (int rc = launch_pf_wdecode(a.table, m.hot, E, mode, a.wop, H, I, st)) return rc;
+        if (int rc = hip_ok(hipEventRecord((hipEvent_t)a.events[0], st))) return rc;
+        for (int i = 1; i < 4; ++i) if (int rc = hip_ok(hipStreamWaitEvent(streams[i], (hipEvent_t)a.events[0], 0))) return rc;
+        const int32_t *pts = m.pt + c, *pes = m.pe + c;
+        static const int heights[4] = {16, 8, 4, 3};             // bit k = height 16 << k
+        auto gemms = [&](int mode) {
+            for (int k = 4; k >= 0; --k)
+                for (int v = 0; v < 2; ++v)
+                    if (a.variants >> v & 1)
+                        if (int rc = launch_pf_gemm(a.table, m.tiles + (size_t)k * m.cap * 4, k < 4 ? E : m.cap, 16 << k, mode | 2 * v | (a.variants == 1 ? 4 : 0), mode ? a.h : a.xg,
+                                                    mode ? nullptr : a.xu, mode ? y : acc, E, H, I, wop ? a.wop : nullptr, streams[stream_of[k]])) return rc;
+            return 0;
+        };
+        for (int i = 0; i < 4; ++i)
+            if (int rc = launch_pf_pre(a.x, a.x_dtype, pts, pes, n, a.table, a.xg, a.xu, a.zg, E, H, I, m.tiles, m.cap, heights[i], streams[i])) return rc;
+        if (int rc = gemms(0)) return rc;
+        for (int i = 0; i < 4; ++i)
+            if (int rc = launch_pf_mid(acc, pes, n, a.table, a.h, a.zg, a.zd, E, H, I, m.tiles, m.cap, heights[i], streams[i])) return rc;
+        if (int rc = gemms(1)) return rc;
+        for (int i = 1; i < 4; ++i)
+        {
+            if (int rc = hip_ok(hipEventRecord((hipEvent_t)a.events[i], streams[i]))) return rc;
+            if (int rc = hip_ok(hipStreamWaitEvent(st, (hipEvent_t)a.events[i], 0))) return rc;
+        }
+        if (int rc = launch_pf_post(y, m.pos, a.sel, a.sel_dtype, a.rw, a.rw_dtype, a.T, a.topk, c, n, a.table, a.out, a.out_dtype, c != 0, a.zd, E, H, I, st)) return rc;
+    }
+    return 0;
+}
+
+int64_t pf_meta_bytes(int P, int R, int E) { return (int64_t)pf_meta(nullptr, P, R, E).bytes; }
 
 }  // namespace nq

@@ -12,6 +12,65 @@
 
 namespace nq {
 
+// ---- caller dtypes: the casts a caller would otherwise launch as separate kernels (x.half(), ids.long(), w.half(),
+// out.to(x.dtype); reference sm120/serve/nq_vllm.py:522,560,573) happen at the loads and the final store, with the same
+// roundings: activations and routing weights pass through fp16, the fp32 result is rounded once to the output type.
+constexpr int DT_BF16 = 1, DT_F32 = 2, DT_I32 = 1, DT_OUT_F16 = 1, DT_OUT_BF16 = 2;   // 0 = the default type of each argument (fp16, int64, fp32 out)
+__device__ __forceinline__ float bf16_to_f(uint16_t v) { return __builtin_bit_cast(float, (uint32_t)v << 16); }
+__device__ __forceinline__ uint16_t f_to_bf16(float f)           // round to nearest even; NaN stays NaN
+{
+    uint32_t u = __builtin_bit_cast(uint32_t, f);
+    if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40u);
+    u += 0x7fffu + ((u >> 16) & 1u);
+    return (uint16_t)(u >> 16);
+}
+__device__ __forceinline__ long long id_at(const void* sel, int dt, size_t i)
+{
+    return dt == DT_I32 ? (long long)((const int32_t*)sel)[i] : (long long)((const int64_t*)sel)[i];
+}
+__device__ __forceinline__ float w_at(const void* rw, int dt, size_t i)   // the weight as fp16 would hold it
+{
+    if (dt == DT_BF16) return (float)(_Float16)bf16_to_f(((const uint16_t*)rw)[i]);
+    if (dt == DT_F32) return (float)(_Float16)((const float*)rw)[i];
+    return (float)((const _Float16*)rw)[i];
+}
+__device__ __forceinline__ half2_t act2_at(const void* x, int dt, size_t i)   // x[i], x[i + 1] (i even) as fp16
+{
+    if (dt == DT_BF16)
+    {
+        const uint32_t v = *(const uint32_t*)((const uint16_t*)x + i);
+        return half2_t{(_Float16)bf16_to_f((uint16_t)v), (_Float16)bf16_to_f((uint16_t)(v >> 16))};
+    }
+    if (dt == DT_F32) { const float2 v = *(const float2*)((const float*)x + i); return half2_t{(_Float16)v.x, (_Float16)v.y}; }
+    return *(const half2_t*)((const _Float16*)x + i);
+}
+__device__ __forceinline__ uint4 act8_at(const void* x, int dt, size_t i)     // x[i .. i + 7] (i a multiple of 8) as fp16
+{
+    if (dt == 0) return *(const uint4*)((const _Float16*)x + i);
+    half8_t h;
+    if (dt == DT_BF16)
+    {
+        const uint4 v = *(const uint4*)((const uint16_t*)x + i);
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int q = 0; q < 4; ++q) { h[2 * q] = (_Float16)bf16_to_f((uint16_t)w[q]); h[2 * q + 1] = (_Float16)bf16_to_f((uint16_t)(w[q] >> 16)); }
+    }
+    else
+    {
+        const float4 a = *(const float4*)((const float*)x + i), b = *(const float4*)((const float*)x + i + 4);
+        const float f[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+        for (int q = 0; q < 8; ++q) h[q] = (_Float16)f[q];
+    }
+    return __builtin_bit_cast(uint4, h);
+}
+__device__ __forceinline__ void res2_store(void* out, int dt, size_t i, float v0, float v1)   // out[i], out[i + 1] (i even)
+{
+    if (dt == DT_OUT_F16) { half2_t h; h.x = (_Float16)v0; h.y = (_Float16)v1; *(half2_t*)((_Float16*)out + i) = h; }
+    else if (dt == DT_OUT_BF16) *(uint32_t*)((uint16_t*)out + i) = (uint32_t)f_to_bf16(v0) | ((uint32_t)f_to_bf16(v1) << 16);
+    else *(float2*)((float*)out + i) = make_float2(v0, v1);
+}
+
 // ---- Hadamard-128 on one wavefront: lane holds elements 2 lane, 2 lane + 1 --------------------------------------------
 // One in-lane butterfly, then six cross-lane stages: lanes l and l ^ m exchange, the lane with bit m clear keeps a + a',
 // the other a' - a (a' = the partner's value), all in fp32 in this order. The exchanges use no LDS: DPP lane selects for
@@ -96,14 +155,14 @@ __device__ __forceinline__ void progress_priority(int c, int NC)
 
 struct LaneCtx
 {
-    size_t rec0;          // record index of this lane in chunk 0 of its k-slice: (unit0) * 32 + 4 g + t4
-    size_t unit0;         // unit index (strip * C + chunk0)
+    uint32_t rec0;        // record index of this lane in chunk 0 of its k-slice: (unit0) * 32 + 4 g + t4
+    uint32_t unit0;       // unit index (strip * C + chunk0)
     size_t nrec;          // records of the whole projection (sub-array stride)
     int src;              // lane holding the next record of the ring
     int g;                // ring index (sign-variant bit)
     const char* xs;       // this lane's B-operand base in LDS (bytes), kg folded in
     int xstep;            // bytes per chunk (0 for lanes without a token)
-    size_t strip, nstrips; int chunk0;   // mask mode: this lane's strip, strips of the projection, first chunk of the k-slice
+    uint32_t strip; size_t nstrips; int chunk0;   // mask mode: this lane's strip, strips of the projection, first chunk of the k-slice
 };
 
 // mask mode: chunk by chunk either the folded decode (refined chunks, residual records compact over them) or the level-2
@@ -113,7 +172,7 @@ __device__ __forceinline__ void gemv_chunks_masked(const Planes& P, const LaneCt
 {
     constexpr int NW = Rec<CODE>::NW;
     const uint64_t f = P.flags[L.strip];
-    uint32_t nvar = P.var ? (uint32_t)P.var[L.unit0] : 0u;
+    uint32_t nvar = P.var ? at_offset<uint8_t>(P.var, L.unit0) : 0u;
     for (int c = 0; c < NC; ++c)
     {
         progress_priority(c, NC);
@@ -126,8 +185,8 @@ __device__ __forceinline__ void gemv_chunks_masked(const Planes& P, const LaneCt
         if (on) { load_record<CODE>(wr, P.res, m.unit * 32 + (L.rec0 & 31), m.nrec); dw = P.dw[m.unit]; }
         if (c + 1 < NC)
         {
-            nb = load_base<BK>(P, L.rec0 + (size_t)(c + 1) * 32, L.nrec);
-            if (P.var) nvar = P.var[L.unit0 + c + 1];
+            nb = load_base<BK>(P, L.rec0 + (uint32_t)(c + 1) * 32, L.nrec);
+            if (P.var) nvar = at_offset<uint8_t>(P.var, L.unit0 + c + 1);
         }
         ext_base<BK>(wb, __shfl(wb[0], L.src));
         const uint32_t sgm = ((var >> L.g) & 1u) * 0x80008000u;
@@ -180,8 +239,8 @@ __device__ __forceinline__ void gemv_chunks(const Planes& P, const LaneCtx& L, i
         if (P.flags) { gemv_chunks_masked<CODE, BK>(P, L, NC, acc, nb); return; }     // block-uniform
     constexpr int NW = RES ? Rec<CODE>::NW : 1;
     uint32_t nr[NW + 2] = {0}, ndw = 0, nvar = 0;
-    if constexpr (RES) { load_record<CODE>(nr, P.res, L.rec0, L.nrec); ndw = P.dw[L.unit0]; }
-    if (P.var) nvar = P.var[L.unit0];
+    if constexpr (RES) { load_record<CODE>(nr, P.res, L.rec0, L.nrec); ndw = at_offset<uint32_t>((gp_u8)P.dw, L.unit0 * 4u); }
+    if (P.var) nvar = at_offset<uint8_t>(P.var, L.unit0);
     for (int c = 0; c < NC; ++c)
     {
         progress_priority(c, NC);
@@ -192,9 +251,9 @@ __device__ __forceinline__ void gemv_chunks(const Planes& P, const LaneCtx& L, i
         const uint32_t dw = ndw, var = nvar;
         if (c + 1 < NC)                                         // prefetch the next chunk's records
         {
-            nb = load_base<BK>(P, L.rec0 + (size_t)(c + 1) * 32, L.nrec);
-            if constexpr (RES) { load_record<CODE>(nr, P.res, L.rec0 + (size_t)(c + 1) * 32, L.nrec); ndw = P.dw[L.unit0 + c + 1]; }
-            if (P.var) nvar = P.var[L.unit0 + c + 1];
+            nb = load_base<BK>(P, L.rec0 + (uint32_t)(c + 1) * 32, L.nrec);
+            if constexpr (RES) { load_record<CODE>(nr, P.res, L.rec0 + (uint32_t)(c + 1) * 32, L.nrec); ndw = at_offset<uint32_t>((gp_u8)P.dw, (L.unit0 + c + 1) * 4u); }
+            if (P.var) nvar = at_offset<uint8_t>(P.var, L.unit0 + c + 1);
         }
         ext_base<BK>(wb, __shfl(wb[0], L.src));
         const uint32_t sgm = ((var >> L.g) & 1u) * 0x80008000u;

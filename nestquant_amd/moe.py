@@ -5,6 +5,7 @@ Host-side mirror of the reference's Python op surface (sm120/moe.py): `entry` :2
 libnq_moe_hip.so, reached through ctypes with raw device pointers; there is no CPU path in this module.
 """
 import ctypes as C
+import os
 
 import torch
 
@@ -288,20 +289,25 @@ def pf_bytes(H, I, R, G=0):
 
 
 def pf_scratch(dev, H, I, R, G=0):
-    """Prefill scratch shared by every layer on `dev`, allocated on first use: xg | xu fp16 [R, H], acc_gu fp32 [R, 2I],
-    h fp16 [R, I], y fp32 [R, H], and wop: decoded weights of up to PF_HOT_SLOTS hot experts. Unlike the reference
-    (sm120/moe.py:263-274), which decodes every expert of a group into dense scratch, only experts with more than one tile go
-    through scratch; the others are decoded in registers inside the grouped GEMM."""
-    k = (str(dev), H, I, R, PF_HOT_SLOTS)
-    if k not in _PF:
+    """Prefill scratch shared by every layer of this shape on `dev`, for at least R pair rows: xg | xu fp16 [R, H], acc_gu fp32
+    [R, 2I], h fp16 [R, I], y fp32 [R, H], and wop: decoded weights of up to PF_HOT_SLOTS hot experts. One set per device and shape,
+    replaced by a larger one (rows rounded up to a power of two) when a call brings more rows than any before. Unlike the
+    reference (sm120/moe.py:263-274), which decodes every expert of a group into dense scratch, only experts with more than one
+    tile go through scratch; the others are decoded in registers inside the grouped GEMM."""
+    k = (str(dev), H, I)
+    slots = max(0, min(PF_HOT_SLOTS, R // PF_HOT_MIN))
+    S = _PF.get(k)
+    if S is None or S["rows"] < R:
+        n = 1 << (max(R, 64) - 1).bit_length()
         f16, f32 = torch.float16, torch.float32
-        slots = max(0, min(PF_HOT_SLOTS, R // PF_HOT_MIN))
-        _PF[k] = dict(wop=torch.empty(slots, 3 * H * I, dtype=f16, device=dev) if slots else None,
-                      xg=torch.empty(R, H, dtype=f16, device=dev), xu=torch.empty(R, H, dtype=f16, device=dev),
-                      acc=torch.empty(R, 2 * I, dtype=f32, device=dev), h=torch.empty(R, I, dtype=f16, device=dev),
-                      y=torch.empty(R, H, dtype=f32, device=dev),
-                      zg=torch.zeros(R, 4, dtype=f32, device=dev), zd=torch.zeros(R, 4, dtype=f32, device=dev))
-    return _PF[k]
+        _PF.pop(k, None); S = None                   # the old set goes back to the allocator before the new one is taken
+        S = _PF[k] = dict(rows=n, wop=None, xg=torch.empty(n, H, dtype=f16, device=dev), xu=torch.empty(n, H, dtype=f16, device=dev),
+                          acc=torch.empty(n, 2 * I, dtype=f32, device=dev), h=torch.empty(n, I, dtype=f16, device=dev),
+                          y=torch.empty(n, H, dtype=f32, device=dev), zg=torch.zeros(n, 4, dtype=f32, device=dev),
+                          zd=torch.zeros(n, 4, dtype=f32, device=dev))
+    if slots != (0 if S["wop"] is None else S["wop"].shape[0]):
+        S["wop"] = torch.empty(slots, 3 * H * I, dtype=torch.float16, device=dev) if slots else None
+    return S
 
 
 def pf_tiles(segs):
@@ -318,100 +324,66 @@ def pf_tiles(segs):
 
 
 _PF_SIDE = {}
-_PF_STREAM_OF = {256: 0, 128: 1, 64: 2, 32: 3, 16: 3}          # stream 0 = the caller's
 
 
-def _pf_chains(Lb, tb, lists, variants, S, x, pts, pes, n, tiles, cap, E, H, I, wop=None):
-    """Everything between the tile plan and the post kernel of one row chunk: rotation of the activations, gate|up GEMM, SwiGLU
-    kernel and down GEMM of every tile height. The heights work on disjoint pair rows, so each is a chain of its own. A GEMM
-    launch ends with the GPU partly idle while its last workgroups drain (a workgroup runs the whole K loop, ~75 us, so a
-    launch of a few dozen tiles is a handful of such rounds); the tallest height stays on the caller's stream and the others
-    go to side streams (default priority) between two events, so that the chains overlap, fill each other's tails and the
-    memory-bound kernels of one height run under the GEMMs of another."""
-    main = torch.cuda.current_stream()
-    side = _PF_SIDE.setdefault(str(tb.device), [])
-    while len(side) < 3:
-        side.append(torch.cuda.Stream(device=tb.device))
-    streams = [main] + side
-    ready = torch.cuda.Event(); ready.record(main)
-    for st in side:
-        st.wait_event(ready)
-    xg, xu, acc, h, y, zg, zd = (S[k].data_ptr() for k in ("xg", "xu", "acc", "h", "y", "zg", "zd"))
+def _pf_side(dev):
+    """three side streams (default priority) and four events of `dev`, created once"""
+    k = str(dev)
+    if k not in _PF_SIDE:
+        with torch.cuda.device(dev):
+            side, ev = [torch.cuda.Stream(device=dev) for _ in range(3)], [torch.cuda.Event() for _ in range(4)]
+            for e in ev:
+                e.record()                           # a torch event exists from its first record on
+        _PF_SIDE[k] = (side, ev, (C.c_void_p * 3)(*[st.cuda_stream for st in side]), (C.c_void_p * 4)(*[e.cuda_event for e in ev]))
+    return _PF_SIDE[k]
 
-    def gemms(mode, A0, A1, Cm):
-        for bm, t, nt in lists:
-            stp = C.c_void_p(streams[_PF_STREAM_OF[bm]].cuda_stream)
-            for v in variants:
-                _lib.check(Lb.nq_pf_gemm(tb.data_ptr(), t.data_ptr(), nt, bm, mode | v, A0, A1, Cm, E, H, I, wop, stp))
 
-    masks = [sum(bm // 16 for bm, _, _ in lists if _PF_STREAM_OF[bm] == i) for i in range(len(streams))]    # bit k = height 16 << k
-    for st, heights in zip(streams, masks):
-        _lib.check(Lb.nq_pf_pre_rows(x.data_ptr(), pts.data_ptr(), pes.data_ptr(), n, tb.data_ptr(), xg, xu, zg, E, H, I,
-                                     tiles.data_ptr(), cap, heights, C.c_void_p(st.cuda_stream)))
-    gemms(0, xg, xu, acc)
-    for st, heights in zip(streams, masks):
-        _lib.check(Lb.nq_pf_mid_rows(acc, pes.data_ptr(), n, tb.data_ptr(), h, zg, zd, E, H, I, tiles.data_ptr(), cap, heights,
-                                     C.c_void_p(st.cuda_stream)))
-    gemms(1, h, None, y)
-    for st in side:
-        done = torch.cuda.Event(); done.record(st); main.wait_event(done)
+def _pf_step(s, x, sel, rw, out, R=None, table=None):
+    """one nq_pf_step call: x [T, H], sel and rw [T, k], out [T, H] in any of the types the decode kernels take and write"""
+    T, k = sel.shape
+    H, I, E, dev, Lb = s.H, s.I, s.E, x.device, s.M
+    tb = s.table if table is None else table
+    P = T * k
+    if P == 0:
+        return out.zero_()
+    R = min(P, R or int(os.environ.get("NQ_PF_ROWS", "32768")))
+    S = pf_scratch(dev, H, I, R)
+    nb = Lb.nq_pf_meta_bytes(T, k, R, E)
+    if nb < 0:
+        raise RuntimeError(Lb.nq_last_error().decode())
+    meta = torch.empty(nb, dtype=torch.uint8, device=dev)
+    _, _, side, events = _pf_side(dev)
+    whole = out if out.dtype == torch.float32 or R == P else torch.empty(T, H, dtype=torch.float32, device=dev)   # chunks add up in fp32
+    # decoded-weight scratch: rows of the common kind only (the variant kernel of the others decodes in the GEMM)
+    wop = S["wop"] if (S["wop"] is not None and P >= PF_HOT_MIN and not s.rare_rows and table is None) else None
+    a = _lib.NqPfArgs()
+    a.x, a.sel, a.rw, a.table, a.out, a.hits = x.data_ptr(), sel.data_ptr(), rw.data_ptr(), tb.data_ptr(), whole.data_ptr(), s.hits_ptr or None
+    a.meta, a.meta_bytes = meta.data_ptr(), nb
+    a.xg, a.xu, a.acc, a.h, a.y, a.zg, a.zd = (S[n].data_ptr() for n in ("xg", "xu", "acc", "h", "y", "zg", "zd"))
+    if wop is not None:
+        a.wop, a.wop_bytes, a.wop_slots, a.hot_min = wop.data_ptr(), wop.numel() * 2, wop.shape[0], PF_HOT_MIN
+    a.side, a.events = side, events
+    a.T, a.topk, a.E, a.H, a.I, a.rows = T, k, E, H, I, R
+    a.x_dtype, a.sel_dtype, a.rw_dtype, a.out_dtype = _DT_IN[x.dtype], _DT_SEL[sel.dtype], _DT_IN[rw.dtype], _DT_OUT[whole.dtype]
+    # mask mode / other base codes run in their own kernel variant; a caller's own table may hold such rows, so it gets both, and
+    # a lone variant is told so: should it meet a row of the other kind after all, the result is NaN, not stale scratch
+    a.variants = 3 if (s.rare_rows or table is not None) else 1
+    _lib.check(Lb.nq_pf_step(C.byref(a), _lib.stream_ptr()))
+    return out if whole is out else out.copy_(whole)
 
 
 def prefill(s, x, sel, rw, out=None, R=None, G=None, table=None):
     """T > Bmax tokens (reference sm120/moe.py:282-326): pairs sorted by expert, each routed expert decoded inside the
     grouped GEMMs at the level of its live table row, same math as the decode path (fp32 accumulation order differs).
-    No host synchronisation (the reference's prefill reads the expert counts back; here the tile lists are built on the
-    device by nq_pf_plan). Exports routing hits like the decode kernel. Calls on one device share the scratch of pf_scratch()
-    (as the reference's do, sm120/moe.py:262-274) and the side streams of _pf_chains, so they must be ordered on one stream."""
+    No host synchronisation (the reference's prefill reads the expert counts back; here the sort and the tile lists are
+    built on the device). Exports routing hits like the decode kernel. Calls on one device share the scratch of pf_scratch()
+    (as the reference's do, sm120/moe.py:262-274) and its side streams, so they must be ordered on one stream."""
     if s.G != 4:
         raise NotImplementedError("prefill decodes rings of G = 4 lanes only (as the reference's pf_decode)")
     assert x.dtype == torch.float16 and rw.dtype == torch.float16 and sel.dtype == torch.int64, (x.dtype, rw.dtype, sel.dtype)
     assert x.is_contiguous()
-    T, k = sel.shape
-    H, I, E, dev, Lb = s.H, s.I, s.E, x.device, s.M
-    tb = s.table if table is None else table
-    st = _lib.stream_ptr()
-    out = torch.zeros(T, H, dtype=torch.float32, device=dev) if out is None else out.zero_()
-    flat = sel.reshape(-1); rwf = rw.reshape(-1)
-    order = torch.argsort(flat, stable=True)
-    pe = flat[order].int(); pt = (order // k).int()
-    pos = torch.empty_like(order, dtype=torch.int32)
-    pos[order] = torch.arange(order.numel(), dtype=torch.int32, device=dev)       # row of pair (t, k) in sorted order
-    selc, rwc = sel.contiguous(), rw.contiguous()
-    one = torch.ones_like(flat, dtype=torch.int32)
-    cnt = torch.zeros(E, dtype=torch.int32, device=dev).scatter_add_(0, flat, one)
-    if s.hits_ptr:
-        hc = torch.zeros(E + 1, dtype=torch.int32, device=dev).scatter_add_(0, torch.where(rwf != 0, flat, E), one)[:E].contiguous()
-        _lib.check(Lb.nq_pf_hits(hc.data_ptr(), s.hits_ptr, E, st))
-    P = T * k
-    if P == 0:
-        return out
-    R = min(P, R or int(__import__("os").environ.get("NQ_PF_ROWS", "32768")))
-    S = pf_scratch(dev, H, I, R)
-    cap = E + R // 256 + 1
-    # mask mode / other base codes run in their own kernel variant; a caller's own table may hold such rows, so it gets both,
-    # and a lone variant is told so (| 4): should it meet a row of the other kind after all, the result is NaN, not stale scratch
-    variants = (0, 2) if (s.rare_rows or table is not None) else (4,)
-    for c in range(0, P, R):
-        d = min(P, c + R); n = d - c
-        # tile lists of the chunk, built on the device from the expert counts: list i = tiles of height 16 << i, entries
-        # without a tile are skipped by the GEMM (no host synchronisation anywhere in the call)
-        tiles = torch.empty(5, cap, 4, dtype=torch.int32, device=dev)
-        # experts with several tiles are decoded once into scratch (rows of the common kind only: the variant kernel of the
-        # others decodes in the GEMM); the side streams of _pf_chains start after these launches
-        wop = S["wop"] if (S["wop"] is not None and n >= PF_HOT_MIN and not s.rare_rows and table is None) else None
-        hot = torch.empty(E, dtype=torch.int32, device=dev) if wop is not None else None
-        _lib.check(Lb.nq_pf_plan(cnt.data_ptr(), E, c, n, tiles.data_ptr(), cap, None if hot is None else hot.data_ptr(), PF_HOT_MIN,
-                                 0 if wop is None else wop.shape[0], st))
-        if wop is not None:
-            for mode in (0, 1):
-                _lib.check(Lb.nq_pf_wdecode(tb.data_ptr(), hot.data_ptr(), E, mode, wop.data_ptr(), wop.numel() * 2, wop.shape[0], H, I, st))
-        lists = [(16 << i, tiles[i], E if i < 4 else cap) for i in (4, 3, 2, 1, 0)]          # tallest first
-        pts, pes = pt[c:d], pe[c:d]
-        _pf_chains(Lb, tb, lists, variants, S, x, pts, pes, n, tiles, cap, E, H, I, None if wop is None else wop.data_ptr())
-        _lib.check(Lb.nq_pf_post(S["y"].data_ptr(), pos.data_ptr(), selc.data_ptr(), rwc.data_ptr(), T, k, c, n, tb.data_ptr(),
-                                 out.data_ptr(), S["zd"].data_ptr(), E, H, I, st))
-    return out
+    out = torch.empty(x.shape[0], s.H, dtype=torch.float32, device=x.device) if out is None else out
+    return _pf_step(s, x, sel.contiguous(), rw.contiguous(), out, R, table)
 
 
 class Mailbox:
@@ -454,12 +426,18 @@ MoELayer.prefill = prefill
 
 
 PF_MIN = 384         # tokens from which a step goes through prefill() (reference NQ_PF_MIN, sm120/serve/nq_vllm.py:187)
+# Steps of more than GROUP_MIN tokens that would take more than three slices go through the grouped kernels of prefill() too (not
+# under graph capture). The reference slices up to 383 tokens into decode calls, and each slice decodes its experts anew: 48 tokens
+# name 200 distinct experts, their twelve slices of four 360. Measured at E = 256, top-8, Bmax 4 (slices / grouped): 9 tokens
+# 522 / 478 us, 16: 934 / 707, 48: 2650 / 1200, 201: 10900 / 1530, 383: 20800 / 1600.
+GROUP_MIN = 12
 
 
 def forward(layer, mailbox, x, topk_weights, topk_ids, pf_min=PF_MIN, sal=None):
     """One MoE layer step as the reference's serving caller runs it (sm120/serve/nq_vllm.py:520-574): apply the mailbox,
-    then up to Bmax tokens in one decode call, pf_min tokens or more through prefill() (never under graph capture), anything
-    between in slices of Bmax tokens. x [T, H] in fp16 / bf16 / fp32, weights [T, topk] likewise, ids int64 / int32;
+    then up to Bmax tokens in one decode call, pf_min tokens or more, or more than three slices' worth, through the grouped kernels
+    of prefill() (never under graph capture), anything between in slices of Bmax tokens. x [T, H] in fp16 / bf16 / fp32, weights
+    [T, topk] likewise, ids int64 / int32;
     returns [T, H] in x's dtype. The decode calls read the caller's dtypes and write the result dtype themselves. `sal`: an
     optional salience.Salience, fed by the decode steps as the reference does (every step of up to Bmax tokens, the slices of
     a step of up to 16 tokens; longer steps count as prefill and are left out)."""
@@ -474,9 +452,15 @@ def forward(layer, mailbox, x, topk_weights, topk_ids, pf_min=PF_MIN, sal=None):
         mailbox.apply()
     if T == 0:
         return torch.empty(0, layer.H, dtype=odt, device=x.device)
-    if T >= pf_min and not torch.cuda.is_current_stream_capturing():
-        return layer.prefill(x.half(), ids.long(), w.half()).to(x.dtype)
     out = torch.empty(T, layer.H, dtype=odt, device=x.device)
+    grouped = T >= pf_min or (T > max(GROUP_MIN, 3 * layer.Bmax) and layer.G == 4 and layer.E <= 4096)
+    if grouped and not torch.cuda.is_current_stream_capturing():
+        if layer.G != 4 or x.dtype not in _DT_IN or w.dtype not in _DT_IN or ids.dtype not in _DT_SEL:
+            return layer.prefill(x.half(), ids.long(), w.half()).to(x.dtype)
+        _pf_step(layer, x, ids, w, out)
+        for i in range(0, T if sal is not None and T <= 16 and T < pf_min else 0, layer.Bmax):
+            sal(x[i:i + layer.Bmax], w[i:i + layer.Bmax], ids[i:i + layer.Bmax])
+        return out
     for i in range(0, T, layer.Bmax):
         j = min(T, i + layer.Bmax)
         layer(x[i:j], ids[i:j], w[i:j], out=out[i:j])

@@ -249,3 +249,40 @@ def test_row_restricted_pre_and_mid_cover_the_rows_of_their_heights_exactly():
                 mine = cls == k
                 assert torch.equal(q[mine], w[mine]) and bool((q[~mine] == 7.0).all()), (fn.__name__, k)
         assert all(torch.equal(a, b) for a, b in zip(fn(31), whole))
+
+
+@pytest.mark.parametrize("T,E,K,Bmax,xd,wd,sd", [
+    (13, 40, 4, 4, torch.bfloat16, torch.float32, torch.int32),        # first grouped size, one-launch plan, rows of every height it has
+    (150, 7, 3, 2, torch.float32, torch.bfloat16, torch.int64),        # 64 rows per expert and more: tall tiles on side streams
+    (229, 300, 8, 8, torch.float16, torch.float16, torch.int32),       # more experts than a workgroup of the sort has threads' worth of groups
+    (5600, 4, 3, 4, torch.float16, torch.float32, torch.int64),        # more pairs than the sort keeps in LDS at a time
+])
+def test_grouped_step_equals_the_decode_slices(T, E, K, Bmax, xd, wd, sd):
+    """moe.forward between the decode call and the long prompts: caller dtypes, ids outside the table, zero weights, an expert at
+    level 0, hits -- against fp32 decode slices of the same layer"""
+    H, I = 256, 256
+    ex = to_dev(experts_on_gpu(H, I, min(E, 12), 70, nested_ids=(1, 3)))
+    L = M.MoELayer(E, H, I, Bmax=Bmax, topk=K)
+    for e in range(E):
+        L.set(e, ex[e % len(ex)], 0 if e == 2 else 4 if ex[e % len(ex)].nested else 2)
+    hits = torch.zeros(E, dtype=torch.int32, device=DEV)
+    L.hits_ptr = hits.data_ptr()
+    g = torch.Generator().manual_seed(T)
+    sel = torch.stack([torch.randperm(E, generator=g)[:K] for _ in range(min(T, 256))]).repeat(-(-T // 256), 1)[:T]
+    sel[3, 0], sel[T // 2, 1], sel[5] = -1, E + 3, 2
+    w = torch.rand(T, K, generator=g) + 0.05
+    w[::7, 0] = 0
+    x = (torch.randn(T, H, generator=g) * 0.3).to(DEV).to(xd)
+    sel, w = sel.to(DEV).to(sd), w.to(DEV).to(wd)
+    y = M.forward(L, None, x, w, sel)
+    want_hits = hits.clone()
+    assert y.dtype == xd and bool(torch.isfinite(y.float()).all())
+    want = torch.empty(T, H, dtype=torch.float32, device=DEV)
+    hits.zero_()
+    for i in range(0, T, Bmax):
+        L(x[i:i + Bmax], sel[i:i + Bmax], w[i:i + Bmax], out=want[i:i + Bmax])
+    torch.cuda.synchronize()
+    assert torch.equal(hits, want_hits)
+    tol = {torch.float32: 5e-5, torch.float16: 1e-3, torch.bfloat16: 8e-3}[xd]
+    assert rel_err(y.float().cpu().numpy(), want.cpu().numpy()) < tol
+    assert not y[5].any()                                         # all its picks at level 0
