@@ -47,6 +47,8 @@ int nq_validate_row(const int64_t* row_host, int H, int I);
  * `row` (device) into fp16 `out`. level 0 = use the row's level, else override. Replaces the NQ_WDUMP debug build +
  * set_wdump (reference sm120/nqmoe.cu:246-288,852-853) and is the bit-exactness probe of the decoder. */
 int nq_dequant(const int64_t* row, int proj, int level, int H, int I, void* out_f16, void* stream);
+/* The same with the row in host memory (its plane addresses are device addresses): nothing has to be copied to the device first. */
+int nq_dequant_row(const int64_t* row_host, int proj, int level, int H, int I, void* out_f16, void* stream);
 
 /* Dense decode of G experts (device int32 ids) at their live table level into Wgu [G][2I][H] and Wdn [G][H][I] fp16;
  * level <= 0 decodes to zeros. Replaces pf_decode (reference sm120/nqmoe.cu:1013-1080,1247-1257). */
@@ -147,6 +149,12 @@ typedef struct NqMoeArgs
                                  the weights are NOT rounded to fp16, and the layer output moves 4.6e-4 (relative l2, mean; 6.3e-4 at
                                  most over 64 routings of the full shape) from the exact form's -- inside the layer's 1e-3 tolerance,
                                  with little room to spare. nq_dequant is never affected. */
+    int32_t with_salience;    /* 0: the struct ends here for the library. 1: the call's routing launch also does what nq_sal does with this
+                                 call's x, rw and sel (the reference launches its salience kernel in front of every decode step,
+                                 sm120/serve/nq_vllm.py:558): */
+    double* sal_acc;          /* fp64 [E] */
+    double* sal_host;         /* [host-mapped] fp64 [E] */
+    float sal_rsf;            /* routed scaling factor */
     int32_t reserved_;
 } NqMoeArgs;
 #define NQ_ROUTE_WS_BYTES 32768

@@ -75,6 +75,18 @@ extern "C" int nq_dequant(const int64_t* row, int proj, int level, int H, int I,
     return launch_dequant(row, proj, level, H, I, out, (hipStream_t)stream);
 }
 
+extern "C" int nq_dequant_row(const int64_t* row, int proj, int level, int H, int I, void* out, void* stream)
+{
+    NQ_REQUIRE(row && out, "nq_dequant_row: null pointer");
+    NQ_REQUIRE(proj == 0 || proj == 1, "nq_dequant_row: proj %d not in {0,1}", proj);
+    NQ_REQUIRE(level == 0 || level == 2 || level == 3 || level == 4, "nq_dequant_row: level %d not in {0,2,3,4}", level);
+    {   // a single projection only needs whole units: N % 16 == 0 and K % 128 == 0
+        const int N = proj == 0 ? 2 * I : H, K = proj == 0 ? H : I;
+        NQ_REQUIRE(H > 0 && I > 0 && N % 16 == 0 && K % 128 == 0 && (int64_t)N * K < ((int64_t)1 << 33), "nq_dequant_row: projection [%d][%d] is not whole 16x128 units", N, K);
+    }
+    return launch_dequant_row(row, proj, level, H, I, out, (hipStream_t)stream);
+}
+
 extern "C" int nq_pf_decode(const int64_t* table, const int32_t* experts, int G, void* Wgu, void* Wdn, int H, int I, void* stream)
 {
     NQ_REQUIRE(G >= 0, "nq_pf_decode: G=%d", G);
@@ -153,6 +165,13 @@ static int moe_args(const char* who, const NqMoeArgs* p, bool own_ws, MoeArgs& a
     }
     NQ_REQUIRE(p->hoist_value_map == 0 || p->hoist_value_map == 1, "%s: hoist_value_map=%d (0 or 1)", who, p->hoist_value_map);
     a.hoist = p->hoist_value_map;
+    NQ_REQUIRE(p->with_salience == 0 || p->with_salience == 1, "%s: with_salience=%d (0 or 1)", who, p->with_salience);
+    if (p->with_salience)
+    {
+        NQ_REQUIRE(p->sal_acc && p->sal_host, "%s: salience needs its accumulator and its host mirror", who);
+        NQ_REQUIRE(!(p->which & 4), "%s: salience is exported by the routing launch, which this call leaves out", who);
+        a.sal_acc = p->sal_acc; a.sal_host = p->sal_host; a.sal_rsf = p->sal_rsf;
+    }
     NQ_REQUIRE(p->common_rows == 0 || p->common_rows == 1, "%s: common_rows=%d (0 or 1)", who, p->common_rows);
     a.common_rows = p->common_rows;
     NQ_REQUIRE(p->G == 0 || p->G == 4 || p->G == 2, "%s: G=%d (rings of 4 lanes, or 2)", who, p->G);

@@ -367,7 +367,7 @@ __device__ __forceinline__ MaskedUnit masked_unit(uint64_t f, uint32_t strip, in
     const int nm = __popcll(f);
     return MaskedUnit{((f >> c) & 1ull) != 0, strip * (uint32_t)nm + (uint32_t)__popcll(f & ((1ull << c) - 1ull)), nstrips * nm * 32};
 }
-__device__ __forceinline__ Planes planes_of(const int64_t* ent, int mode)
+__host__ __device__ __forceinline__ Planes planes_of(const int64_t* ent, int mode)
 {
     const int o = mode == 0 ? 1 : 5;
     Planes P;

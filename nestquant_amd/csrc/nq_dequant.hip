@@ -91,33 +91,38 @@ __device__ __forceinline__ void store_tile(const uint32_t* tile, _Float16* out, 
     }
 }
 
-// planes of projection `mode` (0 gate|up [2I][H], 1 down [H][I]) of the expert described by ent -> out
-__device__ __forceinline__ void dequant_body(const int64_t* ent, int mode, int lv, int H, int I, _Float16* out,
-                                             int pair, uint32_t* tiles)
+// projection `mode` (0 gate|up [2I][H], 1 down [H][I]) of the planes P at level lv -> out; wavefront `wave` of `nwaves` takes every
+// nwaves-th pair of units
+__device__ __forceinline__ void dequant_body(const Planes& P, int mode, int lv, int H, int I, _Float16* out, int wave, int nwaves, uint32_t* tiles)
 {
     const int lane = threadIdx.x & 63, half = lane >> 5;
     const int N = mode == 0 ? 2 * I : H, K = mode == 0 ? H : I, C = K / 128;
     const size_t nunits = (size_t)(N / 16) * C, nrec = nunits * 32;
-    size_t unit = (size_t)pair * 2 + half;
-    const bool live = unit < nunits;
-    if (!live) unit = nunits - 1;                              // keep the wave convergent for the shuffles
+    const int npairs = (int)((nunits + 1) / 2);
     uint32_t* tile = tiles + half * 16 * TS;
-    _Float16* dst = out + (size_t)(unit / C) * 16 * K + (size_t)(unit % C) * 128;
-    if (lv <= 0)
+    for (int pair = wave; pair < npairs; pair += nwaves)         // wave-uniform
     {
-        if (live) for (int i = lane & 31; i < 256; i += 32) *(uint4*)(dst + (size_t)(i >> 4) * K + (i & 15) * 8) = make_uint4(0, 0, 0, 0);
-        return;
-    }
-    const Planes P = planes_of(ent, mode);
-    decode_unit(P, lv, unit, nrec, C, tile, lane);
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    // each half-wave wrote its own tile; the whole wave now drains both tiles
-    for (int h = 0; h < 2; ++h)
-    {
-        const size_t u = (size_t)pair * 2 + h;
-        if (u >= nunits) break;
-        store_tile(tiles + h * 16 * TS, out + (size_t)(u / C) * 16 * K + (size_t)(u % C) * 128, K, lane);
+        size_t unit = (size_t)pair * 2 + half;
+        const bool live = unit < nunits;
+        if (!live) unit = nunits - 1;                            // keep the wave convergent for the shuffles
+        if (lv <= 0)
+        {
+            _Float16* dst = out + (size_t)(unit / C) * 16 * K + (size_t)(unit % C) * 128;
+            if (live) for (int i = lane & 31; i < 256; i += 32) *(uint4*)(dst + (size_t)(i >> 4) * K + (i & 15) * 8) = make_uint4(0, 0, 0, 0);
+            continue;
+        }
+        decode_unit(P, lv, unit, nrec, C, tile, lane);
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        // each half-wave wrote its own tile; the whole wave now drains both tiles
+        for (int h = 0; h < 2; ++h)
+        {
+            const size_t u = (size_t)pair * 2 + h;
+            if (u >= nunits) break;
+            store_tile(tiles + h * 16 * TS, out + (size_t)(u / C) * 16 * K + (size_t)(u % C) * 128, K, lane);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();                         // the tiles are free again
     }
 }
 
@@ -125,12 +130,14 @@ __global__ void __launch_bounds__(256) nq_dequant_k(const int64_t* __restrict__ 
 {
     __shared__ __align__(16) uint32_t tiles[4][2 * 16 * TS];
     const int warp = threadIdx.x >> 6;
-    const int N = mode == 0 ? 2 * I : H, K = mode == 0 ? H : I;
-    const int npairs = ((N / 16) * (K / 128) + 1) / 2;
-    const int pair = blockIdx.x * 4 + warp;
-    if (pair >= npairs) return;                                 // wave-uniform
-    const int lv = level ? level : (int)ent[0];
-    dequant_body(ent, mode, lv, H, I, out, pair, tiles[warp]);
+    dequant_body(planes_of(ent, mode), mode, level ? level : (int)ent[0], H, I, out, blockIdx.x * 4 + warp, gridDim.x * 4, tiles[warp]);
+}
+// the same with the planes as kernel arguments
+__global__ void __launch_bounds__(256) nq_dequant_row_k(Planes P, int mode, int lv, int H, int I, _Float16* out)
+{
+    __shared__ __align__(16) uint32_t tiles[4][2 * 16 * TS];
+    const int warp = threadIdx.x >> 6;
+    dequant_body(P, mode, lv, H, I, out, blockIdx.x * 4 + warp, gridDim.x * 4, tiles[warp]);
 }
 
 // grid (ceil(pairs / 4), G, 2): Wgu [G][2I][H], Wdn [G][H][I]; level from the live table row; level <= 0 -> zeros
@@ -140,20 +147,29 @@ __global__ void __launch_bounds__(256) nq_pf_decode_k(const int64_t* __restrict_
     __shared__ __align__(16) uint32_t tiles[4][2 * 16 * TS];
     const int mode = blockIdx.z, gi = blockIdx.y, warp = threadIdx.x >> 6;
     const int N = mode == 0 ? 2 * I : H, K = mode == 0 ? H : I;
-    const int npairs = ((N / 16) * (K / 128) + 1) / 2;
-    const int pair = blockIdx.x * 4 + warp;
-    if (pair >= npairs) return;
     const int64_t* ent = table + (int64_t)experts[gi] * TBL_W;
     _Float16* out = (mode == 0 ? Wgu : Wdn) + (size_t)gi * N * K;
-    dequant_body(ent, mode, (int)ent[0], H, I, out, pair, tiles[warp]);
+    dequant_body(planes_of(ent, mode), mode, (int)ent[0], H, I, out, blockIdx.x * 4 + warp, gridDim.x * 4, tiles[warp]);
+}
+
+static int dequant_blocks(int proj, int H, int I)
+{
+    const int N = proj == 0 ? 2 * I : H, K = proj == 0 ? H : I;
+    const int npairs = ((N / 16) * (K / 128) + 1) / 2;
+    return (npairs + 3) / 4;                                     // one pair per wavefront: 384 to 1024 workgroups walking several pairs each take as long
 }
 
 int launch_dequant(const int64_t* row, int proj, int level, int H, int I, void* out, hipStream_t st)
 {
-    const int N = proj == 0 ? 2 * I : H, K = proj == 0 ? H : I;
-    const int npairs = ((N / 16) * (K / 128) + 1) / 2;
-    nq_dequant_k<<<dim3((npairs + 3) / 4), 256, 0, st>>>(row, proj, level, H, I, (_Float16*)out);
+    nq_dequant_k<<<dequant_blocks(proj, H, I), 256, 0, st>>>(row, proj, level, H, I, (_Float16*)out);
     NQ_LAUNCH_CHECK("nq_dequant");
+    return 0;
+}
+
+int launch_dequant_row(const int64_t* row, int proj, int level, int H, int I, void* out, hipStream_t st)
+{
+    nq_dequant_row_k<<<dequant_blocks(proj, H, I), 256, 0, st>>>(planes_of(row, proj), proj, level ? level : (int)row[0], H, I, (_Float16*)out);
+    NQ_LAUNCH_CHECK("nq_dequant_row");
     return 0;
 }
 

@@ -42,6 +42,7 @@ struct MoeArgs
     _Float16* xrot;                   // [B * topk][2][H] fp16: rotated activations of every active pick (gate, up), B-operand order
     int hoist;                        // NqMoeArgs::hoist_value_map: level-2 runs without a sign plane apply the value map to the sums
     int mb_apply;                     // this projection launch (the call's last) carries the block that applies the mailbox (set by launch_moe)
+    double* sal_acc; double* sal_host; float sal_rsf;   // salience of the call, exported by its routing launch (sal_acc == nullptr: none)
     int64_t* mb_table; const int64_t* mb_stage; const int32_t* mb_seq; int32_t* mb_applied; int32_t* mb_applied_host;
                                       // mailbox of the call (mb_table == nullptr: none): applied by the last projection launch, published by the next call's routing launch
 };
@@ -52,6 +53,7 @@ int launch_moe_static(MoeArgs a, const int* cfg_gu, const int* cfg_dn, int which
 int query_occ(int mode, int any_rows, int sb, int shm, int* out);
 int launch_mailbox(int64_t* table, const int64_t* stage, const int32_t* seq, int32_t* applied, int32_t* applied_host, int E, hipStream_t st);
 int launch_dequant(const int64_t* row, int proj, int level, int H, int I, void* out, hipStream_t st);
+int launch_dequant_row(const int64_t* row, int proj, int level, int H, int I, void* out, hipStream_t st);
 int launch_pf_decode(const int64_t* table, const int32_t* experts, int G, void* Wgu, void* Wdn, int H, int I, hipStream_t st);
 int launch_pf_pre(const void* x, int xdt, const int32_t* pt, const int32_t* pe, int np, const int64_t* table, void* xg, void* xu, float* zg, int E, int H, int I,
                   const int32_t* tiles, int cap, int heights, hipStream_t st);

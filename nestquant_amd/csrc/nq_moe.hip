@@ -21,7 +21,7 @@
 // pairs are A operands as they leave the decoder, with no cross-lane movement. The B operand (tokens) comes from LDS,
 // staged in the matching column order. Partial sums instead of float atomics make the layer output bitwise repeatable;
 // the arrival counters are zero on entry and are reset by the block that consumes them.
-#include "nq_tile.hpp"
+#include "nq_sal.hpp"
 #include "nq_host.hpp"
 #include <algorithm>
 #include <mutex>
@@ -253,17 +253,26 @@ __device__ __forceinline__ void publish_applied(const int32_t* applied, int32_t*
 // xrot[q][gate|up][chunk] = fp16(Hadamard-128(x[token] * su)) in the MFMA B-operand column order, which the gate|up launch
 // copies into LDS (before, each of the 32 row blocks of a run repeated these rotations: 9 % of the launch's vector
 // instructions). With a mailbox in the call the other three wavefronts of workgroup 0 first publish what earlier calls applied
-// (publish_applied); nothing here reads seq or stage and nothing writes the table.
+// (publish_applied); nothing here reads seq or stage and nothing writes the table. With salience in the call one more workgroup
+// exports it beside the others (a launch of its own in front of the call cost 9 us at one token, 20 us at four).
 __global__ void __launch_bounds__(256) nq_prep_k(MoeArgs a)
 {
     __shared__ PrepRows Q;
     const int lane = threadIdx.x & 63;
+    const int nblk = (int)gridDim.x - (a.sal_acc ? 1 : 0);       // the last workgroup of a call with salience does that and nothing else
+    if ((int)blockIdx.x == nblk)
+    {
+        __shared__ SalShared S;
+        const SalArgs sa{a.x, a.H, a.rw, a.sel, a.B, a.H, a.topk, a.E, a.x_dtype, a.rw_dtype, a.sel_dtype, a.sal_rsf, a.sal_acc, a.sal_host};
+        salience<4>(sa, &S);
+        return;
+    }
     if (threadIdx.x < 64) route(a, a.route, lane, blockIdx.x == 0, &Q);
     else if (blockIdx.x == 0 && a.mb_table && a.mb_applied_host) publish_applied(a.mb_applied, a.mb_applied_host, a.E, threadIdx.x - 64, 192);
     __syncthreads();
     // workgroup 0 has the result to write (it ends ~1 us after the others' routing): with more than one workgroup in the grid the
     // rotation tasks go to the others, so that it is not also the last to finish
-    const int C = a.H / 128, ntask = Q.nq * 2 * C, nrot = gridDim.x > 1 ? gridDim.x - 1 : 1, rot = gridDim.x > 1 ? (int)blockIdx.x - 1 : 0;
+    const int C = a.H / 128, ntask = Q.nq * 2 * C, nrot = nblk > 1 ? nblk - 1 : 1, rot = nblk > 1 ? (int)blockIdx.x - 1 : 0;
     if (rot < 0) return;
     for (int t = rot * 4 + (threadIdx.x >> 6); t < ntask; t += nrot * 4)
     {
@@ -671,7 +680,7 @@ int launch_moe(const MoeArgs& a, const int* cfg_gu, const int* cfg_dn, int which
     if (!reuse)
     {
         const int ntask = S * 2 * (a.H / 128);                   // upper bound: every pick active
-        nq_prep_k<<<std::min((ntask + 3) / 4, 1023) + 1, 256, 0, st>>>(a);       // one workgroup per four rotation tasks, plus the writer
+        nq_prep_k<<<std::min((ntask + 3) / 4, 1023) + 1 + (a.sal_acc ? 1 : 0), 256, 0, st>>>(a);       // one workgroup per four rotation tasks, plus the writer
         NQ_LAUNCH_CHECK("moe_forward (routing)");
     }
     // a call with a mailbox and no projection launch: the apply half as a launch of its own (nothing is published here either)

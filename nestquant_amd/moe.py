@@ -7,6 +7,7 @@ libnq_moe_hip.so, reached through ctypes with raw device pointers; there is no C
 import ctypes as C
 import os
 
+import numpy as np
 import torch
 
 from . import _lib
@@ -35,11 +36,11 @@ def H128(dev="cuda", n=128):
     return (H / n**0.5).to(dev)
 
 
-def entry(ex, level):
-    """table row int64[TBL_W] of expert `ex` at `level` (0, 2, 3, 4). Level 3 points at the one-bit plane p3 (code 10); level 4
+def _entry_words(ex, level):
+    """table row (TBL_W integers) of expert `ex` at `level` (0, 2, 3, 4). Level 3 points at the one-bit plane p3 (code 10); level 4
     points, for experts built with nested=True, at the planes P3 and P4 read as one record (code 11: concatenated, or code 12
     for experts built with interleave=True: interleaved bit by bit), otherwise at the wide residual plane p4 (code rk)."""
-    e = torch.zeros(TBL_W, dtype=torch.int64)
+    e = [0] * TBL_W                                  # a list first: setting elements of a tensor one by one takes 30 us
     e[0] = level
     nested = bool(getattr(ex, "nested", False))
     l3 = level == 3
@@ -74,6 +75,11 @@ def entry(ex, level):
     e[18] = 0 if w == 128 else w
     e[19] = base_code(ex.gu) | base_code(ex.dn) << 8
     return e
+
+
+def entry(ex, level):
+    """_entry_words as an int64 tensor (host)"""
+    return torch.from_numpy(np.array(_entry_words(ex, level), dtype=np.int64))
 
 
 def validate_row(row, H, I):
@@ -114,10 +120,16 @@ def dequant(row_dev, proj, H, I, level=0, out=None):
 
 def dense_W(ex, proj, level, dtype=torch.float16):
     """dense rotated-domain weights [N, K] of projection `proj` (0 gate|up, 1 down) of expert `ex`, decoded on the GPU"""
-    row = entry(ex, level)
-    validate_row(row, ex.H, ex.I)
-    row = row.to(ex.signs.device)
-    return dequant(row, proj, ex.H, ex.I).to(dtype)
+    row = (C.c_int64 * TBL_W)(*_entry_words(ex, level))
+    L = _lib.lib()
+    N, K = (2 * ex.I, ex.H) if proj == 0 else (ex.H, ex.I)
+    rc = L.nq_validate_row(row, ex.H, ex.I)
+    out = None
+    if not rc:                                                   # the row goes along as a kernel argument: no copy to the device
+        out = torch.empty(N, K, dtype=torch.float16, device=ex.signs.device)
+        rc = L.nq_dequant_row(row, proj, 0, ex.H, ex.I, out.data_ptr(), _lib.stream_ptr())
+    _lib.check(rc)
+    return out if dtype == torch.float16 else out.to(dtype)
 
 
 # caller element types the decode kernels read / write directly (codes of include/nq_moe_hip.h)
@@ -145,7 +157,7 @@ class MoELayer:
         S = Bmax * topk
         f32, i32 = torch.float32, torch.int32
         s.cfg_gu, s.cfg_dn = s.default_cfg(H, I)
-        s._tuned = True                               # cfg_for may pick the tuned k-slice lengths; set_cfg switches that off
+        s._tuned, s._cfgs = True, {}                  # cfg_for picks the k-slice lengths by the call's size; set_cfg switches that off
         s.h = torch.zeros(S, I, dtype=torch.float16, device=dev)
         s.cnt_gu = torch.zeros(S * (I // 128), dtype=i32, device=dev); s.cnt_d = torch.zeros(H // 128, dtype=i32, device=dev)
         s.wq = torch.zeros(4, dtype=i32, device=dev)
@@ -161,44 +173,49 @@ class MoELayer:
                                                       # that pick them come out NaN
         s._alloc_partials()
 
-    # k-slice lengths (chunks) per token count 1..8 at the full shape H = 6144, I = 2048, top-8 over 256 experts, measured on
-    # an MI355X with the routing of the layer benchmark; the reference keeps such tables for its GPUs
-    # (sm120/serve/nq_vllm.py:32-33). Index = tokens of the call; other shapes use default_cfg for every count.
-    TUNED_NST = {(6144, 2048): ([12, 12, 24, 24, 24, 24, 24, 24, 24], [4, 4, 4, 4, 4, 4, 4, 4, 4])}
-
-    def cfg_for(s, T):
-        """(cfg_gu, cfg_dn) for a decode call of T tokens: the layer's defaults, with the tuned k-slice length for T where this
-        shape has a table and set_cfg has not replaced the defaults"""
-        t = s.TUNED_NST.get((s.H, s.I)) if s._tuned else None
-        if t is None or T >= len(t[0]):
-            return s.cfg_gu, s.cfg_dn
-        return [s.cfg_gu[0], s.cfg_gu[1], t[0][T]], [s.cfg_dn[0], s.cfg_dn[1], t[1][T]]
+    # k-slice lengths. A projection launch has (row blocks) x (k-slices) x (runs of distinct experts) workgroups, and about 1024 of
+    # them fill the chip (four per CU for gate|up, five for down): fewer leave CUs idle, and every further one costs a head (run
+    # header, activations, first records) of 2 to 4 us. So a slice is as long as keeps the launch at that number, with a run for
+    # every pick (an upper bound), at most 24 chunks for gate|up and 4 for down (whose finisher and SwiGLU staging favour short
+    # slices at every count). Measured best at H = 6144, I = 2048, top-8: 12 chunks at one token, 24 above, down 4; the rule gives
+    # these. The reference keeps tables of measured lengths per GPU (sm120/serve/nq_vllm.py:32-33).
+    @staticmethod
+    def _slice(C, blocks, runs, slots, most):
+        want = min(most, max(1, blocks * C * runs // slots))
+        return max(d for d in range(1, want + 1) if C % d == 0)
 
     @staticmethod
-    def default_cfg(H, I):
-        """[cpw, sb, nst]: k-slice of cpw * nst chunks, sb wavefronts per block"""
-        def pick(C, N, want):
-            nc = max(d for d in range(1, want + 1) if C % d == 0)
-            sb = max(d for d in (4, 2, 1) if (N // 32) % d == 0 and (I // 32) % d == 0)
-            return [1, sb, nc]
-        return pick(H // 128, 2 * I, 12), pick(I // 128, H, 8)
+    def default_cfg(H, I, runs=8):
+        """[cpw, sb, nst]: k-slice of cpw * nst chunks, sb wavefronts per block; for a call of `runs` picks"""
+        sb = lambda N: max(d for d in (4, 2, 1) if (N // 32) % d == 0 and (I // 32) % d == 0)
+        gu, dn = sb(2 * I), sb(H)
+        return ([1, gu, MoELayer._slice(H // 128, 2 * I // 32 // gu, runs, 1024, 24)],
+                [1, dn, MoELayer._slice(I // 128, H // 32 // dn, runs, 1280, 4)])
+
+    def cfg_for(s, T):
+        """(cfg_gu, cfg_dn) for a decode call of T tokens: default_cfg for its picks, unless set_cfg has replaced the defaults"""
+        if not s._tuned:
+            return s.cfg_gu, s.cfg_dn
+        c = s._cfgs.get(T)
+        if c is None:
+            c = s._cfgs[T] = s.default_cfg(s.H, s.I, T * s.topk)
+        return c
 
     def _ny(s, cfg, C):
         return C // (cfg[0] * cfg[2])
 
     def _alloc_partials(s, cfg_gu=None, cfg_dn=None):
         """Partial-sum workspaces for the given (default: the layer's) tilings. At construction they are sized for the finest
-        k-split among the layer's default and its tuned tilings, so the calls a serving loop makes never re-size them. A call
+        k-split among the layer's own tilings (cfg_for, 1 .. Bmax tokens), so the calls a serving loop makes never re-size them. A call
         that brings a finer split of its own replaces them -- graphs captured before hold the old addresses and must be
         captured again -- and that is refused while the stream is capturing (an allocation cannot be captured)."""
         S, dev = s.Bmax * s.topk, s.table.device
         ny_gu, ny_dn = s._ny(cfg_gu or s.cfg_gu, s.H // 128), s._ny(cfg_dn or s.cfg_dn, s.I // 128)
         first = getattr(s, "acc_gu", None) is None
         if first:
-            t = s.TUNED_NST.get((s.H, s.I))
-            if t is not None:
-                ny_gu = max([ny_gu] + [(s.H // 128) // (s.cfg_gu[0] * n) for n in t[0]])
-                ny_dn = max([ny_dn] + [(s.I // 128) // (s.cfg_dn[0] * n) for n in t[1]])
+            own = [s.cfg_for(T) for T in range(1, s.Bmax + 1)]
+            ny_gu = max([ny_gu] + [s._ny(c[0], s.H // 128) for c in own])
+            ny_dn = max([ny_dn] + [s._ny(c[1], s.I // 128) for c in own])
         grow_gu, grow_dn = first or s.acc_gu.shape[0] < ny_gu, first or s.acc_d.shape[0] < ny_dn
         if (grow_gu or grow_dn) and not first and torch.cuda.is_current_stream_capturing():
             raise RuntimeError("this call's k-split needs larger partial-sum workspaces than the layer holds; make one call with "
@@ -222,7 +239,7 @@ class MoELayer:
         s.rare_rows |= bool(row[4] or row[8] or row[19])
         s.table[e].copy_(row.to(s.table.device), non_blocking=False)
 
-    def __call__(s, x, sel, rw, out=None, force_level=0, which=3, cfg_gu=None, cfg_dn=None, table=None, static_ws=False, mailbox=None, hoist=False):
+    def __call__(s, x, sel, rw, out=None, force_level=0, which=3, cfg_gu=None, cfg_dn=None, table=None, static_ws=False, mailbox=None, hoist=False, sal=None):
         """x [B, H], sel [B, topk], rw [B, topk] -> fp32 [B, H] (s.out[:B] unless `out` is given). As in the reference x
         and rw are fp16 and sel int64; the kernels also take x / rw in bf16 or fp32, sel in int32 and `out` in fp16 or
         bf16, with the roundings of x.half(), rw.half() and out.to(dtype) (the casts the reference's caller launches as
@@ -236,6 +253,8 @@ class MoELayer:
         hoist: experts without a sign plane (rows of the common kind) multiply the integers 1024 + S / 1024 + F and apply the value
         map to the sums, so no weight is rounded to fp16: ~4 % faster, ~5e-4 from the default's result (NqMoeArgs.hoist_value_map;
         off by default).
+        sal: a salience.Salience, fed with this call's x, sel and rw by the call's routing launch (what `sal(x, rw, sel)` in front of
+        the call does with a launch of its own; at most 8 picks per token).
         static_ws: go through nq_moe_forward_static, which ignores this layer's workspaces and uses the library's built-in
         device scratch instead (for callers that must not allocate; calls on one GPU then share that scratch)."""
         assert x.dtype in _DT_IN and rw.dtype in _DT_IN and sel.dtype in _DT_SEL, (x.dtype, rw.dtype, sel.dtype)
@@ -245,30 +264,25 @@ class MoELayer:
         assert out.dtype in _DT_OUT and out.is_contiguous(), out.dtype
         tb = s.table if table is None else table
         tg, td = s.cfg_for(B)
-        cg, cd = list(cfg_gu or tg), list(cfg_dn or td)
-        if not static_ws:
+        cg, cd = cfg_gu or tg, cfg_dn or td
+        if not static_ws and (cfg_gu or cfg_dn):
             s._alloc_partials(cg, cd)                # grows only when a call brings a finer k-split than any before
-        a = _lib.NqMoeArgs()
-        a.x, a.sel, a.rw, a.table, a.out = x.data_ptr(), sel.data_ptr(), rw.data_ptr(), tb.data_ptr(), out.data_ptr()
-        a.acc_gu, a.h, a.acc_d, a.hits = s.acc_gu.data_ptr(), s.h.data_ptr(), s.acc_d.data_ptr(), s.hits_ptr or None
-        a.cnt_gu, a.cnt_d = s.cnt_gu.data_ptr(), s.cnt_d.data_ptr()
-        a.acc_gu_elems, a.acc_d_elems, a.h_elems, a.out_elems = s.acc_gu.numel(), s.acc_d.numel(), s.h.numel(), out.numel()
-        a.cnt_gu_elems, a.cnt_d_elems = s.cnt_gu.numel(), s.cnt_d.numel()
-        a.B, a.topk, a.E, a.H, a.I = B, topk, tb.shape[0], x.shape[1], s.I
-        a.cfg_gu = (C.c_int32 * 4)(*(cg + [0] * (4 - len(cg)))); a.cfg_dn = (C.c_int32 * 4)(*(cd + [0] * (4 - len(cd))))
-        a.force_level, a.which = force_level, which
-        a.cnt_h, a.cnt_h_elems = s.cnt_h.data_ptr(), s.cnt_h.numel()
-        a.zd, a.zd_elems = s.zd.data_ptr(), s.zd.numel()
-        a.G = s.G
-        a.route_ws, a.route_ws_bytes = s.route.data_ptr(), s.route.numel()
-        a.xrot, a.xrot_elems = s.xrot.data_ptr(), s.xrot.numel()
-        if mailbox is not None:
-            a.mb_table, a.mb_stage, a.mb_seq = tb.data_ptr(), mailbox.stage.data_ptr(), mailbox.seq.data_ptr()
-            a.mb_applied, a.mb_applied_host = mailbox.applied.data_ptr(), mailbox.applied_host.data_ptr()
-        a.common_rows = int(table is None and not s.rare_rows)     # a caller's own table: unknown
-        a.hoist_value_map = int(bool(hoist))
-        a.x_dtype, a.sel_dtype, a.rw_dtype, a.out_dtype = _DT_IN[x.dtype], _DT_SEL[sel.dtype], _DT_IN[rw.dtype], _DT_OUT[out.dtype]
-        _lib.check((s.M.nq_moe_forward_static if static_ws else s.M.nq_moe_forward)(C.byref(a), _lib.stream_ptr()))
+        # one struct.pack instead of sixty attribute stores on a ctypes structure: 4 us less host time per call
+        mb = (0, 0, 0, 0, 0) if mailbox is None else (tb.data_ptr(), mailbox.stage.data_ptr(), mailbox.seq.data_ptr(), mailbox.applied.data_ptr(),
+                                                      mailbox.applied_host.data_ptr())
+        sl = (0, 0, 0, 0.0) if sal is None else (1, sal.acc.data_ptr(), sal.host.data_ptr(), sal.rsf)
+        raw = _lib.PACK_MOE_ARGS(
+            x.data_ptr(), sel.data_ptr(), rw.data_ptr(), tb.data_ptr(), out.data_ptr(), s.acc_gu.data_ptr(), s.h.data_ptr(), s.acc_d.data_ptr(),
+            s.cnt_gu.data_ptr(), s.cnt_d.data_ptr(), s.hits_ptr or 0,
+            s.acc_gu.numel(), s.acc_d.numel(), s.h.numel(), out.numel(), s.cnt_gu.numel(), s.cnt_d.numel(),
+            B, topk, tb.shape[0], x.shape[1], s.I, cg[0], cg[1], cg[2], cg[3] if len(cg) > 3 else 0, cd[0], cd[1], cd[2], cd[3] if len(cd) > 3 else 0,
+            force_level, which, _DT_IN[x.dtype], _DT_SEL[sel.dtype], _DT_IN[rw.dtype], _DT_OUT[out.dtype],
+            s.cnt_h.data_ptr(), s.cnt_h.numel(), s.zd.data_ptr(), s.zd.numel(),
+            int(table is None and not s.rare_rows), s.G,             # common_rows; a caller's own table: unknown
+            s.route.data_ptr(), s.route.numel(), s.xrot.data_ptr(), s.xrot.numel(), *mb, int(bool(hoist)), *sl, 0)
+        rc = (s.M.nq_moe_forward_static if static_ws else s.M.nq_moe_forward)(raw, _lib.stream_ptr())
+        if rc:
+            _lib.check(rc)
         return out
 
 
@@ -445,9 +459,11 @@ def forward(layer, mailbox, x, topk_weights, topk_ids, pf_min=PF_MIN, sal=None):
     x, w, ids = x.contiguous(), topk_weights.contiguous(), topk_ids.contiguous()
     odt = x.dtype if x.dtype in _DT_OUT else torch.float32
     if 0 < T <= layer.Bmax:
-        if sal is not None:
+        inside = hasattr(sal, "acc") and ids.shape[1] <= 8 and sal.acc.numel() == layer.E       # a Salience: exported by the call itself
+        if sal is not None and not inside:
             sal(x, w, ids)
-        return layer(x, ids, w, out=torch.empty(T, layer.H, dtype=odt, device=x.device), mailbox=mailbox)   # applied by the call's last launch, for the next step
+        return layer(x, ids, w, out=torch.empty(T, layer.H, dtype=odt, device=x.device), mailbox=mailbox,   # applied by the call's last launch, for the next step
+                     sal=sal if inside else None)
     if mailbox is not None:
         mailbox.apply()
     if T == 0:
@@ -530,12 +546,20 @@ Expert.ref = expert_ref
 def proj_gemv(layer, x, e=0, cfg=None):
     """Raw fused decode+GEMV of the gate|up projection of expert e for every token of x [B, H] (B <= 8), without the
     SwiGLU finisher: returns fp32 [B, 2I] = W_gu . fp16(Hadamard(x * su)) (rows < I rotated with su_g, the rest with su_u),
-    read back from the layer's k-slice partial sums after a gate|up-only launch whose finisher output is ignored."""
+    read back from the layer's k-slice partial sums after a gate|up launch that leaves the SwiGLU out."""
     B = x.shape[0]
-    sel = torch.full((B, 1), e, dtype=torch.int64, device=x.device)
-    rw = torch.ones(B, 1, dtype=torch.float16, device=x.device)
-    cfg = list(cfg or layer.cfg_gu)
-    layer(x, sel, rw, which=1, cfg_gu=cfg)
-    ny = (layer.H // 128) // (cfg[0] * cfg[2])
+    C_ = layer.H // 128
+    if cfg is None:
+        # one run: about 512 workgroups and slices of two or three chunks at the full shape are where heads, decode and the number
+        # of partial sums balance, as far as the layer's workspace holds that many slices
+        sb = layer.cfg_gu[1]
+        n = MoELayer._slice(C_, 2 * layer.I // 32 // sb, 1, 512, 24)
+        n = next(d for d in range(n, C_ + 1) if C_ % d == 0 and C_ // d <= layer.acc_gu.shape[0])
+        cfg = [1, sb, n]
+    k = (B, e, x.device)
+    if getattr(layer, "_proj_in", (None,))[0] != k:
+        layer._proj_in = (k, torch.full((B, 1), e, dtype=torch.int64, device=x.device), torch.ones(B, 1, dtype=torch.float16, device=x.device))
+    layer(x, layer._proj_in[1], layer._proj_in[2], which=1 | 8, cfg_gu=list(cfg))      # 8: the launch ends with its partial sums
+    ny = C_ // (cfg[0] * cfg[2])
     n = 2 * layer.I                                               # partial sums are laid out [k-slice][B * topk of the call][2I]
     return layer.acc_gu.view(-1)[: ny * B * n].view(ny, B, n).sum(0)

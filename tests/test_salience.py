@@ -127,3 +127,30 @@ def test_salience_errors_and_forward_hook():
                 O.salience(xt[i:i + 4].float().cpu().numpy(), wt[i:i + 4].half().cpu().numpy(), it[i:i + 4].cpu().numpy(), 1.5, want)
     torch.cuda.synchronize()
     assert np.allclose(S.acc.cpu().numpy(), want, rtol=1e-5, atol=0) and np.array_equal(S.host.numpy(), S.acc.cpu().numpy())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,K,H,xd", [(1, 1, 128, torch.float16), (2, 3, 1152, torch.bfloat16), (8, 8, 384, torch.float32), (3, 8, 6144, torch.bfloat16)])
+def test_salience_inside_the_layer_call_is_the_launch_in_front_of_it(T, K, H, xd):
+    """NqMoeArgs.with_salience: the routing launch exports what nq_sal exports, call after call, and the layer's result is the same"""
+    from nestquant_amd import format as F, moe as M, salience as SA
+    I, E = 128, 9
+    L = M.MoELayer(E, H, I, Bmax=8, topk=K)
+    keep = []
+    for e in range(E):
+        ex = F.Expert(H, I, seed=e, dev="cuda", gen_dev="cuda"); keep.append(ex)
+        L.set(e, ex, 2)
+    g = torch.Generator().manual_seed(T)
+    A, B = SA.Salience(E, rsf=2.5), SA.Salience(E, rsf=2.5)
+    for _ in range(3):
+        x = torch.randn(T, H, generator=g).to(xd).cuda()
+        w = torch.rand(T, K, generator=g).cuda(); w[0, 0] = 0
+        ids = torch.stack([torch.randperm(E, generator=g)[:K] for _ in range(T)]).int().cuda()
+        ids[-1, -1] = E + 1 if K > 1 else 0
+        A(x, w, ids)
+        y = L(x, ids, w).clone()
+        assert torch.equal(L(x, ids, w, sal=B), y)
+    torch.cuda.synchronize()
+    assert A.acc.sum() > 0 or K == 1
+    # the two launches have 512 and 256 threads, so their fp32 norms add up in different orders
+    assert torch.allclose(A.acc, B.acc, rtol=1e-6, atol=0) and torch.equal(B.host, B.acc.cpu())
