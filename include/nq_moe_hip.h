@@ -304,6 +304,21 @@ int nq_pf_hits(const int32_t* counts, int32_t* hits, int E, void* stream);
 int nq_viterbi(const float* w, int T, int L, int K, const float* lut, int64_t* states, void* scratch, int64_t scratch_bytes,
                int position_order, void* stream);
 
+/* The same for plane P4 of the interleaved two-plane level 4 with plane P3 frozen: L <= 256 steps of one bit with eight steps of memory,
+ * values lut[spread(a) | spread(b) << 1]; a int64 [T][L]: P3's windows (low eight bits used), b int64 [T][L]: P4's windows. */
+int nq_viterbi_p4(const float* w, const int64_t* a, int T, int L, const float* lut, int64_t* b, int position_order, void* stream);
+
+/* Encoder: one refinement stage on a frozen base plane, units of 16 x 128 weights as 8 rings of 256 in ring position order
+ * (reference nq_encode.py:186-198,286-316). target fp32 [U][8][256]; sign fp32 [U][8] (+-1 per ring, NULL = +1); st_base, st_res int64
+ * [U][8][256] states; lut fp32 [65536] codebook.
+ * nq_fit_residual: out fp32 [U][8][256] = r / (rms(r) / scale), r = target * sign - lut[st_base] in fp64, rms per unit.
+ * nq_fit_words: delta fp64 [U] = least-squares step size; of the twelve block words around it the first of least cost -> Mb, N int64
+ * [U], and the decoded values Q fp32 [U][8][256]. Cost of an error E (16 x 128): sum of squares (Da NULL), or tr(Do E Da E^T) with
+ * Da fp64 [128][128] and Do fp64 [16][16] (NULL = identity) of unit u at Da + u * da_step, Do + u * do_step. ws: 144 bytes per unit. */
+int nq_fit_residual(const float* target, const float* sign, const int64_t* st_base, const float* lut, double scale, int U, float* out, void* stream);
+int nq_fit_words(const float* target, const float* sign, const int64_t* st_base, const int64_t* st_res, const float* lut, int U, const double* Da, int64_t da_step,
+                 const double* Do, int64_t do_step, void* ws, int64_t ws_bytes, float* Q, int64_t* Mb, int64_t* N, double* delta, void* stream);
+
 /* ---- Refinement-record upgrade engine (host threads + one side stream; replaces the class Engine of the reference's
  * streaming/nqstream.cu:51-277 and its Python surface, :8-26). One engine per record file (one rank) and GPU. Unlike the
  * entry points above, an engine owns memory for its lifetime: n_host pinned host entries of rec_bytes each (bounce

@@ -335,3 +335,31 @@ extern "C" int nq_pf_step(const NqPfArgs* p, void* stream)
     for (int i = 0; i < 4; ++i) NQ_REQUIRE(a.events[i], "nq_pf_step: four events");
     return launch_pf_step(a, (hipStream_t)stream);
 }
+
+extern "C" int nq_fit_residual(const float* target, const float* sign, const int64_t* st_base, const float* lut, double scale, int U, float* out, void* stream)
+{
+    NQ_REQUIRE(U >= 0 && scale > 0, "nq_fit_residual: U=%d scale=%g", U, scale);
+    if (U == 0) return 0;
+    NQ_REQUIRE(target && st_base && lut && out, "nq_fit_residual: null pointer");
+    return launch_fit_residual(target, sign, st_base, lut, scale, U, out, (hipStream_t)stream);
+}
+
+extern "C" int nq_fit_words(const float* target, const float* sign, const int64_t* st_base, const int64_t* st_res, const float* lut, int U, const double* Da, int64_t da_step,
+                            const double* Do, int64_t do_step, void* ws, int64_t ws_bytes, float* Q, int64_t* Mb, int64_t* N, double* delta, void* stream)
+{
+    NQ_REQUIRE(U >= 0 && U <= 65535, "nq_fit_words: U=%d (at most 65535 units a call)", U);
+    if (U == 0) return 0;
+    NQ_REQUIRE(target && st_base && st_res && lut && ws && Q && Mb && N && delta, "nq_fit_words: null pointer");
+    NQ_REQUIRE(Da || !Do, "nq_fit_words: a row metric goes with a column metric");
+    NQ_REQUIRE((da_step == 0 || da_step >= 128 * 128) && (do_step == 0 || do_step >= 256), "nq_fit_words: metric steps %lld, %lld", (long long)da_step, (long long)do_step);
+    NQ_REQUIRE(aligned16(ws) && ws_bytes >= (int64_t)U * 12 * 12, "nq_fit_words: ws needs 144 bytes per unit, 16-byte aligned");
+    return launch_fit_words(target, sign, st_base, st_res, lut, U, Da, da_step, Do, do_step, ws, Q, Mb, N, delta, (hipStream_t)stream);
+}
+
+extern "C" int nq_viterbi_p4(const float* w, const int64_t* a, int T, int L, const float* lut, int64_t* b, int position_order, void* stream)
+{
+    NQ_REQUIRE(T >= 0 && L >= 1 && L <= 256, "nq_viterbi_p4: T=%d L=%d (1..256)", T, L);
+    if (T == 0) return 0;
+    NQ_REQUIRE(w && a && lut && b, "nq_viterbi_p4: null pointer");
+    return launch_viterbi_p4(w, a, T, L, lut, b, position_order != 0, (hipStream_t)stream);
+}

@@ -70,6 +70,10 @@ int launch_pf_gemm(const int64_t* table, const int32_t* tiles, int ntiles, int b
                    int E, int H, int I, const void* Wop, hipStream_t st);
 int launch_pf_step(const ::NqPfArgs& a, hipStream_t st);
 int64_t pf_meta_bytes(int P, int R, int E);
+int launch_fit_residual(const float* target, const float* sign, const int64_t* st_base, const float* lut, double scale, int U, float* out, hipStream_t st);
+int launch_fit_words(const float* target, const float* sign, const int64_t* st_base, const int64_t* st_res, const float* lut, int U, const double* Da, int64_t da_step,
+                     const double* Do, int64_t do_step, void* ws, float* Q, int64_t* Mb, int64_t* N, double* delta, hipStream_t st);
+int launch_viterbi_p4(const float* w, const int64_t* a, int T, int L, const float* lut, int64_t* b, int rev, hipStream_t s);
 int launch_viterbi(const float* w, int T, int L, int K, const float* lut, int64_t* st, uint32_t* back, int slots, int rev, hipStream_t s);
 
 }  // namespace nq

@@ -24,6 +24,15 @@ struct VitArgs { const float* w; const float* lut; int64_t* st; uint32_t* back; 
 // all wavefronts' LDS accesses so far are done; stores to global memory stay in flight (a __syncthreads would wait for them)
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
+// word = word << 1 | this lane's bit of the mask. A mask straight from a comparison needs two wait states before a vector
+// instruction reads it (the compiler does not see into the asm); one that the scalar unit has combined does not.
+template <bool FROM_CMP>
+__device__ __forceinline__ void push_bit(uint32_t& word, unsigned long long mask)
+{
+    if constexpr (FROM_CMP) asm("s_nop 1\n\tv_addc_co_u32 %0, vcc, %0, %0, %1" : "+v"(word) : "s"(mask) : "vcc");
+    else asm("v_addc_co_u32 %0, vcc, %0, %0, %1" : "+v"(word) : "s"(mask) : "vcc");
+}
+
 // one step of the search: costs cur -> nxt (K = 1: the same array), decisions -> the returned word
 template <int K>
 __device__ __forceinline__ uint32_t vit_step(const float (&v)[64 >> (2 * K)][1 << K][1 << K], float wv, const float* cur, float* nxt, int t)
@@ -50,15 +59,22 @@ __device__ __forceinline__ uint32_t vit_step(const float (&v)[64 >> (2 * K)][1 <
                 const float d = v[r][j][q] - wv;
                 x[q] = __builtin_bit_cast(uint32_t, d * d + c[r][q]);
             }
-            uint32_t i;
+            // The decision is the first candidate that equals the minimum. Comparisons leave lane masks in scalar registers, the
+            // scalar unit combines them, and an add with carry shifts a mask's bit into the word: one vector instruction per bit.
             if constexpr (K == 2)
             {
-                const uint32_t m01 = x[1] < x[0] ? x[1] : x[0], m23 = x[3] < x[2] ? x[3] : x[2];
-                const uint32_t i01 = x[1] < x[0] ? 1u : 0u, i23 = x[3] < x[2] ? 3u : 2u;
-                m[j] = m23 < m01 ? m23 : m01; i = m23 < m01 ? i23 : i01;
+                const uint32_t m23 = x[3] < x[2] ? x[3] : x[2];
+                uint32_t mm;
+                asm("v_min3_u32 %0, %1, %2, %3" : "=v"(mm) : "v"(x[0]), "v"(x[1]), "v"(m23));
+                const unsigned long long e0 = __builtin_amdgcn_uicmp(x[0], mm, 33), e1 = __builtin_amdgcn_uicmp(x[1], mm, 33), e2 = __builtin_amdgcn_uicmp(x[2], mm, 33);   // 33: not equal
+                push_bit<false>(word, e0 & e1); push_bit<false>(word, e0 & (~e1 | e2));
+                m[j] = mm;
             }
-            else { m[j] = x[1] < x[0] ? x[1] : x[0]; i = x[1] < x[0] ? 1u : 0u; }
-            word |= i << (K * (r * Q + j));
+            else
+            {
+                push_bit<true>(word, __builtin_amdgcn_uicmp(x[1], x[0], 36));                                      // 36: less
+                m[j] = x[1] < x[0] ? x[1] : x[0];
+            }
         }
         asm volatile("" : "+v"(word));                           // one group at a time: mixing them would not fit the registers
         __builtin_amdgcn_sched_barrier(0);
@@ -94,7 +110,7 @@ __device__ __forceinline__ int vit_trace(const uint32_t* back, int hi, int edge,
             for (int s = 0; s < ROWS && top - s >= 0; ++s)
             {
                 const int g = edge >> K;
-                const uint32_t q = (buf[s * VT + (g & 1023)] >> (K * ((g >> 10) * Q + (edge & (Q - 1))))) & (Q - 1);
+                const uint32_t q = (buf[s * VT + (g & 1023)] >> (32 - K - K * ((g >> 10) * Q + (edge & (Q - 1))))) & (Q - 1);   // first pushed = highest
                 const int st = (int)(q << KR) | edge;
                 sl[top - s] = st;
                 edge = st >> K;
@@ -188,6 +204,111 @@ int launch_viterbi(const float* w, int T, int L, int K, const float* lut, int64_
     if (e != hipSuccess) return set_error("nq_viterbi: LDS %d bytes: %s", shm, hipGetErrorString(e));
     kern<<<T < slots ? T : slots, VT, shm, s>>>(a);
     NQ_LAUNCH_CHECK("nq_viterbi");
+    return 0;
+}
+
+// ---- the second plane of the interleaved two-plane level 4, with the first one frozen (encode.viterbi_ring_given_p3) -------------
+// State b: eight bits of plane P4, one new bit per step; the value at step t is lut[spread(a_t) | spread(b) << 1] with P3's eight bits
+// a_t. 128 edges: one wavefront per ring, lane l owns edges 2 l and 2 l + 1, which share the predecessors l and 64 + l. Costs pass
+// through LDS (256 words per wavefront), decisions are two lane masks per step, kept in LDS for the walk back. The four codebook
+// values of a step do not depend on the search and are requested two steps ahead. Bound by the latency of one step's chain (LDS
+// round trip, three fp32 operations, one selection), so the rings' number counts, not their length.
+constexpr int P4_L = 256, P4_WAVES = 4;
+struct VitP4Args { const float* w; const int64_t* a; const float* lut; int64_t* b; int T, L, rev; };
+
+__device__ __forceinline__ uint32_t spread8(uint32_t v)          // bit i -> bit 2 i
+{
+    v = (v | (v << 4)) & 0x0F0Fu; v = (v | (v << 2)) & 0x3333u;
+    return (v | (v << 1)) & 0x5555u;
+}
+__global__ void __launch_bounds__(64 * P4_WAVES) nq_viterbi_p4_k(VitP4Args A)
+{
+    __shared__ float cost_s[P4_WAVES][2][128];
+    __shared__ unsigned long long back_s[P4_WAVES][P4_L][2];
+    __shared__ float w_s[P4_WAVES][P4_L];
+    __shared__ unsigned short sa_s[P4_WAVES][P4_L];
+    __shared__ unsigned char b_s[P4_WAVES][P4_L];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, L = A.L, ring = blockIdx.x * P4_WAVES + wv;
+    if (ring >= A.T) return;                                     // wave-uniform; nothing below crosses wavefronts
+    auto sync = [] { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); __builtin_amdgcn_wave_barrier(); };
+    for (int i = lane; i < L; i += 64)
+    {
+        const size_t at = (size_t)ring * L + (A.rev ? (L - i) % L : i);
+        w_s[wv][i] = A.w[at]; sa_s[wv][i] = (unsigned short)spread8((uint32_t)A.a[at] & 0xFFu);
+    }
+    uint32_t sb[2][2];                                           // [edge][choice]
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) sb[j][q] = spread8((uint32_t)((q << 7) | (2 * lane + j))) << 1;
+    sync();
+    int start = -1;
+    for (int pass = 0; pass < 2; ++pass)
+    {
+        const int roll = pass == 0 ? L / 2 : 0;
+        float* c0 = cost_s[wv][0]; float* c1 = cost_s[wv][1];
+        c0[2 * lane] = pass == 0 || 2 * lane == start ? 0.f : __builtin_inff();
+        c0[2 * lane + 1] = pass == 0 || 2 * lane + 1 == start ? 0.f : __builtin_inff();
+        auto row = [&](int i) { return i + roll < L ? i + roll : i + roll - L; };
+        float v[3][2][2];
+        auto fetch = [&](int i, float (&d)[2][2]) {
+            const uint32_t sa = sa_s[wv][row(i < L ? i : L - 1)];
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int q = 0; q < 2; ++q) d[j][q] = A.lut[sa | sb[j][q]];
+        };
+        fetch(0, v[0]); fetch(1, v[1]);
+        for (int i = 0; i < L; ++i)
+        {
+            sync();
+            const int ri = row(i);
+            fetch(i + 2, v[2]);
+            const float w = w_s[wv][ri], p0 = c0[lane], p1 = c0[64 + lane];
+            float m[2]; bool hi[2];
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+            {
+                const float d0 = v[0][j][0] - w, d1 = v[0][j][1] - w;
+                const float x0 = d0 * d0 + p0, x1 = d1 * d1 + p1;
+                hi[j] = x1 < x0; m[j] = hi[j] ? x1 : x0;
+            }
+            *(float2*)(c1 + 2 * lane) = make_float2(m[0], m[1]);
+            const unsigned long long b0 = __ballot(hi[0]), b1 = __ballot(hi[1]);
+            if (lane == 0) { back_s[wv][ri][0] = b0; back_s[wv][ri][1] = b1; }
+            float* t = c0; c0 = c1; c1 = t;
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int q = 0; q < 2; ++q) { v[0][j][q] = v[1][j][q]; v[1][j][q] = v[2][j][q]; }
+        }
+        sync();
+        int edge = start;
+        if (pass == 0)
+        {   // the cheapest edge after the last step, the smallest of equals
+            const float e0 = c0[2 * lane], e1 = c0[2 * lane + 1];
+            unsigned long long best = ((unsigned long long)__builtin_bit_cast(uint32_t, e1 < e0 ? e1 : e0) << 32) | (unsigned)(2 * lane + (e1 < e0 ? 1 : 0));
+#pragma unroll
+            for (int k = 32; k; k >>= 1) { const unsigned long long o = __shfl_xor(best, k); best = o < best ? o : best; }
+            edge = (int)(best & 0xFFFFFFFFu);
+        }
+        for (int r = pass == 0 && L > 1 ? roll - 1 : L - 1; r >= 0; --r)          // every lane walks the same way
+        {
+            const int q = (int)(back_s[wv][r][edge & 1] >> (edge >> 1)) & 1, st = (q << 7) | edge;
+            if (lane == 0) b_s[wv][r] = (unsigned char)st;
+            edge = st >> 1;
+        }
+        start = edge;
+        sync();
+    }
+    for (int i = lane; i < L; i += 64) A.b[(size_t)ring * L + (A.rev ? (L - i) % L : i)] = b_s[wv][i];
+}
+
+int launch_viterbi_p4(const float* w, const int64_t* a, int T, int L, const float* lut, int64_t* b, int rev, hipStream_t s)
+{
+    const VitP4Args A{w, a, lut, b, T, L, rev};
+    nq_viterbi_p4_k<<<(T + P4_WAVES - 1) / P4_WAVES, 64 * P4_WAVES, 0, s>>>(A);
+    NQ_LAUNCH_CHECK("nq_viterbi_p4");
     return 0;
 }
 

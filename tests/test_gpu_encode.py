@@ -30,3 +30,58 @@ def test_viterbi_ties_on_a_coarse_codebook():
     w = torch.randint(-3, 4, (4, 64), generator=g).float()
     for K in (1, 2):
         assert torch.equal(EN.viterbi_ring(w.cuda(), lut.cuda(), K).cpu(), EN.viterbi_ring(w, lut, K))
+
+
+@pytest.mark.parametrize("T,L", [(1, 256), (5, 256), (3, 1), (2, 2), (9, 16), (4, 77)])
+def test_second_plane_search_equals_the_torch_form(T, L):
+    """plane P4 with P3 frozen: a partly filled last workgroup, rings of one step up, equal costs"""
+    g = torch.Generator().manual_seed(T * 1000 + L)
+    w = torch.randn(T, L, generator=g)
+    w[::2] = w[::2].round()
+    a = torch.randint(0, 256, (T, L), generator=g)
+    for lut in (EN.codebook(), EN.codebook().round().clamp(-2, 2)):
+        assert torch.equal(EN.viterbi_ring_given_p3(w.cuda(), a.cuda(), lut.cuda()).cpu(), EN.viterbi_ring_given_p3(w, a, lut))
+    if L == 256:
+        st3 = torch.randint(0, 1 << 16, (T, L), generator=g)
+        got, want = EN.viterbi_rings_given_p3(w.cuda(), st3.cuda()), EN.viterbi_rings_given_p3(w, st3)
+        assert all(torch.equal(p.cpu(), q) for p, q in zip(got, want))
+
+
+@pytest.mark.parametrize("U,K,signed,metric", [(1, 2, False, None), (5, 1, True, None), (7, 2, True, "columns"), (3, 1, False, "both"), (2, 2, True, "one")])
+def test_block_word_fit_equals_the_torch_form(U, K, signed, metric):
+    """a refinement stage with plain, column and two-sided cost on the GPU against the same stage in torch on the CPU: the trellis
+    targets may differ in the last bit (sums in another order), so states are given; words and values are then the same"""
+    g = torch.Generator().manual_seed(10 * U + K)
+    target = torch.randn(U, 8, 256, generator=g)
+    target[0] *= 1e-3
+    base = torch.randint(0, 1 << 16, (U, 8, 256), generator=g)
+    res = torch.randint(0, 1 << 16, (U, 8, 256), generator=g)
+    near = EN.codebook()[base] + 0.1 * torch.rand(U, 1, 1, generator=g) * EN.codebook()[res]      # a stage that has something to fit
+    target[-1] = near[-1]
+    sign = (torch.randint(0, 2, (U, 8, 1), generator=g) * 2 - 1).float() if signed else None
+    spd = lambda n, *b: (lambda X: X @ X.transpose(-1, -2) / n + torch.eye(n, dtype=torch.float64))(torch.randn(*b, n, n, generator=g, dtype=torch.float64))
+    Da = None if metric is None else spd(128) if metric == "one" else spd(128, U)
+    Do = spd(16, U) if metric == "both" else None
+
+    def cost(E):
+        idx = EN.ring_index().reshape(-1)
+        X = torch.empty(U, 2048, dtype=torch.float64); X[:, idx] = E.reshape(U, 2048)
+        X = X.reshape(U, 128, 16).transpose(1, 2)
+        Y = X @ Da
+        return ((Y if Do is None else Do @ Y) * X).sum((1, 2))
+    want = EN.encode_residual(target, base, K, sign=sign, states=res, cost=None if Da is None else cost)
+    dev = lambda t: None if t is None else t.cuda()
+    got = EN.encode_residual(target.cuda(), base.cuda(), K, sign=dev(sign), states=res.cuda(), metric=None if Da is None else (Da.cuda(), dev(Do)))
+    for k in ("Mb", "N", "Q"):
+        assert torch.equal(got[k].cpu(), want[k]), k
+    assert torch.allclose(got["delta"].cpu(), want["delta"], rtol=1e-12)
+    # the targets of the stage's own search
+    lut = EN.codebook()
+    r = (target if sign is None else target * sign).double() - lut[base].double()
+    s0 = r.square().mean((1, 2)).sqrt().clamp_min(1e-12) / 1.1
+    out = torch.empty_like(target, device="cuda")
+    from nestquant_amd import _lib
+    args = [t if t is None else t.cuda().contiguous() for t in (target, sign, base, lut)]
+    _lib.check(_lib.lib().nq_fit_residual(*[None if t is None else t.data_ptr() for t in args], 1.1, U, out.data_ptr(), None))
+    torch.cuda.synchronize()
+    assert torch.allclose(out.cpu(), (r / s0[:, None, None]).float(), rtol=2e-7, atol=0)
