@@ -11,8 +11,10 @@
 // pass, reads 2^K costs per group from LDS and writes 2^K. Both directions of that traffic are free of bank conflicts. The
 // decisions of a thread in one step (16 edges x 2 bits, or 32 x 1) fill one word, stored to a scratch of 4 KB per step; the way
 // back is walked by one lane over blocks of steps brought to LDS, the next block in flight.
-// Bound: vector-instruction issue. A step is 65536 candidates of three fp32 operations plus the selection, ~21 instructions per
-// four candidates (K = 2) = 340 per wavefront; with sixteen wavefronts per CU, one ring per CU.
+// Bound: instruction issue of sixteen wavefronts in lockstep. A step is 65536 candidates of three fp32 operations plus the selection,
+// 19 vector instructions per four candidates (K = 2) = 309 per wavefront; one ring per CU. Measured: 935 us for 256 rings (K = 2;
+// 1.6 us per step, the walks back ~100 us), 1160 us (K = 1, whose single array costs a second barrier); with all wavefronts at one
+// priority 1060 and 1230.
 #include "nq_host.hpp"
 
 namespace nq {
@@ -33,6 +35,16 @@ __device__ __forceinline__ void push_bit(uint32_t& word, unsigned long long mask
     else asm("v_addc_co_u32 %0, vcc, %0, %0, %1" : "+v"(word) : "s"(mask) : "vcc");
 }
 
+// Wavefronts lower their priority as they get on with a step: the arbiter otherwise serves the oldest first, and a step ends with
+// the youngest wavefront of every SIMD alone, which cannot issue more than one instruction in six clocks.
+__device__ __forceinline__ void step_priority(int quarter)
+{
+    if (quarter == 0) __builtin_amdgcn_s_setprio(3);
+    else if (quarter == 1) __builtin_amdgcn_s_setprio(2);
+    else if (quarter == 2) __builtin_amdgcn_s_setprio(1);
+    else __builtin_amdgcn_s_setprio(0);
+}
+
 // one step of the search: costs cur -> nxt (K = 1: the same array), decisions -> the returned word
 template <int K>
 __device__ __forceinline__ uint32_t vit_step(const float (&v)[64 >> (2 * K)][1 << K][1 << K], float wv, const float* cur, float* nxt, int t)
@@ -48,6 +60,7 @@ __device__ __forceinline__ uint32_t vit_step(const float (&v)[64 >> (2 * K)][1 <
 #pragma unroll
     for (int r = 0; r < R; ++r)
     {
+        step_priority(4 * r / R);
         uint32_t m[Q];
 #pragma unroll
         for (int j = 0; j < Q; ++j)
@@ -64,8 +77,7 @@ __device__ __forceinline__ uint32_t vit_step(const float (&v)[64 >> (2 * K)][1 <
             if constexpr (K == 2)
             {
                 const uint32_t m23 = x[3] < x[2] ? x[3] : x[2];
-                uint32_t mm;
-                asm("v_min3_u32 %0, %1, %2, %3" : "=v"(mm) : "v"(x[0]), "v"(x[1]), "v"(m23));
+                const uint32_t m01 = x[1] < x[0] ? x[1] : x[0], mm = m23 < m01 ? m23 : m01;            // one three-way minimum
                 const unsigned long long e0 = __builtin_amdgcn_uicmp(x[0], mm, 33), e1 = __builtin_amdgcn_uicmp(x[1], mm, 33), e2 = __builtin_amdgcn_uicmp(x[2], mm, 33);   // 33: not equal
                 push_bit<false>(word, e0 & e1); push_bit<false>(word, e0 & (~e1 | e2));
                 m[j] = mm;
