@@ -94,8 +94,8 @@ struct alignas(64) RunHdr
     int level, ntok;
     int had;                      // width of the Hadamard on the down projection's input: 128 or 512
     int rg, rd;
-    int q0;                       // rotated activations of the run's token j: row q0 + j of MoeArgs::xrot
-    unsigned char slot[MAXTOK];   // pick index (token * topk + k) of the run's tokens
+    int pad;
+    unsigned char slot[MAXTOK];   // pick index (token * topk + k) of the run's tokens: their row of MoeArgs::xrot and of the partial sums
     __device__ __forceinline__ int slot_of(int j) const       // by shifts: a run-time index into slot[] would put the header into scratch memory
     {
         unsigned long long v;
@@ -124,34 +124,56 @@ __device__ __forceinline__ void ld_sys_row(const int64_t* p, int64_t* f)
 }
 
 // ---- routing dedup: picks -> runs (refined experts first, then by first occurrence); slots in pick order ----------------
-// One wavefront per workgroup of nq_prep_k; lane s owns pick s (S <= 64). A run takes at most one pick per token: a token
-// that names the same expert twice opens a second run of that expert, so a run never has more than B tokens. Every lane
-// requests all fields of its own pick's table row together, so the leader's fields cost no second round trip. The routing
-// reads the table and nothing else: no kernel writes the table while a routing launch runs (the mailbox of a call is applied
-// by its last projection launch, see mailbox_apply), so every workgroup of the launch sees the same rows and the rows cannot
-// be torn.
-struct PrepRows { int nq; unsigned char tok[64]; const _Float16* signs[64]; };    // LDS: the rows of xrot, one per active pick
-__device__ __forceinline__ void route(const MoeArgs& a, RouteWs* W, int lane, bool writer, PrepRows* Q)
+// One wavefront; lane s owns pick s (S <= 64). A run takes at most one pick per token: a token that names the same expert twice
+// opens a second run of that expert, so a run never has more than B tokens. Every lane requests all fields of its own pick's table
+// row together, so the leader's fields cost no second round trip. The routing reads the table and nothing else: no kernel writes
+// the table while a routing launch runs (the mailbox of a call is applied by its last projection launch, see mailbox_apply), so
+// every workgroup of the launch sees the same rows and the rows cannot be torn.
+struct PrepRows { int nq; unsigned char pick[64]; const _Float16* signs[64]; };   // LDS: the active picks, in order
+__device__ __forceinline__ bool pick_expert(const MoeArgs& a, int lane, int& e)
+{
+    if (lane >= a.B * a.topk) return false;
+    const long long ee = sel_at(a, lane);
+    if (ee < 0 || ee >= a.E) return false;
+    e = (int)ee;
+    return true;
+}
+// What a workgroup of the rotation needs: the active picks and their sign vectors, no numbering of runs.
+__device__ __forceinline__ void list_picks(const MoeArgs& a, int lane, PrepRows* Q)
+{
+    int e = 0, lv = 0; const _Float16* sg = nullptr;
+    bool ok = false;
+    if (pick_expert(a, lane, e))
+    {
+        const int64_t* ent = a.table + (size_t)e * TBL_W;
+        lv = (int)ent[0]; sg = (const _Float16*)ent[9];
+        ok = rw_at(a, lane) != 0.f && lv > 0;
+    }
+    const unsigned long long okm = __ballot(ok);
+    if (ok)
+    {
+        const int q = __popcll(okm & ((1ull << lane) - 1ull));
+        Q->pick[q] = (unsigned char)lane; Q->signs[q] = sg;
+    }
+    if (lane == 0) Q->nq = __popcll(okm);
+}
+__device__ __forceinline__ void route(const MoeArgs& a, RouteWs* W, int lane)
 {
     const int S = a.B * a.topk;
-    int e = -1, lv = 0; bool ok = false, inrange = false;
+    int e = -1, lv = 0; bool ok = false;
+    const bool inrange = pick_expert(a, lane, e);
     int64_t f[TBL_W];
 #pragma unroll
     for (int i = 0; i < TBL_W; ++i) f[i] = 0;
-    if (lane < S)
+    if (inrange)
     {
-        const long long ee = sel_at(a, lane);
-        if (ee >= 0 && ee < a.E)
-        {
-            e = (int)ee; inrange = true;
-            const int64_t* ent = a.table + (size_t)e * TBL_W;
+        const int64_t* ent = a.table + (size_t)e * TBL_W;
 #pragma unroll
-            for (int i = 0; i < TBL_W; ++i) f[i] = ent[i];
-            lv = (int)f[0];
-            ok = rw_at(a, lane) != 0.f && lv > 0;
-        }
+        for (int i = 0; i < TBL_W; ++i) f[i] = ent[i];
+        lv = (int)f[0];
+        ok = rw_at(a, lane) != 0.f && lv > 0;
     }
-    if (writer && a.hits && inrange && rw_at(a, lane) != 0.f)
+    if (a.hits && inrange && rw_at(a, lane) != 0.f)
         __hip_atomic_fetch_add(a.hits + e, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     const int level = a.force_level ? a.force_level : lv;
     // Runs of refined experts (level 3, 4: twice the decode work per chunk) are numbered before the level-2 ones, each group
@@ -162,27 +184,36 @@ __device__ __forceinline__ void route(const MoeArgs& a, RouteWs* W, int lane, bo
     const unsigned long long below = (1ull << lane) - 1ull;
     const int tok = lane / a.topk, sh = tok * a.topk;
     const unsigned long long mytok = sh < 64 ? (a.topk >= 64 ? ~0ull : ((1ull << a.topk) - 1ull)) << sh : 0ull;
-    int r = 0, cum = 0;
-    int my_run = -1, my_pos = 0, my_ntok = 0, my_q0 = 0;         // the run this lane's pick went into, its place there; for the first lane of a run: its size
-    for (int pass = 0; pass < 2; ++pass)
+    int r = 0;
+    int my_run = -1, my_pos = 0, my_ntok = 0;                    // the run this lane's pick went into, its place there, the run's size
+    unsigned long long eq = 0ull;                                // the active picks of this lane's expert
+#pragma unroll 4
+    for (int j = 0; j < S; ++j)
     {
-        unsigned long long rem = pass == 0 ? heavy : okm & ~heavy;
-        while (rem)
-        {
-            const int leader = __ffsll((long long)rem) - 1;
-            const int ev = __shfl(e, leader);
-            const unsigned long long same = __ballot(((rem >> lane) & 1ull) && e == ev);
-            const unsigned long long m = __ballot(((same >> lane) & 1ull) && (same & mytok & below) == 0ull);   // first pick per token
-            if ((m >> lane) & 1ull)
-            {
-                my_run = r; my_pos = __popcll(m & below); my_ntok = __popcll(m); my_q0 = cum;
-                Q->tok[cum + my_pos] = (unsigned char)tok; Q->signs[cum + my_pos] = (const _Float16*)f[9];
-            }
-            rem &= ~m; ++r; cum += __popcll(m);
-        }
+        const unsigned long long m = __ballot(ok && e == __builtin_amdgcn_readlane(e, j));
+        eq = lane == j ? m : eq;
     }
-    if (lane == 0) Q->nq = cum;
-    if (!writer) return;
+    if (__ballot(ok && (eq & mytok & below)) == 0ull)
+    {   // no token names an expert twice: a run is an expert, and all are numbered at once (one after the other, thirty runs took 5 us)
+        const unsigned long long first = __ballot(ok && (eq & below) == 0ull), fh = first & heavy, fl = first & ~heavy;
+        const int mine = ((heavy >> lane) & 1ull) ? __popcll(fh & below) : __popcll(fh) + __popcll(fl & below);
+        const int run = __shfl(mine, eq ? __ffsll((long long)eq) - 1 : lane);
+        if (ok) { my_run = run; my_pos = __popcll(eq & below); my_ntok = __popcll(eq); }
+        r = __popcll(first);
+    }
+    else
+        for (int pass = 0; pass < 2; ++pass)
+        {
+            unsigned long long rem = pass == 0 ? heavy : okm & ~heavy;
+            while (rem)
+            {
+                const int ev = __builtin_amdgcn_readlane(e, __ffsll((long long)rem) - 1);
+                const unsigned long long same = __ballot(((rem >> lane) & 1ull) && e == ev);
+                const unsigned long long m = __ballot(((same >> lane) & 1ull) && (same & mytok & below) == 0ull);   // first pick per token
+                if ((m >> lane) & 1ull) { my_run = r; my_pos = __popcll(m & below); my_ntok = __popcll(m); }
+                rem &= ~m; ++r;
+            }
+        }
     // the headers, after the numbering: every lane holds its own pick's row, so the first lanes of all runs write their runs'
     // headers side by side (inside the loop above the same stores would be issued once per run, one lane at a time)
     if (my_run >= 0)
@@ -201,7 +232,7 @@ __device__ __forceinline__ void route(const MoeArgs& a, RouteWs* W, int lane, bo
                 R.level = level;
                 R.had = f[18] == 512 ? 512 : 128;
                 R.lr = (const _Float16*)f[14]; R.lr4 = (const _Float16*)f[15]; R.rg = (int)f[16]; R.rd = (int)f[17];
-                R.ntok = my_ntok; R.q0 = my_q0;
+                R.ntok = my_ntok;
             }
         }
     }
@@ -246,42 +277,46 @@ __device__ __forceinline__ void publish_applied(const int32_t* applied, int32_t*
         __hip_atomic_store(applied_host + e, applied[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// First launch of every layer call. Every workgroup repeats the routing (its first wavefront; workgroup 0 writes the result:
-// run headers for both projection launches, which then read one header each instead of repeating the dependent loads
-// sel -> table row in every one of their ~1800 workgroups, the per-pick data of the combine, the hits export); then the
-// wavefronts of the grid share the rotation of the activations: one task per (active pick q, gate or up, 128-column chunk):
-// xrot[q][gate|up][chunk] = fp16(Hadamard-128(x[token] * su)) in the MFMA B-operand column order, which the gate|up launch
-// copies into LDS (before, each of the 32 row blocks of a run repeated these rotations: 9 % of the launch's vector
-// instructions). With a mailbox in the call the other three wavefronts of workgroup 0 first publish what earlier calls applied
-// (publish_applied); nothing here reads seq or stage and nothing writes the table. With salience in the call one more workgroup
-// exports it beside the others (a launch of its own in front of the call cost 9 us at one token, 20 us at four).
+// First launch of every layer call. Workgroup 0 does the routing: run headers for both projection launches, which then read one
+// header each instead of repeating the dependent loads sel -> table row in every one of their ~1800 workgroups, the per-pick
+// data of the combine, the hits export; with a mailbox in the call its other three wavefronts publish what earlier calls applied
+// (publish_applied). Nothing here reads seq or stage and nothing writes the table. With salience in the call workgroup 1 exports
+// it (a launch of its own in front of the call cost 9 us at one token, 20 us at four). All others rotate the activations, one
+// task per (active pick, gate or up, 128-column chunk): xrot[pick][gate|up][chunk] = fp16(Hadamard-128(x[token] * su)) in the
+// MFMA B-operand column order, which the gate|up launch copies into LDS; rows are numbered by pick, so a rotating workgroup
+// needs the list of active picks but not the runs.
+// Bound by latency: three dependent round trips (sel, table row, sign vector and activations) in either branch; 5.2 us at one
+// token, 7.3 us at four with salience (15 us while every workgroup numbered the runs, one after the other, and a single wavefront
+// walked all tokens for the salience).
 __global__ void __launch_bounds__(256) nq_prep_k(MoeArgs a)
 {
     __shared__ PrepRows Q;
     const int lane = threadIdx.x & 63;
-    const int nblk = (int)gridDim.x - (a.sal_acc ? 1 : 0);       // the last workgroup of a call with salience does that and nothing else
-    if ((int)blockIdx.x == nblk)
+    const int extra = a.sal_acc ? 2 : 1;                         // workgroup 0 routes; 1 exports the salience of a call that asks for it
+    if (a.sal_acc && blockIdx.x == 1)
     {
         __shared__ SalShared S;
         const SalArgs sa{a.x, a.H, a.rw, a.sel, a.B, a.H, a.topk, a.E, a.x_dtype, a.rw_dtype, a.sel_dtype, a.sal_rsf, a.sal_acc, a.sal_host};
         salience<4>(sa, &S);
         return;
     }
-    if (threadIdx.x < 64) route(a, a.route, lane, blockIdx.x == 0, &Q);
-    else if (blockIdx.x == 0 && a.mb_table && a.mb_applied_host) publish_applied(a.mb_applied, a.mb_applied_host, a.E, threadIdx.x - 64, 192);
-    __syncthreads();
-    // workgroup 0 has the result to write (it ends ~1 us after the others' routing): with more than one workgroup in the grid the
-    // rotation tasks go to the others, so that it is not also the last to finish
-    const int C = a.H / 128, ntask = Q.nq * 2 * C, nrot = nblk > 1 ? nblk - 1 : 1, rot = nblk > 1 ? (int)blockIdx.x - 1 : 0;
-    if (rot < 0) return;
-    for (int t = rot * 4 + (threadIdx.x >> 6); t < ntask; t += nrot * 4)
+    if (blockIdx.x == 0)
     {
-        const int q = t / (2 * C), r = t - q * 2 * C, up = r / C, c = r - up * C, kk = c * 128 + 2 * lane;
+        if (threadIdx.x < 64) route(a, a.route, lane);
+        else if (a.mb_table && a.mb_applied_host) publish_applied(a.mb_applied, a.mb_applied_host, a.E, threadIdx.x - 64, 192);
+        return;
+    }
+    if (threadIdx.x < 64) list_picks(a, lane, &Q);
+    __syncthreads();
+    const int C = a.H / 128, ntask = Q.nq * 2 * C, nrot = (int)gridDim.x - extra;
+    for (int t = ((int)blockIdx.x - extra) * 4 + (threadIdx.x >> 6); t < ntask; t += nrot * 4)
+    {
+        const int q = t / (2 * C), r = t - q * 2 * C, up = r / C, c = r - up * C, kk = c * 128 + 2 * lane, pick = Q.pick[q];
         const _Float16* su = Q.signs[q] + (up ? 2 * a.H + 3 * a.I : 0);
-        const half2_t xv = x2_at(a, (size_t)Q.tok[q] * a.H + kk), sv = *(const half2_t*)(su + kk);
+        const half2_t xv = x2_at(a, (size_t)(pick / a.topk) * a.H + kk), sv = *(const half2_t*)(su + kk);
         float v0 = (float)xv.x * (float)sv.x, v1 = (float)xv.y * (float)sv.y;
         wht128(v0, v1, lane);
-        _Float16* dst = a.xrot + ((size_t)q * 2 + up) * a.H + c * 128;
+        _Float16* dst = a.xrot + ((size_t)pick * 2 + up) * a.H + c * 128;
         dst[bop_index(2 * lane)] = (_Float16)v0; dst[bop_index(2 * lane + 1)] = (_Float16)v1;
     }
 }
@@ -545,11 +580,11 @@ nq_gemv_k(MoeArgs a, int NC)
     {
         // rotated by nq_prep_k, already in B-operand order: 16 bytes per thread and step
         const bool up = (int)(blockIdx.x * SB * 32) >= a.I;      // gate rows were rotated with su_g, up rows with su_u
-        const _Float16* xr = a.xrot + ((size_t)R.q0 * 2 + (up ? 1 : 0)) * a.H + k0;
+        const _Float16* xr = a.xrot + (up ? a.H : 0) + k0;
         for (int i = threadIdx.x; i < ntok * NC * 16; i += blockDim.x)
         {
             const int j = i / (NC * 16), r = i - j * NC * 16;
-            *(u32x4*)(smem + j * rowstride + r * 16) = *(const u32x4*)(xr + (size_t)j * 2 * a.H + r * 8);
+            *(u32x4*)(smem + j * rowstride + r * 16) = *(const u32x4*)(xr + (size_t)R.slot_of(j) * 2 * a.H + r * 8);
         }
     }
     else if (a.fuse && R.had != 512 && R.lr == nullptr)
@@ -680,7 +715,7 @@ int launch_moe(const MoeArgs& a, const int* cfg_gu, const int* cfg_dn, int which
     if (!reuse)
     {
         const int ntask = S * 2 * (a.H / 128);                   // upper bound: every pick active
-        nq_prep_k<<<std::min((ntask + 3) / 4, 1023) + 1 + (a.sal_acc ? 1 : 0), 256, 0, st>>>(a);       // one workgroup per four rotation tasks, plus the writer
+        nq_prep_k<<<std::min((ntask + 3) / 4, 1023) + (a.sal_acc ? 2 : 1), 256, 0, st>>>(a);       // one workgroup per four rotation tasks, plus the one that routes
         NQ_LAUNCH_CHECK("moe_forward (routing)");
     }
     // a call with a mailbox and no projection launch: the apply half as a launch of its own (nothing is published here either)

@@ -242,7 +242,7 @@ __global__ void __launch_bounds__(256) nq_pf_mid_k(const float* __restrict__ acc
     }
 }
 
-// grid (T), block 256: out[t] (+)= sum over the token's picks whose pair row lies in [row_lo, row_lo + nrows) of
+// grid (T, column parts), block 256: out[t] (+)= sum over the token's picks whose pair row lies in [row_lo, row_lo + nrows) of
 // rw * sv_o (.) Hadamard(y[row]); pos[t][k] = row of pair (t, k) in the expert-sorted order; add: on top of what out holds (fp32),
 // else out is written whole, zeros included. One block owns a token, so
 // the sum needs no atomics and its order is fixed (the reference's pf_post adds with float atomics in arrival order).
@@ -282,7 +282,7 @@ __global__ void __launch_bounds__(256) nq_pf_post_k(const float* __restrict__ y,
     __syncthreads();
     const int np = p_n;
     if (np == 0 && add) return;
-    for (int grp = warp; grp < H / 128; grp += 4)
+    for (int grp = 4 * blockIdx.y + warp; grp < H / 128; grp += 4 * gridDim.y)
     {
         const int col = grp * 128 + 2 * lane;
         float o0 = 0.f, o1 = 0.f;
@@ -777,17 +777,21 @@ __global__ void __launch_bounds__(512) nq_pf_sort_k(PfSort a)
     const int tid = threadIdx.x, lane = tid & 63, E1 = a.E + 1;
     const bool one = a.P <= SORT_TILE;
     auto load = [&](int t0, bool count) {
-        for (int i = tid; i < SORT_TILE; i += 512)
+        for (int i0 = tid; i0 < SORT_TILE; i0 += 8 * 512)
         {
-            if (one && i >= ((a.P + 511) & ~511)) break;
-            int id = 0xFFFF;                                     // past the end: nobody's
-            if (t0 + i < a.P)
+            if (one && i0 - tid >= a.P) break;
+            long long e[8];                                      // eight ids in flight before the first is counted
+#pragma unroll
+            for (int u = 0; u < 8; ++u) e[u] = t0 + i0 + 512 * u < a.P ? id_at(a.sel, a.sdt, t0 + i0 + 512 * u) : -2;
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
             {
-                const long long e = id_at(a.sel, a.sdt, t0 + i);
-                id = e >= 0 && e < a.E ? (int)e : a.E;
-                if (count) atomicAdd(hist + id, 1);
+                const int i = i0 + 512 * u;
+                const bool in = t0 + i < a.P;
+                const int id = !in ? 0xFFFF : e[u] >= 0 && e[u] < a.E ? (int)e[u] : a.E;     // past the end: nobody's
+                if (count && in) atomicAdd(hist + id, 1);
+                ids[i] = (uint16_t)id;
             }
-            ids[i] = (uint16_t)id;
         }
     };
     for (int e = tid; e < E1; e += 512) hist[e] = 0;
@@ -874,7 +878,9 @@ int launch_pf_post(const float* y, const int32_t* pos, const void* sel, int sdt,
                    const int64_t* table, void* out, int odt, int add, const float* zd, int E, int H, int I, hipStream_t st)
 {
     if (!T || (!nrows && add)) return 0;
-    nq_pf_post_k<<<T, 256, 0, st>>>(y, pos, sel, sdt, rw, wdt, topk, row_lo, nrows, table, out, odt, add, zd, E, H, I);
+    // few tokens: several workgroups per token, about a thousand in all (48 tokens of 6144 columns: 43 us with one each, 9 with ten)
+    const int quads = (H / 128 + 3) / 4, parts = T >= 1024 ? 1 : quads < 1024 / T ? quads : 1024 / T;
+    nq_pf_post_k<<<dim3(T, parts), 256, 0, st>>>(y, pos, sel, sdt, rw, wdt, topk, row_lo, nrows, table, out, odt, add, zd, E, H, I);
     NQ_LAUNCH_CHECK("nq_pf_post");
     return 0;
 }

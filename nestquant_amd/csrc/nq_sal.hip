@@ -1,6 +1,6 @@
 // Decode salience export as a launch of its own (reference sm120/nqsal.cu:19-78, called at sm120/serve/nq_vllm.py:558,572): at most 8
 // tokens of 8 picks per call, no host synchronisation, static pointers, so the call can sit in a captured decode step. A layer
-// call can carry it in its routing launch instead (NqMoeArgs.with_salience), where it costs nothing: this launch is 6 us of
+// call can carry it in its routing launch instead (NqMoeArgs.with_salience), where it costs nothing: this launch is 5 us of
 // latency (9.4 us with one wavefront per token and the picks' sums as a chain of lane exchanges).
 #include "nq_sal.hpp"
 #include "nq_host.hpp"
