@@ -264,6 +264,10 @@ int nq_pf_post(const float* y, const int32_t* pos, const int64_t* sel, const voi
 int nq_pf_plan(const int32_t* counts, int E, int row_lo, int nrows, int32_t* tiles, int cap, int32_t* hot, int hot_min, int hot_cap,
                void* stream);
 
+/* out[i] = sum over y < ny of part[y * n + i] in slice order, fp32, n % 4 == 0: the k-slice partial sums that a gate|up call of one
+ * projection (which = 1 | 8) left in acc_gu, added up. */
+int nq_sum_slices(const float* part, int ny, int64_t n, float* out, void* stream);
+
 /* A whole step of T tokens on device data, no host synchronisation: pairs sorted by expert, tile plan, rotation, gate|up, SwiGLU,
  * down, combine -- the chain of the entry points above (reference moe.prefill, sm120/moe.py:282-326) with the casts of its caller
  * (x.half(), ids.long(), w.half(), out.to(dtype), sm120/serve/nq_vllm.py:522,573) at the loads and the final store. Ids outside

@@ -363,3 +363,11 @@ extern "C" int nq_viterbi_p4(const float* w, const int64_t* a, int T, int L, con
     NQ_REQUIRE(w && a && lut && b, "nq_viterbi_p4: null pointer");
     return launch_viterbi_p4(w, a, T, L, lut, b, position_order != 0, (hipStream_t)stream);
 }
+
+extern "C" int nq_sum_slices(const float* part, int ny, int64_t n, float* out, void* stream)
+{
+    NQ_REQUIRE(ny >= 1 && n >= 0 && n % 4 == 0, "nq_sum_slices: ny=%d n=%lld (a multiple of 4)", ny, (long long)n);
+    if (n == 0) return 0;
+    NQ_REQUIRE(part && out && aligned16(part) && aligned16(out), "nq_sum_slices: buffers must be given and 16-byte aligned");
+    return launch_sum_slices(part, ny, n, out, (hipStream_t)stream);
+}

@@ -800,6 +800,25 @@ int launch_moe_static(MoeArgs a, const int* cfg_gu, const int* cfg_dn, int which
     return launch_moe(a, cfg_gu, cfg_dn, which, st);
 }
 
+// out[i] = sum over the ny k-slices of part[y * n + i], in slice order (n a multiple of 4): what is left of a lone projection. Bound by
+// the launch: 24 slices of 8 x 4096 (3 MB, just written, so from the last-level cache) take 2.8 us where a library sum over the first
+// dimension took 5.4 us and chose its blocks on the host first; a projection of eight tokens 21.4 -> 19.3 us.
+__global__ void __launch_bounds__(256) nq_sum_slices_k(const float* __restrict__ part, int ny, int64_t n, float* __restrict__ out)
+{
+    const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (i >= n) return;
+    float4_t s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+    for (int y = 0; y < ny; ++y) s += *(const float4_t*)(part + y * n + i);
+    *(float4_t*)(out + i) = s;
+}
+int launch_sum_slices(const float* part, int ny, int64_t n, float* out, hipStream_t st)
+{
+    nq_sum_slices_k<<<(unsigned)((n / 4 + 255) / 256), 256, 0, st>>>(part, ny, n, out);
+    NQ_LAUNCH_CHECK("nq_sum_slices");
+    return 0;
+}
+
 // resident workgroups per CU, registers and spill bytes of a decode kernel for a launch shape
 int query_occ(int mode, int any_rows, int sb, int shm, int* out)
 {

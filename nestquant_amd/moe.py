@@ -562,4 +562,6 @@ def proj_gemv(layer, x, e=0, cfg=None):
     layer(x, layer._proj_in[1], layer._proj_in[2], which=1 | 8, cfg_gu=list(cfg))      # 8: the launch ends with its partial sums
     ny = C_ // (cfg[0] * cfg[2])
     n = 2 * layer.I                                               # partial sums are laid out [k-slice][B * topk of the call][2I]
-    return layer.acc_gu.view(-1)[: ny * B * n].view(ny, B, n).sum(0)
+    out = torch.empty(B, n, dtype=torch.float32, device=x.device)
+    _lib.check(layer.M.nq_sum_slices(layer.acc_gu.data_ptr(), ny, B * n, out.data_ptr(), _lib.stream_ptr()))
+    return out

@@ -247,3 +247,16 @@ def test_low_rank_plane_fitted_to_the_activations():
         assert e1 < 0.8 * e0, (level, e1, e0)
         print("low-rank plane, level %d: layer vs oracle %.1e; error against the unquantised expert %.4f with the plane, %.4f without" % (
             level, rel_err(y, want), e1, e0))
+
+
+@pytest.mark.parametrize("ny,n", [(1, 4), (3, 1020), (24, 1028), (9, 32768)])
+def test_sum_slices_adds_in_slice_order(ny, n):
+    """k-slice partial sums of a lone projection: one quad, a block less and more than one quad of threads, several blocks"""
+    from nestquant_amd import _lib
+    part = torch.randn(ny, n, generator=torch.Generator().manual_seed(n)).to(DEV)
+    out = torch.full((n + 4,), 7.0, device=DEV)
+    _lib.check(_lib.lib().nq_sum_slices(part.data_ptr(), ny, n, out.data_ptr(), _lib.stream_ptr()))
+    want = torch.zeros(n, device=DEV)
+    for y in range(ny):
+        want += part[y]
+    assert torch.equal(out[:n], want) and bool((out[n:] == 7.0).all())
