@@ -21,26 +21,6 @@ namespace nq {
 
 constexpr int PF_ROW = 256;                    // LDS bytes per staged token and chunk; 16-byte column q of row r sits in slot q ^ (r & 15)
 
-// lane holds columns 2 lane, 2 lane + 1 of a 128-column chunk; columns c and c + 16 are neighbours in the B-operand order,
-// so lanes l and l ^ 8 swap one value each and every lane stores one aligned 4-byte pair
-__device__ __forceinline__ void store_bop(_Float16* dst, float v0, float v1, int lane)
-{
-    const bool hi = (lane >> 3) & 1;
-    const float mine = hi ? v1 : v0, give = hi ? v0 : v1;
-    const float got = dpp_lane<0x128>(give);                      // lane ^ 8 (row rotate): low lanes get the partner's v0, high lanes the partner's v1
-    half2_t w;
-    w.x = (_Float16)(hi ? got : mine); w.y = (_Float16)(hi ? mine : got);
-    const int c = hi ? 2 * (lane ^ 8) + 1 : 2 * lane;           // the pair's low column: (c, c + 16)
-    *(half2_t*)(dst + bop_index(c)) = w;
-}
-
-// order the LDS accesses of one wavefront's lanes among themselves (a wavefront-private buffer needs no workgroup barrier)
-__device__ __forceinline__ void wave_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
 // Is pair row p (of expert e) held by a tile of one of the heights in the bit mask `heights` (bit k = 16 << k)? tiles / cap:
 // the lists of nq_pf_plan_k. The remainder tile of expert e sits at index e of the list of its height and starts at its
 // first row; the rows before it belong to the expert's full 256-row tiles. Rows of no valid expert count as height 256.
@@ -57,192 +37,192 @@ __device__ __forceinline__ bool row_in_heights(const int32_t* __restrict__ tiles
     return (heights >> k) & 1;
 }
 
-// grid (npairs), block 256: wave w handles the 512-column segments w, w + 4, ... of the pair's row, gate and up together.
-// tiles (optional): work only on the rows of the tile heights in `heights`
-__global__ void __launch_bounds__(256) nq_pf_pre_k(const void* __restrict__ x, int xdt, const int32_t* __restrict__ pt, const int32_t* __restrict__ pe,
+// grid (row groups, column parts), block 256: wavefront w of column part y rotates segment 4 y + w (512 columns, four chunks; lanes of
+// chunks beyond H repeat the last one) of `rows` pair rows, gate and up together, holding the scale vectors while the expert stays the same.
+// tiles (optional): work only on the rows of the tile heights in `heights`.
+// A form with two columns per lane (about 50 vector instructions per chunk) was bound by the vector ALU: 8024 rows of 6144 columns
+// 84 us; with eight columns per lane 64, 197 MB written at 3.1 TB/s. Fetching the next row's activations ahead changed nothing.
+__global__ void __launch_bounds__(256) nq_pf_pre_k(const void* __restrict__ x, int xdt, const int32_t* __restrict__ pt, const int32_t* __restrict__ pe, int np, int rows,
                                                     const int64_t* __restrict__ table, _Float16* xg, _Float16* xu, float* zg, int E, int H, int I,
                                                     const int32_t* __restrict__ tiles, int cap, int heights)
 {
     __shared__ float zsh[4][4];
-    const int p = blockIdx.x, lane = threadIdx.x & 63, warp = threadIdx.x >> 6;
-    const int e = pe[p];
-    if (tiles && !row_in_heights(tiles, cap, heights, p, e, E)) return;       // block-uniform
-    const int ng = H / 128;
-    const bool live = e >= 0 && e < E && table[(size_t)e * TBL_W] > 0;
-    const _Float16* signs = live ? (const _Float16*)table[(size_t)e * TBL_W + 9] : nullptr;
-    const size_t xr = live ? (size_t)pt[p] * H : 0;             // first element of the token's row
-    // low-rank plane (table words 14, 16): zg[p] = x V_gu^T over the raw activations, for the mid kernel
-    const _Float16* lr = live ? (const _Float16*)table[(size_t)e * TBL_W + 14] : nullptr;
-    const int rg = lr ? (int)table[(size_t)e * TBL_W + 16] : 0;
-    if (zg && rg)                                                // block-uniform
+    const int lane = threadIdx.x & 63, warp = threadIdx.x >> 6, L = wht_place(lane);
+    const int chunk = (4 * blockIdx.y + warp) * 4 + (lane >> 4), ng = H / 128;
+    const bool mine = chunk < ng;
+    const int col = (mine ? chunk : ng - 1) * 128 + 32 * (L >> 2) + 2 * (L & 3);    // this lane's columns: col + {0, 1} + {0, 8} + {0, 16}
+    const WhtSigns ws = wht_signs(lane);
+    const int p1 = min(np, (int)(blockIdx.x + 1) * rows);
+    half2_t sg[4], su[4];
+    int held = -1;                                               // the expert whose scales sg and su hold
+    for (int p = blockIdx.x * rows; p < p1; ++p)
     {
-        float zz[4] = {0.f, 0.f, 0.f, 0.f};
-        for (int k = 2 * threadIdx.x; k < H; k += 512)
+        const int e = pe[p];
+        if (tiles && !row_in_heights(tiles, cap, heights, p, e, E)) continue;     // block-uniform, like every branch on e
+        const bool live = e >= 0 && e < E && table[(size_t)e * TBL_W] > 0;
+        const size_t xr = live ? (size_t)pt[p] * H : 0;         // first element of the token's row
+        // low-rank plane (table words 14, 16): zg[p] = x V_gu^T over the raw activations, for the mid kernel
+        const _Float16* lr = live ? (const _Float16*)table[(size_t)e * TBL_W + 14] : nullptr;
+        const int rg = lr ? (int)table[(size_t)e * TBL_W + 16] : 0;
+        if (zg && rg && blockIdx.y == 0)
         {
-            const half2_t xv = act2_at(x, xdt, xr + k);
+            float zz[4] = {0.f, 0.f, 0.f, 0.f};
+            for (int k = 2 * threadIdx.x; k < H; k += 512)
+            {
+                const half2_t xv = act2_at(x, xdt, xr + k);
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (r < rg) { const half2_t vv = *(const half2_t*)(lr + (size_t)r * H + k); zz[r] += (float)xv.x * (float)vv.x + (float)xv.y * (float)vv.y; }
+            }
+            __syncthreads();                                     // the previous row's sums have been read
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-                if (r < rg) { const half2_t vv = *(const half2_t*)(lr + (size_t)r * H + k); zz[r] += (float)xv.x * (float)vv.x + (float)xv.y * (float)vv.y; }
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-        {
-#pragma unroll
-            for (int m = 32; m >= 1; m >>= 1) zz[r] += __shfl_xor(zz[r], m);
-            if (lane == 0) zsh[warp][r] = zz[r];
-        }
-        __syncthreads();
-        if (threadIdx.x < 4) zg[(size_t)p * 4 + threadIdx.x] = zsh[0][threadIdx.x] + zsh[1][threadIdx.x] + zsh[2][threadIdx.x] + zsh[3][threadIdx.x];
-    }
-    // A wavefront takes 512-column segments: x and the two scale vectors arrive as one 16-byte load per lane each and pass
-    // through a wavefront-private LDS buffer to the WHT's layout (lane = columns 2 lane, 2 lane + 1 of a 128-column chunk);
-    // the eight rotated chunks (4 chunks x gate / up) go back through the same buffer in B-operand order and leave as
-    // 16-byte stores. Full segments only when H is a multiple of 512; the remaining chunks take the narrow path below.
-    __shared__ __align__(16) _Float16 seg[4][3 * 512];
-    _Float16* sb = seg[warp];
-    const int nseg = H / 512;
-    for (int sgi = warp; sgi < nseg; sgi += 4)
-    {
-        const int k0 = sgi * 512;
-        float v[2][4][2];
-        if (live)
-        {
-            const _Float16* sug = signs, *suu = signs + 2 * H + 3 * I;
-            const uint4 xi = act8_at(x, xdt, xr + k0 + 8 * lane), gi = *(const uint4*)(sug + k0 + 8 * lane), ui = *(const uint4*)(suu + k0 + 8 * lane);
-            *(uint4*)(sb + 8 * lane) = xi; *(uint4*)(sb + 512 + 8 * lane) = gi; *(uint4*)(sb + 1024 + 8 * lane) = ui;
-            wave_sync();
-#pragma unroll
-            for (int c = 0; c < 4; ++c)
             {
-                const half2_t xv = *(const half2_t*)(sb + 128 * c + 2 * lane), sg = *(const half2_t*)(sb + 512 + 128 * c + 2 * lane),
-                              su = *(const half2_t*)(sb + 1024 + 128 * c + 2 * lane);
-                v[0][c][0] = (float)xv.x * (float)sg.x; v[0][c][1] = (float)xv.y * (float)sg.y;
-                v[1][c][0] = (float)xv.x * (float)su.x; v[1][c][1] = (float)xv.y * (float)su.y;
+#pragma unroll
+                for (int m = 32; m >= 1; m >>= 1) zz[r] += __shfl_xor(zz[r], m);
+                if (lane == 0) zsh[warp][r] = zz[r];
             }
-#pragma unroll
-            for (int up = 0; up < 2; ++up)
-#pragma unroll
-                for (int c = 0; c < 4; ++c) wht128(v[up][c][0], v[up][c][1], lane);
+            __syncthreads();
+            if (threadIdx.x < 4) zg[(size_t)p * 4 + threadIdx.x] = zsh[0][threadIdx.x] + zsh[1][threadIdx.x] + zsh[2][threadIdx.x] + zsh[3][threadIdx.x];
         }
-        else
-        {
-#pragma unroll
-            for (int up = 0; up < 2; ++up)
-#pragma unroll
-                for (int c = 0; c < 4; ++c) v[up][c][0] = v[up][c][1] = 0.f;
-        }
-        wave_sync();       // every lane has read its inputs before the buffer is reused
-#pragma unroll
-        for (int up = 0; up < 2; ++up)
-#pragma unroll
-            for (int c = 0; c < 4; ++c) store_bop(sb + up * 512 + c * 128, v[up][c][0], v[up][c][1], lane);
-        wave_sync();
-        *(uint4*)(xg + (size_t)p * H + k0 + 8 * lane) = *(const uint4*)(sb + 8 * lane);
-        *(uint4*)(xu + (size_t)p * H + k0 + 8 * lane) = *(const uint4*)(sb + 512 + 8 * lane);
-        wave_sync();       // the stores' LDS reads are done before the next segment's writes
-    }
-    for (int task = 8 * nseg + warp; task < 2 * ng; task += 4)       // chunks beyond the last full segment (task = 2 * chunk + up)
-    {
-        const int up = task & 1, grp = task >> 1, k = grp * 128 + 2 * lane;
-        _Float16* dst = (up ? xu : xg) + (size_t)p * H + grp * 128;
-        float v0 = 0.f, v1 = 0.f;
+        uint4 bg = make_uint4(0, 0, 0, 0), bu = bg;              // rows of no live expert are zero
         if (live)
         {
-            const _Float16* su = up ? signs + 2 * H + 3 * I : signs;
-            const half2_t xv = act2_at(x, xdt, xr + k), sv = *(const half2_t*)(su + k);
-            v0 = (float)xv.x * (float)sv.x; v1 = (float)xv.y * (float)sv.y;
-            wht128(v0, v1, lane);
+            half2_t xv[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) xv[q] = act2_at(x, xdt, xr + col + 8 * q);
+            if (e != held)
+            {
+                const _Float16 *sug = (const _Float16*)table[(size_t)e * TBL_W + 9], *suu = sug + 2 * H + 3 * I;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) { sg[q] = *(const half2_t*)(sug + col + 8 * q); su[q] = *(const half2_t*)(suu + col + 8 * q); }
+                held = e;
+            }
+            float g[8], u[8];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+            {
+                const float x0 = (float)xv[q].x, x1 = (float)xv[q].y;
+                g[2 * q] = x0 * (float)sg[q].x; g[2 * q + 1] = x1 * (float)sg[q].y;
+                u[2 * q] = x0 * (float)su[q].x; u[2 * q + 1] = x1 * (float)su[q].y;
+            }
+            wht8_bop(g, ws); wht8_bop(u, ws);
+            bg = bop_block(g); bu = bop_block(u);
         }
-        store_bop(dst, v0, v1, lane);
+        if (mine)
+        {
+            const size_t at = (size_t)p * H + chunk * 128 + 8 * L;
+            *(uint4*)(xg + at) = bg;
+            *(uint4*)(xu + at) = bu;
+        }
     }
 }
 
-// grid (npairs), block 256: acc_gu [P][2I] fp32 (gate | up) -> h [P][I] fp16 in B-operand order. With in_had_down = 512
-// (table word 18) the four wavefronts hold the four 128-column groups of a 512-column block and combine their WHT_128
-// results through LDS with the Sylvester H_4 / 2 before the single rounding to fp16.
+// grid (row groups), block 256: acc_gu [P][2I] fp32 (gate | up) -> h [P][I] fp16 in B-operand order. The wavefronts take the tasks
+// (pair row of the group, segment of 512 columns) in turn; lanes of chunks beyond I repeat the last one. With in_had_down = 512
+// (table word 18) the four chunks of a segment are combined with the Sylvester H_4 / 2 before the single rounding to fp16.
 // tiles (optional): work only on the rows of the tile heights in `heights`, as nq_pf_pre_k
-__global__ void __launch_bounds__(256) nq_pf_mid_k(const float* __restrict__ acc_gu, const int32_t* __restrict__ pe,
+// Bound by memory, 5 bytes per output element and no reuse: 8024 rows of 2 x 2048 sums 66 -> 40 us (4.1 TB/s) with eight columns per
+// lane, for the same reason as there.
+constexpr int MID_ROWS = 8;                                      // most rows of a group
+__global__ void __launch_bounds__(256) nq_pf_mid_k(const float* __restrict__ acc_gu, const int32_t* __restrict__ pe, int np, int rows,
                                                     const int64_t* __restrict__ table, _Float16* h, const float* zg, float* zd, int E, int H, int I,
                                                     const int32_t* __restrict__ tiles, int cap, int heights)
 {
-    __shared__ float wsh[4][128];
-    __shared__ float zsh[4][4];
-    const int p = blockIdx.x, lane = threadIdx.x & 63, warp = threadIdx.x >> 6;
-    const int e = pe[p];
-    if (tiles && !row_in_heights(tiles, cap, heights, p, e, E)) return;       // block-uniform
-    const bool live = e >= 0 && e < E && table[(size_t)e * TBL_W] > 0;
-    const _Float16* signs = live ? (const _Float16*)table[(size_t)e * TBL_W + 9] : nullptr;
-    const bool wide = live && table[(size_t)e * TBL_W + 18] == 512;      // block-uniform
-    // low-rank plane: g / u += zg (U2 [+ U4 at level 4]); zd[p] = sw V_dn^T for the post kernel
-    const _Float16* lr = live ? (const _Float16*)table[(size_t)e * TBL_W + 14] : nullptr;
-    const _Float16* lr4 = live ? (const _Float16*)table[(size_t)e * TBL_W + 15] : nullptr;
-    const int rg = lr && zg ? (int)table[(size_t)e * TBL_W + 16] : 0, rd = lr && zd ? (int)table[(size_t)e * TBL_W + 17] : 0;
-    const bool l4 = live && table[(size_t)e * TBL_W] == 4;
-    const _Float16* U2g = lr + (size_t)rg * H, *U2u = U2g + (size_t)rg * I, *Vd = U2u + (size_t)rg * I, *U4g = lr4, *U4u = lr4 + (size_t)rg * I;
-    float zr[4] = {0.f, 0.f, 0.f, 0.f}, zacc[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int r = 0; r < rg; ++r) zr[r] = zg[(size_t)p * 4 + r];
-    for (int grp = warp; grp < I / 128; grp += 4)
+    __shared__ float zsh[MID_ROWS][4][4];
+    const int lane = threadIdx.x & 63, warp = threadIdx.x >> 6, L = wht_place(lane);
+    const int p0 = blockIdx.x * rows, nr = min(rows, np - p0), ni = I / 128, nseg = (ni + 3) / 4;
+    const WhtSigns ws = wht_signs(lane);
+    if (zd)
     {
-        const int col = grp * 128 + 2 * lane;
-        _Float16* dst = h + (size_t)p * I + grp * 128;
-        float v0 = 0.f, v1 = 0.f;
+        for (int i = threadIdx.x; i < MID_ROWS * 16; i += 256) (&zsh[0][0][0])[i] = 0.f;
+        __syncthreads();
+    }
+    for (int t = warp; t < nr * nseg; t += 4)                    // e, live, ... are the same for the whole wavefront
+    {
+        const int row = t / nseg, p = p0 + row, chunk = (t - row * nseg) * 4 + (lane >> 4);
+        const int e = pe[p];
+        if (tiles && !row_in_heights(tiles, cap, heights, p, e, E)) continue;
+        const bool mine = chunk < ni, live = e >= 0 && e < E && table[(size_t)e * TBL_W] > 0;
+        uint4 b = make_uint4(0, 0, 0, 0);
         if (live)
         {
+            const _Float16* signs = (const _Float16*)table[(size_t)e * TBL_W + 9];
             const _Float16 *sv_g = signs + H, *sv_u = sv_g + I, *su_d = sv_u + I;
-            const float2 pg = *(const float2*)(acc_gu + (size_t)p * 2 * I + col), pu = *(const float2*)(acc_gu + (size_t)p * 2 * I + I + col);
-            float g0 = pg.x, g1 = pg.y, u0 = pu.x, u1 = pu.y;
-            wht128(g0, g1, lane); wht128(u0, u1, lane);
-            const half2_t svg = *(const half2_t*)(sv_g + col), svu = *(const half2_t*)(sv_u + col), sud = *(const half2_t*)(su_d + col);
-            g0 *= (float)svg.x; g1 *= (float)svg.y; u0 *= (float)svu.x; u1 *= (float)svu.y;
+            const int col = (mine ? chunk : ni - 1) * 128 + 8 * L;
+            float g[8], u[8];
+            const float* ag = acc_gu + (size_t)p * 2 * I + col;
+            *(float4_t*)g = *(const float4_t*)ag; *(float4_t*)(g + 4) = *(const float4_t*)(ag + 4);
+            *(float4_t*)u = *(const float4_t*)(ag + I); *(float4_t*)(u + 4) = *(const float4_t*)(ag + I + 4);
+            const half8_t svg = *(const half8_t*)(sv_g + col), svu = *(const half8_t*)(sv_u + col), sud = *(const half8_t*)(su_d + col);
+            wht8_row(g, ws); wht8_row(u, ws);
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                if (r < rg)
+            for (int i = 0; i < 8; ++i) { g[i] *= (float)svg[i]; u[i] *= (float)svu[i]; }
+            // low-rank plane: g / u += zg (U2 [+ U4 at level 4]); zd[p] = sw V_dn^T for the post kernel
+            const _Float16* lr = (const _Float16*)table[(size_t)e * TBL_W + 14];
+            const int rg = lr && zg ? (int)table[(size_t)e * TBL_W + 16] : 0, rd = lr && zd ? (int)table[(size_t)e * TBL_W + 17] : 0;
+            const _Float16* U2g = lr + (size_t)rg * H, *U2u = U2g + (size_t)rg * I, *Vd = U2u + (size_t)rg * I;
+            if (rg)
+            {
+                const _Float16* lr4 = table[(size_t)e * TBL_W] == 4 ? (const _Float16*)table[(size_t)e * TBL_W + 15] : nullptr;
+                for (int r = 0; r < rg; ++r)
                 {
-                    half2_t ug = *(const half2_t*)(U2g + (size_t)r * I + col), uu = *(const half2_t*)(U2u + (size_t)r * I + col);
-                    g0 += zr[r] * (float)ug.x; g1 += zr[r] * (float)ug.y; u0 += zr[r] * (float)uu.x; u1 += zr[r] * (float)uu.y;
-                    if (l4)
+                    const float z = zg[(size_t)p * 4 + r];
+                    half8_t ug = *(const half8_t*)(U2g + (size_t)r * I + col), uu = *(const half8_t*)(U2u + (size_t)r * I + col);
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) { g[i] += z * (float)ug[i]; u[i] += z * (float)uu[i]; }
+                    if (lr4)
                     {
-                        ug = *(const half2_t*)(U4g + (size_t)r * I + col); uu = *(const half2_t*)(U4u + (size_t)r * I + col);
-                        g0 += zr[r] * (float)ug.x; g1 += zr[r] * (float)ug.y; u0 += zr[r] * (float)uu.x; u1 += zr[r] * (float)uu.y;
+                        ug = *(const half8_t*)(lr4 + (size_t)r * I + col); uu = *(const half8_t*)(lr4 + (size_t)(rg + r) * I + col);
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) { g[i] += z * (float)ug[i]; u[i] += z * (float)uu[i]; }
                     }
                 }
-            const float sw0 = g0 / (1.f + __expf(-g0)) * u0, sw1 = g1 / (1.f + __expf(-g1)) * u1;
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                if (r < rd) { const half2_t vv = *(const half2_t*)(Vd + (size_t)r * I + col); zacc[r] += sw0 * (float)vv.x + sw1 * (float)vv.y; }
-            v0 = sw0 * (float)sud.x; v1 = sw1 * (float)sud.y;
-            wht128(v0, v1, lane);
-        }
-        if (wide)
-        {   // I % 512 == 0, so all four wavefronts are in this iteration: grp = 4 * block + warp
-            wsh[warp][2 * lane] = v0; wsh[warp][2 * lane + 1] = v1;
-            __syncthreads();
-            v0 = v1 = 0.f;
-#pragma unroll
-            for (int pp = 0; pp < 4; ++pp)
-            {
-                const float sg = (__builtin_popcount(warp & pp) & 1) ? -0.5f : 0.5f;
-                v0 += sg * wsh[pp][2 * lane]; v1 += sg * wsh[pp][2 * lane + 1];
             }
-            __syncthreads();
+            float v[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = g[i] / (1.f + __expf(-g[i])) * u[i];
+            for (int r = 0; r < rd; ++r)
+            {
+                const half8_t vv = *(const half8_t*)(Vd + (size_t)r * I + col);
+                float z = 0.f;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) z += v[i] * (float)vv[i];
+                if (!mine) z = 0.f;
+#pragma unroll
+                for (int m = 32; m >= 1; m >>= 1) z += __shfl_xor(z, m);
+                if (lane == 0) zsh[row][warp][r] += z;           // this wavefront's own sums, segment by segment
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] *= (float)sud[i];
+            wht8_row(v, ws);
+            if (table[(size_t)e * TBL_W + 18] == 512)            // I % 512 == 0: every chunk of the segment is there
+            {
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+                {
+                    float o = 0.f;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) o += ((__builtin_popcount((lane >> 4) & q) & 1) ? -0.5f : 0.5f) * __shfl(v[i], 16 * q + (lane & 15));
+                    v[i] = o;
+                }
+            }
+            b = bop_block_of_row(v, lane);
         }
-        store_bop(dst, v0, v1, lane);
+        if (mine) *(uint4*)(h + (size_t)p * I + chunk * 128 + 8 * L) = b;
     }
-    if (rd)                                                      // block-uniform
+    if (!zd) return;
+    __syncthreads();
+    for (int i = threadIdx.x; i < nr * 4; i += 256)
     {
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-        {
-#pragma unroll
-            for (int m = 32; m >= 1; m >>= 1) zacc[r] += __shfl_xor(zacc[r], m);
-            if (lane == 0) zsh[warp][r] = zacc[r];
-        }
-        __syncthreads();
-        if (threadIdx.x < 4) zd[(size_t)p * 4 + threadIdx.x] = zsh[0][threadIdx.x] + zsh[1][threadIdx.x] + zsh[2][threadIdx.x] + zsh[3][threadIdx.x];
+        const int p = p0 + i / 4, r = i & 3, e = pe[p];
+        if (e < 0 || e >= E || table[(size_t)e * TBL_W] <= 0 || !table[(size_t)e * TBL_W + 14] || table[(size_t)e * TBL_W + 17] <= r) continue;
+        if (tiles && !row_in_heights(tiles, cap, heights, p, e, E)) continue;
+        zd[(size_t)p * 4 + r] = zsh[i / 4][0][r] + zsh[i / 4][1][r] + zsh[i / 4][2][r] + zsh[i / 4][3][r];
     }
 }
 
-// grid (T, column parts), block 256: out[t] (+)= sum over the token's picks whose pair row lies in [row_lo, row_lo + nrows) of
+// grid (T, column parts), block 64 or 256: out[t] (+)= sum over the token's picks whose pair row lies in [row_lo, row_lo + nrows) of
 // rw * sv_o (.) Hadamard(y[row]); pos[t][k] = row of pair (t, k) in the expert-sorted order; add: on top of what out holds (fp32),
 // else out is written whole, zeros included. One block owns a token, so
 // the sum needs no atomics and its order is fixed (the reference's pf_post adds with float atomics in arrival order).
@@ -282,40 +262,57 @@ __global__ void __launch_bounds__(256) nq_pf_post_k(const float* __restrict__ y,
     __syncthreads();
     const int np = p_n;
     if (np == 0 && add) return;
-    for (int grp = 4 * blockIdx.y + warp; grp < H / 128; grp += 4 * gridDim.y)
+    const int nw = blockDim.x >> 6, ng = H / 128, L = wht_place(lane);
+    const WhtSigns ws = wht_signs(lane);                         // eight columns per lane: 8024 rows 62 -> 46 us (4.5 TB/s)
+    for (int sg = nw * blockIdx.y + warp; 4 * sg < ng; sg += nw * gridDim.y)       // segments of 512 columns, eight per lane; lanes beyond H repeat the last chunk
     {
-        const int col = grp * 128 + 2 * lane;
-        float o0 = 0.f, o1 = 0.f;
+        const int chunk = 4 * sg + (lane >> 4), col = (chunk < ng ? chunk : ng - 1) * 128 + 8 * L;
+        float o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
         for (int k0 = 0; k0 < np; k0 += 4)                       // four picks at a time, reads first
         {
-            float2 v[4]; half2_t sv[4];
+            float v[4][8]; half8_t sv[4];
 #pragma unroll
             for (int u = 0; u < 4; ++u)
             {
                 const int k = k0 + u < np ? k0 + u : k0;
-                v[u] = *(const float2*)(y + (size_t)p_row[k] * H + col);
-                sv[u] = *(const half2_t*)(p_sv[k] + col);
+                const float* row = y + (size_t)p_row[k] * H + col;
+                *(float4_t*)v[u] = *(const float4_t*)row; *(float4_t*)(v[u] + 4) = *(const float4_t*)(row + 4);
+                sv[u] = *(const half8_t*)(p_sv[k] + col);
             }
 #pragma unroll
             for (int u = 0; u < 4; ++u)
             {
                 if (k0 + u >= np) break;
-                float v0 = v[u].x, v1 = v[u].y;
-                wht128(v0, v1, lane);
+                wht8_row(v[u], ws);
                 const float w = p_w[k0 + u];
-                v0 *= (float)sv[u].x; v1 *= (float)sv[u].y;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) v[u][i] *= (float)sv[u][i];
                 for (int r = 0; r < p_rd[k0 + u]; ++r)           // y += (sw V_dn^T) (U2_d [+ U4_d])
                 {
                     const float zr = zd[(size_t)p_row[k0 + u] * 4 + r];
-                    half2_t ud = *(const half2_t*)(p_u2[k0 + u] + (size_t)r * H + col);
-                    v0 += zr * (float)ud.x; v1 += zr * (float)ud.y;
-                    if (p_u4[k0 + u]) { ud = *(const half2_t*)(p_u4[k0 + u] + (size_t)r * H + col); v0 += zr * (float)ud.x; v1 += zr * (float)ud.y; }
+                    half8_t ud = *(const half8_t*)(p_u2[k0 + u] + (size_t)r * H + col);
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) v[u][i] += zr * (float)ud[i];
+                    if (p_u4[k0 + u])
+                    {
+                        ud = *(const half8_t*)(p_u4[k0 + u] + (size_t)r * H + col);
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) v[u][i] += zr * (float)ud[i];
+                    }
                 }
-                o0 += w * v0; o1 += w * v1;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) o[i] += w * v[u][i];
             }
         }
-        if (add) { const float2 cur = *(const float2*)((const float*)out + (size_t)t * H + col); o0 = cur.x + o0; o1 = cur.y + o1; }   // fp32 results only
-        res2_store(out, odt, (size_t)t * H + col, o0, o1);
+        if (chunk >= ng) continue;
+        const size_t at = (size_t)t * H + col;
+        if (add)                                                 // fp32 results only
+#pragma unroll
+            for (int i = 0; i < 8; ++i) o[i] = ((const float*)out)[at + i] + o[i];
+        if (odt == DT_OUT_F16) *(uint4*)((_Float16*)out + at) = make_uint4(pack_f16(o[0], o[1]), pack_f16(o[2], o[3]), pack_f16(o[4], o[5]), pack_f16(o[6], o[7]));
+        else
+#pragma unroll
+            for (int i = 0; i < 8; i += 2) res2_store(out, odt, at + i, o[i], o[i + 1]);
     }
 }
 
@@ -858,11 +855,14 @@ __global__ void __launch_bounds__(512) nq_pf_sort_k(PfSort a)
     for (int i = base + tid; i < a.cap; i += 512) T4[i] = make_int4(-1, 0, 0, 0);
 }
 
+// pair rows per workgroup of the row kernels: what leaves about two thousand workgroups (eight per CU), at most eight
+static int row_group(int np, int parts) { return std::min(MID_ROWS, std::max(1, (int)((int64_t)np * parts / 2048))); }
 int launch_pf_pre(const void* x, int xdt, const int32_t* pt, const int32_t* pe, int np, const int64_t* table, void* xg, void* xu, float* zg, int E, int H, int I,
                   const int32_t* tiles, int cap, int heights, hipStream_t st)
 {
     if (!np) return 0;
-    nq_pf_pre_k<<<np, 256, 0, st>>>(x, xdt, pt, pe, table, (_Float16*)xg, (_Float16*)xu, zg, E, H, I, tiles, cap, heights);
+    const int parts = (H / 128 + 15) / 16, rows = row_group(np, parts);
+    nq_pf_pre_k<<<dim3((np + rows - 1) / rows, parts), 256, 0, st>>>(x, xdt, pt, pe, np, rows, table, (_Float16*)xg, (_Float16*)xu, zg, E, H, I, tiles, cap, heights);
     NQ_LAUNCH_CHECK("nq_pf_pre");
     return 0;
 }
@@ -870,7 +870,8 @@ int launch_pf_mid(const float* acc_gu, const int32_t* pe, int np, const int64_t*
                   const int32_t* tiles, int cap, int heights, hipStream_t st)
 {
     if (!np) return 0;
-    nq_pf_mid_k<<<np, 256, 0, st>>>(acc_gu, pe, table, (_Float16*)h, zg, zd, E, H, I, tiles, cap, heights);
+    const int rows = row_group(np, 1);
+    nq_pf_mid_k<<<(np + rows - 1) / rows, 256, 0, st>>>(acc_gu, pe, np, rows, table, (_Float16*)h, zg, zd, E, H, I, tiles, cap, heights);
     NQ_LAUNCH_CHECK("nq_pf_mid");
     return 0;
 }
@@ -878,9 +879,10 @@ int launch_pf_post(const float* y, const int32_t* pos, const void* sel, int sdt,
                    const int64_t* table, void* out, int odt, int add, const float* zd, int E, int H, int I, hipStream_t st)
 {
     if (!T || (!nrows && add)) return 0;
-    // few tokens: several workgroups per token, about a thousand in all (48 tokens of 6144 columns: 43 us with one each, 9 with ten)
-    const int quads = (H / 128 + 3) / 4, parts = T >= 1024 ? 1 : quads < 1024 / T ? quads : 1024 / T;
-    nq_pf_post_k<<<dim3(T, parts), 256, 0, st>>>(y, pos, sel, sdt, rw, wdt, topk, row_lo, nrows, table, out, odt, add, zd, E, H, I);
+    // few tokens: one wavefront per segment of 512 columns, each a workgroup of its own, so that every CU has some
+    const int segs = (H / 128 + 3) / 4;
+    const dim3 grid = T >= 1024 ? dim3(T, 1) : dim3(T, segs);
+    nq_pf_post_k<<<grid, T >= 1024 ? 256 : 64, 0, st>>>(y, pos, sel, sdt, rw, wdt, topk, row_lo, nrows, table, out, odt, add, zd, E, H, I);
     NQ_LAUNCH_CHECK("nq_pf_post");
     return 0;
 }

@@ -116,6 +116,91 @@ __device__ __forceinline__ void wht128(float& a, float& b, int lane)
     a *= 0.08838834764f; b *= 0.08838834764f;
 }
 
+// ---- Hadamard-128 on sixteen lanes: eight elements per lane, four chunks per wavefront ---------------------------------
+// The throughput form for kernels that rotate many rows: three butterflies in the lane, four between lanes of a DPP row, 64 instructions
+// for 512 elements (wht128 takes about 50 for 128). A lane's place L = 0..15 in its chunk is chosen so that the four
+// lane bits of L are exchanged by the lane masks 1, 2, 7, 8, each one DPP select (wht_place: lane = L0 ^ 2 L1 ^ 7 L2 ^ 8 L3). A lane whose bit is set would
+// hold a' - a; it keeps a - a' instead, one multiply-add by +-1 with the exchange inside it, and since a lane's sign is common to all
+// it holds and to its partners in the later exchanges, the last multiplication puts it right. The sums and their roundings are
+// those of wht128. Which columns a place and its eight elements stand for: wht8_bop, wht8_row.
+__device__ __forceinline__ int wht_place(int lane) { return (lane & 4) ? (lane & 15) ^ 3 : lane & 15; }
+struct WhtSigns { float s0, s1, s2, s3, scale; };
+__device__ __forceinline__ WhtSigns wht_signs(int lane)
+{
+    const int L = wht_place(lane);
+    const float s0 = (L & 1) ? -1.f : 1.f, s1 = (L & 2) ? -1.f : 1.f, s2 = (L & 4) ? -1.f : 1.f, s3 = (L & 8) ? -1.f : 1.f;
+    return WhtSigns{s0, s1, s2, s3, 0.08838834764f * s0 * s1 * s2 * s3};
+}
+// v[i] = v[i] + s * (v[i] of the partner lane). Asm, because the compiler puts the select into a move of its own; a DPP read needs two
+// wait states after the write of its register, which it cannot see, so they are written out.
+#define NQ_WHT_LANES(NAME, SELECT) \
+__device__ __forceinline__ void NAME(float* v, float s) \
+{ \
+    asm("s_nop 1\n\t" \
+        "v_fmac_f32_dpp %0, %0, %8 " SELECT " row_mask:0xf bank_mask:0xf\n\tv_fmac_f32_dpp %1, %1, %8 " SELECT " row_mask:0xf bank_mask:0xf\n\t" \
+        "v_fmac_f32_dpp %2, %2, %8 " SELECT " row_mask:0xf bank_mask:0xf\n\tv_fmac_f32_dpp %3, %3, %8 " SELECT " row_mask:0xf bank_mask:0xf\n\t" \
+        "v_fmac_f32_dpp %4, %4, %8 " SELECT " row_mask:0xf bank_mask:0xf\n\tv_fmac_f32_dpp %5, %5, %8 " SELECT " row_mask:0xf bank_mask:0xf\n\t" \
+        "v_fmac_f32_dpp %6, %6, %8 " SELECT " row_mask:0xf bank_mask:0xf\n\tv_fmac_f32_dpp %7, %7, %8 " SELECT " row_mask:0xf bank_mask:0xf" \
+        : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]) : "v"(s)); \
+}
+NQ_WHT_LANES(wht_lanes1, "quad_perm:[1,0,3,2]")                  // lane ^ 1
+NQ_WHT_LANES(wht_lanes2, "quad_perm:[2,3,0,1]")                  // lane ^ 2
+NQ_WHT_LANES(wht_lanes7, "row_half_mirror")                      // lane ^ 7
+NQ_WHT_LANES(wht_lanes8, "row_ror:8")                            // lane ^ 8
+#undef NQ_WHT_LANES
+template <int D> __device__ __forceinline__ void wht_inside(float* v)
+{
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+        if (!(i & D)) { const float a = v[i], b = v[i + D]; v[i] = a + b; v[i + D] = a - b; }
+}
+// place L = 4 mm + kg of the chunk; v[j + 2 a + 4 b] = column 32 mm + 2 kg + j + 8 a + 16 b
+__device__ __forceinline__ void wht8_bop(float* v, const WhtSigns& w)
+{
+    wht_inside<1>(v); wht_lanes1(v, w.s0); wht_lanes2(v, w.s1);        // columns apart by 1, 2, 4
+    wht_inside<2>(v); wht_inside<4>(v);                                          // 8, 16
+    wht_lanes7(v, w.s2); wht_lanes8(v, w.s3);                        // 32, 64
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] *= w.scale;
+}
+// v[j] = column 8 L + j
+__device__ __forceinline__ void wht8_row(float* v, const WhtSigns& w)
+{
+    wht_inside<1>(v); wht_inside<2>(v); wht_inside<4>(v);
+    wht_lanes1(v, w.s0); wht_lanes2(v, w.s1); wht_lanes7(v, w.s2); wht_lanes8(v, w.s3);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] *= w.scale;
+}
+__device__ __forceinline__ uint32_t pack_f16(float lo, float hi)
+{
+    half2_t h; h.x = (_Float16)lo; h.y = (_Float16)hi;
+    return __builtin_bit_cast(uint32_t, h);
+}
+// the 16-byte block (mm, kg) of the B-operand order from wht8_bop's arrangement: halfs 2 i + hi = column i's pair (c, c + 16)
+__device__ __forceinline__ uint4 bop_block(const float* v)
+{
+    return make_uint4(pack_f16(v[0], v[4]), pack_f16(v[1], v[5]), pack_f16(v[2], v[6]), pack_f16(v[3], v[7]));
+}
+// the same from wht8_row's arrangement: two exchanges within the four lanes that hold columns 32 mm .. 32 mm + 31 (places 4 mm + q,
+// q = bit 3 of the column + 2 * bit 4): first with the lane 16 columns on, which makes the pairs, then with the one 8 columns on.
+template <int CTRL> __device__ __forceinline__ uint32_t dpp_word(uint32_t v) { return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, true); }
+__device__ __forceinline__ uint4 bop_block_of_row(const float* v, int lane)
+{
+    const int L = wht_place(lane);
+    const bool hi = L & 2, up = L & 1;
+    uint32_t d[4];                                               // columns (0, 1), (2, 3), (4, 5), (6, 7)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) d[i] = pack_f16(v[2 * i], v[2 * i + 1]);
+    // kg = 0, 1 go to the lane with column bit 4 clear, kg = 2, 3 to the other
+    const uint32_t g0 = dpp_word<0x4E>(hi ? d[0] : d[2]), g1 = dpp_word<0x4E>(hi ? d[1] : d[3]);
+    const uint32_t l0 = hi ? g0 : d[0], l1 = hi ? g1 : d[1], h0 = hi ? d[2] : g0, h1 = hi ? d[3] : g1;      // of the lower, of the upper 16 columns
+    const uint32_t p0 = __builtin_amdgcn_perm(h0, l0, 0x05040100u), p1 = __builtin_amdgcn_perm(h0, l0, 0x07060302u);   // first kg: pairs of j = 0, 1
+    const uint32_t p2 = __builtin_amdgcn_perm(h1, l1, 0x05040100u), p3 = __builtin_amdgcn_perm(h1, l1, 0x07060302u);   // second kg
+    // the first kg goes to the lane with column bit 3 clear, the second to the other; its own columns' bit 3 orders the halves
+    const uint32_t q0 = dpp_word<0xB1>(up ? p0 : p2), q1 = dpp_word<0xB1>(up ? p1 : p3);
+    return up ? make_uint4(q0, q1, p2, p3) : make_uint4(p0, p1, q0, q1);
+}
+
 // LDS position (in halfs) of column c of a 128-column chunk in the B-operand order:
 // 16-byte block (mm, kg) holds, for i = 0..3, columns 32 mm + 2 kg + 8 (i >> 1) + (i & 1) and that + 16
 __device__ __forceinline__ int bop_index(int c)

@@ -286,3 +286,36 @@ def test_grouped_step_equals_the_decode_slices(T, E, K, Bmax, xd, wd, sd):
     tol = {torch.float32: 5e-5, torch.float16: 1e-3, torch.bfloat16: 8e-3}[xd]
     assert rel_err(y.float().cpu().numpy(), want.cpu().numpy()) < tol
     assert not y[5].any()                                         # all its picks at level 0
+
+
+@pytest.mark.parametrize("H,I,n", [(128, 128, 1), (640, 384, 37), (2176, 512, 2050), (256, 768, 4100)])
+def test_row_kernels_against_a_float64_hadamard(H, I, n):
+    """nq_pf_pre and nq_pf_mid where chunks do not fill a wavefront's four and where a workgroup takes one, two, more rows"""
+    from nestquant_amd import _lib
+    Lb = _lib.lib()
+    E, T = 3, 11
+    ex = to_dev(experts_on_gpu(H, I, E, 31))
+    L = M.MoELayer(E, H, I, Bmax=4, topk=1)
+    for e in range(E):
+        L.set(e, ex[e], 2)
+    g = torch.Generator().manual_seed(n)
+    pe, pt = torch.randint(-1, E, (n,), generator=g).int().sort().values, torch.randint(0, T, (n,), generator=g).int()
+    x, acc = (torch.randn(T, H, generator=g) * 0.3).half(), torch.randn(n, 2 * I, generator=g)
+    xg = torch.full((n, H), 7.0, dtype=torch.float16, device=DEV); xu, h = torch.full_like(xg, 7.0), torch.full((n, I), 7.0, dtype=torch.float16, device=DEV)
+    xd, ad, ped, ptd = x.to(DEV), acc.to(DEV), pe.to(DEV), pt.to(DEV)
+    _lib.check(Lb.nq_pf_pre(xd.data_ptr(), ptd.data_ptr(), ped.data_ptr(), n, L.table.data_ptr(), xg.data_ptr(), xu.data_ptr(), None, E, H, I, None))
+    _lib.check(Lb.nq_pf_mid(ad.data_ptr(), ped.data_ptr(), n, L.table.data_ptr(), h.data_ptr(), None, None, E, H, I, None))
+    had = torch.ones(1, 1, dtype=torch.float64)
+    for _ in range(7):
+        had = torch.cat([torch.cat([had, had], 1), torch.cat([had, -had], 1)])
+    wht = lambda v: (v.view(n, -1, 128) @ had / 128**0.5).view(n, -1)
+    place = torch.tensor([((c >> 5) * 4 + (c >> 1 & 3)) * 8 + 2 * (2 * (c >> 3 & 1) + (c & 1)) + (c >> 4 & 1) for c in range(128)])
+    bop = lambda v: torch.empty_like(v).view(n, -1, 128).index_copy_(2, place, v.view(n, -1, 128)).view(n, -1)
+    sg = torch.stack([e.signs.cpu().double() for e in ex])[pe.clamp(min=0).long()]
+    live = (pe >= 0).double()[:, None]
+    xs = x.double()[pt.long()]
+    for got, su in ((xg, sg[:, :H]), (xu, sg[:, 2 * H + 3 * I:])):
+        assert rel_err(got.cpu().double().numpy(), (bop(wht(xs * su)) * live).numpy()) < 5e-4
+    gate, up = wht(acc[:, :I].double().contiguous()) * sg[:, H:H + I], wht(acc[:, I:].double().contiguous()) * sg[:, H + I:H + 2 * I]
+    want = bop(wht(torch.nn.functional.silu(gate) * up * sg[:, H + 2 * I:H + 3 * I])) * live
+    assert rel_err(h.cpu().double().numpy(), want.numpy()) < 5e-4
