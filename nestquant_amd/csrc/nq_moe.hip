@@ -442,9 +442,43 @@ __device__ __forceinline__ void finish_gu(const MoeArgs& a, const RunHdr& R, flo
     if (threadIdx.x == 0) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// What the combine needs to know of the call's picks, lane s holding pick s: one coalesced read of PickInfo for all of them, issued
+// under the decode's last partial sums. Read pick by pick inside the combine (weight -> sign vector's address -> its values, then the
+// low-rank address) these were four dependent round trips per token on the launch's last workgroup. Layer of H 512, I 256, 4 picks, 2
+// tokens: 17.5 -> 16.95 us a call; at 6144 x 2048 the same within 0.3 % (there other workgroups still decode under it).
+struct PickLanes
+{
+    float w; unsigned long long signs; int rd;                   // rd: rank of the low-rank plane's down half, 0 without one
+    __device__ __forceinline__ float weight(int s) const { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), s)); }
+    __device__ __forceinline__ const _Float16* sign_row(int s) const
+    {
+        const unsigned lo = __builtin_amdgcn_readlane((int)(unsigned)signs, s), hi = __builtin_amdgcn_readlane((int)(signs >> 32), s);
+        return (const _Float16*)(((unsigned long long)hi << 32) | lo);
+    }
+    __device__ __forceinline__ int rank(int s) const { return __builtin_amdgcn_readlane(rd, s); }
+};
+__device__ __forceinline__ PickLanes pick_lanes(const PickInfo& R, int lane)
+{
+    PickLanes P;
+    P.w = R.w[lane]; P.signs = (unsigned long long)R.signs[lane]; P.rd = R.lr[lane] ? R.rd[lane] : 0;
+    return P;
+}
+// the output scales of picks k and k + SB of token b for this lane's two columns (nothing for picks that do not contribute)
+__device__ __forceinline__ void pick_scales(const MoeArgs& a, const PickLanes& P, int b, int k, int SB, int col, half2_t* sv)
+{
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+    {
+        const int kq = k + q * SB, s = (b * a.topk + kq) & 63;
+        sv[q] = half2_t{};
+        if (b < a.B && kq < a.topk && P.weight(s) != 0.f) sv[q] = *(const half2_t*)(P.sign_row(s) + a.H + 3 * a.I + col);
+    }
+}
+
 // combine of the down projection for output rows [grp * 128, +128): out[b] = sum_k rw[b,k] * sv_o[e] (.) WHT(sum_y part_d[slot])
-// picks of a token are spread over the block's wavefronts and reduced through LDS (red: SB * 128 floats)
-__device__ __forceinline__ void finish_dn(const MoeArgs& a, const PickInfo& R, int grp, int NY, int warp, int SB, int lane, float* red)
+// picks of a token are spread over the block's wavefronts and reduced through LDS (red: SB * 128 floats). `next`: the scales of the
+// wavefront's first two picks, requested before the arrival counter; those of every later step are requested one step ahead.
+__device__ __forceinline__ void finish_dn(const MoeArgs& a, const PickInfo& R, const PickLanes& P, half2_t* next, int grp, int NY, int warp, int SB, int lane, float* red)
 {
     const int S = a.B * a.topk, col = grp * 128 + 2 * lane;
     for (int b = 0; b < a.B; ++b)
@@ -454,17 +488,17 @@ __device__ __forceinline__ void finish_dn(const MoeArgs& a, const PickInfo& R, i
         {
             float2 pv[2] = {make_float2(0.f, 0.f), make_float2(0.f, 0.f)};
             float w[2] = {0.f, 0.f};
-            half2_t sv[2] = {};
+            half2_t sv[2] = {next[0], next[1]};
             const float* rows2[2] = {a.part_d, a.part_d};
 #pragma unroll
             for (int q = 0; q < 2; ++q)
             {
-                const int kq = k + q * SB, s = b * a.topk + kq;
-                if (kq >= a.topk || R.w[s] == 0.f) continue;     // what route() saw: no second look at the table
-                w[q] = R.w[s]; rows2[q] = a.part_d + (size_t)s * a.H + col;
-
-                sv[q] = *(const half2_t*)(R.signs[s] + a.H + 3 * a.I + col);
+                const int kq = k + q * SB, s = (b * a.topk + kq) & 63;
+                if (kq >= a.topk || P.weight(s) == 0.f) continue;    // what route() saw: no second look at the table
+                w[q] = P.weight(s); rows2[q] = a.part_d + (size_t)s * a.H + col;
             }
+            const bool more = k + 2 * SB < a.topk;
+            pick_scales(a, P, more ? b : b + 1, more ? k + 2 * SB : warp, SB, col, next);
             if (w[0] == 0.f && w[1] == 0.f) continue;
             sum_partials<2>(rows2, (size_t)S * a.H, NY, pv);
 #pragma unroll
@@ -474,7 +508,7 @@ __device__ __forceinline__ void finish_dn(const MoeArgs& a, const PickInfo& R, i
                 wht128(v0, v1, lane);
                 if (w[q] == 0.f) continue;
                 v0 *= (float)sv[q].x; v1 *= (float)sv[q].y;
-                const int s = b * a.topk + k + q * SB, prd = R.lr[s] ? R.rd[s] : 0;
+                const int s = b * a.topk + k + q * SB, prd = P.rank(s);
                 if (prd)
                 {   // y += (sw V_dn^T) (U2_d [+ U4_d]): z_d summed over the I / 128 groups written by the gate|up finishers
                     const int prg = R.rg[s];
@@ -655,6 +689,8 @@ nq_gemv_k(MoeArgs a, int NC)
     else dispatch_code(P.code, [&](auto tag) { gemv_chunks<true, decltype(tag)::value, 0, false>(P, L, NC, acc, nb0); });
 
     __builtin_amdgcn_s_setprio(3);                               // the tail is a chain of latencies: nothing should wait behind decoders
+    PickLanes picks = {};
+    if constexpr (MODE == 1) picks = pick_lanes(a.route->picks, lane);
 
     // ---- k-slice partial sums: lane (t4, n) holds rows 16 (strip0 + t4 / 2) + 4 (t4 & 1) + i (+ 8 for acc[1]) of token n
     if (n < ntok)
@@ -675,13 +711,16 @@ nq_gemv_k(MoeArgs a, int NC)
     int* cnt = MODE == 0 ? a.cnt_gu + blockIdx.z * (a.I / 128) + grp : a.cnt_d + grp;
     const int expect = (MODE == 0 ? 2 : nruns) * NY * (128 / (SB * 32));
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");             // this wavefront's partial sums are acknowledged
+    half2_t scales[2] = {};
+    const int wv = __builtin_amdgcn_readfirstlane(warp);
+    if constexpr (MODE == 1) pick_scales(a, picks, 0, wv, SB, grp * 128 + 2 * lane, scales);
     __syncthreads();
     if (threadIdx.x == 0)
         last = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == expect - 1;
     __syncthreads();
     if (!last) return;                                           // block-uniform
     if constexpr (MODE == 0) finish_gu(a, R, zl, blockIdx.z, grp, NY, warp, SB, lane, last);
-    else finish_dn(a, a.route->picks, grp, NY, warp, SB, lane, (float*)smem);
+    else finish_dn(a, a.route->picks, picks, scales, grp, NY, wv, SB, lane, (float*)smem);
     if (threadIdx.x == 0) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
