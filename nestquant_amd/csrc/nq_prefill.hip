@@ -1020,17 +1020,21 @@ int launch_pf_step(const NqPfArgs& a, hipStream_t st)
                                                     mode ? nullptr : a.xu, mode ? y : acc, E, H, I, wop ? a.wop : nullptr, streams[stream_of[k]])) return rc;
             return 0;
         };
-        for (int i = 0; i < 4; ++i)
-            if (int rc = launch_pf_pre(a.x, a.x_dtype, pts, pes, n, a.table, a.xg, a.xu, a.zg, E, H, I, m.tiles, m.cap, heights[i], streams[i])) return rc;
-        if (int rc = gemms(0)) return rc;
-        for (int i = 0; i < 4; ++i)
-            if (int rc = launch_pf_mid(acc, pes, n, a.table, a.h, a.zg, a.zd, E, H, I, m.tiles, m.cap, heights[i], streams[i])) return rc;
-        if (int rc = gemms(1)) return rc;
-        for (int i = 1; i < 4; ++i)
+        auto chains = [&]() {
+            for (int i = 0; i < 4; ++i)
+                if (int rc = launch_pf_pre(a.x, a.x_dtype, pts, pes, n, a.table, a.xg, a.xu, a.zg, E, H, I, m.tiles, m.cap, heights[i], streams[i])) return rc;
+            if (int rc = gemms(0)) return rc;
+            for (int i = 0; i < 4; ++i)
+                if (int rc = launch_pf_mid(acc, pes, n, a.table, a.h, a.zg, a.zd, E, H, I, m.tiles, m.cap, heights[i], streams[i])) return rc;
+            return gemms(1);
+        };
+        const int failed = chains();
+        for (int i = 1; i < 4; ++i)                              // joined in any case: the caller gives the buffers back in its stream's order
         {
             if (int rc = hip_ok(hipEventRecord((hipEvent_t)a.events[i], streams[i]))) return rc;
             if (int rc = hip_ok(hipStreamWaitEvent(st, (hipEvent_t)a.events[i], 0))) return rc;
         }
+        if (failed) return failed;
         if (int rc = launch_pf_post(y, m.pos, a.sel, a.sel_dtype, a.rw, a.rw_dtype, a.T, a.topk, c, n, a.table, a.out, a.out_dtype, c != 0, a.zd, E, H, I, st)) return rc;
     }
     return 0;

@@ -286,7 +286,6 @@ class MoELayer:
         return out
 
 
-_PF = {}
 PF_TILES = (16, 32, 64, 128, 256)            # token-tile heights the grouped GEMM is compiled for
 # An expert with at least PF_HOT_MIN pair rows in a chunk (more than one 256-row tile) can be decoded once per call into a scratch
 # of decoded weights (at most PF_HOT_SLOTS experts at 6 H I bytes each) instead of once per tile; see nq_pf_wdecode. Off by
@@ -296,32 +295,42 @@ PF_TILES = (16, 32, 64, 128, 256)            # token-tile heights the grouped GE
 PF_HOT_MIN, PF_HOT_SLOTS = 257, 0
 
 
+_PF_REGIONS = ("xg", "xu", "acc", "h", "y", "zg", "zd")
+
+
+def _pf_offsets(H, I, R):
+    """byte offsets of _PF_REGIONS in a block for R pair rows, each on 256 bytes, and the block's size"""
+    at, off = 0, []
+    for row in (2 * H, 2 * H, 8 * I, 2 * I, 4 * H, 16, 16):
+        off.append(at)
+        at += -(-R * row // 256) * 256
+    return off, at
+
+
+def _pf_slots(R):
+    """slots of the decoded-weight scratch for R pair rows"""
+    return max(0, min(PF_HOT_SLOTS, R // PF_HOT_MIN))
+
+
 def pf_bytes(H, I, R, G=0):
     """bytes of prefill scratch for R pair rows (G is accepted for signature compatibility: the decoded-weight scratch is sized
     by the rows, not by a group of experts)"""
-    return R * (2 * H * 2 + 2 * I * 4 + I * 2 + H * 4 + 32) + max(0, min(PF_HOT_SLOTS, R // PF_HOT_MIN)) * 6 * H * I
+    return _pf_offsets(H, I, R)[1] + _pf_slots(R) * 6 * H * I
 
 
 def pf_scratch(dev, H, I, R, G=0):
-    """Prefill scratch shared by every layer of this shape on `dev`, for at least R pair rows: xg | xu fp16 [R, H], acc_gu fp32
-    [R, 2I], h fp16 [R, I], y fp32 [R, H], and wop: decoded weights of up to PF_HOT_SLOTS hot experts. One set per device and shape,
-    replaced by a larger one (rows rounded up to a power of two) when a call brings more rows than any before. Unlike the
-    reference (sm120/moe.py:263-274), which decodes every expert of a group into dense scratch, only experts with more than one
-    tile go through scratch; the others are decoded in registers inside the grouped GEMM."""
-    k = (str(dev), H, I)
-    slots = max(0, min(PF_HOT_SLOTS, R // PF_HOT_MIN))
-    S = _PF.get(k)
-    if S is None or S["rows"] < R:
-        n = 1 << (max(R, 64) - 1).bit_length()
-        f16, f32 = torch.float16, torch.float32
-        _PF.pop(k, None); S = None                   # the old set goes back to the allocator before the new one is taken
-        S = _PF[k] = dict(rows=n, wop=None, xg=torch.empty(n, H, dtype=f16, device=dev), xu=torch.empty(n, H, dtype=f16, device=dev),
-                          acc=torch.empty(n, 2 * I, dtype=f32, device=dev), h=torch.empty(n, I, dtype=f16, device=dev),
-                          y=torch.empty(n, H, dtype=f32, device=dev), zg=torch.zeros(n, 4, dtype=f32, device=dev),
-                          zd=torch.zeros(n, 4, dtype=f32, device=dev))
-    if slots != (0 if S["wop"] is None else S["wop"].shape[0]):
-        S["wop"] = torch.empty(slots, 3 * H * I, dtype=torch.float16, device=dev) if slots else None
-    return S
+    """Prefill scratch for R pair rows on `dev`, not initialised: xg | xu fp16 [R, H], acc fp32 [R, 2I], h fp16 [R, I], y fp32
+    [R, H], the low-rank plane's zg | zd fp32 [R, 4], and wop: decoded weights of up to PF_HOT_SLOTS hot experts (None without).
+    A set belongs to whoever asks for it, and every step takes one of its own from torch's allocator: what another layer, stream
+    or thread has in flight, or a captured graph holds, is never shared. Unlike the reference (sm120/moe.py:262-274), which
+    keeps one set per device and decodes every expert of a group into it, only experts with more than one tile go through
+    decoded weights; the others are decoded in registers inside the grouped GEMM."""
+    f16, f32 = torch.float16, torch.float32
+    off, size = _pf_offsets(H, I, R)
+    block, slots = torch.empty(size, dtype=torch.uint8, device=dev), _pf_slots(R)
+    S = {n: block[o:o + R * w * dt.itemsize].view(dt).view(R, w)
+         for n, o, w, dt in zip(_PF_REGIONS, off, (H, H, 2 * I, I, H, 4, 4), (f16, f16, f32, f16, f32, f32, f32))}
+    return dict(S, rows=R, wop=torch.empty(slots, 3 * H * I, dtype=f16, device=dev) if slots else None)
 
 
 def pf_tiles(segs):
@@ -340,16 +349,23 @@ def pf_tiles(segs):
 _PF_SIDE = {}
 
 
-def _pf_side(dev):
-    """three side streams (default priority) and four events of `dev`, created once"""
-    k = str(dev)
-    if k not in _PF_SIDE:
+def _pf_side(dev, stream):
+    """(streams, events, their handles): three side streams (default priority) and four events for steps that the caller puts on
+    `stream` of `dev`. An event is only ever recorded on one stream, so of two threads on one stream each waits for its own
+    work, at most for more; steps on different streams share no event (streams of torch's pool may coincide, which only orders
+    more). At most 64 sets are kept."""
+    k = (dev.index, stream)
+    S = _PF_SIDE.get(k)
+    if S is None:
         with torch.cuda.device(dev):
             side, ev = [torch.cuda.Stream(device=dev) for _ in range(3)], [torch.cuda.Event() for _ in range(4)]
             for e in ev:
-                e.record()                           # a torch event exists from its first record on
-        _PF_SIDE[k] = (side, ev, (C.c_void_p * 3)(*[st.cuda_stream for st in side]), (C.c_void_p * 4)(*[e.cuda_event for e in ev]))
-    return _PF_SIDE[k]
+                e.record(side[0])                    # a torch event exists from its first record on (not on `stream`, which may be capturing)
+        S = (side, ev, (C.c_void_p * 3)(*[st.cuda_stream for st in side]), (C.c_void_p * 4)(*[e.cuda_event for e in ev]))
+        if len(_PF_SIDE) >= 64:
+            _PF_SIDE.clear()
+        _PF_SIDE[k] = S
+    return S
 
 
 def _pf_step(s, x, sel, rw, out, R=None, table=None):
@@ -361,28 +377,31 @@ def _pf_step(s, x, sel, rw, out, R=None, table=None):
     if P == 0:
         return out.zero_()
     R = min(P, R or int(os.environ.get("NQ_PF_ROWS", "32768")))
-    S = pf_scratch(dev, H, I, R)
     nb = Lb.nq_pf_meta_bytes(T, k, R, E)
     if nb < 0:
         raise RuntimeError(Lb.nq_last_error().decode())
-    meta = torch.empty(nb, dtype=torch.uint8, device=dev)
-    _, _, side, events = _pf_side(dev)
-    whole = out if out.dtype == torch.float32 or R == P else torch.empty(T, H, dtype=torch.float32, device=dev)   # chunks add up in fp32
     # decoded-weight scratch: rows of the common kind only (the variant kernel of the others decodes in the GEMM)
-    wop = S["wop"] if (S["wop"] is not None and P >= PF_HOT_MIN and not s.rare_rows and table is None) else None
-    a = _lib.NqPfArgs()
+    slots = _pf_slots(R) if P >= PF_HOT_MIN and not s.rare_rows and table is None else 0
+    off, size = _pf_offsets(H, I, R)
+    meta_at, wop_at = size, size + -(-nb // 256) * 256
+    # one block per call, the step's own: it goes back to the allocator in the order of the caller's stream, which the side streams join
+    block = torch.empty(wop_at + slots * 6 * H * I, dtype=torch.uint8, device=dev)
+    stream = _lib.stream_ptr()
+    held = _pf_side(dev, stream)
+    whole = out if out.dtype == torch.float32 or R == P else torch.empty(T, H, dtype=torch.float32, device=dev)   # chunks add up in fp32
+    a, at = _lib.NqPfArgs(), block.data_ptr()
     a.x, a.sel, a.rw, a.table, a.out, a.hits = x.data_ptr(), sel.data_ptr(), rw.data_ptr(), tb.data_ptr(), whole.data_ptr(), s.hits_ptr or None
-    a.meta, a.meta_bytes = meta.data_ptr(), nb
-    a.xg, a.xu, a.acc, a.h, a.y, a.zg, a.zd = (S[n].data_ptr() for n in ("xg", "xu", "acc", "h", "y", "zg", "zd"))
-    if wop is not None:
-        a.wop, a.wop_bytes, a.wop_slots, a.hot_min = wop.data_ptr(), wop.numel() * 2, wop.shape[0], PF_HOT_MIN
-    a.side, a.events = side, events
+    a.meta, a.meta_bytes = at + meta_at, nb
+    a.xg, a.xu, a.acc, a.h, a.y, a.zg, a.zd = (at + o for o in off)
+    if slots:
+        a.wop, a.wop_bytes, a.wop_slots, a.hot_min = at + wop_at, slots * 6 * H * I, slots, PF_HOT_MIN
+    a.side, a.events = held[2], held[3]
     a.T, a.topk, a.E, a.H, a.I, a.rows = T, k, E, H, I, R
     a.x_dtype, a.sel_dtype, a.rw_dtype, a.out_dtype = _DT_IN[x.dtype], _DT_SEL[sel.dtype], _DT_IN[rw.dtype], _DT_OUT[whole.dtype]
     # mask mode / other base codes run in their own kernel variant; a caller's own table may hold such rows, so it gets both, and
     # a lone variant is told so: should it meet a row of the other kind after all, the result is NaN, not stale scratch
     a.variants = 3 if (s.rare_rows or table is not None) else 1
-    _lib.check(Lb.nq_pf_step(C.byref(a), _lib.stream_ptr()))
+    _lib.check(Lb.nq_pf_step(C.byref(a), stream))
     return out if whole is out else out.copy_(whole)
 
 
@@ -390,8 +409,8 @@ def prefill(s, x, sel, rw, out=None, R=None, G=None, table=None):
     """T > Bmax tokens (reference sm120/moe.py:282-326): pairs sorted by expert, each routed expert decoded inside the
     grouped GEMMs at the level of its live table row, same math as the decode path (fp32 accumulation order differs).
     No host synchronisation (the reference's prefill reads the expert counts back; here the sort and the tile lists are
-    built on the device). Exports routing hits like the decode kernel. Calls on one device share the scratch of pf_scratch()
-    (as the reference's do, sm120/moe.py:262-274) and its side streams, so they must be ordered on one stream."""
+    built on the device). Exports routing hits like the decode kernel. A call's scratch is its own (pf_scratch; the reference's calls
+    share one set per device, sm120/moe.py:262-274) and its side streams belong to the caller's stream."""
     if s.G != 4:
         raise NotImplementedError("prefill decodes rings of G = 4 lanes only (as the reference's pf_decode)")
     assert x.dtype == torch.float16 and rw.dtype == torch.float16 and sel.dtype == torch.int64, (x.dtype, rw.dtype, sel.dtype)

@@ -319,3 +319,65 @@ def test_row_kernels_against_a_float64_hadamard(H, I, n):
     gate, up = wht(acc[:, :I].double().contiguous()) * sg[:, H:H + I], wht(acc[:, I:].double().contiguous()) * sg[:, H + I:H + 2 * I]
     want = bop(wht(torch.nn.functional.silu(gate) * up * sg[:, H + 2 * I:H + 3 * I])) * live
     assert rel_err(h.cpu().double().numpy(), want.numpy()) < 5e-4
+
+
+class _StepSpy:
+    """the library, remembering of each nq_pf_step call where its scratch is and which events it records"""
+
+    def __init__(s):
+        from nestquant_amd import _lib
+        s.lib, s.calls = _lib.lib(), []
+
+    def __getattr__(s, name):
+        return getattr(s.lib, name)
+
+    def nq_pf_step(s, ref, stream):
+        a = ref._obj
+        s.calls.append((a.xg, a.y + a.rows * a.H * 4, set(a.events)))
+        return s.lib.nq_pf_step(ref, stream)
+
+
+@pytest.mark.parametrize("T,E", [(40, 40), (150, 7)])             # the one-launch plan, and the tall tiles on side streams
+def test_steps_on_two_streams_share_no_scratch_and_no_event(T, E):
+    """two layers of one shape, each on a stream of its own, with both steps in flight at once (a sleep in front of each): no
+    common scratch or event, and the results of the layers one after the other"""
+    H, I, K = 256, 256, 4
+    spy, layers, want = _StepSpy(), [], []
+    ex = to_dev(experts_on_gpu(H, I, min(E, 8), 310, nested_ids=(1, 3)))
+    for i in range(2):
+        L = M.MoELayer(E, H, I, Bmax=4, topk=K, mod=spy)
+        for e in range(E):
+            L.set(e, ex[(e + 3 * i) % len(ex)], 2)
+        g = torch.Generator().manual_seed(50 + i)
+        sel, rw = gumbel_topk(T, E, K, seed=8 + i)
+        layers.append((L, (torch.randn(T, H, generator=g) * 0.3).to(DEV), rw, sel))
+        want.append(M.forward(L, None, *layers[i][1:]))
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    for L, *a in layers:
+        for s in streams:
+            with torch.cuda.stream(s):
+                M.forward(L, None, *a)                            # the streams' first step
+    torch.cuda.synchronize()
+    for _ in range(3):
+        del spy.calls[:]
+        got = []
+        for (L, *a), s in zip(layers, streams):
+            with torch.cuda.stream(s):
+                torch.cuda._sleep(20_000_000)
+                got.append(M.forward(L, None, *a))
+        assert not streams[0].query()                             # the first step has not run when the second one is enqueued
+        (lo, hi, ev), (lo2, hi2, ev2) = spy.calls
+        assert (hi <= lo2 or hi2 <= lo) and not ev & ev2
+        torch.cuda.synchronize()
+        assert all(torch.equal(g, w) for g, w in zip(got, want))
+
+
+def test_scratch_is_as_large_as_pf_bytes_says():
+    for H, I, R in ((256, 128, 1), (6144, 2048, 777)):
+        S = None
+        before = torch.cuda.memory_allocated()
+        S = M.pf_scratch(torch.device(DEV), H, I, R)
+        assert 0 <= torch.cuda.memory_allocated() - before - M.pf_bytes(H, I, R) < 2 << 20       # the allocator's rounding
+        assert S["rows"] == R and {n: tuple(S[n].shape) for n in S if n not in ("rows", "wop")} == dict(
+            xg=(R, H), xu=(R, H), acc=(R, 2 * I), h=(R, I), y=(R, H), zg=(R, 4), zd=(R, 4))
+        assert S["wop"] is None and M.pf_scratch(torch.device(DEV), H, I, R)["xg"].data_ptr() != S["xg"].data_ptr()
