@@ -459,8 +459,9 @@ MoELayer.prefill = prefill
 
 
 PF_MIN = 384         # tokens from which a step goes through prefill() (reference NQ_PF_MIN, sm120/serve/nq_vllm.py:187)
-# Steps of more than GROUP_MIN tokens that would take more than three slices go through the grouped kernels of prefill() too (not
-# under graph capture). The reference slices up to 383 tokens into decode calls, and each slice decodes its experts anew: 48 tokens
+# Steps of more than GROUP_MIN tokens that would take more than three slices go through the grouped kernels of prefill() too, eagerly
+# and under graph capture alike (a step's scratch comes from torch's allocator, which hands out the graph's own memory then).
+# The reference slices up to 383 tokens into decode calls, and each slice decodes its experts anew: 48 tokens
 # name 200 distinct experts, their twelve slices of four 360. Measured at E = 256, top-8, Bmax 4 (slices / grouped): 9 tokens
 # 522 / 478 us, 16: 934 / 707, 48: 2650 / 1200, 201: 10900 / 1530, 383: 20800 / 1600.
 GROUP_MIN = 12
@@ -468,9 +469,9 @@ GROUP_MIN = 12
 
 def forward(layer, mailbox, x, topk_weights, topk_ids, pf_min=PF_MIN, sal=None):
     """One MoE layer step as the reference's serving caller runs it (sm120/serve/nq_vllm.py:520-574): apply the mailbox,
-    then up to Bmax tokens in one decode call, pf_min tokens or more, or more than three slices' worth, through the grouped kernels
-    of prefill() (never under graph capture), anything between in slices of Bmax tokens. x [T, H] in fp16 / bf16 / fp32, weights
-    [T, topk] likewise, ids int64 / int32;
+    then up to Bmax tokens in one decode call, more than three slices' worth through the grouped kernels of prefill(), pf_min
+    tokens or more through prefill() (under graph capture in slices, as the reference's caller does), anything between in slices of
+    Bmax tokens. x [T, H] in fp16 / bf16 / fp32, weights [T, topk] likewise, ids int64 / int32;
     returns [T, H] in x's dtype. The decode calls read the caller's dtypes and write the result dtype themselves. `sal`: an
     optional salience.Salience, fed by the decode steps as the reference does (every step of up to Bmax tokens, the slices of
     a step of up to 16 tokens; longer steps count as prefill and are left out)."""
@@ -488,8 +489,11 @@ def forward(layer, mailbox, x, topk_weights, topk_ids, pf_min=PF_MIN, sal=None):
     if T == 0:
         return torch.empty(0, layer.H, dtype=odt, device=x.device)
     out = torch.empty(T, layer.H, dtype=odt, device=x.device)
-    grouped = T >= pf_min or (T > max(GROUP_MIN, 3 * layer.Bmax) and layer.G == 4 and layer.E <= 4096)
-    if grouped and not torch.cuda.is_current_stream_capturing():
+    if T >= pf_min:
+        grouped = not torch.cuda.is_current_stream_capturing()
+    else:
+        grouped = T > max(GROUP_MIN, 3 * layer.Bmax) and layer.G == 4 and layer.E <= 4096
+    if grouped:
         if layer.G != 4 or x.dtype not in _DT_IN or w.dtype not in _DT_IN or ids.dtype not in _DT_SEL:
             return layer.prefill(x.half(), ids.long(), w.half()).to(x.dtype)
         _pf_step(layer, x, ids, w, out)

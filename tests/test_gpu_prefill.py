@@ -381,3 +381,40 @@ def test_scratch_is_as_large_as_pf_bytes_says():
         assert S["rows"] == R and {n: tuple(S[n].shape) for n in S if n not in ("rows", "wop")} == dict(
             xg=(R, H), xu=(R, H), acc=(R, 2 * I), h=(R, I), y=(R, H), zg=(R, 4), zd=(R, 4))
         assert S["wop"] is None and M.pf_scratch(torch.device(DEV), H, I, R)["xg"].data_ptr() != S["xg"].data_ptr()
+
+
+@pytest.mark.parametrize("T,E", [(13, 40), (150, 7)])             # the one-launch plan, and the tall tiles on side streams
+def test_a_captured_grouped_step_equals_the_eager_one(T, E):
+    """the same kernels under capture: equal bits on every replay, with new inputs in the graph's buffers, longer and shorter eager
+    steps and foreign memory in between"""
+    H, I, K = 256, 256, 3
+    ex = to_dev(experts_on_gpu(H, I, min(E, 8), 610, nested_ids=(1, 3)))
+    L = M.MoELayer(E, H, I, Bmax=4, topk=K)
+    for e in range(E):
+        L.set(e, ex[e % len(ex)], 4 if ex[e % len(ex)].nested else 2)
+    MB = M.Mailbox(L)
+    g = torch.Generator().manual_seed(T)
+    x = (torch.randn(T, H, generator=g) * 0.3).to(DEV).bfloat16()
+    sel, w = gumbel_topk(T, E, K, seed=2)
+    M.forward(L, MB, x, w, sel)
+    torch.cuda.synchronize()
+    st = torch.cuda.Stream()                                     # the step's first call on this stream is the captured one
+    M._PF_SIDE.pop((0, st.cuda_stream), None)
+    gr = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(gr, stream=st):
+        y = M.forward(L, MB, x, w, sel)
+    for i in range(4):
+        x.copy_((torch.randn(T, H, generator=g) * 0.3).to(DEV))
+        s2, w2 = gumbel_topk(T, E, K, seed=3 + i)
+        sel.copy_(s2); w.copy_(w2)
+        for n in (T, 3 * T, 700 + 900 * i):                      # a longer step each time: its scratch is new memory
+            xe = (torch.randn(n, H, generator=g) * 0.3).to(DEV)
+            se, we = gumbel_topk(n, E, K, seed=n)
+            M.forward(L, MB, xe, we, se)
+        want = M.forward(L, MB, x, w, sel)
+        junk = [torch.full((1 << 18,), float("nan"), device=DEV) for _ in range(8)]
+        y.fill_(float("nan"))
+        gr.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want), i
+        del junk
