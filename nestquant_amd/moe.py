@@ -138,6 +138,23 @@ _DT_SEL = {torch.int64: 0, torch.int32: 1}
 _DT_OUT = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
 
 
+_LONE = {}
+
+
+def _lone_picks(dev, E):
+    """(ids int32 [>= E, 8] with row e = e, ones fp16 [8]) of a device: the routing of a lone projection of expert e for up to eight
+    tokens. Constants, made with the first layer of a device and whole before another stream or a capture may see them."""
+    k = str(dev)
+    t = _LONE.get(k)
+    if t is None or t[0].shape[0] < E:
+        n = max(E, 256)
+        t = (torch.arange(n, dtype=torch.int32, device=dev)[:, None].repeat(1, 8), torch.ones(8, dtype=torch.float16, device=dev))
+        if t[0].is_cuda:
+            torch.cuda.current_stream(t[0].device).synchronize()
+        _LONE[k] = t
+    return t
+
+
 class MoELayer:
     """Device table [E, TBL_W] + workspaces for up to Bmax tokens; table rows are flipped in place (graph-safe).
 
@@ -165,6 +182,7 @@ class MoELayer:
         s.out = torch.zeros(Bmax, H, dtype=f32, device=dev)
         s.route = torch.zeros(_lib.ROUTE_WS_BYTES, dtype=torch.uint8, device=dev)    # the routing launch's result for the projection launches
         s.xrot = torch.zeros(S, 2, H, dtype=torch.float16, device=dev)               # and the rotated activations of every pick
+        s._lone, s._lone_views = _lone_picks(s.table.device, E), {}                  # proj_gemv
         s.hits_ptr = 0
         s.rare_rows = False                           # set once a row in mask mode or with a base window code other than 0 is
                                                       # installed (set / Mailbox.post): the decode call then runs the kernel that
@@ -579,10 +597,14 @@ def proj_gemv(layer, x, e=0, cfg=None):
         n = MoELayer._slice(C_, 2 * layer.I // 32 // sb, 1, 512, 24)
         n = next(d for d in range(n, C_ + 1) if C_ % d == 0 and C_ // d <= layer.acc_gu.shape[0])
         cfg = [1, sb, n]
-    k = (B, e, x.device)
-    if getattr(layer, "_proj_in", (None,))[0] != k:
-        layer._proj_in = (k, torch.full((B, 1), e, dtype=torch.int64, device=x.device), torch.ones(B, 1, dtype=torch.float16, device=x.device))
-    layer(x, layer._proj_in[1], layer._proj_in[2], which=1 | 8, cfg_gu=list(cfg))      # 8: the launch ends with its partial sums
+    picks = layer._lone_views.get((B, e))
+    if picks is None:
+        if 0 <= e < layer.E and B <= 8:
+            picks = layer._lone_views[B, e] = (layer._lone[0][e, :B].view(B, 1), layer._lone[1][:B].view(B, 1))
+        else:                                                     # the layer call has its answer to both
+            picks = torch.full((B, 1), e, dtype=torch.int64, device=x.device), torch.ones(B, 1, dtype=torch.float16, device=x.device)
+    sel, rw = picks
+    layer(x, sel, rw, which=1 | 8, cfg_gu=list(cfg))              # 8: the launch ends with its partial sums
     ny = C_ // (cfg[0] * cfg[2])
     n = 2 * layer.I                                               # partial sums are laid out [k-slice][B * topk of the call][2I]
     out = torch.empty(B, n, dtype=torch.float32, device=x.device)

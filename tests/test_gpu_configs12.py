@@ -260,3 +260,33 @@ def test_sum_slices_adds_in_slice_order(ny, n):
     for y in range(ny):
         want += part[y]
     assert torch.equal(out[:n], want) and bool((out[n:] == 7.0).all())
+
+
+def test_projection_captured_before_its_first_eager_call():
+    """a graph only records: what a lone projection needs beside its inputs is there from the layer's construction, so eager calls
+    and a second graph before the first replay are right, for every expert and token count"""
+    H, I, E = 256, 128, 3
+    ex = [F.Expert(H, I, seed=90 + i, dev=DEV) for i in range(E)]
+    L = M.MoELayer(E, H, I, Bmax=8, topk=1)
+    for e in range(E):
+        L.set(e, ex[e], 2)
+    g = torch.Generator().manual_seed(1)
+    x = (torch.randn(3, H, generator=g) * 0.05).half().to(DEV)
+    W = [M.dense_W(e, 0, 2, torch.float32) for e in ex]
+    had = lambda v: (v.view(3, -1, 128) @ M.H128(DEV)).view(3, H).half().float()
+    want = [torch.cat([had(x.float() * ex[e].signs[:H].float()) @ W[e][:I].T, had(x.float() * ex[e].signs[2 * H + 3 * I:].float()) @ W[e][I:].T], 1)
+            for e in range(E)]
+    torch.cuda.synchronize()
+    graphs = []
+    for e in (2, 2, 1):
+        gr = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(gr):
+            graphs.append((gr, e, M.proj_gemv(L, x, e)))
+        for f in (e, *range(E)):                                 # between capture and replay
+            assert rel_err(M.proj_gemv(L, x, f).cpu().numpy(), want[f].cpu().numpy()) < 1e-4, (e, f)
+    for gr, e, y in graphs * 2:
+        y.fill_(float("nan"))
+        gr.replay()
+        assert rel_err(y.cpu().numpy(), want[e].cpu().numpy()) < 1e-4, e
+    for f in range(E):
+        assert rel_err(M.proj_gemv(L, x[:1], f).cpu().numpy(), want[f][:1].cpu().numpy()) < 1e-4
