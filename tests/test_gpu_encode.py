@@ -85,3 +85,19 @@ def test_block_word_fit_equals_the_torch_form(U, K, signed, metric):
     _lib.check(_lib.lib().nq_fit_residual(*[None if t is None else t.data_ptr() for t in args], 1.1, U, out.data_ptr(), None))
     torch.cuda.synchronize()
     assert torch.allclose(out.cpu(), (r / s0[:, None, None]).float(), rtol=2e-7, atol=0)
+
+
+def test_viterbi_search_looks_at_its_codebook():
+    """a short codebook raises as the torch form does; one that fp32 cannot hold, or of another layout, takes the torch form"""
+    g = torch.Generator().manual_seed(3)
+    w = torch.randn(2, 9, generator=g)
+    lut = EN.codebook()
+    for bad in (lut[:65535], lut[:16], lut[:0]):
+        for dev in ("cpu", "cuda"):
+            with pytest.raises(IndexError):
+                EN.viterbi_ring(w.to(dev), bad.to(dev))
+    with pytest.raises(RuntimeError):
+        EN.viterbi_ring(w.cuda(), lut)                            # on another device
+    near = lut.double() + 1e-9 * torch.randn(1 << 16, generator=g, dtype=torch.float64)
+    for other in (near, lut.half(), lut.repeat(2), lut.repeat_interleave(2)[::2], (lut * 16).round().int()):
+        assert torch.equal(EN.viterbi_ring(w.cuda(), other.cuda()).cpu(), EN.viterbi_ring(w, other)), other.dtype
