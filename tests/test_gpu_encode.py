@@ -101,3 +101,21 @@ def test_viterbi_search_looks_at_its_codebook():
     near = lut.double() + 1e-9 * torch.randn(1 << 16, generator=g, dtype=torch.float64)
     for other in (near, lut.half(), lut.repeat(2), lut.repeat_interleave(2)[::2], (lut * 16).round().int()):
         assert torch.equal(EN.viterbi_ring(w.cuda(), other.cuda()).cpu(), EN.viterbi_ring(w, other)), other.dtype
+
+
+def test_second_plane_search_looks_at_its_inputs():
+    """windows of another shape, type or device and short codebooks do on the GPU what they do in torch on the CPU"""
+    g = torch.Generator().manual_seed(4)
+    w, lut = torch.randn(3, 6, generator=g), EN.codebook()
+    win = lambda *s: torch.randint(0, 256, s, generator=g)
+    for a in (win(1, 6), win(3, 9), win(3, 6).int(), win(3, 6).short()):
+        assert torch.equal(EN.viterbi_ring_given_p3(w.cuda(), a.cuda(), lut.cuda()).cpu(), EN.viterbi_ring_given_p3(w, a, lut)), (a.shape, a.dtype)
+    near = lut.double() + 1e-9 * torch.randn(1 << 16, generator=g, dtype=torch.float64)
+    assert torch.equal(EN.viterbi_ring_given_p3(w.cuda(), win(3, 6).cuda().fill_(5), near.cuda()).cpu(), EN.viterbi_ring_given_p3(w, win(3, 6).fill_(5), near))
+    for bad in (win(3, 5), win(2, 6), win(6), torch.rand(3, 6)):
+        with pytest.raises((IndexError, RuntimeError)):
+            EN.viterbi_ring_given_p3(w.cuda(), bad.cuda(), lut.cuda())
+    with pytest.raises(RuntimeError):
+        EN.viterbi_ring_given_p3(w.cuda(), win(3, 6), lut.cuda())
+    with pytest.raises(IndexError):
+        EN.viterbi_ring_given_p3(w.cuda(), win(3, 6).cuda(), lut.cuda()[:4096])
