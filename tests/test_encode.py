@@ -5,6 +5,7 @@ closed form and by exhaustive search, and decode(encode) through the oracle at e
 import itertools
 
 import numpy as np
+import pytest
 import torch
 
 from nestquant_amd import encode as EN
@@ -349,3 +350,19 @@ def test_low_rank_plane_detect_metric_fit():
     cost = lambda D: float((((W.double() - D.double()) @ H) * (W.double() - D.double())).sum())
     assert cost(w2) < 0.75 * cost(d2) and cost(w4) < 0.75 * cost(d4)   # the span holds 57 of H's trace of 183.5
     assert w4.dtype == torch.float32 and float((w4 - d4 - (U2.float() + U4.float()).T @ V.float()).abs().max()) < 1e-3
+
+
+@pytest.mark.parametrize("shape", [(2, 128), (2, 300), (2, 1), (2, 2, 256), (256,)])
+def test_ring_searches_refuse_rings_of_another_length(shape, monkeypatch):
+    """also where the search would go to a kernel, which takes any length up to 1024"""
+    searched = []
+    monkeypatch.setattr(EN, "_native", lambda *a: True)
+    monkeypatch.setattr(EN, "_viterbi_gpu", lambda *a: searched.append(a))
+    monkeypatch.setattr(EN, "_viterbi_p4_gpu", lambda *a: searched.append(a))
+    with pytest.raises(IndexError):
+        EN.viterbi_rings(torch.zeros(*shape), 2)
+    with pytest.raises(IndexError):
+        EN.viterbi_rings_given_p3(torch.zeros(*shape), torch.zeros(*shape, dtype=torch.int64))
+    with pytest.raises(IndexError):
+        EN.viterbi_rings_given_p3(torch.zeros(2, 256), torch.zeros(*shape, dtype=torch.int64))
+    assert not searched
