@@ -119,3 +119,29 @@ def test_second_plane_search_looks_at_its_inputs():
         EN.viterbi_ring_given_p3(w.cuda(), win(3, 6), lut.cuda())
     with pytest.raises(IndexError):
         EN.viterbi_ring_given_p3(w.cuda(), win(3, 6).cuda(), lut.cuda()[:4096])
+
+
+def test_block_word_fit_looks_at_its_inputs():
+    """states, signs and scales of another type or shape do on the GPU what they do in torch on the CPU: int32 states count as the
+    same states, broadcast ones are broadcast, others raise"""
+    g = torch.Generator().manual_seed(5)
+    U = 3
+    st, res = (torch.randint(0, 1 << 16, (U, 8, 256), generator=g) for _ in range(2))
+    target = EN.codebook()[st] + 0.2 * EN.codebook()[res]
+    sign = (torch.randint(0, 2, (U, 8, 1), generator=g) * 2 - 1).float()
+    dev = lambda t: t.cuda() if isinstance(t, torch.Tensor) else t
+    want = EN.encode_residual(target, st, 1, states=res)
+    for a, b in ((st.int(), res), (st, res.int())):
+        got = EN.encode_residual(target.cuda(), a.cuda(), 1, states=b.cuda())
+        assert all(torch.equal(got[k].cpu(), want[k]) for k in ("Mb", "N", "Q", "states"))
+    for base, kw in ((st[:1], dict(states=res)), (st, dict(states=res[:1])), (st, dict(states=res, sign=sign[:1])),
+                     (st, dict(states=res, sign=sign.expand(U, 8, 256))), (st, dict(states=res, sign=sign.double())),
+                     (st, dict(states=res, scale=torch.tensor([1.0, 1.1, 1.2]))), (st.transpose(1, 2).contiguous().transpose(1, 2), dict(states=res))):
+        want = EN.encode_residual(target, base, 1, **kw)
+        got = EN.encode_residual(target.cuda(), base.cuda(), 1, **{k: dev(v) for k, v in kw.items()})
+        assert got["Q"].dtype == want["Q"].dtype and all(torch.equal(got[k].cpu(), want[k]) for k in ("Mb", "N", "Q")), (base.shape, list(kw))
+    for base, b in ((st[:2], res), (st[:, :4], res), (st.reshape(U, 2048), res), (st, res[:, :, :128]), (st.float(), res), (st, res.float())):
+        with pytest.raises((RuntimeError, NotImplementedError)):
+            EN.encode_residual(target.cuda(), base.cuda(), 1, states=b.cuda())
+    with pytest.raises(RuntimeError):
+        EN.encode_residual(target.cuda(), st.cuda(), 1, states=res)                   # on another device
