@@ -366,3 +366,24 @@ def test_ring_searches_refuse_rings_of_another_length(shape, monkeypatch):
     with pytest.raises(IndexError):
         EN.viterbi_rings_given_p3(torch.zeros(2, 256), torch.zeros(*shape, dtype=torch.int64))
     assert not searched
+
+
+@pytest.mark.parametrize("both", [False, True])
+def test_a_metric_alone_is_the_cost(both):
+    """metric without a cost function: the block words that the same cost picks, also in torch"""
+    g = torch.Generator().manual_seed(9)
+    U = 4
+    st, res = (torch.randint(0, 1 << 16, (U, 8, 256), generator=g) for _ in range(2))
+    target = EN.codebook()[st] + 0.3 * torch.randn(U, 8, 256, generator=g)
+    spd = lambda n: (lambda X: X @ X.transpose(-1, -2) / n)(torch.randn(U, n, n // 8, generator=g, dtype=torch.float64))
+    Da, Do = spd(128), spd(16) if both else None
+
+    def cost(E):
+        X = EN.from_rings(E.reshape(-1, 256), 16 * U, 128).reshape(U, 16, 128)
+        Y = X @ Da
+        return ((Do @ Y if both else Y) * X).sum((1, 2))
+    want = EN.encode_residual(target, st, 1, states=res, cost=cost)
+    got = EN.encode_residual(target, st, 1, states=res, metric=(Da, Do))
+    plain = EN.encode_residual(target, st, 1, states=res)
+    assert all(torch.equal(got[k], want[k]) for k in ("Mb", "N", "Q"))
+    assert not (torch.equal(plain["Mb"], want["Mb"]) and torch.equal(plain["N"], want["N"]))       # the metric matters here
