@@ -387,3 +387,8 @@ def test_a_metric_alone_is_the_cost(both):
     plain = EN.encode_residual(target, st, 1, states=res)
     assert all(torch.equal(got[k], want[k]) for k in ("Mb", "N", "Q"))
     assert not (torch.equal(plain["Mb"], want["Mb"]) and torch.equal(plain["N"], want["N"]))       # the metric matters here
+
+
+def test_constant_tables_take_keywords():
+    assert torch.equal(EN.codebook(dev="cpu", state_bits=8), EN.codebook("cpu", 8)) and EN.codebook(state_bits=8).shape == (256,)
+    assert torch.equal(EN.ring_index(dev="cpu"), EN.ring_index()) and torch.equal(EN.hadamard128(dev="cpu"), EN.hadamard128())
