@@ -392,3 +392,13 @@ def test_a_metric_alone_is_the_cost(both):
 def test_constant_tables_take_keywords():
     assert torch.equal(EN.codebook(dev="cpu", state_bits=8), EN.codebook("cpu", 8)) and EN.codebook(state_bits=8).shape == (256,)
     assert torch.equal(EN.ring_index(dev="cpu"), EN.ring_index()) and torch.equal(EN.hadamard128(dev="cpu"), EN.hadamard128())
+
+
+def test_constant_tables_are_the_callers_to_change():
+    W = torch.randn(128, 128, generator=torch.Generator().manual_seed(1))
+    want = EN.blocked_had(W, 1)
+    for get in (EN.codebook, EN.ring_index, EN.hadamard128):
+        kept = get().clone()
+        get().mul_(0)
+        assert torch.equal(get(), kept), get.__name__
+    assert torch.equal(EN.blocked_had(W, 1), want)
