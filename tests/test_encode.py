@@ -402,3 +402,32 @@ def test_constant_tables_are_the_callers_to_change():
         get().mul_(0)
         assert torch.equal(get(), kept), get.__name__
     assert torch.equal(EN.blocked_had(W, 1), want)
+
+
+def test_constant_tables_do_not_depend_on_who_asked_first(monkeypatch):
+    """the current device, the default type and inference mode of the first caller are not the next one's"""
+    monkeypatch.setattr(EN, "_CONST", {})
+    made = []
+
+    @EN._per_device
+    def table(dev="cpu", n=2):
+        made.append(torch.device(dev))
+        return torch.ones(n)
+    current = [1]
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: current[0])
+    table("cuda"); table("cuda:1")
+    current[0] = 0
+    table("cuda"); table(torch.device("cuda", 0))
+    assert made == [torch.device("cuda", 1), torch.device("cuda", 0)]
+    torch.set_default_dtype(torch.float64)
+    try:
+        double = EN.hadamard128()
+    finally:
+        torch.set_default_dtype(torch.float32)
+    assert double.dtype == torch.float64 and EN.hadamard128().dtype == torch.float32
+    EN._CONST.clear()
+    with torch.inference_mode():
+        EN.hadamard128()
+    W = torch.ones(1, 128, requires_grad=True)
+    EN.blocked_had(W, 1).sum().backward()
+    assert W.grad is not None
