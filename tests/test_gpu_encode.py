@@ -145,3 +145,17 @@ def test_block_word_fit_looks_at_its_inputs():
             EN.encode_residual(target.cuda(), base.cuda(), 1, states=b.cuda())
     with pytest.raises(RuntimeError):
         EN.encode_residual(target.cuda(), st.cuda(), 1, states=res)                   # on another device
+
+
+def test_side_stream_of_a_fit_outlives_another_threads_clean_up(monkeypatch):
+    """a thread that drops the kept side streams between two steps of another one"""
+    class Emptied(dict):
+        def __setitem__(s, k, v):
+            super().__setitem__(k, v)
+            s.clear()
+    monkeypatch.setattr(EN, "_SIDE", Emptied())
+    W = torch.randn(128, 128, generator=torch.Generator().manual_seed(2)).cuda()
+    a = EN.encode_nested(W)
+    monkeypatch.undo()
+    b = EN.encode_nested(W)
+    assert all(torch.equal(a[k], b[k]) for k in ("base", "p3", "d3", "p4", "d4"))
