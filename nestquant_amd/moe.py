@@ -497,7 +497,8 @@ def forward(layer, mailbox, x, topk_weights, topk_ids, pf_min=PF_MIN, sal=None):
     x, w, ids = x.contiguous(), topk_weights.contiguous(), topk_ids.contiguous()
     odt = x.dtype if x.dtype in _DT_OUT else torch.float32
     if 0 < T <= layer.Bmax:
-        inside = hasattr(sal, "acc") and ids.shape[1] <= 8 and sal.acc.numel() == layer.E       # a Salience: exported by the call itself
+        # a Salience whose call is its own, with operands that call would take: exported by the layer call itself
+        inside = getattr(type(sal).__call__, "layer_can", False) and ids.shape[1] <= 8 and sal.acc.numel() == layer.E
         if sal is not None and not inside:
             sal(x, w, ids)
         return layer(x, ids, w, out=torch.empty(T, layer.H, dtype=odt, device=x.device), mailbox=mailbox,   # applied by the call's last launch, for the next step

@@ -45,3 +45,5 @@ class Salience:
 
     def __call__(s, x, w, ids):
         sal(x, w, ids, s.rsf, s.acc, s.host.data_ptr())
+
+    __call__.layer_can = True         # the layer call's routing launch does the same (moe.forward asks); what a subclass does instead, it does not

@@ -154,3 +154,40 @@ def test_salience_inside_the_layer_call_is_the_launch_in_front_of_it(T, K, H, xd
     assert A.acc.sum() > 0 or K == 1
     # the two launches have 512 and 256 threads, so their fp32 norms add up in different orders
     assert torch.allclose(A.acc, B.acc, rtol=1e-6, atol=0) and torch.equal(B.host, B.acc.cpu())
+
+
+def _host_salience(cls, E):
+    s = object.__new__(cls)                                       # without the pinned mirror, which needs a GPU
+    s.acc, s.host, s.rsf = torch.zeros(E, dtype=torch.float64), torch.zeros(E, dtype=torch.float64), 1.0
+    return s
+
+
+class _LayerStub:
+    """what moe.forward asks of a layer for a decode call; remembers which salience the call was to export"""
+    H, E, Bmax, G = 128, 6, 4, 4
+
+    def __call__(s, x, sel, rw, out=None, mailbox=None, sal=None):
+        s.sal = sal
+        return out
+
+
+def test_a_salience_with_a_call_of_its_own_is_called():
+    from nestquant_amd import moe as M, salience as SAL
+    x, w, ids = torch.zeros(2, 128), torch.ones(2, 3), torch.zeros(2, 3, dtype=torch.int64)
+
+    class Doubled(SAL.Salience):
+        def __call__(s, x, w, ids):
+            calls.append(s)
+
+    class Other:
+        acc = torch.zeros(6, dtype=torch.float64)
+
+        def __call__(s, x, w, ids):
+            calls.append(s)
+    for own in (_host_salience(Doubled, 6), Other()):
+        calls, L = [], _LayerStub()
+        M.forward(L, None, x, w, ids, sal=own)
+        assert calls == [own] and L.sal is None
+    L, plain = _LayerStub(), _host_salience(SAL.Salience, 6)
+    M.forward(L, None, x, w, ids, sal=plain)
+    assert L.sal is plain
