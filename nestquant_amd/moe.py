@@ -498,7 +498,8 @@ def forward(layer, mailbox, x, topk_weights, topk_ids, pf_min=PF_MIN, sal=None):
     odt = x.dtype if x.dtype in _DT_OUT else torch.float32
     if 0 < T <= layer.Bmax:
         # a Salience whose call is its own, with operands that call would take: exported by the layer call itself
-        inside = getattr(type(sal).__call__, "layer_can", False) and ids.shape[1] <= 8 and sal.acc.numel() == layer.E
+        inside = getattr(type(sal).__call__, "layer_can", False) and ids.shape[1] <= 8 and sal.acc.numel() == layer.E \
+            and sal.acc.dtype == torch.float64 and sal.acc.is_contiguous() and w.numel() == ids.numel() == T * ids.shape[1]
         if sal is not None and not inside:
             sal(x, w, ids)
         return layer(x, ids, w, out=torch.empty(T, layer.H, dtype=odt, device=x.device), mailbox=mailbox,   # applied by the call's last launch, for the next step

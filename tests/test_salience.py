@@ -191,3 +191,15 @@ def test_a_salience_with_a_call_of_its_own_is_called():
     L, plain = _LayerStub(), _host_salience(SAL.Salience, 6)
     M.forward(L, None, x, w, ids, sal=plain)
     assert L.sal is plain
+
+
+def test_salience_operands_are_looked_at_either_way():
+    """what the salience call refuses is not left to the routing launch, which would not notice"""
+    from nestquant_amd import moe as M, salience as SAL
+    x, w, ids = torch.zeros(2, 128, dtype=torch.float16), torch.ones(2, 3, dtype=torch.float16), torch.zeros(2, 3, dtype=torch.int64)
+    for acc, ww in ((torch.zeros(6), w), (torch.zeros(6, dtype=torch.int64), w), (torch.zeros(12, dtype=torch.float64)[::2], w),
+                    (torch.zeros(6, dtype=torch.float64), w[:, :2])):
+        s = _host_salience(SAL.Salience, 6)
+        s.acc = acc
+        with pytest.raises(RuntimeError):
+            M.forward(_LayerStub(), None, x, ww, ids, sal=s)
