@@ -509,12 +509,13 @@ def forward(layer, mailbox, x, topk_weights, topk_ids, pf_min=PF_MIN, sal=None):
     if T == 0:
         return torch.empty(0, layer.H, dtype=odt, device=x.device)
     out = torch.empty(T, layer.H, dtype=odt, device=x.device)
+    plain = layer.G == 4 and x.dtype in _DT_IN and w.dtype in _DT_IN and ids.dtype in _DT_SEL
     if T >= pf_min:
         grouped = not torch.cuda.is_current_stream_capturing()
-    else:
-        grouped = T > max(GROUP_MIN, 3 * layer.Bmax) and layer.G == 4 and layer.E <= 4096
+    else:                                            # what the slices refuse stays refused
+        grouped = T > max(GROUP_MIN, 3 * layer.Bmax) and plain and layer.E <= 4096
     if grouped:
-        if layer.G != 4 or x.dtype not in _DT_IN or w.dtype not in _DT_IN or ids.dtype not in _DT_SEL:
+        if not plain:
             return layer.prefill(x.half(), ids.long(), w.half()).to(x.dtype)
         _pf_step(layer, x, ids, w, out)
         for i in range(0, T if sal is not None and T <= 16 and T < pf_min else 0, layer.Bmax):
