@@ -2,7 +2,9 @@
 //   nq_dequant_k   : one projection of one expert (the reference's NQ_WDUMP debug dump, sm120/nqmoe.cu:246-288,852-853)
 //   nq_pf_decode_k : G experts, both projections (reference nq_pf_decode, sm120/nqmoe.cu:1013-1080)
 // A wavefront decodes two adjacent units (64 records = 1 KiB of base codes, one coalesced load), stages the 2 x 16 x 128
-// fp16 tile in LDS and writes 256-byte row segments. HBM-bound on the fp16 writes: 2 B written per 0.25-0.5 B read.
+// fp16 tile in LDS and writes 256-byte row segments, one pair per wavefront: a loop over pairs, with its fence and barrier behind the
+// stores, costs 11 % (16 experts of 6144 x 2048 at level 3, us per expert: 22.2 with it, 19.7 without; level 4 21.9 and 19.2, level 2
+// 16.2 and 16.5; torch fills the same memory in 11.0).
 #include "nq_decode.hpp"
 #include "nq_host.hpp"
 
@@ -91,38 +93,32 @@ __device__ __forceinline__ void store_tile(const uint32_t* tile, _Float16* out, 
     }
 }
 
-// projection `mode` (0 gate|up [2I][H], 1 down [H][I]) of the planes P at level lv -> out; wavefront `wave` of `nwaves` takes every
-// nwaves-th pair of units
-__device__ __forceinline__ void dequant_body(const Planes& P, int mode, int lv, int H, int I, _Float16* out, int wave, int nwaves, uint32_t* tiles)
+// units 2 pair and 2 pair + 1 of projection `mode` (0 gate|up [2I][H], 1 down [H][I]) of the planes P at level lv -> out
+__device__ __forceinline__ void dequant_body(const Planes& P, int mode, int lv, int H, int I, _Float16* out, int pair, uint32_t* tiles)
 {
     const int lane = threadIdx.x & 63, half = lane >> 5;
     const int N = mode == 0 ? 2 * I : H, K = mode == 0 ? H : I, C = K / 128;
     const size_t nunits = (size_t)(N / 16) * C, nrec = nunits * 32;
-    const int npairs = (int)((nunits + 1) / 2);
+    size_t unit = (size_t)pair * 2 + half;
+    const bool live = unit < nunits;
+    if ((size_t)pair * 2 >= nunits) return;                      // wave-uniform: the last workgroup's spare wavefronts
+    if (!live) unit = nunits - 1;                                // keep the wave convergent for the shuffles
     uint32_t* tile = tiles + half * 16 * TS;
-    for (int pair = wave; pair < npairs; pair += nwaves)         // wave-uniform
+    if (lv <= 0)
     {
-        size_t unit = (size_t)pair * 2 + half;
-        const bool live = unit < nunits;
-        if (!live) unit = nunits - 1;                            // keep the wave convergent for the shuffles
-        if (lv <= 0)
-        {
-            _Float16* dst = out + (size_t)(unit / C) * 16 * K + (size_t)(unit % C) * 128;
-            if (live) for (int i = lane & 31; i < 256; i += 32) *(uint4*)(dst + (size_t)(i >> 4) * K + (i & 15) * 8) = make_uint4(0, 0, 0, 0);
-            continue;
-        }
-        decode_unit(P, lv, unit, nrec, C, tile, lane);
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        // each half-wave wrote its own tile; the whole wave now drains both tiles
-        for (int h = 0; h < 2; ++h)
-        {
-            const size_t u = (size_t)pair * 2 + h;
-            if (u >= nunits) break;
-            store_tile(tiles + h * 16 * TS, out + (size_t)(u / C) * 16 * K + (size_t)(u % C) * 128, K, lane);
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();                         // the tiles are free again
+        _Float16* dst = out + (size_t)(unit / C) * 16 * K + (size_t)(unit % C) * 128;
+        if (live) for (int i = lane & 31; i < 256; i += 32) *(uint4*)(dst + (size_t)(i >> 4) * K + (i & 15) * 8) = make_uint4(0, 0, 0, 0);
+        return;
+    }
+    decode_unit(P, lv, unit, nrec, C, tile, lane);
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    // each half-wave wrote its own tile; the whole wave now drains both tiles
+    for (int h = 0; h < 2; ++h)
+    {
+        const size_t u = (size_t)pair * 2 + h;
+        if (u >= nunits) break;
+        store_tile(tiles + h * 16 * TS, out + (size_t)(u / C) * 16 * K + (size_t)(u % C) * 128, K, lane);
     }
 }
 
@@ -130,14 +126,14 @@ __global__ void __launch_bounds__(256) nq_dequant_k(const int64_t* __restrict__ 
 {
     __shared__ __align__(16) uint32_t tiles[4][2 * 16 * TS];
     const int warp = threadIdx.x >> 6;
-    dequant_body(planes_of(ent, mode), mode, level ? level : (int)ent[0], H, I, out, blockIdx.x * 4 + warp, gridDim.x * 4, tiles[warp]);
+    dequant_body(planes_of(ent, mode), mode, level ? level : (int)ent[0], H, I, out, blockIdx.x * 4 + warp, tiles[warp]);
 }
 // the same with the planes as kernel arguments
 __global__ void __launch_bounds__(256) nq_dequant_row_k(Planes P, int mode, int lv, int H, int I, _Float16* out)
 {
     __shared__ __align__(16) uint32_t tiles[4][2 * 16 * TS];
     const int warp = threadIdx.x >> 6;
-    dequant_body(P, mode, lv, H, I, out, blockIdx.x * 4 + warp, gridDim.x * 4, tiles[warp]);
+    dequant_body(P, mode, lv, H, I, out, blockIdx.x * 4 + warp, tiles[warp]);
 }
 
 // grid (ceil(pairs / 4), G, 2): Wgu [G][2I][H], Wdn [G][H][I]; level from the live table row; level <= 0 -> zeros
@@ -149,14 +145,14 @@ __global__ void __launch_bounds__(256) nq_pf_decode_k(const int64_t* __restrict_
     const int N = mode == 0 ? 2 * I : H, K = mode == 0 ? H : I;
     const int64_t* ent = table + (int64_t)experts[gi] * TBL_W;
     _Float16* out = (mode == 0 ? Wgu : Wdn) + (size_t)gi * N * K;
-    dequant_body(planes_of(ent, mode), mode, (int)ent[0], H, I, out, blockIdx.x * 4 + warp, gridDim.x * 4, tiles[warp]);
+    dequant_body(planes_of(ent, mode), mode, (int)ent[0], H, I, out, blockIdx.x * 4 + warp, tiles[warp]);
 }
 
 static int dequant_blocks(int proj, int H, int I)
 {
     const int N = proj == 0 ? 2 * I : H, K = proj == 0 ? H : I;
     const int npairs = ((N / 16) * (K / 128) + 1) / 2;
-    return (npairs + 3) / 4;                                     // one pair per wavefront: 384 to 1024 workgroups walking several pairs each take as long
+    return (npairs + 3) / 4;                                     // a pair per wavefront
 }
 
 int launch_dequant(const int64_t* row, int proj, int level, int H, int I, void* out, hipStream_t st)
