@@ -954,10 +954,15 @@ static PfMeta pf_meta(void* ws, int P, int R, int E)
     return m;
 }
 
-// Steps whose experts hold few rows each take the one-launch plan of short tiles. The line: at 32 pair rows per expert on average
-// hardly an expert of an even routing exceeds one 64-row tile, and what a skewed routing's few popular ones decode twice costs
-// less than the side streams' extra launches and the taller bodies' lower occupancy; above it the tall tiles save decodes.
-static bool pf_is_short(int64_t P, int E) { return P <= 32 * (int64_t)E; }
+// Which steps take the one-launch plan of short tiles. An expert of n rows is decoded n / 64 times there, n / 256 times by the tall
+// tiles, which cost side streams, a launch per height and lower occupancy: about 0.1 ms a step. us short / tall:
+//   few rows per expert, up to 32 on average (E = 256 of 6144 x 2048, top-8, all level 4): even routing of 200 tokens 2301 / 2342, 400
+//   2351 / 2537, 1000 2756 / 2913; Zipf(1.1) popularity 200 1977 / 2126, 400 2470 / 2416, 1000 3173 / 2999, where the popular experts'
+//   further decodes cost up to 6 %. Beyond the line 1400 tokens 3058 / 3271 and 3641 / 3336, 2048 4203 / 3924 and 4437 / 3896.
+//   little work beside the 0.1 ms, rows * H * I <= 2^34 (a decode's price goes with H I): 512 x 256, 16 experts, 1000 tokens
+//   51 / 141; 2048 x 1024, 64 experts, 750 tokens 217 / 277; 6144 x 2048, 8 experts, 93 tokens 146 / 201. At the line 0.84 to 1.02 of
+//   tall over ten shapes, at twice the line 1.06 to 1.27 for all but one.
+static bool pf_is_short(int64_t P, int E, int H, int I) { return P <= 32 * (int64_t)E || P * H * I <= (int64_t)1 << 34; }
 
 template <bool MASKED>
 static int launch_short(const PfGemm& a, int ntiles, int N, hipStream_t st)
@@ -972,7 +977,7 @@ int launch_pf_step(const NqPfArgs& a, hipStream_t st)
     const int P = a.T * a.topk, R = a.rows < P ? a.rows : P, E = a.E, H = a.H, I = a.I;
     const PfMeta m = pf_meta(a.meta, P, R, E);
     if (m.bytes > (size_t)a.meta_bytes) return set_error("nq_pf_step: meta needs %zu bytes, has %lld", m.bytes, (long long)a.meta_bytes);
-    const bool brief = R == P && !a.wop && pf_is_short(P, E);
+    const bool brief = R == P && !a.wop && pf_is_short(P, E, H, I);
     {
         const PfSort s{a.sel, a.rw, a.sel_dtype, a.rw_dtype, P, a.topk, E, a.table, m.cnt, m.pe, m.pt, m.pos, a.hits, brief ? m.tiles : nullptr, m.scap};
         const int shm = SORT_TILE * 2 + 3 * (E + 1) * 4;

@@ -253,14 +253,25 @@ def test_row_restricted_pre_and_mid_cover_the_rows_of_their_heights_exactly():
 
 @pytest.mark.parametrize("T,E,K,Bmax,xd,wd,sd", [
     (13, 40, 4, 4, torch.bfloat16, torch.float32, torch.int32),        # first grouped size, one-launch plan, rows of every height it has
-    (150, 7, 3, 2, torch.float32, torch.bfloat16, torch.int64),        # 64 rows per expert and more: tall tiles on side streams
+    (150, 7, 3, 2, torch.float32, torch.bfloat16, torch.int64),        # 64 rows per expert and more: several short tiles of one expert
     (229, 300, 8, 8, torch.float16, torch.float16, torch.int32),       # more experts than a workgroup of the sort has threads' worth of groups
     (5600, 4, 3, 4, torch.float16, torch.float32, torch.int64),        # more pairs than the sort keeps in LDS at a time
 ])
 def test_grouped_step_equals_the_decode_slices(T, E, K, Bmax, xd, wd, sd):
     """moe.forward between the decode call and the long prompts: caller dtypes, ids outside the table, zero weights, an expert at
     level 0, hits -- against fp32 decode slices of the same layer"""
-    H, I = 256, 256
+    grouped_step_against_slices(256, 256, T, E, K, Bmax, xd, wd, sd)
+
+
+@pytest.mark.parametrize("H,I,T,E,K,Bmax,xd,wd,sd", [
+    (2560, 2304, 383, 9, 8, 4, torch.float32, torch.bfloat16, torch.int64),     # just beyond the one-launch plan: tall tiles on side streams
+    (2048, 1024, 5500, 4, 2, 8, torch.bfloat16, torch.float32, torch.int32),    # many 256-row tiles
+])
+def test_tall_grouped_step_equals_the_decode_slices(H, I, T, E, K, Bmax, xd, wd, sd):
+    grouped_step_against_slices(H, I, T, E, K, Bmax, xd, wd, sd)
+
+
+def grouped_step_against_slices(H, I, T, E, K, Bmax, xd, wd, sd):
     ex = to_dev(experts_on_gpu(H, I, min(E, 12), 70, nested_ids=(1, 3)))
     L = M.MoELayer(E, H, I, Bmax=Bmax, topk=K)
     for e in range(E):
@@ -337,13 +348,12 @@ class _StepSpy:
         return s.lib.nq_pf_step(ref, stream)
 
 
-@pytest.mark.parametrize("T,E", [(40, 40), (150, 7)])             # the one-launch plan, and the tall tiles on side streams
-def test_steps_on_two_streams_share_no_scratch_and_no_event(T, E):
+@pytest.mark.parametrize("H,I,T,E,K", [(256, 256, 40, 40, 4), (2560, 2304, 383, 8, 8)])      # the one-launch plan, and the tall tiles on side streams
+def test_steps_on_two_streams_share_no_scratch_and_no_event(H, I, T, E, K):
     """two layers of one shape, each on a stream of its own, with both steps in flight at once (a sleep in front of each): no
     common scratch or event, and the results of the layers one after the other"""
-    H, I, K = 256, 256, 4
     spy, layers, want = _StepSpy(), [], []
-    ex = to_dev(experts_on_gpu(H, I, min(E, 8), 310, nested_ids=(1, 3)))
+    ex = to_dev(experts_on_gpu(H, I, min(E, 4), 310, nested_ids=(1, 3)))
     for i in range(2):
         L = M.MoELayer(E, H, I, Bmax=4, topk=K, mod=spy)
         for e in range(E):
@@ -383,12 +393,11 @@ def test_scratch_is_as_large_as_pf_bytes_says():
         assert S["wop"] is None and M.pf_scratch(torch.device(DEV), H, I, R)["xg"].data_ptr() != S["xg"].data_ptr()
 
 
-@pytest.mark.parametrize("T,E", [(13, 40), (150, 7)])             # the one-launch plan, and the tall tiles on side streams
-def test_a_captured_grouped_step_equals_the_eager_one(T, E):
+@pytest.mark.parametrize("H,I,T,E,K", [(256, 256, 13, 40, 3), (2560, 2304, 383, 8, 8)])      # the one-launch plan, and the tall tiles on side streams
+def test_a_captured_grouped_step_equals_the_eager_one(H, I, T, E, K):
     """the same kernels under capture: equal bits on every replay, with new inputs in the graph's buffers, longer and shorter eager
     steps and foreign memory in between"""
-    H, I, K = 256, 256, 3
-    ex = to_dev(experts_on_gpu(H, I, min(E, 8), 610, nested_ids=(1, 3)))
+    ex = to_dev(experts_on_gpu(H, I, min(E, 4), 610, nested_ids=(1, 3)))
     L = M.MoELayer(E, H, I, Bmax=4, topk=K)
     for e in range(E):
         L.set(e, ex[e % len(ex)], 4 if ex[e % len(ex)].nested else 2)
