@@ -427,3 +427,76 @@ def test_a_captured_grouped_step_equals_the_eager_one(H, I, T, E, K):
         torch.cuda.synchronize()
         assert torch.equal(y, want), i
         del junk
+
+
+@pytest.mark.parametrize("H,I", [(640, 384), (256, 1024)])
+def test_row_kernels_keep_infinities_and_nan_in_their_chunk(H, I):
+    """nq_pf_pre and nq_pf_mid over rows with infinities, NaN, sums beyond fp16 and gates whose exponential overflows: what float64
+    gives in the 128 columns they share a Hadamard with, nothing anywhere else"""
+    from nestquant_amd import _lib
+    Lb = _lib.lib()
+    E, n = 2, 12
+    ex = to_dev(experts_on_gpu(H, I, E, 33))
+    L = M.MoELayer(E, H, I, Bmax=4, topk=1)
+    for e in range(E):
+        L.set(e, ex[e], 2)
+    g = torch.Generator().manual_seed(H)
+    x, acc = (torch.randn(n, H, generator=g) * 0.3).half(), torch.randn(n, 2 * I, generator=g)
+    clean = x.clone(), acc.clone()
+    inf, nan = float("inf"), float("nan")
+    for r, v in enumerate((inf, -inf, nan)):
+        x[r, 5 + 128 * (r % 2)] = v; acc[r, 200 + r] = v; acc[r + 3, I + 7 + r] = v
+    x[3, 130], x[3, 140] = inf, inf                              # inf - inf in half of the outputs
+    x[4, :128] = 65504.0                                         # their sum does not fit fp16
+    acc[6, :128] = -200.0; acc[7, 128:256] = 200.0               # exp(200) does not fit fp32; the gate is 0, or the value itself
+    pe, pt = torch.arange(n).mul(E).div(n, rounding_mode="floor").int().to(DEV), torch.arange(n).int().to(DEV)
+
+    def run(x, acc):
+        xg = torch.full((n, H), 7.0, dtype=torch.float16, device=DEV); xu, h = torch.full_like(xg, 7.0), torch.full((n, I), 7.0, dtype=torch.float16, device=DEV)
+        xd, ad = x.to(DEV), acc.to(DEV)
+        _lib.check(Lb.nq_pf_pre(xd.data_ptr(), pt.data_ptr(), pe.data_ptr(), n, L.table.data_ptr(), xg.data_ptr(), xu.data_ptr(), None, E, H, I, None))
+        _lib.check(Lb.nq_pf_mid(ad.data_ptr(), pe.data_ptr(), n, L.table.data_ptr(), h.data_ptr(), None, None, E, H, I, None))
+        return [t.cpu().double() for t in (xg, xu, h)]
+    had = torch.ones(1, 1, dtype=torch.float64)
+    for _ in range(7):
+        had = torch.cat([torch.cat([had, had], 1), torch.cat([had, -had], 1)])
+    wht = lambda v: ((v.reshape(n, -1, 1, 128) * had).sum(-1) / 128**0.5).reshape(n, -1)      # sums, no products with zero
+    place = torch.tensor([((c >> 5) * 4 + (c >> 1 & 3)) * 8 + 2 * (2 * (c >> 3 & 1) + (c & 1)) + (c >> 4 & 1) for c in range(128)])
+    bop = lambda v: torch.empty_like(v).view(n, -1, 128).index_copy_(2, place, v.view(n, -1, 128)).view(n, -1)
+    sg = torch.stack([e.signs.cpu().double() for e in ex])[pe.cpu().long()]
+
+    def want(x, acc):
+        xs = x.double()
+        gate, up = wht(acc[:, :I].double()) * sg[:, H:H + I], wht(acc[:, I:].double()) * sg[:, H + I:H + 2 * I]
+        act = torch.nn.functional.silu(gate) * up
+        return [bop(wht(xs * sg[:, :H])).half().double(), bop(wht(xs * sg[:, 2 * H + 3 * I:])).half().double(),
+                bop(wht(act * sg[:, H + 2 * I:H + 3 * I])).half().double()]
+    for got, base, ref in zip(run(x, acc), run(*clean), want(x, acc)):
+        for kind in (torch.isnan, torch.isposinf, torch.isneginf):
+            assert torch.equal(kind(got), kind(ref)), kind.__name__
+        ok = torch.isfinite(ref)
+        assert 0 < int((~ok).sum()) < ok.numel() // 2 and rel_err(got[ok].numpy(), ref[ok].numpy()) < 5e-4
+        same = (got == base).view(n, -1, 128).all(-1)            # whole chunks
+        assert bool(same[8:].all()) and int((~same).sum()) <= 12
+
+
+@pytest.mark.parametrize("H,I,T,E,K", [(256, 256, 40, 40, 4), (2560, 2304, 383, 8, 8)])      # the one-launch plan, and the tall tiles on side streams
+def test_a_token_that_is_not_finite_is_its_own_affair(H, I, T, E, K):
+    """NaN or an infinity in a token's activations or weights reaches that token's result, as in the decode call, and no other's"""
+    ex = to_dev(experts_on_gpu(H, I, 4, 710, nested_ids=(1, 3)))
+    L = M.MoELayer(E, H, I, Bmax=4, topk=K)
+    for e in range(E):
+        L.set(e, ex[e % 4], 4 if ex[e % 4].nested else 2)
+    g = torch.Generator().manual_seed(T)
+    x = (torch.randn(T, H, generator=g) * 0.3).to(DEV)
+    sel, w = gumbel_topk(T, E, K, seed=4)
+    w = w.float()
+    clean = M.forward(L, None, x, w, sel)
+    x[1, 3], x[T // 2, H - 1], w[T - 1, 0], w[6, 1] = float("nan"), float("inf"), float("inf"), float("nan")
+    hit = torch.zeros(T, dtype=torch.bool, device=DEV)
+    hit[[1, T // 2, T - 1, 6]] = True
+    y = M.forward(L, None, x, w, sel)
+    slices = torch.cat([L(x[i:i + 4], sel[i:i + 4], w[i:i + 4]).clone() for i in range(0, T, 4)])
+    torch.cuda.synchronize()
+    assert torch.equal(y[~hit], clean[~hit])
+    assert torch.equal(torch.isfinite(y), torch.isfinite(slices)) and not torch.isfinite(y[hit]).any()
