@@ -304,7 +304,7 @@ int nq_pf_hits(const int32_t* counts, int32_t* hits, int E, void* stream);
  * or 2 new bits per step and the values lut [65536]; states [T][L] = the states of the path of least squared error, ties to the
  * smallest predecessor (reference threads/05-exl3-harness/harness.py:297-364). position_order = 0: w and states in step order; 1: in
  * ring position order (step i <-> position (L - i) mod L). scratch: 4096 * L bytes for each ring searched at a time (one workgroup
- * each; one per CU is the most that is of use). w must not hold NaN. */
+ * each; one per CU is the most that is of use). A target that is not finite makes every path equally dear from its step on. */
 int nq_viterbi(const float* w, int T, int L, int K, const float* lut, int64_t* states, void* scratch, int64_t scratch_bytes,
                int position_order, void* stream);
 

@@ -159,3 +159,15 @@ def test_side_stream_of_a_fit_outlives_another_threads_clean_up(monkeypatch):
     monkeypatch.undo()
     b = EN.encode_nested(W)
     assert all(torch.equal(a[k], b[k]) for k in ("base", "p3", "d3", "p4", "d4"))
+
+
+@pytest.mark.parametrize("K", [1, 2])
+def test_searches_over_targets_that_are_not_finite(K):
+    """an infinite or NaN target makes every path equally dear from its step on: ties to the smallest predecessor, as in torch"""
+    g = torch.Generator().manual_seed(K)
+    w = torch.randn(4, 24, generator=g)
+    w[0, 3], w[1, 20], w[2, 11], w[3, 0] = float("inf"), -float("inf"), float("nan"), 3e20      # whose square is infinite
+    lut = EN.codebook()
+    assert torch.equal(EN.viterbi_ring(w.cuda(), lut.cuda(), K).cpu(), EN.viterbi_ring(w, lut, K))
+    a = torch.randint(0, 256, (4, 24), generator=g)
+    assert torch.equal(EN.viterbi_ring_given_p3(w.cuda(), a.cuda(), lut.cuda()).cpu(), EN.viterbi_ring_given_p3(w, a, lut))
