@@ -271,8 +271,9 @@ int nq_sum_slices(const float* part, int ny, int64_t n, float* out, void* stream
 /* A whole step of T tokens on device data, no host synchronisation: pairs sorted by expert, tile plan, rotation, gate|up, SwiGLU,
  * down, combine -- the chain of the entry points above (reference moe.prefill, sm120/moe.py:282-326) with the casts of its caller
  * (x.half(), ids.long(), w.half(), out.to(dtype), sm120/serve/nq_vllm.py:522,573) at the loads and the final store. Ids outside
- * [0, E) contribute nothing. Steps with at most 32 pairs per expert on average run on `stream` alone, longer ones fork onto the side
- * streams and join again. Calls that share scratch, side streams or events must be ordered on one stream. */
+ * [0, E) contribute nothing. Steps with at most 32 pairs per expert on average or pairs * H * I <= 2^34 run on `stream` alone, longer
+ * ones fork onto the side streams and join again, also when a launch between fails. Calls that share scratch must be ordered on one
+ * stream; side streams and events belong to the calls of one stream. */
 typedef struct NqPfArgs
 {
     const void* x;                 /* [T][H], type x_dtype */

@@ -4,10 +4,12 @@
 // (--pmc FETCH_SIZE / WRITE_SIZE) can wrap; `--calib` adds one 256 MiB device copy as the known-size kernel that scales
 // those counters.
 //
-//   nq_bench_native [--experts 64] [--batch 1] [--steps 32] [--calib] [--level L] [--prefill ROWS] [--hoist]
+//   nq_bench_native [--experts 64] [--batch 1] [--steps 32] [--calib] [--level L] [--prefill ROWS] [--step TOKENS] [--hoist]
+//   nq_bench_native --viterbi RINGS [--steps 32]
 //
 // --prefill ROWS times the decode-fused grouped GEMMs of the prefill path instead (nq_pf_gemm, gate|up then down): every
-// expert gets ROWS pair rows (<= 256, one tile each); --level L puts every expert at level L.
+// expert gets ROWS pair rows (<= 256, one tile each); --level L puts every expert at level L. --step TOKENS times whole grouped
+// steps (nq_pf_step) of that many tokens, top-8, evenly routed. --viterbi RINGS times the encoder's trellis search, K = 2 and K = 1.
 //
 // Planes are pseudo-random words (the decoder's cost does not depend on the values); levels cycle 2,2,2,3,4,2,2,4 so
 // every step mixes levels; each step routes to 8 experts not used by the step before.
@@ -41,9 +43,36 @@ __global__ void fill_block_words(uint32_t* p, size_t n, uint32_t seed)       // 
 __global__ void fill_half(uint16_t* p, size_t n, uint16_t v) { for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) p[i] = v; }
 __global__ void copy_words(const uint4* __restrict__ a, uint4* __restrict__ b, size_t n) { for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) b[i] = a[i]; }
 
+__global__ void fill_float(float* p, size_t n, float scale) { for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) p[i] = ((float)((uint32_t)i * 2654435761u >> 8) / 8388608.f - 1.f) * scale; }
+
+template <class F> static float timed_ms(int steps, F&& f)                      // one untimed call, then `steps` between two events
+{
+    hipEvent_t e0, e1; HIPCHK(hipEventCreate(&e0)); HIPCHK(hipEventCreate(&e1));
+    f(); HIPCHK(hipDeviceSynchronize());
+    HIPCHK(hipEventRecord(e0, nullptr));
+    for (int i = 0; i < steps; ++i) f();
+    HIPCHK(hipEventRecord(e1, nullptr)); HIPCHK(hipEventSynchronize(e1));
+    float ms; HIPCHK(hipEventElapsedTime(&ms, e0, e1));
+    return ms / steps;
+}
+static int viterbi(int rings, int steps)
+{
+    const int L = 256, slots = rings < 256 ? rings : 256;
+    float *w, *lut; int64_t* st; void* scratch;
+    HIPCHK(hipMalloc(&w, (size_t)rings * L * 4)); HIPCHK(hipMalloc(&lut, 65536 * 4)); HIPCHK(hipMalloc(&st, (size_t)rings * L * 8));
+    HIPCHK(hipMalloc(&scratch, (size_t)slots * L * 4096));
+    fill_float<<<256, 256>>>(w, (size_t)rings * L, 2.f); fill_float<<<64, 256>>>(lut, 65536, 3.f);
+    for (int K = 2; K >= 1; --K)
+    {
+        const float ms = timed_ms(steps, [&] { NQCHK(nq_viterbi(w, rings, L, K, lut, st, scratch, (int64_t)slots * L * 4096, 1, nullptr)); });
+        printf("nq_bench_native viterbi: %d rings of %d steps, K = %d: %.1f us\n", rings, L, K, ms * 1e3);
+    }
+    return 0;
+}
+
 int main(int argc, char** argv)
 {
-    int E = 64, B = 1, steps = 32, calib = 0, level = 0, pf_rows = 0, hoist = 0;
+    int E = 64, B = 1, steps = 32, calib = 0, level = 0, pf_rows = 0, pf_step = 0, rings = 0, hoist = 0;
     for (int i = 1; i < argc; ++i)
     {
         if (!strcmp(argv[i], "--experts") && i + 1 < argc) E = atoi(argv[++i]);
@@ -53,8 +82,12 @@ int main(int argc, char** argv)
         else if (!strcmp(argv[i], "--hoist")) hoist = 1;
         else if (!strcmp(argv[i], "--level") && i + 1 < argc) level = atoi(argv[++i]);
         else if (!strcmp(argv[i], "--prefill") && i + 1 < argc) pf_rows = atoi(argv[++i]);
-        else { fprintf(stderr, "usage: %s [--experts E>=16] [--batch B<=8] [--steps K] [--calib] [--level 2|3|4] [--prefill ROWS<=256] [--hoist]\n", argv[0]); return 2; }
+        else if (!strcmp(argv[i], "--step") && i + 1 < argc) pf_step = atoi(argv[++i]);
+        else if (!strcmp(argv[i], "--viterbi") && i + 1 < argc) rings = atoi(argv[++i]);
+        else { fprintf(stderr, "usage: %s [--experts E>=16] [--batch B<=8] [--steps K] [--calib] [--level 2|3|4] [--prefill ROWS<=256] [--step TOKENS<=4096] [--hoist] | --viterbi RINGS<=4096\n", argv[0]); return 2; }
     }
+    if (steps < 1 || rings < 0 || rings > 4096 || pf_step < 0 || pf_step > 4096) { fprintf(stderr, "need steps >= 1, RINGS and TOKENS <= 4096\n"); return 2; }
+    if (rings) return viterbi(rings, steps);
     if ((level && level != 2 && level != 3 && level != 4) || pf_rows < 0 || pf_rows > 256) { fprintf(stderr, "need level in {2,3,4} and 0 <= ROWS <= 256\n"); return 2; }
     if (E < 16 || B < 1 || B > 8) { fprintf(stderr, "need E >= 16 and 1 <= B <= 8\n"); return 2; }
     const int H = 6144, I = 2048, topk = 8, S = B * topk;
@@ -115,6 +148,30 @@ int main(int argc, char** argv)
         const double flop = 2.0 * np * 3.0 * H * I;
         printf("nq_bench_native prefill: E=%d tiles of %d rows (height %d), level %d: %.3f ms per gate|up + down pair, %.1f TFLOP/s, %.2f us per tile\n",
                E, pf_rows, bm, level, ms / steps, flop / (ms / steps * 1e-3) / 1e12, ms * 1e3 / steps / E);
+        return 0;
+    }
+
+    if (pf_step)
+    {
+        const int T = pf_step, P = T * topk;
+        NqPfArgs a; memset(&a, 0, sizeof a);
+        auto alloc = [](size_t bytes) { void* p; HIPCHK(hipMalloc(&p, bytes)); return p; };
+        std::vector<int64_t> hs((size_t)P);
+        for (int t = 0; t < T; ++t)
+            for (int k = 0; k < topk; ++k) hs[(size_t)t * topk + k] = (topk * (int64_t)t * 5 + k) % E;       // eight neighbours: distinct
+        int64_t* sel = (int64_t*)alloc((size_t)P * 8); HIPCHK(hipMemcpy(sel, hs.data(), hs.size() * 8, hipMemcpyHostToDevice));
+        uint16_t *x = (uint16_t*)alloc((size_t)T * H * 2), *rw = (uint16_t*)alloc((size_t)P * 2);
+        fill_half<<<1024, 256>>>(x, (size_t)T * H, 0x2A66); fill_half<<<64, 256>>>(rw, P, 0x3000);
+        a.x = x; a.sel = sel; a.rw = rw; a.table = d_table; a.out = alloc((size_t)T * H * 4);
+        a.meta_bytes = nq_pf_meta_bytes(T, topk, P, E); a.meta = alloc(a.meta_bytes);
+        a.xg = alloc((size_t)P * H * 2); a.xu = alloc((size_t)P * H * 2); a.h = alloc((size_t)P * I * 2);
+        a.acc = alloc((size_t)P * 2 * I * 4); a.y = alloc((size_t)P * H * 4); a.zg = (float*)alloc((size_t)P * 16); a.zd = (float*)alloc((size_t)P * 16);
+        for (int i = 0; i < 3; ++i) { hipStream_t q; HIPCHK(hipStreamCreateWithFlags(&q, hipStreamNonBlocking)); a.side[i] = q; }
+        for (int i = 0; i < 4; ++i) { hipEvent_t q; HIPCHK(hipEventCreateWithFlags(&q, hipEventDisableTiming)); a.events[i] = q; }
+        a.T = T; a.topk = topk; a.E = E; a.H = H; a.I = I; a.rows = P; a.variants = 1;
+        HIPCHK(hipDeviceSynchronize());
+        const float ms = timed_ms(steps, [&] { NQCHK(nq_pf_step(&a, nullptr)); });
+        printf("nq_bench_native step: E=%d, %d tokens, level %d: %.1f us, %.1f TFLOP/s\n", E, T, level, ms * 1e3, 2.0 * P * 3.0 * H * I / (ms * 1e-3) / 1e12);
         return 0;
     }
 

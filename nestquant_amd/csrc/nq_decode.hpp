@@ -206,9 +206,10 @@ template <int O> __device__ __forceinline__ uint32_t window_reg(const uint32_t* 
     if constexpr (s == 0) return w[i]; else return __builtin_amdgcn_alignbit(w[i + 1], w[i], s);
 }
 // The low half is cut out by a 16-bit add of 0 (it clears the upper half): of the instructions that do it, the 16-bit ones are the
-// only ones that pair with another wavefront's byte sum, funnel shift or 32-bit multiply. In a loop of one of those and one
-// cut the cut costs 0.9 ns per wavefront and SIMD as v_add_u16 and 1.85 ns as v_and_b32 or v_bfe_u32 (four wavefronts per SIMD);
-// decode layer of four tokens 246 -> 238 us, of one token 74.6 -> 72.9.
+// only ones that pair with another wavefront's byte sum, funnel shift or 32-bit multiply. In a loop of one of those (2.1 ns per
+// wavefront and SIMD alone, four wavefronts per SIMD) and one cut, the cut adds 0.6 to 0.7 ns as v_add_u16, 1.2 to 2.1 as v_and_b32,
+// 1.7 to 2.5 as v_bfe_u32; beside a dot product it is 1.6 as either (profiles/gfx950_vector_issue_rates.txt). Decode layer of four
+// tokens 246 -> 238 us, of one token 74.6 -> 72.9.
 template <int O> __device__ __forceinline__ uint32_t state(uint32_t r)
 {
     if constexpr ((O & 31) < 16)

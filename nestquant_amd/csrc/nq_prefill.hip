@@ -40,8 +40,9 @@ __device__ __forceinline__ bool row_in_heights(const int32_t* __restrict__ tiles
 // grid (row groups, column parts), block 256: wavefront w of column part y rotates segment 4 y + w (512 columns, four chunks; lanes of
 // chunks beyond H repeat the last one) of `rows` pair rows, gate and up together, holding the scale vectors while the expert stays the same.
 // tiles (optional): work only on the rows of the tile heights in `heights`.
-// A form with two columns per lane (about 50 vector instructions per chunk) was bound by the vector ALU: 8024 rows of 6144 columns
-// 84 us; with eight columns per lane 64, 197 MB written at 3.1 TB/s. Fetching the next row's activations ahead changed nothing.
+// Bound by memory, 197 MB written and 57 read at 4.0 TB/s with 8024 rows of 6144 columns: 64 us, one vector instruction per 7 clocks
+// and SIMD (profiles/grouped_steps.txt). With two columns per lane (about 50 vector instructions per chunk) it took 84. Fetching
+// the next row's activations ahead changed nothing.
 __global__ void __launch_bounds__(256) nq_pf_pre_k(const void* __restrict__ x, int xdt, const int32_t* __restrict__ pt, const int32_t* __restrict__ pe, int np, int rows,
                                                     const int64_t* __restrict__ table, _Float16* xg, _Float16* xu, float* zg, int E, int H, int I,
                                                     const int32_t* __restrict__ tiles, int cap, int heights)
@@ -122,8 +123,8 @@ __global__ void __launch_bounds__(256) nq_pf_pre_k(const void* __restrict__ x, i
 // (pair row of the group, segment of 512 columns) in turn; lanes of chunks beyond I repeat the last one. With in_had_down = 512
 // (table word 18) the four chunks of a segment are combined with the Sylvester H_4 / 2 before the single rounding to fp16.
 // tiles (optional): work only on the rows of the tile heights in `heights`, as nq_pf_pre_k
-// Bound by memory, 5 bytes per output element and no reuse: 8024 rows of 2 x 2048 sums 66 -> 40 us (4.1 TB/s) with eight columns per
-// lane, for the same reason as there.
+// Bound by memory, 5 bytes per output element and no reuse: 8024 rows of 2 x 2048 sums 66 -> 41 us (4.1 TB/s) with eight columns per
+// lane, which halves the vector instructions as there.
 constexpr int MID_ROWS = 8;                                      // most rows of a group
 __global__ void __launch_bounds__(256) nq_pf_mid_k(const float* __restrict__ acc_gu, const int32_t* __restrict__ pe, int np, int rows,
                                                     const int64_t* __restrict__ table, _Float16* h, const float* zg, float* zd, int E, int H, int I,
@@ -754,7 +755,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
 
 // Tiles of up to 64 rows of any height in one launch (the plan of nq_pf_sort_k). Steps of a few hundred tokens over many experts
 // have nothing taller, so a projection is one launch on the caller's stream instead of five on four; with at most 64 rows a tile
-// costs what decoding its expert costs, and the registers of the 64-row body (126) still let four wavefronts share a SIMD.
+// costs what decoding its expert costs, and the registers of the 64-row body (126) still let four wavefronts share a SIMD. Bound by
+// instruction issue: one vector instruction per 4.0 to 4.2 clocks and SIMD at 200 and 1000 tokens (profiles/grouped_steps.txt).
 template <bool MASKED>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MASKED ? 2 : 4))) nq_pf_short_k(PfGemm a)
 {
@@ -769,7 +771,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MASKED
 }
 
 // ---- pairs sorted by expert ----------------------------------------------------------------------------------------------
-// One launch in place of a library sort, its gathers and the counting scatter (a dozen launches, 150 us of them at 32768 pairs).
+// One launch in place of a library sort, its gathers and the counting scatter (a dozen launches, 150 us of them at 32768 pairs):
+// 11 us at 384 pairs, 21 at 8024, 84 to 89 at 32768, where every workgroup reads and counts all picks.
 // Every workgroup counts all picks in LDS, so that it knows where each expert's rows start without waiting for another one; its
 // eight wavefronts then gather the pairs of one expert each, in pair order, from the picks kept in LDS as 16-bit ids. Picks outside
 // [0, E) form a last group of rows of no expert (pe = -1), which every later kernel passes over. Workgroup 0 also writes the

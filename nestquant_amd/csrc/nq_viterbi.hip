@@ -12,9 +12,9 @@
 // decisions of a thread in one step (16 edges x 2 bits, or 32 x 1) fill one word, stored to a scratch of 4 KB per step; the way
 // back is walked by one lane over blocks of steps brought to LDS, the next block in flight.
 // Bound: instruction issue of sixteen wavefronts in lockstep. A step is 65536 candidates of three fp32 operations plus the selection,
-// 19 vector instructions per four candidates (K = 2) = 309 per wavefront; one ring per CU. Measured: 935 us for 256 rings (K = 2;
-// 1.6 us per step, the walks back ~100 us), 1160 us (K = 1, whose single array costs a second barrier); with all wavefronts at one
-// priority 1060 and 1230.
+// 19 vector instructions per four candidates (K = 2) = 309 per wavefront, which issue at one per 3.1 clocks and SIMD over the whole
+// launch (K = 1: 4.0; profiles/encoder_searches.txt); one ring per CU. Measured: 935 to 990 us for 256 rings (K = 2; 1.6 us per step,
+// the walks back ~100 us), 1160 us (K = 1, whose single array costs a second barrier); with all wavefronts at one priority 1060 and 1230.
 #include "nq_host.hpp"
 
 namespace nq {
