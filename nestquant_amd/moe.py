@@ -288,6 +288,9 @@ class MoELayer:
         # one struct.pack instead of sixty attribute stores on a ctypes structure: 4 us less host time per call
         mb = (0, 0, 0, 0, 0) if mailbox is None else (tb.data_ptr(), mailbox.stage.data_ptr(), mailbox.seq.data_ptr(), mailbox.applied.data_ptr(),
                                                       mailbox.applied_host.data_ptr())
+        if sal is not None and not (sal.acc.dtype == sal.host.dtype == torch.float64 and sal.acc.is_contiguous() and sal.host.is_contiguous()
+                                    and sal.acc.numel() >= tb.shape[0] <= sal.host.numel() and rw.numel() == sel.numel()):
+            raise RuntimeError("salience: acc and its host mirror must be contiguous float64 with an entry per expert, rw one weight per pick")
         sl = (0, 0, 0, 0.0) if sal is None else (1, sal.acc.data_ptr(), sal.host.data_ptr(), sal.rsf)
         raw = _lib.PACK_MOE_ARGS(
             x.data_ptr(), sel.data_ptr(), rw.data_ptr(), tb.data_ptr(), out.data_ptr(), s.acc_gu.data_ptr(), s.h.data_ptr(), s.acc_d.data_ptr(),

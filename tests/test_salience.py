@@ -203,3 +203,28 @@ def test_salience_operands_are_looked_at_either_way():
         s.acc = acc
         with pytest.raises(RuntimeError):
             M.forward(_LayerStub(), None, x, ww, ids, sal=s)
+
+
+def test_layer_call_looks_at_its_salience(monkeypatch):
+    """the routing launch indexes accumulator and mirror by expert: a shorter or otherwise typed one is refused by the host"""
+    from nestquant_amd import _lib, moe as M, salience as SAL
+
+    class Lib:
+        calls = 0
+
+        def nq_moe_forward(s, raw, stream):
+            s.calls += 1
+            return 0
+    monkeypatch.setattr(_lib, "stream_ptr", lambda: 0)
+    L = M.MoELayer(6, 128, 128, Bmax=2, topk=2, dev="cpu", mod=Lib())
+    x, sel, rw = torch.zeros(1, 128, dtype=torch.float16), torch.zeros(1, 2, dtype=torch.int64), torch.ones(1, 2, dtype=torch.float16)
+    f64 = lambda n: torch.zeros(n, dtype=torch.float64)
+    for acc, host, w in ((f64(5), f64(6), rw), (f64(6), f64(5), rw), (torch.zeros(6), f64(6), rw), (f64(6), torch.zeros(6), rw),
+                         (f64(12)[::2], f64(6), rw), (f64(6), f64(6), rw[:, :1].contiguous())):
+        s = _host_salience(SAL.Salience, 6)
+        s.acc, s.host = acc, host
+        with pytest.raises(RuntimeError):
+            L(x, sel, w, sal=s)
+    assert L.M.calls == 0
+    L(x, sel, rw, sal=_host_salience(SAL.Salience, 6))
+    assert L.M.calls == 1
