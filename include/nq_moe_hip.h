@@ -272,7 +272,7 @@ int nq_sum_slices(const float* part, int ny, int64_t n, float* out, void* stream
  * down, combine -- the chain of the entry points above (reference moe.prefill, sm120/moe.py:282-326) with the casts of its caller
  * (x.half(), ids.long(), w.half(), out.to(dtype), sm120/serve/nq_vllm.py:522,573) at the loads and the final store. Ids outside
  * [0, E) contribute nothing. Steps with at most 32 pairs per expert on average or pairs * H * I <= 2^34 run on `stream` alone, longer
- * ones fork onto the side streams and join again, also when a launch between fails. Calls that share scratch must be ordered on one
+ * ones fork onto the side streams, where there are some, and join again, also when a launch between fails. The bits do not depend on it. Calls that share scratch must be ordered on one
  * stream; side streams and events belong to the calls of one stream. */
 typedef struct NqPfArgs
 {
@@ -287,8 +287,8 @@ typedef struct NqPfArgs
     void *acc, *y;                 /* fp32 [rows][2I], [rows][H] */
     float *zg, *zd;                /* fp32 [rows][4] each, or NULL when no expert has a low-rank plane */
     void* wop; int64_t wop_bytes;  /* optional scratch of decoded weights (nq_pf_wdecode) with wop_slots slots for experts of >= hot_min rows */
-    void* side[3];                 /* streams of default priority */
-    void* events[4];               /* events without timing of the same device */
+    void* side[3];                 /* streams of default priority, or NULL: the step stays on `stream` */
+    void* events[4];               /* events without timing of the same device, with side streams */
     int32_t T, topk, E, H, I;
     int32_t rows;                  /* pair rows the scratch holds; more pairs are worked through in chunks (out must then be fp32) */
     int32_t x_dtype, sel_dtype, rw_dtype, out_dtype;   /* as in NqMoeArgs */

@@ -331,8 +331,8 @@ extern "C" int nq_pf_step(const NqPfArgs* p, void* stream)
     NQ_REQUIRE(a.rows >= 1 && (a.out_dtype == 0 || a.rows >= (int64_t)a.T * a.topk), "nq_pf_step: rows=%d; a result of another type than fp32 needs all %d pairs in one chunk", a.rows, a.T * a.topk);
     NQ_REQUIRE((int64_t)a.E + a.rows / 256 + 1 <= 65535, "nq_pf_step: rows=%d exceed one launch", a.rows);
     NQ_REQUIRE(!a.wop || (a.hot_min >= 1 && a.wop_slots >= 1 && a.wop_bytes >= (int64_t)a.wop_slots * 3 * a.H * a.I * 2), "nq_pf_step: the decoded-weight scratch needs %d slots of 3 * H * I halfs", a.wop_slots);
-    for (int i = 0; i < 3; ++i) NQ_REQUIRE(a.side[i], "nq_pf_step: three side streams");
-    for (int i = 0; i < 4; ++i) NQ_REQUIRE(a.events[i], "nq_pf_step: four events");
+    for (int i = 0; i < 3; ++i) NQ_REQUIRE(!a.side[i] == !a.side[0], "nq_pf_step: three side streams or none");
+    for (int i = 0; i < 4; ++i) NQ_REQUIRE(!a.side[0] || a.events[i], "nq_pf_step: four events with the side streams");
     return launch_pf_step(a, (hipStream_t)stream);
 }
 

@@ -965,7 +965,10 @@ static PfMeta pf_meta(void* ws, int P, int R, int E)
 //   little work beside the 0.1 ms, rows * H * I <= 2^34 (a decode's price goes with H I): 512 x 256, 16 experts, 1000 tokens
 //   51 / 141; 2048 x 1024, 64 experts, 750 tokens 217 / 277; 6144 x 2048, 8 experts, 93 tokens 146 / 201. At the line 0.84 to 1.02 of
 //   tall over ten shapes, at twice the line 1.06 to 1.27 for all but one.
-static bool pf_is_short(int64_t P, int E, int H, int I) { return P <= 32 * (int64_t)E || P * H * I <= (int64_t)1 << 34; }
+// Without side streams the tall tiles' launches follow one another and the line lies at 2^36: 6144 x 2048, 16 experts, 383 tokens 540 / 505
+// and (Zipf) 530 / 917, 1000 tokens, beyond it, 1205 / 1066 and 1204 / 1296; 64 experts 633 / 746 and 741 / 1448, 1338 / 1409 and
+// 1400 / 1760, 2000 tokens 2498 / 2158 and 2466 / 2478.
+static bool pf_is_short(int64_t P, int E, int H, int I, bool fork) { return P <= 32 * (int64_t)E || P * H * I <= (int64_t)1 << (fork ? 34 : 36); }
 
 template <bool MASKED>
 static int launch_short(const PfGemm& a, int ntiles, int N, hipStream_t st)
@@ -980,7 +983,7 @@ int launch_pf_step(const NqPfArgs& a, hipStream_t st)
     const int P = a.T * a.topk, R = a.rows < P ? a.rows : P, E = a.E, H = a.H, I = a.I;
     const PfMeta m = pf_meta(a.meta, P, R, E);
     if (m.bytes > (size_t)a.meta_bytes) return set_error("nq_pf_step: meta needs %zu bytes, has %lld", m.bytes, (long long)a.meta_bytes);
-    const bool brief = R == P && !a.wop && pf_is_short(P, E, H, I);
+    const bool fork = a.side[0] != nullptr, brief = R == P && !a.wop && pf_is_short(P, E, H, I, fork);
     {
         const PfSort s{a.sel, a.rw, a.sel_dtype, a.rw_dtype, P, a.topk, E, a.table, m.cnt, m.pe, m.pt, m.pos, a.hits, brief ? m.tiles : nullptr, m.scap};
         const int shm = SORT_TILE * 2 + 3 * (E + 1) * 4;
@@ -1006,7 +1009,9 @@ int launch_pf_step(const NqPfArgs& a, hipStream_t st)
     // Tile heights 256 | 128 | 64, 32, 16 as four chains: the tallest on the caller's stream, the others on side streams between two
     // events. A GEMM launch ends with the GPU partly idle while its last workgroups drain; the chains fill each other's tails, and
     // the memory-bound kernels of one height run under the GEMMs of another.
-    hipStream_t streams[4] = {st, (hipStream_t)a.side[0], (hipStream_t)a.side[1], (hipStream_t)a.side[2]};
+    // Without side streams the chains follow one another on the caller's.
+    hipStream_t streams[4] = {st, st, st, st};
+    for (int i = 0; fork && i < 3; ++i) streams[i + 1] = (hipStream_t)a.side[i];
     static const int stream_of[5] = {3, 3, 2, 1, 0};             // by height 16 << k
     auto hip_ok = [](hipError_t e) { return e == hipSuccess ? 0 : set_error("nq_pf_step: %s", hipGetErrorString(e)); };
     for (int c = 0; c < P; c += R)
@@ -1016,8 +1021,8 @@ int launch_pf_step(const NqPfArgs& a, hipStream_t st)
         if (int rc = launch_pf_plan(m.cnt, E, c, n, m.tiles, m.cap, wop ? m.hot : nullptr, a.hot_min, a.wop_slots, st)) return rc;
         for (int mode = 0; wop && mode < 2; ++mode)
             if (int rc = launch_pf_wdecode(a.table, m.hot, E, mode, a.wop, H, I, st)) return rc;
-        if (int rc = hip_ok(hipEventRecord((hipEvent_t)a.events[0], st))) return rc;
-        for (int i = 1; i < 4; ++i) if (int rc = hip_ok(hipStreamWaitEvent(streams[i], (hipEvent_t)a.events[0], 0))) return rc;
+        if (fork) if (int rc = hip_ok(hipEventRecord((hipEvent_t)a.events[0], st))) return rc;
+        for (int i = 1; fork && i < 4; ++i) if (int rc = hip_ok(hipStreamWaitEvent(streams[i], (hipEvent_t)a.events[0], 0))) return rc;
         const int32_t *pts = m.pt + c, *pes = m.pe + c;
         static const int heights[4] = {16, 8, 4, 3};             // bit k = height 16 << k
         auto gemms = [&](int mode) {
@@ -1037,7 +1042,7 @@ int launch_pf_step(const NqPfArgs& a, hipStream_t st)
             return gemms(1);
         };
         const int failed = chains();
-        for (int i = 1; i < 4; ++i)                              // joined in any case: the caller gives the buffers back in its stream's order
+        for (int i = 1; fork && i < 4; ++i)                      // joined in any case: the caller gives the buffers back in its stream's order
         {
             if (int rc = hip_ok(hipEventRecord((hipEvent_t)a.events[i], streams[i]))) return rc;
             if (int rc = hip_ok(hipStreamWaitEvent(st, (hipEvent_t)a.events[i], 0))) return rc;

@@ -381,7 +381,7 @@ def _pf_side(dev, stream):
         with torch.cuda.device(dev):
             side, ev = [torch.cuda.Stream(device=dev) for _ in range(3)], [torch.cuda.Event() for _ in range(4)]
             for e in ev:
-                e.record(side[0])                    # a torch event exists from its first record on (not on `stream`, which may be capturing)
+                e.record(side[0])                    # a torch event exists from its first record on
         S = (side, ev, (C.c_void_p * 3)(*[st.cuda_stream for st in side]), (C.c_void_p * 4)(*[e.cuda_event for e in ev]))
         if len(_PF_SIDE) >= 64:
             _PF_SIDE.clear()
@@ -408,7 +408,8 @@ def _pf_step(s, x, sel, rw, out, R=None, table=None):
     # one block per call, the step's own: it goes back to the allocator in the order of the caller's stream, which the side streams join
     block = torch.empty(wop_at + slots * 6 * H * I, dtype=torch.uint8, device=dev)
     stream = _lib.stream_ptr()
-    held = _pf_side(dev, stream)
+    # a step that is being captured stays on its stream: streams of torch's pool may coincide with one that somebody is using
+    held = None if torch.cuda.is_current_stream_capturing() else _pf_side(dev, stream)
     whole = out if out.dtype == torch.float32 or R == P else torch.empty(T, H, dtype=torch.float32, device=dev)   # chunks add up in fp32
     a, at = _lib.NqPfArgs(), block.data_ptr()
     a.x, a.sel, a.rw, a.table, a.out, a.hits = x.data_ptr(), sel.data_ptr(), rw.data_ptr(), tb.data_ptr(), whole.data_ptr(), s.hits_ptr or None
@@ -416,7 +417,8 @@ def _pf_step(s, x, sel, rw, out, R=None, table=None):
     a.xg, a.xu, a.acc, a.h, a.y, a.zg, a.zd = (at + o for o in off)
     if slots:
         a.wop, a.wop_bytes, a.wop_slots, a.hot_min = at + wop_at, slots * 6 * H * I, slots, PF_HOT_MIN
-    a.side, a.events = held[2], held[3]
+    if held is not None:
+        a.side, a.events = held[2], held[3]
     a.T, a.topk, a.E, a.H, a.I, a.rows = T, k, E, H, I, R
     a.x_dtype, a.sel_dtype, a.rw_dtype, a.out_dtype = _DT_IN[x.dtype], _DT_SEL[sel.dtype], _DT_IN[rw.dtype], _DT_OUT[whole.dtype]
     # mask mode / other base codes run in their own kernel variant; a caller's own table may hold such rows, so it gets both, and

@@ -412,6 +412,7 @@ def test_a_captured_grouped_step_equals_the_eager_one(H, I, T, E, K):
     gr = torch.cuda.CUDAGraph()
     with torch.cuda.graph(gr, stream=st):
         y = M.forward(L, MB, x, w, sel)
+    assert (0, st.cuda_stream) not in M._PF_SIDE                 # and it stays on the stream
     for i in range(4):
         x.copy_((torch.randn(T, H, generator=g) * 0.3).to(DEV))
         s2, w2 = gumbel_topk(T, E, K, seed=3 + i)
@@ -427,6 +428,27 @@ def test_a_captured_grouped_step_equals_the_eager_one(H, I, T, E, K):
         torch.cuda.synchronize()
         assert torch.equal(y, want), i
         del junk
+
+
+def test_a_captured_prompt_equals_the_eager_one():
+    """prefill() captured: the tall tiles one after the other on the graph's stream"""
+    H, I, T, E = 2560, 2304, 1500, 8
+    ex = to_dev(experts_on_gpu(H, I, 4, 620, nested_ids=(1, 3)))
+    L = M.MoELayer(E, H, I, Bmax=4)
+    for e in range(E):
+        L.set(e, ex[e % 4], 4 if ex[e % 4].nested else 2)
+    x = (torch.randn(T, H, generator=torch.Generator().manual_seed(3)) * 0.3).to(DEV).half()
+    sel, w = gumbel_topk(T, E, 8, seed=2)
+    want = L.prefill(x, sel, w)
+    torch.cuda.synchronize()
+    gr = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(gr):
+        y = L.prefill(x, sel, w)
+    for _ in range(3):
+        y.fill_(float("nan"))
+        gr.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want) and torch.equal(L.prefill(x, sel, w), want)
 
 
 @pytest.mark.parametrize("H,I", [(640, 384), (256, 1024)])
