@@ -5,16 +5,23 @@
 // bit for bit: every candidate is (value - target)^2 + cost in fp32 with the torch code's roundings (no contraction), and ties go
 // to the smallest predecessor.
 //
-// One workgroup of 1024 threads per ring. "Edge" = the low 16 - K bits of a state (E of them); the candidates of edge e are its
-// 2^K states, each with predecessor edge (q << (16 - 2 K)) | (e >> K), so 2^K neighbouring edges (a group) share their
-// predecessors: thread t owns the groups t + 1024 r, keeps the 64 codebook values of their states in registers through a
-// pass, reads 2^K costs per group from LDS and writes 2^K. Both directions of that traffic are free of bank conflicts. The
-// decisions of a thread in one step (16 edges x 2 bits, or 32 x 1) fill one word, stored to a scratch of 4 KB per step; the way
-// back is walked by one lane over blocks of steps brought to LDS, the next block in flight.
-// Bound: instruction issue of sixteen wavefronts in lockstep. A step is 65536 candidates of three fp32 operations plus the selection,
-// 19 vector instructions per four candidates (K = 2) = 309 per wavefront, which issue at one per 3.1 clocks and SIMD over the whole
-// launch (K = 1: 4.0; profiles/encoder_searches.txt); one ring per CU. Measured: 935 to 990 us for 256 rings (K = 2; 1.6 us per step,
-// the walks back ~100 us), 1160 us (K = 1, whose single array costs a second barrier); with all wavefronts at one priority 1060 and 1230.
+// One workgroup of 1024 threads per ring. "Edge" = the low 16 - K bits of a state (E of them); the
+// candidates of edge e are its 2^K states, each with predecessor edge (q << (16 - 2 K)) | (e >> K), so 2^K neighbouring edges (a
+// group) share their predecessors: thread t owns the groups t + 1024 r, keeps the 64 codebook values of their states in registers through
+// a pass, reads 2^K costs per group from LDS and writes 2^K. Both directions of that traffic are free of bank conflicts.
+// The decisions of a thread in one step (16 edges x 2 bits, or 32 x 1) fill one word, stored to a scratch of 4 KB per step; the way
+// back is walked by one lane over blocks of steps brought to LDS, the next block on its way meanwhile.
+//
+// Bound: instruction issue of sixteen wavefronts in lockstep, and with all CUs at work the clock that the power limit leaves. A step is 65536
+// candidates of three fp32 operations plus the selection. ns per four candidates (K = 2), wavefront and SIMD in a loop of nothing else:
+// the twelve fp32 operations 12.8; with three minima 14.1 (a three-way one and one of two 15.0); with the decision besides, as comparisons
+// whose lane masks are carried into the word, 20.9; as minima of doubles, below, 18.5. At K = 1 the sign of a difference shifted into
+// the word (9.3 for two candidates) is ahead of the carried mask (9.6) by more than that inside the kernel, of minima of doubles too.
+// Measured, us for 128 / 256 / 512 rings of 256 steps: K = 2 725 / 935 / 1785 (858 / 1019 / 2034 with the carried masks, decisions in steps
+// that nobody walks back over, and a walk that waited for each of its blocks), K = 1 932 / 1050 / 1990 (1084 / 1190 / 2300; its
+// single array costs a second barrier). The walks back are about 40 of them. Without any decisions 640 and 758 (K = 2): keeping
+// every seventh step's costs instead and finding the decisions anew from them cost more in traffic than that gives.
+#include "nq_decode.hpp"
 #include "nq_host.hpp"
 
 namespace nq {
@@ -26,15 +33,6 @@ struct VitArgs { const float* w; const float* lut; int64_t* st; uint32_t* back; 
 // all wavefronts' LDS accesses so far are done; stores to global memory stay in flight (a __syncthreads would wait for them)
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// word = word << 1 | this lane's bit of the mask. A mask straight from a comparison needs two wait states before a vector
-// instruction reads it (the compiler does not see into the asm); one that the scalar unit has combined does not.
-template <bool FROM_CMP>
-__device__ __forceinline__ void push_bit(uint32_t& word, unsigned long long mask)
-{
-    if constexpr (FROM_CMP) asm("s_nop 1\n\tv_addc_co_u32 %0, vcc, %0, %0, %1" : "+v"(word) : "s"(mask) : "vcc");
-    else asm("v_addc_co_u32 %0, vcc, %0, %0, %1" : "+v"(word) : "s"(mask) : "vcc");
-}
-
 // Wavefronts lower their priority as they get on with a step: the arbiter otherwise serves the oldest first, and a step ends with
 // the youngest wavefront of every SIMD alone, which cannot issue more than one instruction in six clocks.
 __device__ __forceinline__ void step_priority(int quarter)
@@ -45,11 +43,28 @@ __device__ __forceinline__ void step_priority(int quarter)
     else __builtin_amdgcn_s_setprio(0);
 }
 
-// one step of the search: costs cur -> nxt (K = 1: the same array), decisions -> the returned word
-template <int K>
-__device__ __forceinline__ uint32_t vit_step(const float (&v)[64 >> (2 * K)][1 << K][1 << K], float wv, const float* cur, float* nxt, int t)
+template <int K> constexpr int VIT_R = 64 >> (2 * K);           // groups per thread
+template <int K> using Values = float[VIT_R<K>][1 << K][1 << K];                         // [group][edge of the group][candidate]
+
+// The least of candidates and which one it was, in one instruction: a cost's bits as the upper half of a double, the candidate's number as the
+// lower half. Costs are >= +0 and never NaN (vit_target, vit_value), so doubles order as (cost, number) do, subnormal ones included: the first of the
+// least wins.
+typedef uint32_t Tagged __attribute__((ext_vector_type(2)));     // number, cost
+__device__ __forceinline__ Tagged vit_min(Tagged a, Tagged b)
 {
-    constexpr int Q = 1 << K, R = 64 >> (2 * K), G = 1024 * R;
+    double d;
+    asm("v_min_f64 %0, %1, %2" : "=v"(d) : "v"(__builtin_bit_cast(double, a)), "v"(__builtin_bit_cast(double, b)));
+    return __builtin_bit_cast(Tagged, d);
+}
+// a target that is not a finite number makes all candidates equally dear, infinitely so; a value that is no number is never near
+__device__ __forceinline__ float vit_target(float w) { return __builtin_fabsf(w) <= 3.4028234e38f ? w : 3e38f; }
+__device__ __forceinline__ float vit_value(float v) { return v == v ? v : __builtin_inff(); }
+
+// one step of the search: costs cur -> nxt (K = 1: the same array); DECIDE: the decisions -> the returned word
+template <int K, bool DECIDE>
+__device__ __forceinline__ uint32_t vit_step(const Values<K>& v, float wv, const float* cur, float* nxt, Tagged (&x)[1 << K], int t)
+{
+    constexpr int Q = 1 << K, R = VIT_R<K>, G = 1024 * R;
     float c[R][Q];
 #pragma unroll
     for (int r = 0; r < R; ++r)
@@ -61,45 +76,45 @@ __device__ __forceinline__ uint32_t vit_step(const float (&v)[64 >> (2 * K)][1 <
     for (int r = 0; r < R; ++r)
     {
         step_priority(4 * r / R);
-        uint32_t m[Q];
+        uint32_t m_of[Q];
 #pragma unroll
         for (int j = 0; j < Q; ++j)
         {
-            uint32_t x[Q];                                       // costs are >= +0: their bit patterns order as they do
+            auto cand = [&](int q) { const float d = v[r][j][q] - wv; return __builtin_bit_cast(uint32_t, d * d + c[r][q]); };
+            uint32_t m;
+            if constexpr (K == 2 && DECIDE)
+            {
 #pragma unroll
-            for (int q = 0; q < Q; ++q)
-            {
-                const float d = v[r][j][q] - wv;
-                x[q] = __builtin_bit_cast(uint32_t, d * d + c[r][q]);
-            }
-            // The decision is the first candidate that equals the minimum. Comparisons leave lane masks in scalar registers, the
-            // scalar unit combines them, and an add with carry shifts a mask's bit into the word: one vector instruction per bit.
-            if constexpr (K == 2)
-            {
-                const uint32_t m23 = x[3] < x[2] ? x[3] : x[2];
-                const uint32_t m01 = x[1] < x[0] ? x[1] : x[0], mm = m23 < m01 ? m23 : m01;            // one three-way minimum
-                const unsigned long long e0 = __builtin_amdgcn_uicmp(x[0], mm, 33), e1 = __builtin_amdgcn_uicmp(x[1], mm, 33), e2 = __builtin_amdgcn_uicmp(x[2], mm, 33);   // 33: not equal
-                push_bit<false>(word, e0 & e1); push_bit<false>(word, e0 & (~e1 | e2));
-                m[j] = mm;
+                for (int q = 0; q < Q; ++q) x[q].y = cand(q);
+                const Tagged b = vit_min(vit_min(x[0], x[1]), vit_min(x[2], x[3]));
+                asm("v_lshl_or_b32 %0, %0, 2, %1" : "+v"(word) : "v"(b.x));           // (as an expression it becomes a tree that keeps all numbers alive)
+                m = b.y;
             }
             else
             {
-                push_bit<true>(word, __builtin_amdgcn_uicmp(x[1], x[0], 36));                                      // 36: less
-                m[j] = x[1] < x[0] ? x[1] : x[0];
+                const uint32_t x0 = cand(0), x1 = cand(1);
+                m = x1 < x0 ? x1 : x0;
+                if constexpr (K == 2)
+                {
+                    uint32_t n;                                  // (two minima of two: a three-way one issues at half the rate)
+                    asm("v_min_u32 %0, %1, %2" : "=v"(n) : "v"(cand(2)), "v"(cand(3)));
+                    asm("v_min_u32 %0, %1, %2" : "=v"(m) : "v"(m), "v"(n));
+                }
+                else if constexpr (DECIDE) asm("v_alignbit_b32 %0, %0, %1, 31" : "+v"(word) : "v"(x1 - x0));     // word << 1 | sign of the difference
             }
+            m_of[j] = m;
         }
-        asm volatile("" : "+v"(word));                           // one group at a time: mixing them would not fit the registers
-        __builtin_amdgcn_sched_barrier(0);
-        if constexpr (K == 2) *(uint4*)(nxt + 4 * (t + 1024 * r)) = make_uint4(m[0], m[1], m[2], m[3]);
-        else *(uint2*)(nxt + 2 * (t + 1024 * r)) = make_uint2(m[0], m[1]);
+        __builtin_amdgcn_sched_barrier(0);                       // one group at a time: mixing them would not fit the registers
+        if constexpr (K == 2) *(uint4*)(nxt + 4 * (t + 1024 * r)) = make_uint4(m_of[0], m_of[1], m_of[2], m_of[3]);
+        else *(uint2*)(nxt + 2 * (t + 1024 * r)) = make_uint2(m_of[0], m_of[1]);
     }
     return word;
 }
 
-// walk back over the rows hi .. 0 of the decisions: sl[row] = state at that row. back rows are 4 KB; 16 rows per block, the
-// block after next requested while a lane walks. Returns (to thread 0) the edge entering row 0.
+// walk back over the rows hi .. 0 of the decisions: sl[row] = state at that row. back rows are 4 KB; 16 rows per block, walked by one lane
+// while the next block is written to the other half of buf and the one after that is on its way. Returns the edge entering row 0.
 template <int K>
-__device__ __forceinline__ int vit_trace(const uint32_t* back, int hi, int edge, uint32_t* buf, int* sl, int t)
+__device__ __forceinline__ int vit_trace(const uint32_t* back, int hi, int edge, uint32_t* buf, int* sl, int& edge_sh, int t)
 {
     constexpr int Q = 1 << K, KR = 16 - K, ROWS = 16;
     uint4 nx[ROWS / 4];
@@ -111,49 +126,55 @@ __device__ __forceinline__ int vit_trace(const uint32_t* back, int hi, int edge,
             nx[u] = row >= 0 ? *(const uint4*)(back + (size_t)row * VT + 4 * (t & 255)) : make_uint4(0, 0, 0, 0);
         }
     };
-    request(hi);
-    for (int top = hi; top >= 0; top -= ROWS)
-    {
+    auto place = [&](uint32_t* half) {
 #pragma unroll
-        for (int u = 0; u < ROWS / 4; ++u) *(uint4*)(buf + (4 * u + (t >> 8)) * VT + 4 * (t & 255)) = nx[u];
-        if (top >= ROWS) request(top - ROWS);
-        lds_barrier();
+        for (int u = 0; u < ROWS / 4; ++u) *(uint4*)(half + (4 * u + (t >> 8)) * VT + 4 * (t & 255)) = nx[u];
+    };
+    request(hi);
+    place(buf);
+    if (hi >= ROWS) request(hi - ROWS);
+    for (int top = hi, b = 0; top >= 0; top -= ROWS, b ^= 1)
+    {
+        lds_barrier();                                           // block b is there, block b ^ 1 has been walked
+        if (top >= ROWS) place(buf + (b ^ 1) * ROWS * VT);
+        if (top >= 2 * ROWS) request(top - 2 * ROWS);
         if (t == 0)
             for (int s = 0; s < ROWS && top - s >= 0; ++s)
             {
                 const int g = edge >> K;
-                const uint32_t q = (buf[s * VT + (g & 1023)] >> (32 - K - K * ((g >> 10) * Q + (edge & (Q - 1))))) & (Q - 1);   // first pushed = highest
+                const uint32_t q = (buf[(b * ROWS + s) * VT + (g & 1023)] >> (32 - K - K * ((g >> 10) * Q + (edge & (Q - 1))))) & (Q - 1);   // first pushed = highest
                 const int st = (int)(q << KR) | edge;
                 sl[top - s] = st;
                 edge = st >> K;
             }
-        lds_barrier();
     }
-    return edge;
+    if (t == 0) edge_sh = edge;
+    lds_barrier();
+    return edge_sh;
 }
 
 template <int K>
 __global__ void __launch_bounds__(VT) nq_viterbi_k(VitArgs a)
 {
-    constexpr int Q = 1 << K, KR = 16 - K, E = 1 << KR, R = 64 >> (2 * K);
+    constexpr int Q = 1 << K, KR = 16 - K, E = 1 << KR, R = VIT_R<K>;
     extern __shared__ __align__(16) float cost[];                // 128 KB: two arrays of E costs (K = 2), or one (K = 1); then the walk's blocks
     __shared__ float wl[VIT_LMAX];
     __shared__ int sl[VIT_LMAX];
     __shared__ unsigned long long red[VT / 64];
-    __shared__ int start_sh;
+    __shared__ int edge_sh;
     const int t = threadIdx.x, L = a.L;
     uint32_t* back = a.back + (size_t)blockIdx.x * L * VT;
     for (int ring = blockIdx.x; ring < a.T; ring += gridDim.x)
     {
-        for (int i = t; i < L; i += VT) wl[i] = a.w[(size_t)ring * L + (a.rev ? (L - i) % L : i)];
+        for (int i = t; i < L; i += VT) wl[i] = vit_target(a.w[(size_t)ring * L + (a.rev ? (L - i) % L : i)]);
         int start = -1;
 #pragma clang loop unroll(disable)
         for (int pass = 0; pass < 2; ++pass)
         {
-            asm volatile("" : "+s"(pass));                       // one copy of the loop below
-            const int roll = pass == 0 ? L / 2 : 0, keep = pass == 0 && L > 1 ? L - roll : 0;
+            asm volatile("" : "+s"(pass));                       // one copy of the loops below
+            const int roll = pass == 0 ? L / 2 : 0, keep = pass == 0 && L > 1 ? L - roll : 0;     // nobody walks back over the steps before `keep`
             for (int e = t; e < E; e += VT) cost[e] = pass == 0 || e == start ? 0.f : __builtin_inff();
-            float v[R][Q][Q];                                    // the pass's codebook values: loaded here so that nothing else shares their registers
+            Values<K> v;                                         // the pass's codebook values: loaded here so that nothing else shares their registers
             uint32_t off = Q * t * 4u;
             asm volatile("" : "+v"(off));
 #pragma unroll
@@ -163,18 +184,27 @@ __global__ void __launch_bounds__(VT) nq_viterbi_k(VitArgs a)
                 {
                     const char* base = (const char*)(a.lut + (q << KR) + Q * 1024 * r);
 #pragma unroll
-                    for (int j = 0; j < Q; ++j) v[r][j][q] = *(const float*)(base + off + 4 * j);
+                    for (int j = 0; j < Q; ++j) v[r][j][q] = vit_value(*(const float*)(base + off + 4 * j));
                 }
+            Tagged x[Q];                                         // their numbers stay where they are through all steps
+#pragma unroll
+            for (int q = 0; q < Q; ++q) { uint32_t num = q; asm volatile("" : "+v"(num)); x[q].x = num; }
             lds_barrier();
-            for (int i = 0; i < L; ++i)
-            {
-                const int ri = i + roll < L ? i + roll : i + roll - L;
-                float* cur = K == 2 ? cost + (i & 1) * E : cost;
-                float* nxt = K == 2 ? cost + (~i & 1) * E : cost;
-                const uint32_t word = vit_step<K>(v, wl[ri], cur, nxt, t);
-                if (i >= keep) back[(size_t)ri * VT + t] = word;
-                lds_barrier();
-            }
+            auto steps = [&](auto decide, int from, int to) {
+                constexpr bool D = decltype(decide)::value != 0;
+                for (int i = from; i < to; ++i)
+                {
+                    const int ri = i + roll < L ? i + roll : i + roll - L;
+                    float* cur = K == 2 ? cost + (i & 1) * E : cost;
+                    float* nxt = K == 2 ? cost + (~i & 1) * E : cost;
+                    const uint32_t word = vit_step<K, D>(v, wl[ri], cur, nxt, x, t);
+                    if (D) back[(size_t)ri * VT + t] = word;
+                    lds_barrier();
+                }
+            };
+            steps(CodeTag<0>{}, 0, keep);
+            steps(CodeTag<1>{}, keep, L);
+            __builtin_amdgcn_s_setprio(0);
             int edge = start;
             if (pass == 0)
             {   // the cheapest edge after the last step, the smallest of equals
@@ -194,13 +224,7 @@ __global__ void __launch_bounds__(VT) nq_viterbi_k(VitArgs a)
                 edge = (int)(best & 0xFFFFFFFFu);
             }
             __syncthreads();                                     // the decisions of all wavefronts are in memory
-            edge = vit_trace<K>(back, pass == 0 && L > 1 ? roll - 1 : L - 1, edge, (uint32_t*)cost, sl, t);
-            if (pass == 0)
-            {
-                if (t == 0) start_sh = edge;
-                lds_barrier();
-                start = start_sh;
-            }
+            start = vit_trace<K>(back, pass == 0 && L > 1 ? roll - 1 : L - 1, edge, (uint32_t*)cost, sl, edge_sh, t);
         }
         for (int i = t; i < L; i += VT) a.st[(size_t)ring * L + (a.rev ? (L - i) % L : i)] = sl[i];
         lds_barrier();                                           // sl and wl are free again

@@ -171,3 +171,15 @@ def test_searches_over_targets_that_are_not_finite(K):
     assert torch.equal(EN.viterbi_ring(w.cuda(), lut.cuda(), K).cpu(), EN.viterbi_ring(w, lut, K))
     a = torch.randint(0, 256, (4, 24), generator=g)
     assert torch.equal(EN.viterbi_ring_given_p3(w.cuda(), a.cuda(), lut.cuda()).cpu(), EN.viterbi_ring_given_p3(w, a, lut))
+
+
+@pytest.mark.parametrize("K", [1, 2])
+@pytest.mark.parametrize("scale", [1e-21, 3e-20, 1e18])
+def test_searches_at_the_ends_of_the_range_of_costs(K, scale):
+    """costs that are zero, subnormal or close to overflow order as they do in torch, ties included (L 17 and 40: one block of the walk
+    back and a remainder, two blocks and a remainder)"""
+    g = torch.Generator().manual_seed(K)
+    lut = EN.codebook().round().clamp(-5, 5) * scale
+    for L in (17, 40):
+        w = torch.randint(-6, 7, (3, L), generator=g).float() * scale
+        assert torch.equal(EN.viterbi_ring(w.cuda(), lut.cuda(), K).cpu(), EN.viterbi_ring(w, lut, K))
