@@ -268,6 +268,14 @@ int nq_pf_plan(const int32_t* counts, int E, int row_lo, int nrows, int32_t* til
  * projection (which = 1 | 8) left in acc_gu, added up. */
 int nq_sum_slices(const float* part, int ny, int64_t n, float* out, void* stream);
 
+/* One expert's gate|up projection alone, in one launch: out [B][2I] fp32 = W_gu . fp16(Hadamard-128(x * su)) for x [B][H] (B <= 8), gate rows
+ * rotated with su_g, up rows with su_u; row = the expert's table row (device). k-slices of `chunks` 128-column chunks (a divisor of H / 128, at
+ * most 48), sb = 1, 2 or 4 wavefronts per block. part: (H / 128 / chunks) * B * 2I floats, not initialised, holds the k-slice partial sums
+ * [slice][B][2I] afterwards (with one slice untouched); cnt: 2I / 128 counters, zero on entry and exit. Rows of the common kind only (base
+ * window code 0, no mask-mode flags): another kind comes out NaN, level 0 zero. */
+int nq_proj(const void* x, int x_dtype, int B, const int64_t* row, int H, int I, int G, int chunks, int sb, float* part, int64_t part_elems,
+            int32_t* cnt, int64_t cnt_elems, float* out, void* stream);
+
 /* A whole step of T tokens on device data, no host synchronisation: pairs sorted by expert, tile plan, rotation, gate|up, SwiGLU,
  * down, combine -- the chain of the entry points above (reference moe.prefill, sm120/moe.py:282-326) with the casts of its caller
  * (x.half(), ids.long(), w.half(), out.to(dtype), sm120/serve/nq_vllm.py:522,573) at the loads and the final store. Ids outside

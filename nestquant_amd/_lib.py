@@ -72,6 +72,7 @@ SIGNATURES = {
     "nq_pf_mid_rows": (C.c_int, [_vp, _i32p, _i, _i64p, _vp, _vp, _vp, _i, _i, _i, _i32p, _i, _i, _vp]),
     "nq_pf_post": (C.c_int, [_vp, _i32p, _i64p, _vp, _i, _i, _i, _i, _i64p, _vp, _vp, _i, _i, _i, _vp]),
     "nq_pf_plan": (C.c_int, [_i32p, _i, _i, _i, _i32p, _i, _i32p, _i, _i, _vp]),
+    "nq_proj": (C.c_int, [_vp, _i, _i, _vp, _i, _i, _i, _i, _i, _vp, C.c_int64, _vp, C.c_int64, _vp, _vp]),
     "nq_sum_slices": (C.c_int, [_vp, _i, C.c_int64, _vp, _vp]),
     "nq_pf_step": (C.c_int, [C.POINTER(NqPfArgs), _vp]),
     "nq_pf_meta_bytes": (C.c_int64, [_i, _i, _i, _i]),

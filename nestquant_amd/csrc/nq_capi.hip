@@ -364,6 +364,18 @@ extern "C" int nq_viterbi_p4(const float* w, const int64_t* a, int T, int L, con
     return launch_viterbi_p4(w, a, T, L, lut, b, position_order != 0, (hipStream_t)stream);
 }
 
+extern "C" int nq_proj(const void* x, int x_dtype, int B, const int64_t* row, int H, int I, int G, int chunks, int sb, float* part, int64_t part_elems,
+                       int32_t* cnt, int64_t cnt_elems, float* out, void* stream)
+{
+    NQ_REQUIRE(x && row && part && cnt && out, "nq_proj: null pointer");
+    NQ_REQUIRE(B >= 1 && B <= 8 && x_dtype >= 0 && x_dtype <= 2, "nq_proj: B=%d (1..8) x_dtype=%d", B, x_dtype);
+    NQ_REQUIRE(shape_ok(H, I) && (G == 4 || G == 2), "nq_proj: H=%d I=%d must be positive multiples of 128, G=%d (rings of 4 lanes, or 2)", H, I, G);
+    NQ_REQUIRE(chunks >= 1 && chunks <= 48 && H / 128 % chunks == 0 && (sb == 1 || sb == 2 || sb == 4), "nq_proj: k-slice %d chunks of %d, %d wavefronts per block (1, 2 or 4)", chunks, H / 128, sb);
+    NQ_REQUIRE(aligned16(x) && aligned16(part) && aligned16(out), "nq_proj: x, part and out must be 16-byte aligned");
+    NQ_REQUIRE(part_elems >= (int64_t)(H / 128 / chunks) * B * 2 * I && cnt_elems >= 2 * I / 128, "workspace too small: part or cnt");
+    return launch_proj(x, x_dtype, B, row, H, I, G, chunks, sb, part, cnt, out, (hipStream_t)stream);
+}
+
 extern "C" int nq_sum_slices(const float* part, int ny, int64_t n, float* out, void* stream)
 {
     NQ_REQUIRE(ny >= 1 && n >= 0 && n % 4 == 0, "nq_sum_slices: ny=%d n=%lld (a multiple of 4)", ny, (long long)n);

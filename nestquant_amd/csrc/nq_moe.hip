@@ -839,6 +839,124 @@ int launch_moe_static(MoeArgs a, const int* cfg_gu, const int* cfg_dn, int which
     return launch_moe(a, cfg_gu, cfg_dn, which, st);
 }
 
+// ---- a lone projection ---------------------------------------------------------------------------------------------------------
+// out[B][2I] = W_gu . fp16(Hadamard-128(x * su)) of one expert for B tokens in one launch: what a gate|up launch of one run computes,
+// whose routing the host knows. grid (row blocks, k-slices), block 64 * SB; a workgroup reads the table row, rotates its own k-slice of
+// the tokens (eight columns per lane, four chunks per wavefront at a time: a tenth of its decode) and decodes as nq_gemv_k does. The
+// last workgroup of a 128-row group adds the group's slices in slice order. Common rows only, as nq_gemv_k<0, false>: another kind comes out NaN.
+// Bound by latency beside the decode: table row, then records and sign vector, then 5.8 us of decode issue at level 3 (6144 x 4096), then
+// acknowledged stores, arrival counter and the slices' sums. Eight tokens, us a call: levels 2 / 3 / 4 10.7 / 13.7 / 13.8, where routing
+// launch, gate|up launch and slice sums took 20.4 / 19.0 / 19.0; slices of 2, 3, 6 or 8 chunks 13.5, 13.6, 14.2, 16.9 at level 3.
+struct ProjArgs { const void* x; const int64_t* row; float* part; int* cnt; float* out; int x_dtype, B, H, I, G; };
+__device__ __forceinline__ float4_t ld_dev4_issue(const float* p)
+{
+    float4_t v;
+    asm volatile("global_load_dwordx4 %0, %1, off sc0 sc1" : "=v"(v) : "v"(p) : "memory");
+    return v;
+}
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) nq_proj_k(ProjArgs a, int NC)
+{
+    extern __shared__ __align__(16) char smem[];
+    __builtin_amdgcn_s_setprio(3);
+    __shared__ int last;
+    const int lane = threadIdx.x & 63, warp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), SB = blockDim.x >> 6;
+    int64_t ent[TBL_W];                                          // block-uniform: through the scalar cache
+    const __attribute__((address_space(4))) int64_t* src = (const __attribute__((address_space(4))) int64_t*)a.row;
+#pragma unroll
+    for (int i = 0; i < TBL_W; ++i) ent[i] = src[i];
+    const int N = 2 * a.I, C = a.H / 128, NY = C / NC, chunk0 = blockIdx.y * NC, rowstride = NC * 256 + 16;
+    const int t4 = lane >> 4, ss = (lane >> 3) & 1, g = lane & 7, n = lane & 15;
+    // the tokens' k-slice, before the row is there: chunk-tasks (token, chunk), four per wavefront at a time
+    const int L8 = wht_place(lane), tasks = a.B * NC, col8 = 32 * (L8 >> 2) + 2 * (L8 & 3);
+    const int strip = 2 * (blockIdx.x * SB + warp) + ss;
+    const int level = (int)ent[0];
+    const Planes P = planes_of(ent, 0);
+    const bool live = level > 0, foreign = P.bcode != 0 || (P.flags != nullptr && level != 2);
+    LaneCtx L;
+    L.unit0 = (uint32_t)strip * C + chunk0; L.rec0 = L.unit0 * 32 + 4 * g + t4;
+    L.nrec = (size_t)(N / 16) * C * 32;
+    L.src = a.G == 2 ? lane ^ 16 : (lane + 16) & 63;
+    L.g = g; L.strip = (uint32_t)strip; L.nstrips = (size_t)(N / 16); L.chunk0 = chunk0;
+    char* zero = smem + a.B * rowstride;
+    L.xs = (n < a.B ? smem + n * rowstride : zero) + t4 * 16; L.xstep = n < a.B ? 256 : 0;
+    u32x4 nb0 = {0u, 0u, 0u, 0u};
+    if (live && !foreign) nb0 = load_base<0>(P, L.rec0, L.nrec);
+    const WhtSigns ws = wht_signs(lane);
+    const _Float16* su = (const _Float16*)ent[9] + ((int)(blockIdx.x * SB * 32) >= a.I ? 2 * a.H + 3 * a.I : 0);
+    for (int q0 = 4 * warp; live && q0 < tasks; q0 += 4 * SB)
+    {
+        const int q = min(q0 + (lane >> 4), tasks - 1), j = q / NC, c = q - j * NC;       // lanes beyond the last task repeat it
+        const size_t at = (size_t)j * a.H + (chunk0 + c) * 128 + col8;
+        half2_t xv[4], sv[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) { xv[i] = act2_at(a.x, a.x_dtype, at + 8 * i); sv[i] = *(const half2_t*)(su + (chunk0 + c) * 128 + col8 + 8 * i); }
+        float v[8];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) { v[2 * i] = (float)xv[i].x * (float)sv[i].x; v[2 * i + 1] = (float)xv[i].y * (float)sv[i].y; }
+        wht8_bop(v, ws);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) asm volatile("" : "+v"(v[i]));                // scaled in fp32, then rounded to fp16, as nq_prep_k does (see finish_gu)
+        *(uint4*)(smem + j * rowstride + c * 256 + 16 * L8) = bop_block(v);
+    }
+    if (threadIdx.x < 64) ((uint32_t*)zero)[threadIdx.x] = 0u;
+    __syncthreads();
+
+    float4_t acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    if (foreign) { const float nan = __builtin_nanf(""); acc[0] = float4_t{nan, nan, nan, nan}; acc[1] = acc[0]; }
+    else if (level == 2) gemv_chunks<false, 0, 0, false>(P, L, NC, acc, nb0);
+    else if (live) dispatch_code(P.code, [&](auto tag) { gemv_chunks<true, decltype(tag)::value, 0, false>(P, L, NC, acc, nb0); });
+    __builtin_amdgcn_s_setprio(3);
+
+    const int row = 16 * (2 * (blockIdx.x * SB + warp) + (t4 >> 1)) + 4 * (t4 & 1);
+    if (NY == 1)
+    {
+        if (n < a.B) { float* o = a.out + (size_t)n * N + row; *(float4_t*)o = acc[0]; *(float4_t*)(o + 8) = acc[1]; }
+        return;
+    }
+    if (n < a.B)
+    {
+        float* part = a.part + ((size_t)blockIdx.y * a.B + n) * N + row;
+        st_dev4(part, acc[0]); st_dev4(part + 8, acc[1]);
+    }
+    // the hand-off of nq_gemv_k: acknowledged stores, then the group's counter; the last to arrive reads the slices device-coherently
+    const int grp = blockIdx.x * SB * 32 / 128, expect = NY * (128 / (SB * 32));
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) last = __hip_atomic_fetch_add(a.cnt + grp, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == expect - 1;
+    __syncthreads();
+    if (!last) return;
+    for (int i = threadIdx.x; i < a.B * 32; i += blockDim.x)     // four rows of one token each
+    {
+        const size_t at = (size_t)(i >> 5) * N + grp * 128 + 4 * (i & 31);
+        float4_t s = {0.f, 0.f, 0.f, 0.f};
+        for (int y = 0; y < NY; y += 8)
+        {
+            float4_t v[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) v[k] = ld_dev4_issue(a.part + (size_t)(y + k < NY ? y + k : y) * a.B * N + at);
+#pragma unroll
+            for (int k = 0; k < 8; k += 4) asm volatile("s_waitcnt vmcnt(0)" : "+v"(v[k]), "+v"(v[k + 1]), "+v"(v[k + 2]), "+v"(v[k + 3]) :: "memory");
+#pragma unroll
+            for (int k = 0; k < 8; ++k) if (y + k < NY) s += v[k];
+        }
+        *(float4_t*)(a.out + at) = s;
+    }
+    if (threadIdx.x == 0) __hip_atomic_store(a.cnt + grp, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+int launch_proj(const void* x, int x_dtype, int B, const int64_t* row, int H, int I, int G, int NC, int SB, float* part, int* cnt, float* out, hipStream_t st)
+{
+    const ProjArgs a{x, row, part, cnt, out, x_dtype, B, H, I, G};
+    const int shm = B * (NC * 256 + 16) + 256;
+    if (shm > 48 * 1024)
+    {
+        const hipError_t e = hipFuncSetAttribute((const void*)nq_proj_k, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
+        if (e != hipSuccess) return set_error("nq_proj: LDS %d bytes: %s", shm, hipGetErrorString(e));
+    }
+    nq_proj_k<<<dim3(2 * I / 32 / SB, H / 128 / NC), 64 * SB, shm, st>>>(a, NC);
+    NQ_LAUNCH_CHECK("nq_proj");
+    return 0;
+}
+
 // out[i] = sum over the ny k-slices of part[y * n + i], in slice order (n a multiple of 4): what is left of a lone projection. Bound by
 // the launch: 24 slices of 8 x 4096 (3 MB, just written, so from the last-level cache) take 2.8 us where a library sum over the first
 // dimension took 5.4 us and chose its blocks on the host first; a projection of eight tokens 21.4 -> 19.3 us.

@@ -596,10 +596,14 @@ Expert.ref = expert_ref
 
 def proj_gemv(layer, x, e=0, cfg=None):
     """Raw fused decode+GEMV of the gate|up projection of expert e for every token of x [B, H] (B <= 8), without the
-    SwiGLU finisher: returns fp32 [B, 2I] = W_gu . fp16(Hadamard(x * su)) (rows < I rotated with su_g, the rest with su_u),
-    read back from the layer's k-slice partial sums after a gate|up launch that leaves the SwiGLU out."""
+    SwiGLU finisher: returns fp32 [B, 2I] = W_gu . fp16(Hadamard(x * su)) (rows < I rotated with su_g, the rest with su_u)."""
     B = x.shape[0]
     C_ = layer.H // 128
+    # One launch (nq_proj) for rows of the common kind where nobody counts the picks; what that leaves, and what it would refuse, goes through
+    # a layer call of one run and the sum of its slices. At 6144 x 4096, eight tokens: 10.7 / 13.7 / 13.8 us a call at levels 2 / 3 / 4, three
+    # launches 20.4 / 19.0 / 19.0.
+    lone = not layer.rare_rows and not layer.hits_ptr and 0 <= e < layer.E and 0 < B <= min(8, layer.Bmax) and x.dtype in _DT_IN \
+        and x.is_contiguous() and x.shape == (B, layer.H) and layer.cnt_gu.numel() >= 2 * layer.I // 128
     if cfg is None:
         # one run: about 512 workgroups and slices of two or three chunks at the full shape are where heads, decode and the number
         # of partial sums balance, as far as the layer's workspace holds that many slices
@@ -607,6 +611,16 @@ def proj_gemv(layer, x, e=0, cfg=None):
         n = MoELayer._slice(C_, 2 * layer.I // 32 // sb, 1, 512, 24)
         n = next(d for d in range(n, C_ + 1) if C_ % d == 0 and C_ // d <= layer.acc_gu.shape[0])
         cfg = [1, sb, n]
+    n = 2 * layer.I
+    if lone and len(cfg) == 3 and cfg[0] >= 1 and cfg[2] >= 1 and C_ % (cfg[0] * cfg[2]) == 0:
+        if C_ // (cfg[0] * cfg[2]) * B * n > layer.acc_gu.numel():
+            layer._alloc_partials(cfg)
+        out = torch.empty(B, n, dtype=torch.float32, device=x.device)
+        rc = layer.M.nq_proj(x.data_ptr(), _DT_IN[x.dtype], B, layer.table.data_ptr() + 8 * TBL_W * e, layer.H, layer.I, layer.G, cfg[0] * cfg[2], cfg[1],
+                             layer.acc_gu.data_ptr(), layer.acc_gu.numel(), layer.cnt_gu.data_ptr(), layer.cnt_gu.numel(), out.data_ptr(), _lib.stream_ptr())
+        if rc:
+            _lib.check(rc)
+        return out
     picks = layer._lone_views.get((B, e))
     if picks is None:
         if 0 <= e < layer.E and B <= 8:
@@ -615,8 +629,7 @@ def proj_gemv(layer, x, e=0, cfg=None):
             picks = torch.full((B, 1), e, dtype=torch.int64, device=x.device), torch.ones(B, 1, dtype=torch.float16, device=x.device)
     sel, rw = picks
     layer(x, sel, rw, which=1 | 8, cfg_gu=list(cfg))              # 8: the launch ends with its partial sums
-    ny = C_ // (cfg[0] * cfg[2])
-    n = 2 * layer.I                                               # partial sums are laid out [k-slice][B * topk of the call][2I]
+    ny = C_ // (cfg[0] * cfg[2])                                  # partial sums are laid out [k-slice][B * topk of the call][2I]
     out = torch.empty(B, n, dtype=torch.float32, device=x.device)
     _lib.check(layer.M.nq_sum_slices(layer.acc_gu.data_ptr(), ny, B * n, out.data_ptr(), _lib.stream_ptr()))
     return out

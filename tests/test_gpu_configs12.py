@@ -290,3 +290,35 @@ def test_projection_captured_before_its_first_eager_call():
         assert rel_err(y.cpu().numpy(), want[e].cpu().numpy()) < 1e-4, e
     for f in range(E):
         assert rel_err(M.proj_gemv(L, x[:1], f).cpu().numpy(), want[f][:1].cpu().numpy()) < 1e-4
+
+
+@pytest.mark.parametrize("H,I,B,level,cfg,dt,G", [
+    (128, 128, 1, 2, None, torch.float16, 4),                     # one chunk: no partial sums
+    (256, 128, 3, 4, [1, 4, 1], torch.bfloat16, 4),               # two slices
+    (640, 256, 8, 3, [1, 2, 1], torch.float16, 4),                # five chunks, two wavefronts per block, the most tokens
+    (640, 256, 5, 2, [1, 1, 5], torch.float32, 4),                # one wavefront per block, five token rows in its only slice
+    (1536, 384, 7, 4, [1, 4, 4], torch.float16, 4),               # chunk-tasks that do not fill the last wavefront
+    (2304, 128, 8, 3, [1, 4, 1], torch.float16, 4),               # eighteen slices: more than two batches of the sum
+    (512, 128, 2, 4, None, torch.float16, 2),                     # rings of two lanes
+])
+def test_projection_launch_equals_a_layer_call_of_one_run(H, I, B, level, cfg, dt, G):
+    """the one-launch projection against the layer call and slice sum that it stands for (which it still is where the picks are counted):
+    the same products, with at most a few activations rounded to the other fp16 neighbour (2^-11 of one of H terms each); bitwise
+    repeatable, counters left at zero, level 0 zero, a foreign row NaN"""
+    ex = F.Expert(H, I, seed=3, dev="cpu", nested=True)
+    ex.gu.to(DEV); ex.dn.to(DEV); ex.signs = ex.signs.to(DEV)
+    ex.gu.slot = ex.gu.nested_plane(); ex.dn.slot = ex.dn.nested_plane()
+    L = M.MoELayer(3, H, I, Bmax=8, topk=1, G=G)
+    L.set(1, ex, level)
+    x = (torch.randn(B, H, generator=torch.Generator().manual_seed(B)) * 0.3).to(dt).to(DEV)
+    hits = torch.zeros(3, dtype=torch.int32, device=DEV)
+    got = M.proj_gemv(L, x, 1, cfg)
+    assert torch.equal(got, M.proj_gemv(L, x, 1, cfg)) and not L.cnt_gu.any()
+    L.hits_ptr = hits.data_ptr()
+    want = M.proj_gemv(L, x, 1, cfg)
+    L.hits_ptr = 0
+    assert hits.tolist() == [0, B, 0]
+    assert rel_err(got.cpu().numpy(), want.cpu().numpy()) < 4 * 2.0 ** -11 / H ** 0.5
+    assert not M.proj_gemv(L, x, 0, cfg).any()                    # level 0
+    L.table[2].copy_(L.table[1]); L.table[2, 19] = 1              # a base plane of another window code, written past the layer
+    assert M.proj_gemv(L, x, 2, cfg).isnan().all()
