@@ -331,6 +331,12 @@ int nq_viterbi_p4(const float* w, const int64_t* a, int T, int L, const float* l
 int nq_fit_residual(const float* target, const float* sign, const int64_t* st_base, const float* lut, double scale, int U, float* out, void* stream);
 int nq_fit_words(const float* target, const float* sign, const int64_t* st_base, const int64_t* st_res, const float* lut, int U, const double* Da, int64_t da_step,
                  const double* Do, int64_t do_step, void* ws, int64_t ws_bytes, float* Q, int64_t* Mb, int64_t* N, double* delta, void* stream);
+/* A fitted plane as the decoder reads it: states int64 [strips * chunks][8][256] -> words int32 [units * 32][2 K], the lane records of its K
+ * new bits per step (32 records a unit: ring, lane of four). Optionally dw int32 [units] = Mb | N << 8; var uint8 [units] = ring g negated in
+ * bit g, from sign fp32 [units][8]; Q fp32 [16 strips][128 chunks] = values fp32 [units][8][256], or lut[state] * sign where values is NULL
+ * (sign NULL = +1). *bad is set to 1 if the states of a ring do not close, else left alone. */
+int nq_fit_pack(const int64_t* states, int K, const float* values, const float* sign, const float* lut, const int64_t* Mb, const int64_t* N, int strips, int chunks,
+                int32_t* words, int32_t* dw, uint8_t* var, float* Q, int32_t* bad, void* stream);
 
 /* ---- Refinement-record upgrade engine (host threads + one side stream; replaces the class Engine of the reference's
  * streaming/nqstream.cu:51-277 and its Python surface, :8-26). One engine per record file (one rank) and GPU. Unlike the

@@ -81,6 +81,7 @@ SIGNATURES = {
     "nq_viterbi_p4": (C.c_int, [_vp, _vp, _i, _i, _vp, _vp, _i, _vp]),
     "nq_fit_residual": (C.c_int, [_vp, _vp, _vp, _vp, C.c_double, _i, _vp, _vp]),
     "nq_fit_words": (C.c_int, [_vp, _vp, _vp, _vp, _vp, _i, _vp, C.c_int64, _vp, C.c_int64, _vp, C.c_int64, _vp, _vp, _vp, _vp, _vp]),
+    "nq_fit_pack": (C.c_int, [_vp, _i, _vp, _vp, _vp, _vp, _vp, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp]),
     # record upgrade engine (host threads; structures mirrored in stream_engine.py)
     "nq_stream_open": (C.c_void_p, [C.c_char_p, C.c_char_p, C.c_int64, _i, _i, _i, _i]),
     "nq_stream_upgrade": (C.c_int, [_vp, C.c_int64, C.c_int64, _vp, _vp, C.POINTER(C.c_int64), _vp, C.c_int32]),

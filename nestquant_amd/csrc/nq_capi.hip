@@ -356,6 +356,18 @@ extern "C" int nq_fit_words(const float* target, const float* sign, const int64_
     return launch_fit_words(target, sign, st_base, st_res, lut, U, Da, da_step, Do, do_step, ws, Q, Mb, N, delta, (hipStream_t)stream);
 }
 
+extern "C" int nq_fit_pack(const int64_t* states, int K, const float* values, const float* sign, const float* lut, const int64_t* Mb, const int64_t* N, int strips, int chunks,
+                           int32_t* words, int32_t* dw, uint8_t* var, float* Q, int32_t* bad, void* stream)
+{
+    NQ_REQUIRE(K == 1 || K == 2, "nq_fit_pack: K=%d (1 or 2)", K);
+    NQ_REQUIRE(strips >= 0 && chunks >= 1 && (int64_t)strips * chunks <= INT32_MAX / 64, "nq_fit_pack: %d x %d units", strips, chunks);
+    if (strips == 0) return 0;
+    NQ_REQUIRE(states && words && bad, "nq_fit_pack: null pointer");
+    NQ_REQUIRE(!Q || values || lut, "nq_fit_pack: a matrix needs values or a codebook");
+    NQ_REQUIRE((!dw || (Mb && N)) && (!var || sign), "nq_fit_pack: block words need Mb and N, the sign plane its signs");
+    return launch_fit_pack(states, K, values, sign, lut, Mb, N, strips * chunks, chunks, words, dw, var, Q, bad, (hipStream_t)stream);
+}
+
 extern "C" int nq_viterbi_p4(const float* w, const int64_t* a, int T, int L, const float* lut, int64_t* b, int position_order, void* stream)
 {
     NQ_REQUIRE(T >= 0 && L >= 1 && L <= 256, "nq_viterbi_p4: T=%d L=%d (1..256)", T, L);

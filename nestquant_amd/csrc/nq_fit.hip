@@ -6,6 +6,7 @@
 //   nq_fit_delta_k     delta per unit and the twelve candidates
 //   nq_fit_cost_k      cost of candidate c of unit u: sum of squared errors, or tr(Do E Da E^T) with the unit's metrics
 //   nq_fit_pick_k      the first candidate of least cost; its values
+//   nq_fit_pack_k      a plane as the decoder reads it, and its values as a matrix
 //
 // A unit is 16 x 128 weights, held as 8 rings of 256 (ring position order), 2048 values on one workgroup of 256 threads. In torch
 // the same is about three hundred launches over a few hundred kilobytes per stage, with a synchronisation at each of the twelve
@@ -162,6 +163,68 @@ __global__ void __launch_bounds__(256) nq_fit_pick_k(const float* __restrict__ s
         Q[at] = fold_value(byte_sum((uint32_t)st_base[at]), byte_sum((uint32_t)st_res[at]), dw, k) * sign_of(sign, u, i);
     }
     if (t == 0) { Mb[u] = dw & 0xFF; N[u] = dw >> 8; }
+}
+
+// What a fit hands out for one plane, one unit per workgroup: the states' new bits as lane records, the block words, the ring signs as a
+// byte, and the values as a matrix (from the codebook, or given in ring order). In torch some forty launches a plane, and the check of
+// the ring, which stops the host, in each: three planes of a 128 x 256 weight took 0.96 ms. A ring is whole if every state's upper bits are the
+// next one's lower bits; the first that is not sets *bad, which the host reads once for all planes.
+struct PackArgs
+{
+    const int64_t* st; const float* values; const float* sign; const float* lut; const int64_t* Mb; const int64_t* N;
+    int32_t* words; int32_t* dw; uint8_t* var; float* Q; int32_t* bad; int K, C;
+};
+__global__ void __launch_bounds__(256) nq_fit_pack_k(PackArgs a)
+{
+    __shared__ uint16_t st[8][256];
+    __shared__ float tile[16][129];
+    const int u = blockIdx.x, t = threadIdx.x, K = a.K;
+    const size_t u0 = (size_t)u * UNIT;
+    int whole = 1;
+#pragma unroll
+    for (int g = 0; g < 8; ++g)
+    {
+        const int64_t s = a.st[u0 + g * 256 + t];
+        whole &= s >= 0 && s < 65536;
+        st[g][t] = (uint16_t)s;
+    }
+    __syncthreads();
+    for (int g = 0; g < 8; ++g)
+    {
+        const uint32_t s = st[g][t];
+        whole &= (s >> K) == (st[g][(t + 1) & 255] & (0xFFFFu >> K));
+        if (!a.Q) continue;
+        int row, col;
+        ring_to_unit(g * 256 + t, row, col);
+        tile[row][col] = a.values ? a.values[u0 + g * 256 + t] : a.lut[s] * sign_of(a.sign, u, g * 256);
+    }
+    if (!whole) *a.bad = 1;
+    const int per = 32 / K, ring_words = 8 * K;                  // steps of a word, words of a ring (four records of 2 K)
+    for (int w = t; w < 8 * ring_words; w += 256)
+    {
+        const int g = w / ring_words, p0 = (w - g * ring_words) * per;
+        uint32_t v = 0;
+        for (int j = 0; j < per; ++j) v |= (st[g][p0 + j] & ((1u << K) - 1u)) << (K * j);
+        a.words[(size_t)u * 8 * ring_words + w] = (int32_t)v;
+    }
+    if (t == 0 && a.dw) a.dw[u] = (int32_t)(uint32_t)(a.Mb[u] | a.N[u] << 8);
+    if (t == 0 && a.var)
+    {
+        uint32_t m = 0;
+        for (int g = 0; g < 8; ++g) m |= (a.sign[u * 8 + g] < 0.f ? 1u : 0u) << g;
+        a.var[u] = (uint8_t)m;
+    }
+    if (!a.Q) return;
+    __syncthreads();
+    const size_t cols = (size_t)a.C * 128, at = (size_t)(u / a.C) * 16 * cols + (size_t)(u % a.C) * 128;
+    for (int i = t; i < UNIT; i += 256) a.Q[at + (i >> 7) * cols + (i & 127)] = tile[i >> 7][i & 127];
+}
+int launch_fit_pack(const int64_t* st, int K, const float* values, const float* sign, const float* lut, const int64_t* Mb, const int64_t* N, int U, int C,
+                    int32_t* words, int32_t* dw, uint8_t* var, float* Q, int32_t* bad, hipStream_t s)
+{
+    nq_fit_pack_k<<<U, 256, 0, s>>>(PackArgs{st, values, sign, lut, Mb, N, words, dw, var, Q, bad, K, C});
+    NQ_LAUNCH_CHECK("nq_fit_pack");
+    return 0;
 }
 
 int launch_fit_residual(const float* target, const float* sign, const int64_t* st_base, const float* lut, double scale, int U, float* out, hipStream_t st)

@@ -75,6 +75,8 @@ int64_t pf_meta_bytes(int P, int R, int E);
 int launch_fit_residual(const float* target, const float* sign, const int64_t* st_base, const float* lut, double scale, int U, float* out, hipStream_t st);
 int launch_fit_words(const float* target, const float* sign, const int64_t* st_base, const int64_t* st_res, const float* lut, int U, const double* Da, int64_t da_step,
                      const double* Do, int64_t do_step, void* ws, float* Q, int64_t* Mb, int64_t* N, double* delta, hipStream_t st);
+int launch_fit_pack(const int64_t* st, int K, const float* values, const float* sign, const float* lut, const int64_t* Mb, const int64_t* N, int U, int C,
+                    int32_t* words, int32_t* dw, uint8_t* var, float* Q, int32_t* bad, hipStream_t s);
 int launch_viterbi_p4(const float* w, const int64_t* a, int T, int L, const float* lut, int64_t* b, int rev, hipStream_t s);
 int launch_viterbi(const float* w, int T, int L, int K, const float* lut, int64_t* st, uint32_t* back, int slots, int rev, hipStream_t s);
 

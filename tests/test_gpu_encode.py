@@ -183,3 +183,40 @@ def test_searches_at_the_ends_of_the_range_of_costs(K, scale):
     for L in (17, 40):
         w = torch.randint(-6, 7, (3, L), generator=g).float() * scale
         assert torch.equal(EN.viterbi_ring(w.cuda(), lut.cuda(), K).cpu(), EN.viterbi_ring(w, lut, K))
+
+
+@pytest.mark.parametrize("N,K,signed,nested", [(16, 128, False, False), (48, 384, True, True), (128, 256, True, False), (32, 128, False, True)])
+def test_planes_are_packed_as_in_torch(N, K, signed, nested):
+    """records, block words, sign bytes and matrices of a fit, from whole rings of random bits, at one unit and at several strips and chunks;
+    a ring that does not close, in any plane, raises as it does in torch"""
+    g = torch.Generator().manual_seed(N + K)
+    U = (N // 16) * (K // 128)
+
+    def states(k):
+        sym = torch.randint(0, 1 << k, (U * 8, 256), generator=g)
+        return sum(sym[:, (torch.arange(256) + i) % 256] << (k * i) for i in range(16 // k)).reshape(U, 8, 256)
+    word = lambda n: torch.randint(0, n, (U,), generator=g)
+    e = lambda k: dict(states=states(k), Q=torch.randn(U, 8, 256, generator=g), Mb=word(256), N=word(256))
+    fits = {3: e(1), 4: e(2)}
+    if nested:
+        fits["4n"] = dict(e(2), p4_bits=torch.randint(0, 2, (U, 8, 256), generator=g))
+    sign = (torch.randint(0, 2, (U, 8, 1), generator=g) * 2 - 1).float() if signed else None
+    st2 = states(2)
+    dev = lambda f: {k: {n: t.cuda() for n, t in v.items()} for k, v in f.items()}
+    put = lambda t: None if t is None else t.cuda()
+    want, got = EN.pack_planes({}, N, K, st2, fits, sign), EN.pack_planes({}, N, K, st2.cuda(), dev(fits), put(sign))
+    assert want.keys() == got.keys()
+    for k in want:
+        assert (want[k] is None and got[k] is None) or (want[k].dtype == got[k].dtype and torch.equal(want[k], got[k].cpu())), k
+    if signed:                                                   # a type that the kernel does not read
+        got = EN.pack_planes({}, N, K, st2.cuda(), dev(fits), sign.cuda().double())
+        assert torch.equal(got["Q"].cpu(), want["Q"].double()) and torch.equal(got["base"].cpu(), want["base"])
+    for lvl in (2, 3, 4):
+        f, s = {k: dict(v) for k, v in fits.items()}, st2.clone()
+        broken = s if lvl == 2 else f[lvl]["states"].clone()
+        broken[U - 1, 7, 255] ^= 1 << 15                          # the last state's first bit, whose ring it closes
+        if lvl != 2:
+            f[lvl]["states"] = broken
+        for args in ((s, f, sign), (s.cuda(), dev(f), put(sign))):
+            with pytest.raises(AssertionError, match="tail-biting"):
+                EN.pack_planes({}, N, K, *args)
