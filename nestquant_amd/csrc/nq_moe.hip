@@ -55,6 +55,9 @@ __device__ __forceinline__ void ld_wait(float2& a, float2& b, float2& c, float2&
 {
     asm volatile("s_waitcnt vmcnt(0)" : "+v"(a), "+v"(b), "+v"(c), "+v"(d) :: "memory");
 }
+// A launch's last workgroups run the tail's code cold: straight on, 2 KB of it cost 2300 clk instead of 1030, and each jump over code that
+// is not wanted waits for a line from the L2. What few calls need stands out of line.
+__device__ __forceinline__ bool rare(bool c) { return __builtin_expect(c, 0); }
 // sums over k-slices y of the two floats at p[q] + y * stride, for NR rows q at once: the reads of all rows are in flight
 // together, four slices per row at a time (device-coherent reads)
 template <int NR>
@@ -463,86 +466,143 @@ __device__ __forceinline__ PickLanes pick_lanes(const PickInfo& R, int lane)
     P.w = R.w[lane]; P.signs = (unsigned long long)R.signs[lane]; P.rd = R.lr[lane] ? R.rd[lane] : 0;
     return P;
 }
-// the output scales of picks k and k + SB of token b for this lane's two columns (nothing for picks that do not contribute)
-__device__ __forceinline__ void pick_scales(const MoeArgs& a, const PickLanes& P, int b, int k, int SB, int col, half2_t* sv)
+// the output scales of picks k and k + SB of the first token for this lane's two columns (nothing for picks that do not contribute)
+__device__ __forceinline__ void pick_scales(const MoeArgs& a, const PickLanes& P, int k, int SB, int col, half2_t* sv)
 {
 #pragma unroll
     for (int q = 0; q < 2; ++q)
     {
-        const int kq = k + q * SB, s = (b * a.topk + kq) & 63;
+        const int kq = k + q * SB;
         sv[q] = half2_t{};
-        if (b < a.B && kq < a.topk && P.weight(s) != 0.f) sv[q] = *(const half2_t*)(P.sign_row(s) + a.H + 3 * a.I + col);
+        if (kq < a.topk && P.weight(kq & 63) != 0.f) sv[q] = *(const half2_t*)(P.sign_row(kq & 63) + a.H + 3 * a.I + col);
     }
+}
+// o += weight of pick s * (its output scales (.) WHT(its partial sums pv) + its low-rank term), for this lane's two columns
+__device__ __forceinline__ void add_pick(const MoeArgs& a, const PickInfo& R, const PickLanes& P, int s, float w, float2 pv, half2_t sv, int col, int lane, float& o0, float& o1)
+{
+    float v0 = pv.x, v1 = pv.y;
+    wht128(v0, v1, lane);
+    if (w == 0.f) return;
+    v0 *= (float)sv.x; v1 *= (float)sv.y;
+    const int prd = P.rank(s);
+    if (rare(prd))
+    {   // y += (sw V_dn^T) (U2_d [+ U4_d]): z_d summed over the I / 128 groups written by the gate|up finishers
+        const int prg = R.rg[s];
+        const _Float16* U2d = R.lr[s] + (size_t)prg * (a.H + 2 * a.I) + (size_t)prd * a.I;
+        const _Float16* U4d = R.lr4[s] + (size_t)prg * 2 * a.I;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (r < prd)
+            {
+                float zr = 0.f;
+                for (int gq = 0; gq < a.I / 128; ++gq) zr += a.zd[((size_t)s * (a.I / 128) + gq) * 4 + r];
+                half2_t ud = *(const half2_t*)(U2d + (size_t)r * a.H + col);
+                v0 += zr * (float)ud.x; v1 += zr * (float)ud.y;
+                if (R.lv[s] == 4) { ud = *(const half2_t*)(U4d + (size_t)r * a.H + col); v0 += zr * (float)ud.x; v1 += zr * (float)ud.y; }
+            }
+    }
+    o0 += w * v0; o1 += w * v1;
+}
+// out[o], out[o + 1] = the sums of a token's n <= 4 wavefronts (those beyond n are not written: their reads are turned to the last)
+__device__ __forceinline__ void sum_waves(const MoeArgs& a, size_t o, const float* red, int n)
+{
+    float2 v[4];
+#pragma unroll
+    for (int w = 0; w < 4; ++w) v[w] = *(const float2*)(red + min(w, n - 1) * 128);
+    float r0 = 0.f, r1 = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+        if (w < n) { r0 += v[w].x; r1 += v[w].y; }
+    out2_store(a, o, r0, r1);
 }
 
 // combine of the down projection for output rows [grp * 128, +128): out[b] = sum_k rw[b,k] * sv_o[e] (.) WHT(sum_y part_d[slot])
-// picks of a token are spread over the block's wavefronts and reduced through LDS (red: SB * 128 floats). `next`: the scales of the
-// wavefront's first two picks, requested before the arrival counter; those of every later step are requested one step ahead.
+// picks of a token are spread over the block's wavefronts and reduced through LDS. One token: two picks of a wavefront in flight
+// (red: SB * 128 floats); `next`: the scales of the first two, requested before the arrival counter.
 __device__ __forceinline__ void finish_dn(const MoeArgs& a, const PickInfo& R, const PickLanes& P, half2_t* next, int grp, int NY, int warp, int SB, int lane, float* red)
 {
-    const int S = a.B * a.topk, col = grp * 128 + 2 * lane;
-    for (int b = 0; b < a.B; ++b)
+    const int col = grp * 128 + 2 * lane;
+    float o0 = 0.f, o1 = 0.f;
+    for (int k = warp; k < a.topk; k += 2 * SB)
     {
-        float o0 = 0.f, o1 = 0.f;
-        for (int k = warp; k < a.topk; k += 2 * SB)              // two picks of this wavefront at a time, their reads in flight together
+        float2 pv[2] = {make_float2(0.f, 0.f), make_float2(0.f, 0.f)};
+        float w[2] = {0.f, 0.f};
+        half2_t sv[2] = {next[0], next[1]};
+        const float* rows2[2] = {a.part_d, a.part_d};
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
         {
-            float2 pv[2] = {make_float2(0.f, 0.f), make_float2(0.f, 0.f)};
-            float w[2] = {0.f, 0.f};
-            half2_t sv[2] = {next[0], next[1]};
-            const float* rows2[2] = {a.part_d, a.part_d};
-#pragma unroll
-            for (int q = 0; q < 2; ++q)
-            {
-                const int kq = k + q * SB, s = (b * a.topk + kq) & 63;
-                if (kq >= a.topk || P.weight(s) == 0.f) continue;    // what route() saw: no second look at the table
-                w[q] = P.weight(s); rows2[q] = a.part_d + (size_t)s * a.H + col;
-            }
-            const bool more = k + 2 * SB < a.topk;
-            pick_scales(a, P, more ? b : b + 1, more ? k + 2 * SB : warp, SB, col, next);
-            if (w[0] == 0.f && w[1] == 0.f) continue;
-            sum_partials<2>(rows2, (size_t)S * a.H, NY, pv);
-#pragma unroll
-            for (int q = 0; q < 2; ++q)
-            {
-                float v0 = pv[q].x, v1 = pv[q].y;
-                wht128(v0, v1, lane);
-                if (w[q] == 0.f) continue;
-                v0 *= (float)sv[q].x; v1 *= (float)sv[q].y;
-                const int s = b * a.topk + k + q * SB, prd = P.rank(s);
-                if (prd)
-                {   // y += (sw V_dn^T) (U2_d [+ U4_d]): z_d summed over the I / 128 groups written by the gate|up finishers
-                    const int prg = R.rg[s];
-                    const _Float16* U2d = R.lr[s] + (size_t)prg * (a.H + 2 * a.I) + (size_t)prd * a.I;
-                    const _Float16* U4d = R.lr4[s] + (size_t)prg * 2 * a.I;
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        if (r < prd)
-                        {
-                            float zr = 0.f;
-                            for (int gq = 0; gq < a.I / 128; ++gq) zr += a.zd[((size_t)s * (a.I / 128) + gq) * 4 + r];
-                            half2_t ud = *(const half2_t*)(U2d + (size_t)r * a.H + col);
-                            v0 += zr * (float)ud.x; v1 += zr * (float)ud.y;
-                            if (R.lv[s] == 4) { ud = *(const half2_t*)(U4d + (size_t)r * a.H + col); v0 += zr * (float)ud.x; v1 += zr * (float)ud.y; }
-                        }
-                }
-                o0 += w[q] * v0; o1 += w[q] * v1;
-            }
+            const int s = k + q * SB;
+            if (s >= a.topk || P.weight(s & 63) == 0.f) continue;    // what route() saw: no second look at the table
+            w[q] = P.weight(s & 63); rows2[q] = a.part_d + (size_t)s * a.H + col;
         }
-        red[warp * 128 + 2 * lane] = o0; red[warp * 128 + 2 * lane + 1] = o1;
-        __syncthreads();
-        if (warp == 0)
-        {
-            float r0 = 0.f, r1 = 0.f;
-            for (int w2 = 0; w2 < SB; ++w2) { r0 += red[w2 * 128 + 2 * lane]; r1 += red[w2 * 128 + 2 * lane + 1]; }
-            out2_store(a, (size_t)b * a.H + col, r0, r1);
-        }
-        __syncthreads();
+        if (k + 2 * SB < a.topk) pick_scales(a, P, k + 2 * SB, SB, col, next);
+        if (w[0] == 0.f && w[1] == 0.f) continue;
+        sum_partials<2>(rows2, (size_t)a.topk * a.H, NY, pv);
+#pragma unroll
+        for (int q = 0; q < 2; ++q) add_pick(a, R, P, (k + q * SB) & 63, w[q], pv[q], sv[q], col, lane, o0, o1);
     }
+    *(float2*)(red + warp * 128 + 2 * lane) = make_float2(o0, o1);
+    __syncthreads();
+    if (warp == 0) sum_waves(a, col, red + 2 * lane, SB);
+}
+
+// Several tokens: all at once (red: B * SB * 128 floats), N picks of a wavefront in flight with their scales, one barrier. Token by token as
+// above, with two barriers each, the last workgroup's tail grew with the tokens: us a call, before and now: 512 x 256, 2 tokens 16.9 -> 15.6;
+// 1024 x 384, 4 tokens 29.8 -> 28.3; 4736 x 1152, 3 tokens 72.9 -> 70.9; 2048 x 1024, 4 tokens 52.8 -> 51.8, 8 tokens 83.2 -> 80.0; 6144 x 2048, 4
+// tokens 204.0 -> 202.4. For one token the walk over tokens costs more than it gives (30.7 against 30.5 at 2048 x 1024); N = 2 where
+// that is all a wavefront has (four reads' worth of dummies cost 1 us at 512 x 256), else 4.
+template <int N>
+__device__ __forceinline__ void finish_dn_all(const MoeArgs& a, const PickInfo& R, const PickLanes& P, int grp, int NY, int warp, int SB, int lane, float* red)
+{
+    const int col = grp * 128 + 2 * lane;
+    float o0 = 0.f, o1 = 0.f;
+    int b = warp < a.topk ? 0 : a.B, k = warp;                   // the wavefront's next pick: of every token the picks warp, warp + SB, ...
+    while (b < a.B)
+    {
+        int tb[N], ts[N];                                        // token (-1: nothing), pick; the sign of ts: the token's last of this wavefront
+        bool end[N];
+        float w[N];
+        half2_t sv[N];
+        float2 pv[N];
+        const float* rows[N];
+        bool any = false;
+#pragma unroll
+        for (int q = 0; q < N; ++q)
+        {
+            tb[q] = b; ts[q] = (b * a.topk + k) & 63; end[q] = k + SB >= a.topk;
+            w[q] = b < a.B ? P.weight(ts[q]) : 0.f;              // what route() saw: no second look at the table
+            sv[q] = half2_t{};
+            rows[q] = a.part_d; pv[q] = make_float2(0.f, 0.f);
+            if (w[q] != 0.f)
+            {
+                sv[q] = *(const half2_t*)(P.sign_row(ts[q]) + a.H + 3 * a.I + col);
+                rows[q] = a.part_d + (size_t)ts[q] * a.H + col;
+                any = true;
+            }
+            k += SB;
+            if (k >= a.topk) { k = warp; ++b; }
+        }
+        if (any) sum_partials<N>(rows, (size_t)a.B * a.topk * a.H, NY, pv);
+#pragma unroll
+        for (int q = 0; q < N; ++q)
+        {
+            if (tb[q] >= a.B) break;
+            add_pick(a, R, P, ts[q], w[q], pv[q], sv[q], col, lane, o0, o1);
+            if (end[q])
+            {
+                *(float2*)(red + (tb[q] * SB + warp) * 128 + 2 * lane) = make_float2(o0, o1);
+                o0 = o1 = 0.f;
+            }
+        }
+    }
+    __syncthreads();
+    for (int t = warp; t < a.B; t += SB) sum_waves(a, (size_t)t * a.H + col, red + t * SB * 128 + 2 * lane, min(SB, a.topk));
 }
 
 // MODE 0: gate|up (N = 2I, K = H, input x rotated here). MODE 1: down (N = H, K = I, input h).
 // grid (N / 32 / SB, C / NC, S); block 64 * SB threads (SB = 1, 2 or 4: a block covers at most one 128-row group);
-// dynamic LDS = rows * (NC * 256 + 16) + 256 bytes (>= SB * 512 for the combine), one row per token of the call
+// dynamic LDS = rows * (NC * 256 + 16) + 256 bytes (>= rows * SB * 512 for the combine), one row per token of the call
 // ANYROW = false: the kernel of a layer whose rows are all of the common kind, base window code 0 and no mask-mode flags (the
 // host says so, MoeArgs::common_rows). A run whose row is nevertheless of another kind is not decoded as if it were common:
 // its plane is not read and its partial sums are NaN, so every token that picked it comes out NaN. ANYROW = true also
@@ -711,16 +771,18 @@ nq_gemv_k(MoeArgs a, int NC)
     int* cnt = MODE == 0 ? a.cnt_gu + blockIdx.z * (a.I / 128) + grp : a.cnt_d + grp;
     const int expect = (MODE == 0 ? 2 : nruns) * NY * (128 / (SB * 32));
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");             // this wavefront's partial sums are acknowledged
-    half2_t scales[2] = {};
     const int wv = __builtin_amdgcn_readfirstlane(warp);
-    if constexpr (MODE == 1) pick_scales(a, picks, 0, wv, SB, grp * 128 + 2 * lane, scales);
+    half2_t scales[2] = {};
+    if constexpr (MODE == 1) if (a.B == 1) pick_scales(a, picks, wv, SB, grp * 128 + 2 * lane, scales);
     __syncthreads();
     if (threadIdx.x == 0)
         last = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == expect - 1;
     __syncthreads();
     if (!last) return;                                           // block-uniform
     if constexpr (MODE == 0) finish_gu(a, R, zl, blockIdx.z, grp, NY, warp, SB, lane, last);
-    else finish_dn(a, a.route->picks, picks, scales, grp, NY, wv, SB, lane, (float*)smem);
+    else if (!rare(a.B != 1)) finish_dn(a, a.route->picks, picks, scales, grp, NY, wv, SB, lane, (float*)smem);
+    else if (a.B * a.topk <= 2 * SB) finish_dn_all<2>(a, a.route->picks, picks, grp, NY, wv, SB, lane, (float*)smem);
+    else finish_dn_all<4>(a, a.route->picks, picks, grp, NY, wv, SB, lane, (float*)smem);
     if (threadIdx.x == 0) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
@@ -767,7 +829,7 @@ int launch_moe(const MoeArgs& a, const int* cfg_gu, const int* cfg_dn, int which
         const int NC = cf[0] * cf[2], SB = cf[1];
         const int N = mode == 0 ? 2 * a.I : a.H, K = mode == 0 ? a.H : a.I, C = K / 128;
         const int NX = N / 32 / SB, NY = C / NC;
-        const int shm = std::max(a.B * (NC * 256 + 16) + 256, SB * 512);
+        const int shm = std::max(a.B * (NC * 256 + 16) + 256, (mode == 1 ? a.B : 1) * SB * 512);
         const bool any = a.common_rows != 1;
         MoeArgs b = a;
         b.fuse = which == 3 || defer;                             // both launches belong to this call (or the caller says the other one follows)

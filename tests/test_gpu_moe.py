@@ -633,3 +633,32 @@ def test_finisher_in_the_down_launch_gives_the_same_bits(golden_dir):
         torch.cuda.synchronize()
         assert torch.isfinite(y3).all() and y3.abs().max() > 0 and torch.equal(y3, y12) and torch.equal(y3, y18), B
         assert not L.cnt_gu.any() and not L.cnt_d.any() and not L.cnt_h.any()
+
+
+@pytest.mark.parametrize("B,topk,SB,low_rank", [(2, 1, 4, False), (2, 3, 2, False), (3, 2, 4, False), (2, 4, 4, False), (3, 5, 4, True), (8, 8, 4, False), (8, 8, 1, False), (5, 6, 2, True)])
+def test_tokens_of_one_call_are_combined_as_alone(B, topk, SB, low_rank):
+    """The down launch combines one token in one way and several in another (two or four picks of a wavefront in flight, one
+    barrier), with the same sums in the same order: bitwise the single calls, with fewer picks than wavefronts, with a remainder,
+    with weights of zero, ids that name no expert, a token with no pick at all, and low-rank rows."""
+    H, I, E = 384, 256, 8
+    ex = to_dev(experts_on_gpu(H, I, E, 70, nested_ids=(1, 4)))
+    gen = torch.Generator().manual_seed(7)
+    for e in range(1, E if low_rank else 0, 2):
+        ex[e].set_lr(*[torch.randn(s, generator=gen).half() * 0.1 for s in ((2, H), (2, I), (2, I), (2, I), (2, I), (3, I), (3, H), (3, H))])
+    L = M.MoELayer(E, H, I, Bmax=8, topk=topk)
+    for e in range(E):
+        L.set(e, ex[e], 4 if e in (1, 4) else 2)
+    rng = np.random.default_rng(100 * B + topk)
+    x = torch.from_numpy((rng.standard_normal((B, H)) * 0.5).astype(np.float16)).to(DEV)
+    sel = np.stack([rng.permutation(E)[:topk] for _ in range(B)]).astype(np.int32)
+    rw = rng.uniform(0.1, 1.0, (B, topk)).astype(np.float32)
+    rw[0, topk // 2] = 0.0
+    sel[B - 1, 0] = E + 3
+    rw[B // 2] = 0.0
+    sel, rw = torch.from_numpy(sel).to(DEV), torch.from_numpy(rw).to(DEV)
+    cg, cd = [1, 4, 1], [1, SB, 1]
+    for _ in range(2):
+        y = L(x, sel, rw, cfg_gu=cg, cfg_dn=cd).clone()
+        for b in range(B):
+            assert torch.equal(y[b:b + 1], L(x[b:b + 1], sel[b:b + 1], rw[b:b + 1], cfg_gu=cg, cfg_dn=cd)), b
+    assert not y[B // 2].any() and not L.cnt_d.any()
