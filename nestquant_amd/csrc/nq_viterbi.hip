@@ -5,7 +5,7 @@
 // bit for bit: every candidate is (value - target)^2 + cost in fp32 with the torch code's roundings (no contraction), and ties go
 // to the smallest predecessor.
 //
-// One workgroup of 1024 threads per ring. "Edge" = the low 16 - K bits of a state (E of them); the
+// One workgroup of 1024 threads per ring, or per pass over it (launch_viterbi). "Edge" = the low 16 - K bits of a state (E of them); the
 // candidates of edge e are its 2^K states, each with predecessor edge (q << (16 - 2 K)) | (e >> K), so 2^K neighbouring edges (a
 // group) share their predecessors: thread t owns the groups t + 1024 r, keeps the 64 codebook values of their states in registers through
 // a pass, reads 2^K costs per group from LDS and writes 2^K. Both directions of that traffic are free of bank conflicts.
@@ -28,7 +28,7 @@ namespace nq {
 
 constexpr int VT = 1024, VIT_LMAX = 1024;
 
-struct VitArgs { const float* w; const float* lut; int64_t* st; uint32_t* back; int T, L, rev; };
+struct VitArgs { const float* w; const float* lut; int64_t* st; uint32_t* back; int T, L, rev; int from, to; };
 
 // all wavefronts' LDS accesses so far are done; stores to global memory stay in flight (a __syncthreads would wait for them)
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
@@ -153,7 +153,7 @@ __device__ __forceinline__ int vit_trace(const uint32_t* back, int hi, int edge,
     return edge_sh;
 }
 
-template <int K>
+template <int K, bool HALVES>
 __global__ void __launch_bounds__(VT) nq_viterbi_k(VitArgs a)
 {
     constexpr int Q = 1 << K, KR = 16 - K, E = 1 << KR, R = VIT_R<K>;
@@ -164,13 +164,15 @@ __global__ void __launch_bounds__(VT) nq_viterbi_k(VitArgs a)
     __shared__ int edge_sh;
     const int t = threadIdx.x, L = a.L;
     uint32_t* back = a.back + (size_t)blockIdx.x * L * VT;
-    for (int ring = blockIdx.x; ring < a.T; ring += gridDim.x)
-    {
+    for (int u = (HALVES ? a.from : 0) + blockIdx.x; u < (HALVES ? a.to : a.T); u += gridDim.x)
+    {   // a whole ring, or one pass over it: pass 1 of ring u, pass 2 of ring u - T, whose first state pass 1 has left in st
+        const int first = HALVES && u >= a.T ? 1 : 0, last = HALVES ? first + 1 : 2, ring = HALVES && first ? u - a.T : u;
         for (int i = t; i < L; i += VT) wl[i] = vit_target(a.w[(size_t)ring * L + (a.rev ? (L - i) % L : i)]);
-        int start = -1;
+        int start = HALVES && first ? (int)a.st[(size_t)ring * L] : -1;
 #pragma clang loop unroll(disable)
-        for (int pass = 0; pass < 2; ++pass)
+        for (int pass = first; pass < last; ++pass)
         {
+            if (HALVES) pass = __builtin_amdgcn_readfirstlane(pass);
             asm volatile("" : "+s"(pass));                       // one copy of the loops below
             const int roll = pass == 0 ? L / 2 : 0, keep = pass == 0 && L > 1 ? L - roll : 0;     // nobody walks back over the steps before `keep`
             for (int e = t; e < E; e += VT) cost[e] = pass == 0 || e == start ? 0.f : __builtin_inff();
@@ -226,20 +228,29 @@ __global__ void __launch_bounds__(VT) nq_viterbi_k(VitArgs a)
             __syncthreads();                                     // the decisions of all wavefronts are in memory
             start = vit_trace<K>(back, pass == 0 && L > 1 ? roll - 1 : L - 1, edge, (uint32_t*)cost, sl, edge_sh, t);
         }
-        for (int i = t; i < L; i += VT) a.st[(size_t)ring * L + (a.rev ? (L - i) % L : i)] = sl[i];
+        if (HALVES && last == 1) { if (t == 0) a.st[(size_t)ring * L] = start; }
+        else for (int i = t; i < L; i += VT) a.st[(size_t)ring * L + (a.rev ? (L - i) % L : i)] = sl[i];
         lds_barrier();                                           // sl and wl are free again
     }
 }
 
 int launch_viterbi(const float* w, int T, int L, int K, const float* lut, int64_t* st, uint32_t* back, int slots, int rev, hipStream_t s)
 {
-    const VitArgs a{w, lut, st, back, T, L, rev};
     const int shm = 2 * 16384 * 4;
-    auto kern = K == 2 ? nq_viterbi_k<2> : nq_viterbi_k<1>;
+    // Rings that leave more than half of the last round's workgroups idle are searched pass by pass, in launches of `slots` passes (all first ones,
+    // then all second ones: T > slots, so the two of a ring are in different launches): halves of a round are then filled. us for 320 / 384 rings
+    // of 256 steps on 256 CUs: K = 2 1480 / 1560 -> 1265 / 1380, K = 1 1874 / 1872 -> 1523 / 1590. Elsewhere both take as many rounds.
+    const bool halves = T > slots && (2 * (int64_t)T + slots - 1) / slots < 2 * (((int64_t)T + slots - 1) / slots);
+    auto kern = halves ? (K == 2 ? nq_viterbi_k<2, true> : nq_viterbi_k<1, true>) : (K == 2 ? nq_viterbi_k<2, false> : nq_viterbi_k<1, false>);
     const hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
     if (e != hipSuccess) return set_error("nq_viterbi: LDS %d bytes: %s", shm, hipGetErrorString(e));
-    kern<<<T < slots ? T : slots, VT, shm, s>>>(a);
-    NQ_LAUNCH_CHECK("nq_viterbi");
+    const int64_t units = halves ? 2 * (int64_t)T : T;
+    for (int64_t from = 0; from < units; from += halves ? slots : units)
+    {
+        const int64_t to = halves && from + slots < units ? from + slots : units;
+        kern<<<(int)(to - from < slots ? to - from : slots), VT, shm, s>>>(VitArgs{w, lut, st, back, T, L, rev, (int)from, (int)to});
+        NQ_LAUNCH_CHECK("nq_viterbi");
+    }
     return 0;
 }
 

@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-from nestquant_amd import encode as EN
+from nestquant_amd import _lib, encode as EN
 
 pytestmark = pytest.mark.gpu
 
@@ -21,6 +21,20 @@ def test_viterbi_search_equals_the_torch_form(T, L, K):
     assert torch.equal(EN.viterbi_ring(w.cuda(), lut.cuda(), K).cpu(), want)
     if L == 256:
         assert torch.equal(EN.viterbi_rings(w.cuda(), K).cpu(), EN.viterbi_rings(w, K))
+
+
+@pytest.mark.parametrize("K", [1, 2])
+@pytest.mark.parametrize("T,slots,L,position", [(3, 2, 40, False), (4, 3, 9, True), (5, 2, 1, False), (6, 5, 2, True), (7, 3, 33, True), (9, 4, 17, False)])
+def test_viterbi_search_pass_by_pass(T, slots, L, position, K):
+    """more rings than the scratch holds at a time, with a last round that is at most half full: passes instead of rings, the same
+    states as with a scratch for all of them (whole rings)"""
+    g = torch.Generator().manual_seed(T + L)
+    w, lut = (torch.randn(T, L, generator=g) * 1.3).cuda(), EN.codebook().cuda()
+    def run(n):
+        st, scratch = torch.full((T, L), -1, dtype=torch.int64, device="cuda"), torch.empty(n * L * 1024, dtype=torch.int32, device="cuda")
+        _lib.check(_lib.lib().nq_viterbi(w.data_ptr(), T, L, K, lut.data_ptr(), st.data_ptr(), scratch.data_ptr(), scratch.numel() * 4, int(position), _lib.stream_ptr()))
+        return st.cpu()
+    assert torch.equal(run(slots), run(T))
 
 
 def test_viterbi_ties_on_a_coarse_codebook():
