@@ -330,20 +330,22 @@ __global__ void nq_pf_hits_k(const int32_t* counts, int32_t* hits, int E)
 // it, at index e of list k; the full tiles follow at indices E.. of list 4. tiles: int32 [5][cap][4] = (expert, first row in
 // the chunk, rows, 0); entries without a tile get expert -1, which the GEMM skips. Replaces the host loop over the expert
 // counts and with it the call's one host synchronisation.
-__device__ __forceinline__ void block_scan(int* a, int* b, int E)
-{   // inclusive prefix sum of a[0..E) in place (b: scratch of the same size); all threads of the block call it
-    int *src = a, *dst = b;
-    for (int off = 1; off < E; off <<= 1)
-    {
-        for (int e = threadIdx.x; e < E; e += blockDim.x) dst[e] = src[e] + (e >= off ? src[e - off] : 0);
-        __syncthreads();
-        int* t = src; src = dst; dst = t;
-    }
-    if (src != a)
-    {
-        for (int e = threadIdx.x; e < E; e += blockDim.x) a[e] = src[e];
-        __syncthreads();
-    }
+__device__ __forceinline__ void block_scan(int* a, int n)
+{   // inclusive prefix sum of a[0..n) in LDS, in place; all threads of the block call it (at most 16 wavefronts), a[] written before a barrier
+    __shared__ int part[16];
+    const int lane = threadIdx.x & 63, warp = threadIdx.x >> 6, per = (n + (int)blockDim.x - 1) / (int)blockDim.x;
+    const int lo = min(n, (int)threadIdx.x * per), hi = min(n, lo + per);
+    int s = 0;
+    for (int i = lo; i < hi; ++i) s += a[i];
+    int v = s;                                                   // sum of this and the wavefront's earlier threads
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) { const int o = __shfl_up(v, m); if (lane >= m) v += o; }
+    if (lane == 63) part[warp] = v;
+    __syncthreads();
+    v -= s;
+    for (int w = 0; w < warp; ++w) v += part[w];
+    for (int i = lo; i < hi; ++i) a[i] = v += a[i];
+    __syncthreads();
 }
 
 // hot (may be null): experts with at least hot_min rows in the chunk get a slot 0 .. hot_cap - 1 of the decoded-weight scratch (in
@@ -355,7 +357,7 @@ __global__ void __launch_bounds__(256) nq_pf_plan_k(const int32_t* __restrict__ 
     int *incl = plan_sh, *tmp = plan_sh + E, *full = plan_sh + 2 * E, *hrank = plan_sh + 3 * E;
     for (int e = threadIdx.x; e < E; e += blockDim.x) incl[e] = counts[e] > 0 ? counts[e] : 0;
     __syncthreads();
-    block_scan(incl, tmp, E);
+    block_scan(incl, E);
     const int row_hi = row_lo + nrows;
     for (int e = threadIdx.x; e < E; e += blockDim.x)
     {
@@ -366,11 +368,11 @@ __global__ void __launch_bounds__(256) nq_pf_plan_k(const int32_t* __restrict__ 
         hrank[e] = hot != nullptr && n >= hot_min ? 1 : 0;
     }
     __syncthreads();
-    block_scan(hrank, tmp, E);                                   // inclusive: hot experts up to and including e
+    block_scan(hrank, E);                                   // inclusive: hot experts up to and including e
     int* fincl = tmp;                                            // inclusive scan of the full-tile counts
     for (int e = threadIdx.x; e < E; e += blockDim.x) fincl[e] = full[e];
     __syncthreads();
-    block_scan(fincl, full, E);                                  // clobbers full[]: recomputed below
+    block_scan(fincl, E);
     int4* T4 = (int4*)tiles;
     for (int e = threadIdx.x; e < E; e += blockDim.x)
     {
@@ -771,105 +773,116 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MASKED
 }
 
 // ---- pairs sorted by expert ----------------------------------------------------------------------------------------------
-// One launch in place of a library sort, its gathers and the counting scatter (a dozen launches, 150 us of them at 32768 pairs):
-// 11 us at 384 pairs, 21 at 8024, 84 to 89 at 32768, where every workgroup reads and counts all picks.
-// Every workgroup counts all picks in LDS, so that it knows where each expert's rows start without waiting for another one; its
-// eight wavefronts then gather the pairs of one expert each, in pair order, from the picks kept in LDS as 16-bit ids. Picks outside
-// [0, E) form a last group of rows of no expert (pe = -1), which every later kernel passes over. Workgroup 0 also writes the
-// tile list of nq_pf_short_k: at most 64 rows per tile, experts above level 2 first (their tiles take twice as long, so they
-// start first), unused entries -1.
-constexpr int SORT_TILE = 16384, SHORT_ROWS = 64;
+// One launch in place of a library sort, its gathers and the counting scatter. Every workgroup counts all picks in LDS, those before its
+// own share of the pairs apart, so that it knows where its pairs of an expert begin without waiting for another workgroup; then it ranks its
+// pairs, 512 at a time, one per lane: within a wavefront by the ids' bits, between wavefronts by taking turns at the experts' cursors.
+// Rows of an expert are in pair order. Picks outside [0, E) form a last group of rows of no expert (pe = -1), which every later kernel
+// passes over. One workgroup more writes the counts, the hits and the tile list of nq_pf_short_k: at most 64 rows per tile, experts above
+// level 2 first (their tiles take twice as long, so they start first), unused entries -1.
+// Bound by the counting's LDS atomics beyond a few thousand pairs, by latency below. us at 384 / 1608 / 8024 / 32768 pairs of 256 experts: 7.7 / 8.3 / 10.2 / 20.2, where
+// eight experts a workgroup, each gathered by one wavefront that looked at every pair, took 10.7 / 11.9 / 21.1 / 89.7.
+constexpr int SORT_BLOCK = 512, SORT_WGS = 256, SHORT_ROWS = 64;
 struct PfSort
 {
     const void* sel; const void* rw; int sdt, wdt; int P, topk, E;
     const int64_t* table; int32_t* cnt; int32_t* pe; int32_t* pt; int32_t* pos; int* hits; int32_t* tiles; int cap;
+    int per;                                                     // blocks of SORT_BLOCK pairs per workgroup
 };
-__global__ void __launch_bounds__(512) nq_pf_sort_k(PfSort a)
+__global__ void __launch_bounds__(1024) nq_pf_sort_k(PfSort a)
 {
-    extern __shared__ __align__(16) uint16_t ids[];              // [SORT_TILE], then hist | start | tmp, E + 1 each
-    int* hist = (int*)(ids + SORT_TILE); int* incl = hist + a.E + 1; int* tmp = incl + a.E + 1;
-    const int tid = threadIdx.x, lane = tid & 63, E1 = a.E + 1;
-    const bool one = a.P <= SORT_TILE;
-    auto load = [&](int t0, bool count) {
-        for (int i0 = tid; i0 < SORT_TILE; i0 += 8 * 512)
-        {
-            if (one && i0 - tid >= a.P) break;
-            long long e[8];                                      // eight ids in flight before the first is counted
+    extern __shared__ int sort_sh[];
+    const int E1 = a.E + 1, tid = threadIdx.x, lane = tid & 63, warp = tid >> 6;
+    int *bef = sort_sh, *tot = bef + E1, *ext = tot + E1;       // pairs before this workgroup's, all pairs, scans
+    const bool list = blockIdx.x == gridDim.x - 1;               // block-uniform
+    const int begin = list ? a.P : min((int64_t)a.P, (int64_t)blockIdx.x * a.per * SORT_BLOCK), end = min((int64_t)a.P, (int64_t)begin + a.per * SORT_BLOCK);
+    auto id_of = [&](int i) { const long long e = id_at(a.sel, a.sdt, i); return e >= 0 && e < a.E ? (int)e : a.E; };
+    int id = tid < SORT_BLOCK && begin + tid < end ? id_of(begin + tid) : -1;        // requested before the counting
+    int lv[4] = {};                                              // levels of experts tid + 1024 k (E <= 4096)
+    if (list && a.tiles)
 #pragma unroll
-            for (int u = 0; u < 8; ++u) e[u] = t0 + i0 + 512 * u < a.P ? id_at(a.sel, a.sdt, t0 + i0 + 512 * u) : -2;
-#pragma unroll
-            for (int u = 0; u < 8; ++u)
-            {
-                const int i = i0 + 512 * u;
-                const bool in = t0 + i < a.P;
-                const int id = !in ? 0xFFFF : e[u] >= 0 && e[u] < a.E ? (int)e[u] : a.E;     // past the end: nobody's
-                if (count && in) atomicAdd(hist + id, 1);
-                ids[i] = (uint16_t)id;
-            }
-        }
-    };
-    for (int e = tid; e < E1; e += 512) hist[e] = 0;
+        for (int k = 0; k < 4; ++k)
+            if (tid + 1024 * k < a.E) lv[k] = (int)a.table[(size_t)(tid + 1024 * k) * TBL_W];
+    for (int e = tid; e < E1; e += 1024) { bef[e] = 0; tot[e] = 0; ext[e] = 0; }
     __syncthreads();
-    for (int t0 = 0; t0 < a.P; t0 += SORT_TILE) { if (t0) __syncthreads(); load(t0, true); }
-    __syncthreads();
-    for (int e = tid; e < E1; e += 512) incl[e] = hist[e];
-    __syncthreads();
-    block_scan(incl, tmp, E1);
-    const int e = blockIdx.x * 8 + (tid >> 6);
-    int row = e < E1 ? incl[e] - hist[e] : 0, nz = 0;            // next row of this wavefront's expert
-    const int mine = e < E1 ? e : -1;
-    if (mine >= 0 && mine < a.E && lane == 0) a.cnt[mine] = hist[mine];
-    for (int t0 = 0; t0 < a.P; t0 += SORT_TILE)
+    for (int64_t i0 = tid; i0 < a.P; i0 += 8 * 1024)
     {
-        if (!one) { __syncthreads(); load(t0, false); __syncthreads(); }
-        const int n = a.P - t0 < SORT_TILE ? a.P - t0 : SORT_TILE;
-        for (int i = 0; i < n; i += 512)
-        {
-            const uint4 v = *(const uint4*)(ids + i + 8 * lane);
-            const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+        int e[8]; bool hit[8];                                   // eight in flight before the first is counted
 #pragma unroll
-            for (int j = 0; j < 8; ++j)                          // rows of an expert: by blocks of 512 pairs, then by j, then by lane
-            {
-                const bool eq = (int)((w[j >> 1] >> (16 * (j & 1))) & 0xFFFFu) == mine;
-                const unsigned long long m = __ballot(eq);
-                if (!m) continue;
-                if (eq)
-                {
-                    const int pair = t0 + i + 8 * lane + j, r = row + __popcll(m & ((1ull << lane) - 1ull));
-                    a.pos[pair] = r; a.pt[r] = pair / a.topk; a.pe[r] = mine < a.E ? mine : -1;
-                }
-                if (a.hits) nz += __popcll(__ballot(eq && w_at(a.rw, a.wdt, t0 + i + 8 * lane + j) != 0.f));
-                row += __popcll(m);
-            }
+        for (int u = 0; u < 8; ++u)
+        {
+            const int64_t i = i0 + 1024 * u;
+            e[u] = i < a.P ? id_of((int)i) : -1;
+            hit[u] = list && a.hits && i < a.P && w_at(a.rw, a.wdt, i) != 0.f;
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+        {
+            if (e[u] >= 0) atomicAdd((i0 + 1024 * u < begin ? bef : tot) + e[u], 1);
+            if (hit[u]) atomicAdd(ext + e[u], 1);
         }
     }
-    if (a.hits && nz && mine >= 0 && mine < a.E && lane == 0) __hip_atomic_fetch_add(a.hits + mine, nz, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    if (blockIdx.x != 0 || !a.tiles) return;
     __syncthreads();
-    // start rows into incl, then per class (0: above level 2, 1: level 2) a scan of the tile counts
+    if (list && a.hits)
+        for (int e = tid; e < a.E; e += 1024)
+            if (ext[e]) __hip_atomic_fetch_add(a.hits + e, ext[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    for (int e = tid; e < E1; e += 1024) ext[e] = tot[e] += bef[e];
+    __syncthreads();
+    block_scan(ext, E1);
+    if (!list)
+    {
+        for (int e = tid; e < E1; e += 1024) bef[e] += ext[e] - tot[e];              // row of the expert's next pair here
+        const int bits = 32 - __builtin_clz(a.E);
+        for (int p0 = begin; p0 < end; p0 += SORT_BLOCK)
+        {
+            if (p0 > begin) id = tid < SORT_BLOCK && p0 + tid < end ? id_of(p0 + tid) : -1;
+            unsigned long long same = __ballot(id >= 0);         // the lanes with this lane's id
+            for (int b = 0; b < bits; ++b)
+            {
+                const unsigned long long m = __ballot((id >> b) & 1);
+                same &= ((id >> b) & 1) ? m : ~m;
+            }
+            const int before = __popcll(same & ((1ull << lane) - 1ull));
+            int row = 0;
+            for (int w = 0; w < SORT_BLOCK / 64; ++w)
+            {
+                __syncthreads();
+                if (w == warp && id >= 0 && before == 0) { row = bef[id]; bef[id] = row + __popcll(same); }
+            }
+            row = __shfl(row, id >= 0 ? __ffsll((long long)same) - 1 : lane) + before;
+            if (id >= 0)
+            {
+                const int pair = p0 + tid;
+                a.pos[pair] = row; a.pt[row] = pair / a.topk; a.pe[row] = id < a.E ? id : -1;
+            }
+        }
+        return;
+    }
+    for (int e = tid; e < a.E; e += 1024) a.cnt[e] = tot[e];
+    if (!a.tiles) return;
+    // per class (0: above level 2, 1: level 2) a scan of the tile counts
     int4* T4 = (int4*)a.tiles;
+    int* nt = bef;
     int base = 0;
-    for (int x = tid; x < a.E; x += 512) incl[x] -= hist[x];
-    int* nt = (int*)ids;                                         // E <= 4096 ints fit the id buffer
     for (int cls = 0; cls < 2; ++cls)
     {
         __syncthreads();
-        for (int x = tid; x < a.E; x += 512)
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
         {
-            const int lv = (int)a.table[(size_t)x * TBL_W];
-            nt[x] = lv > 0 && (lv > 2) == (cls == 0) ? (hist[x] + SHORT_ROWS - 1) / SHORT_ROWS : 0;
+            const int x = tid + 1024 * k;
+            if (x < a.E) nt[x] = lv[k] > 0 && (lv[k] > 2) == (cls == 0) ? (tot[x] + SHORT_ROWS - 1) / SHORT_ROWS : 0;
         }
         __syncthreads();
-        block_scan(nt, tmp, a.E);
-        for (int x = tid; x < a.E; x += 512)
+        block_scan(nt, a.E);
+        for (int x = tid; x < a.E; x += 1024)
         {
-            const int k = nt[x] - (x ? nt[x - 1] : 0), at = base + nt[x] - k;
+            const int k = nt[x] - (x ? nt[x - 1] : 0), at = base + nt[x] - k, n = tot[x], start = ext[x] - n;
             for (int q = 0; q < k; ++q)
-                T4[at + q] = make_int4(x, incl[x] + SHORT_ROWS * q, hist[x] - SHORT_ROWS * q < SHORT_ROWS ? hist[x] - SHORT_ROWS * q : SHORT_ROWS, 0);
+                T4[at + q] = make_int4(x, start + SHORT_ROWS * q, n - SHORT_ROWS * q < SHORT_ROWS ? n - SHORT_ROWS * q : SHORT_ROWS, 0);
         }
         base += nt[a.E - 1];
     }
-    for (int i = base + tid; i < a.cap; i += 512) T4[i] = make_int4(-1, 0, 0, 0);
+    for (int i = base + tid; i < a.cap; i += 1024) T4[i] = make_int4(-1, 0, 0, 0);
 }
 
 // pair rows per workgroup of the row kernels: what leaves about two thousand workgroups (eight per CU), at most eight
@@ -985,11 +998,15 @@ int launch_pf_step(const NqPfArgs& a, hipStream_t st)
     if (m.bytes > (size_t)a.meta_bytes) return set_error("nq_pf_step: meta needs %zu bytes, has %lld", m.bytes, (long long)a.meta_bytes);
     const bool fork = a.side[0] != nullptr, brief = R == P && !a.wop && pf_is_short(P, E, H, I, fork);
     {
-        const PfSort s{a.sel, a.rw, a.sel_dtype, a.rw_dtype, P, a.topk, E, a.table, m.cnt, m.pe, m.pt, m.pos, a.hits, brief ? m.tiles : nullptr, m.scap};
-        const int shm = SORT_TILE * 2 + 3 * (E + 1) * 4;
-        const hipError_t e = hipFuncSetAttribute((const void*)nq_pf_sort_k, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
-        if (e != hipSuccess) return set_error("nq_pf_sort: LDS %d bytes: %s", shm, hipGetErrorString(e));
-        nq_pf_sort_k<<<(E + 8) / 8, 512, shm, st>>>(s);
+        const int blocks = (int)(((int64_t)P + SORT_BLOCK - 1) / SORT_BLOCK), per = (blocks + SORT_WGS - 1) / SORT_WGS;
+        const PfSort s{a.sel, a.rw, a.sel_dtype, a.rw_dtype, P, a.topk, E, a.table, m.cnt, m.pe, m.pt, m.pos, a.hits, brief ? m.tiles : nullptr, m.scap, per};
+        const int shm = 3 * (E + 1) * 4;
+        if (shm > 48 * 1024)
+        {
+            const hipError_t e = hipFuncSetAttribute((const void*)nq_pf_sort_k, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
+            if (e != hipSuccess) return set_error("nq_pf_sort: LDS %d bytes: %s", shm, hipGetErrorString(e));
+        }
+        nq_pf_sort_k<<<(per ? (blocks + per - 1) / per : 0) + 1, 1024, shm, st>>>(s);
         NQ_LAUNCH_CHECK("nq_pf_sort");
     }
     float *acc = (float*)a.acc, *y = (float*)a.y;

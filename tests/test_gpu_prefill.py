@@ -522,3 +522,33 @@ def test_a_token_that_is_not_finite_is_its_own_affair(H, I, T, E, K):
     torch.cuda.synchronize()
     assert torch.equal(y[~hit], clean[~hit])
     assert torch.equal(torch.isfinite(y), torch.isfinite(slices)) and not torch.isfinite(y[hit]).any()
+
+
+@pytest.mark.parametrize("T,E,K,sd", [(1, 1, 1, torch.int32), (16, 4096, 32, torch.int64), (171, 5, 3, torch.int32), (73, 256, 7, torch.int64), (128, 300, 8, torch.int32),
+                                      (4096, 256, 8, torch.int32), (2049, 63, 64, torch.int64), (33001, 1000, 8, torch.int32)])
+def test_pairs_are_sorted_by_expert_in_pair_order(monkeypatch, T, E, K, sd):
+    """the sort of a grouped step against torch's stable one: a share of 512 pairs per workgroup, one more or fewer, several such
+    blocks per workgroup, ids of one bit and of thirteen, ids outside the table (a group behind all others), one popular expert"""
+    L = M.MoELayer(E, 128, 128, Bmax=1, topk=K)                      # every row of the table at level 0: nothing is decoded
+    g = torch.Generator().manual_seed(T)
+    sel = torch.randint(-1, E + 1, (T, K), generator=g)
+    sel[torch.rand(T, K, generator=g) < 0.3] = E // 2
+    rw = (torch.rand(T, K, generator=g) > 0.2).float()
+    hits = torch.zeros(E, dtype=torch.int32, device=DEV)
+    L.hits_ptr = hits.data_ptr()
+    made, empty = [], torch.empty
+    monkeypatch.setattr(torch, "empty", lambda *a, **k: made.append(empty(*a, **k)) or made[-1])
+    M._pf_step(L, torch.ones(T, 128, dtype=torch.float16, device=DEV), sel.to(DEV, sd), rw.to(DEV), torch.zeros(T, 128, device=DEV), R=T * K)
+    monkeypatch.undo()
+    P, key = T * K, torch.where((sel < 0) | (sel >= E), E, sel).reshape(-1)
+    block = next(t for t in made if t.dtype == torch.uint8).cpu()
+    at, parts = M._pf_offsets(128, 128, P)[1], []
+    for n in (E, P, P, P):
+        parts.append(block[at:at + 4 * n].view(torch.int32).long())
+        at += (4 * n + 15) // 16 * 16
+    cnt, pe, pt, pos = parts
+    order = torch.argsort(key, stable=True)
+    assert torch.equal(cnt, torch.bincount(key, minlength=E + 1)[:E])
+    assert torch.equal(pos[order], torch.arange(P)) and torch.equal(pt, order // K)
+    assert torch.equal(pe, torch.where(key[order] < E, key[order], -1))
+    assert torch.equal(hits.cpu().long(), torch.bincount(key[rw.reshape(-1) != 0], minlength=E + 1)[:E])
