@@ -48,6 +48,7 @@ class NqPfArgs(C.Structure):
 
 
 ROUTE_WS_BYTES = 32768          # NQ_ROUTE_WS_BYTES
+CNT_STEP = 64                   # NQ_CNT_STEP
 
 
 # name -> (restype, argtypes); every symbol declared in include/nq_moe_hip.h

@@ -110,6 +110,13 @@ extern "C" int nq_sal(const void* x, int x_dtype, int64_t x_row_stride, const vo
 
 // checks shared by the two decode entry points; own_ws: the caller brings the workspaces (nq_moe_forward), else they are
 // carved from the library's built-in scratch (nq_moe_forward_static) and the workspace fields of *p are not looked at
+// Ints between two arrival counters of a launch: NQ_CNT_STEP if the workspace has room for it. Every workgroup of a launch adds to one counter,
+// and additions to one line of memory follow one another at about 9 ns each, whichever counter they are for: in the down launch of
+// 2048 x 1024, 6 picks, 768 of them in two microseconds, the last was through 7 us later. us a call, side by side and apart: that one 30.2 ->
+// 23.4; 2048 x 1024, 4 tokens 51.2 -> 42.0; 896 x 512, 8 tokens 56.3 -> 44.3; 1024 x 384, 4 tokens 27.9 -> 24.6; 6144 x 2048, one to eight
+// tokens the same (spread over 20 us and more). 64, 128, 256, 1024 or 4096 bytes apart: the same; 32 a third of the way back.
+static int counter_step(int64_t elems, int64_t n) { return elems >= n * NQ_CNT_STEP ? NQ_CNT_STEP : 1; }
+
 static int moe_args(const char* who, const NqMoeArgs* p, bool own_ws, MoeArgs& a)
 {
     NQ_REQUIRE(p, "%s: null args", who);
@@ -150,7 +157,7 @@ static int moe_args(const char* who, const NqMoeArgs* p, bool own_ws, MoeArgs& a
         NQ_REQUIRE(p->cnt_h && p->cnt_h_elems >= S * (p->I / 128), "workspace too small: cnt_h");
         NQ_REQUIRE(p->zd && p->zd_elems >= S * (p->I / 128) * 4, "workspace too small: zd");
         a.part_gu = (float*)p->acc_gu; a.h = (_Float16*)p->h; a.part_d = (float*)p->acc_d;
-        a.cnt_gu = p->cnt_gu; a.cnt_d = p->cnt_d; a.cnt_h = p->cnt_h; a.zd = (float*)p->zd;
+        a.cnt_gu = p->cnt_gu; a.cnt_d = p->cnt_d; a.cnt_d_step = counter_step(p->cnt_d_elems, p->H / 128); a.cnt_h = p->cnt_h; a.zd = (float*)p->zd;
         NQ_REQUIRE(p->route_ws && p->route_ws_bytes >= NQ_ROUTE_WS_BYTES && ((uintptr_t)p->route_ws & 63) == 0,
                    "workspace too small: route_ws needs %d bytes, 64-byte aligned", NQ_ROUTE_WS_BYTES);
         a.route = (RouteWs*)p->route_ws;
@@ -385,7 +392,7 @@ extern "C" int nq_proj(const void* x, int x_dtype, int B, const int64_t* row, in
     NQ_REQUIRE(chunks >= 1 && chunks <= 48 && H / 128 % chunks == 0 && (sb == 1 || sb == 2 || sb == 4), "nq_proj: k-slice %d chunks of %d, %d wavefronts per block (1, 2 or 4)", chunks, H / 128, sb);
     NQ_REQUIRE(aligned16(x) && aligned16(part) && aligned16(out), "nq_proj: x, part and out must be 16-byte aligned");
     NQ_REQUIRE(part_elems >= (int64_t)(H / 128 / chunks) * B * 2 * I && cnt_elems >= 2 * I / 128, "workspace too small: part or cnt");
-    return launch_proj(x, x_dtype, B, row, H, I, G, chunks, sb, part, cnt, out, (hipStream_t)stream);
+    return launch_proj(x, x_dtype, B, row, H, I, G, chunks, sb, part, cnt, counter_step(cnt_elems, 2 * I / 128), out, (hipStream_t)stream);
 }
 
 extern "C" int nq_sum_slices(const float* part, int ny, int64_t n, float* out, void* stream)

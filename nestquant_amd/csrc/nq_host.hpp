@@ -38,6 +38,7 @@ struct MoeArgs
     int common_rows;                  // 1 = every row that can be picked has base window code 0 and no mask-mode flags; 0 = unknown
     int fuse;                         // both launches belong to this call: for runs whose row has neither a low-rank plane nor the
                                       // 512-wide rotation the down launch's staging does the gate|up finisher (set by launch_moe)
+    int cnt_d_step;                   // ints between two counters of cnt_d
     RouteWs* route;                   // NQ_ROUTE_WS_BYTES of device memory: what the routing launch hands to the projection launches
     _Float16* xrot;                   // [B * topk][2][H] fp16: rotated activations of every active pick (gate, up), B-operand order
     int hoist;                        // NqMoeArgs::hoist_value_map: level-2 runs without a sign plane apply the value map to the sums
@@ -51,7 +52,7 @@ struct MoeArgs
 int launch_moe(const MoeArgs& a, const int* cfg_gu, const int* cfg_dn, int which, hipStream_t st);
 int launch_moe_static(MoeArgs a, const int* cfg_gu, const int* cfg_dn, int which, hipStream_t st);
 int query_occ(int mode, int any_rows, int sb, int shm, int* out);
-int launch_proj(const void* x, int x_dtype, int B, const int64_t* row, int H, int I, int G, int NC, int SB, float* part, int* cnt, float* out, hipStream_t st);
+int launch_proj(const void* x, int x_dtype, int B, const int64_t* row, int H, int I, int G, int NC, int SB, float* part, int* cnt, int cnt_step, float* out, hipStream_t st);
 int launch_sum_slices(const float* part, int ny, int64_t n, float* out, hipStream_t st);
 int launch_mailbox(int64_t* table, const int64_t* stage, const int32_t* seq, int32_t* applied, int32_t* applied_host, int E, hipStream_t st);
 int launch_dequant(const int64_t* row, int proj, int level, int H, int I, void* out, hipStream_t st);

@@ -622,6 +622,8 @@ nq_gemv_k(MoeArgs a, int NC)
     __shared__ float zl[MAXTOK][4];                              // gate|up finisher: x V_gu^T of the run's tokens (low-rank plane)
     __shared__ int last;
     const int lane = threadIdx.x & 63, warp = threadIdx.x >> 6, SB = blockDim.x >> 6;
+    int cnt_step = a.cnt_d_step;
+    if constexpr (MODE == 1) asm volatile("" : "+s"(cnt_step));  // read with the first arguments, not in the tail
     if (a.mb_apply && blockIdx.z == gridDim.z - 1)
     {   // the extra plane of blocks of the last projection launch of a call with a mailbox: one of them applies it
         if (blockIdx.x == 0 && blockIdx.y == 0) mailbox_apply(a.mb_table, a.mb_stage, a.mb_seq, a.mb_applied, a.E);
@@ -768,7 +770,7 @@ nq_gemv_k(MoeArgs a, int NC)
     // ---- arrival counter of the 128-row group this block belongs to; the last block to arrive finishes the group
     const int rows0 = blockIdx.x * SB * 32;
     const int grp = MODE == 0 ? (rows0 % a.I) / 128 : rows0 / 128;
-    int* cnt = MODE == 0 ? a.cnt_gu + blockIdx.z * (a.I / 128) + grp : a.cnt_d + grp;
+    int* cnt = MODE == 0 ? a.cnt_gu + blockIdx.z * (a.I / 128) + grp : a.cnt_d + grp * cnt_step;
     const int expect = (MODE == 0 ? 2 : nruns) * NY * (128 / (SB * 32));
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");             // this wavefront's partial sums are acknowledged
     const int wv = __builtin_amdgcn_readfirstlane(warp);
@@ -884,9 +886,11 @@ int launch_moe_static(MoeArgs a, const int* cfg_gu, const int* cfg_dn, int which
     const size_t ny_gu = (size_t)(a.H / 128) / (cfg_gu[0] * cfg_gu[2]), ny_dn = (size_t)(a.I / 128) / (cfg_dn[0] * cfg_dn[2]);
     size_t off = 0;
     auto take = [&](size_t bytes) { const size_t o = off; off += (bytes + 255) & ~(size_t)255; return o; };
-    const size_t o_cnt = take((2 * S * G128 + (size_t)a.H / 128) * sizeof(int));       // cnt_gu | cnt_h | cnt_d: cleared below
     const size_t o_gu = take(ny_gu * S * 2 * a.I * sizeof(float)), o_d = take(ny_dn * S * a.H * sizeof(float));
     const size_t o_h = take(S * a.I * sizeof(_Float16)), o_zd = take(S * G128 * 4 * sizeof(float)), o_route = take(sizeof(RouteWs)), o_xrot = take(S * 2 * a.H * sizeof(_Float16));
+    const size_t before = off, wide = (2 * S * G128 + (size_t)a.H / 128 * NQ_CNT_STEP) * sizeof(int);      // the counters as far apart as there is room
+    a.cnt_d_step = before + wide <= STATIC_SCRATCH_BYTES ? NQ_CNT_STEP : 1;
+    const size_t o_cnt = take((2 * S * G128 + (size_t)a.H / 128 * a.cnt_d_step) * sizeof(int));             // cnt_gu | cnt_h | cnt_d: cleared below
     if (off > STATIC_SCRATCH_BYTES)
         return set_error("nq_moe_forward_static: this call needs %zu bytes of workspace (B=%d topk=%d H=%d I=%d, %zu and %zu k-slices), the built-in "
                          "scratch holds %zu: use coarser k-slices, or nq_moe_forward with workspaces of the caller's", off, a.B, a.topk, a.H, a.I, ny_gu, ny_dn,
@@ -895,7 +899,7 @@ int launch_moe_static(MoeArgs a, const int* cfg_gu, const int* cfg_dn, int which
     a.part_gu = (float*)(base + o_gu); a.part_d = (float*)(base + o_d); a.h = (_Float16*)(base + o_h); a.zd = (float*)(base + o_zd);
     a.route = (RouteWs*)(base + o_route); a.xrot = (_Float16*)(base + o_xrot);
     // the counters must be zero on entry; a fill kernel, not hipMemsetAsync, so that the call can be recorded into a graph
-    const int ncnt = (int)(2 * S * G128 + (size_t)a.H / 128);
+    const int ncnt = (int)(2 * S * G128 + (size_t)a.H / 128 * a.cnt_d_step);
     nq_clear_k<<<(ncnt + 255) / 256, 256, 0, st>>>(a.cnt_gu, ncnt);
     NQ_LAUNCH_CHECK("nq_moe_forward_static");
     return launch_moe(a, cfg_gu, cfg_dn, which, st);
@@ -909,7 +913,7 @@ int launch_moe_static(MoeArgs a, const int* cfg_gu, const int* cfg_dn, int which
 // Bound by latency beside the decode: table row, then records and sign vector, then 5.8 us of decode issue at level 3 (6144 x 4096), then
 // acknowledged stores, arrival counter and the slices' sums. Eight tokens, us a call: levels 2 / 3 / 4 10.7 / 13.7 / 13.8, where routing
 // launch, gate|up launch and slice sums took 20.4 / 19.0 / 19.0; slices of 2, 3, 6 or 8 chunks 13.5, 13.6, 14.2, 16.9 at level 3.
-struct ProjArgs { const void* x; const int64_t* row; float* part; int* cnt; float* out; int x_dtype, B, H, I, G; };
+struct ProjArgs { const void* x; const int64_t* row; float* part; int* cnt; float* out; int x_dtype, B, H, I, G, cnt_step; };
 __device__ __forceinline__ float4_t ld_dev4_issue(const float* p)
 {
     float4_t v;
@@ -984,7 +988,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))
     const int grp = blockIdx.x * SB * 32 / 128, expect = NY * (128 / (SB * 32));
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (threadIdx.x == 0) last = __hip_atomic_fetch_add(a.cnt + grp, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == expect - 1;
+    if (threadIdx.x == 0) last = __hip_atomic_fetch_add(a.cnt + grp * a.cnt_step, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == expect - 1;
     __syncthreads();
     if (!last) return;
     for (int i = threadIdx.x; i < a.B * 32; i += blockDim.x)     // four rows of one token each
@@ -1003,11 +1007,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))
         }
         *(float4_t*)(a.out + at) = s;
     }
-    if (threadIdx.x == 0) __hip_atomic_store(a.cnt + grp, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (threadIdx.x == 0) __hip_atomic_store(a.cnt + grp * a.cnt_step, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-int launch_proj(const void* x, int x_dtype, int B, const int64_t* row, int H, int I, int G, int NC, int SB, float* part, int* cnt, float* out, hipStream_t st)
+int launch_proj(const void* x, int x_dtype, int B, const int64_t* row, int H, int I, int G, int NC, int SB, float* part, int* cnt, int cnt_step, float* out, hipStream_t st)
 {
-    const ProjArgs a{x, row, part, cnt, out, x_dtype, B, H, I, G};
+    const ProjArgs a{x, row, part, cnt, out, x_dtype, B, H, I, G, cnt_step};
     const int shm = B * (NC * 256 + 16) + 256;
     if (shm > 48 * 1024)
     {

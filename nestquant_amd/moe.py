@@ -176,7 +176,7 @@ class MoELayer:
         s.cfg_gu, s.cfg_dn = s.default_cfg(H, I)
         s._tuned, s._cfgs = True, {}                  # cfg_for picks the k-slice lengths by the call's size; set_cfg switches that off
         s.h = torch.zeros(S, I, dtype=torch.float16, device=dev)
-        s.cnt_gu = torch.zeros(S * (I // 128), dtype=i32, device=dev); s.cnt_d = torch.zeros(H // 128, dtype=i32, device=dev)
+        s.cnt_gu = torch.zeros(max(S * (I // 128), _lib.CNT_STEP * 2 * I // 128), dtype=i32, device=dev); s.cnt_d = torch.zeros(_lib.CNT_STEP * H // 128, dtype=i32, device=dev)
         s.wq = torch.zeros(4, dtype=i32, device=dev)
         s.zd = torch.zeros(S * (I // 128) * 4, dtype=f32, device=dev); s.cnt_h = torch.zeros(S * (I // 128), dtype=i32, device=dev)
         s.out = torch.zeros(Bmax, H, dtype=f32, device=dev)

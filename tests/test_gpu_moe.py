@@ -12,7 +12,7 @@ import numpy as np
 import pytest
 import torch
 
-from nestquant_amd import format as F, moe as M, routing as RT
+from nestquant_amd import _lib, format as F, moe as M, routing as RT
 from oracle import nq_oracle as O
 from tests.util import oracle_plane, rel_err
 
@@ -662,3 +662,29 @@ def test_tokens_of_one_call_are_combined_as_alone(B, topk, SB, low_rank):
         for b in range(B):
             assert torch.equal(y[b:b + 1], L(x[b:b + 1], sel[b:b + 1], rw[b:b + 1], cfg_gu=cg, cfg_dn=cd)), b
     assert not y[B // 2].any() and not L.cnt_d.any()
+
+
+@pytest.mark.parametrize("H,I,B,topk", [(128, 128, 1, 1), (384, 256, 3, 4), (2048, 128, 8, 8)])
+def test_arrival_counters_side_by_side_or_apart(H, I, B, topk):
+    """a workspace with room for counters NQ_CNT_STEP ints apart, with exactly that room, one short of it (side by side) and just the
+    H / 128 of the contract: the same bits, and every counter back at zero"""
+    E = 8
+    ex = to_dev(experts_on_gpu(H, I, E, 40, nested_ids=(2,)))
+    L = M.MoELayer(E, H, I, Bmax=8, topk=topk)
+    for e in range(E):
+        L.set(e, ex[e], 4 if e == 2 else 2)
+    rng = np.random.default_rng(H + B)
+    x = torch.from_numpy((rng.standard_normal((B, H)) * 0.5).astype(np.float16)).to(DEV)
+    sel = torch.from_numpy(np.stack([rng.permutation(E)[:topk] for _ in range(B)]).astype(np.int32)).to(DEV)
+    rw = torch.from_numpy(rng.uniform(0.1, 1.0, (B, topk)).astype(np.float32)).to(DEV)
+    wide = L.cnt_d
+    assert wide.numel() == _lib.CNT_STEP * H // 128
+    want = L(x, sel, rw).clone()
+    for n in (_lib.CNT_STEP * H // 128 - 1, H // 128):
+        guarded = torch.zeros(n + 64, dtype=torch.int32, device=DEV)
+        guarded[n:] = -7
+        L.cnt_d = guarded[:n]
+        for _ in range(2):
+            assert torch.equal(L(x, sel, rw), want), n
+        assert not L.cnt_d.any() and bool((guarded[n:] == -7).all())
+    assert not wide.any()
