@@ -160,25 +160,31 @@ __device__ __forceinline__ void list_picks(const MoeArgs& a, int lane, PrepRows*
     }
     if (lane == 0) Q->nq = __popcll(okm);
 }
-__device__ __forceinline__ void route(const MoeArgs& a, RouteWs* W, int lane)
+// pick `lane`: its expert (-1: none), the fields of the expert's row, the level it runs at, and whether it contributes
+struct Pick { int e, level; bool inrange, ok; int64_t f[TBL_W]; };
+__device__ __forceinline__ Pick load_pick(const MoeArgs& a, int lane)
+{
+    Pick p;
+    p.e = -1; p.ok = false;
+    int lv = 0;
+    p.inrange = pick_expert(a, lane, p.e);
+#pragma unroll
+    for (int i = 0; i < TBL_W; ++i) p.f[i] = 0;
+    if (p.inrange)
+    {
+        const int64_t* ent = a.table + (size_t)p.e * TBL_W;
+#pragma unroll
+        for (int i = 0; i < TBL_W; ++i) p.f[i] = ent[i];
+        lv = (int)p.f[0];
+        p.ok = rw_at(a, lane) != 0.f && lv > 0;
+    }
+    p.level = a.force_level ? a.force_level : lv;
+    return p;
+}
+struct Place { int run, pos, ntok, nruns; };                     // the run this lane's pick goes into (-1: none), its place there, the run's size; the number of runs
+__device__ __forceinline__ Place number_runs(const MoeArgs& a, int e, bool ok, int level, int lane)
 {
     const int S = a.B * a.topk;
-    int e = -1, lv = 0; bool ok = false;
-    const bool inrange = pick_expert(a, lane, e);
-    int64_t f[TBL_W];
-#pragma unroll
-    for (int i = 0; i < TBL_W; ++i) f[i] = 0;
-    if (inrange)
-    {
-        const int64_t* ent = a.table + (size_t)e * TBL_W;
-#pragma unroll
-        for (int i = 0; i < TBL_W; ++i) f[i] = ent[i];
-        lv = (int)f[0];
-        ok = rw_at(a, lane) != 0.f && lv > 0;
-    }
-    if (a.hits && inrange && rw_at(a, lane) != 0.f)
-        __hip_atomic_fetch_add(a.hits + e, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    const int level = a.force_level ? a.force_level : lv;
     // Runs of refined experts (level 3, 4: twice the decode work per chunk) are numbered before the level-2 ones, each group
     // by first occurrence: workgroups are dispatched in run order, so the long ones start first and spread over all CUs, and
     // the short ones fill in around them (gate|up 44.0 -> 42.6 us, down 28.4 -> 27.2 us on the benchmark's level mix).
@@ -187,8 +193,7 @@ __device__ __forceinline__ void route(const MoeArgs& a, RouteWs* W, int lane)
     const unsigned long long below = (1ull << lane) - 1ull;
     const int tok = lane / a.topk, sh = tok * a.topk;
     const unsigned long long mytok = sh < 64 ? (a.topk >= 64 ? ~0ull : ((1ull << a.topk) - 1ull)) << sh : 0ull;
-    int r = 0;
-    int my_run = -1, my_pos = 0, my_ntok = 0;                    // the run this lane's pick went into, its place there, the run's size
+    Place p{-1, 0, 0, 0};
     unsigned long long eq = 0ull;                                // the active picks of this lane's expert
 #pragma unroll 4
     for (int j = 0; j < S; ++j)
@@ -201,8 +206,8 @@ __device__ __forceinline__ void route(const MoeArgs& a, RouteWs* W, int lane)
         const unsigned long long first = __ballot(ok && (eq & below) == 0ull), fh = first & heavy, fl = first & ~heavy;
         const int mine = ((heavy >> lane) & 1ull) ? __popcll(fh & below) : __popcll(fh) + __popcll(fl & below);
         const int run = __shfl(mine, eq ? __ffsll((long long)eq) - 1 : lane);
-        if (ok) { my_run = run; my_pos = __popcll(eq & below); my_ntok = __popcll(eq); }
-        r = __popcll(first);
+        if (ok) { p.run = run; p.pos = __popcll(eq & below); p.ntok = __popcll(eq); }
+        p.nruns = __popcll(first);
     }
     else
         for (int pass = 0; pass < 2; ++pass)
@@ -213,10 +218,32 @@ __device__ __forceinline__ void route(const MoeArgs& a, RouteWs* W, int lane)
                 const int ev = __builtin_amdgcn_readlane(e, __ffsll((long long)rem) - 1);
                 const unsigned long long same = __ballot(((rem >> lane) & 1ull) && e == ev);
                 const unsigned long long m = __ballot(((same >> lane) & 1ull) && (same & mytok & below) == 0ull);   // first pick per token
-                if ((m >> lane) & 1ull) { my_run = r; my_pos = __popcll(m & below); my_ntok = __popcll(m); }
-                rem &= ~m; ++r;
+                if ((m >> lane) & 1ull) { p.run = p.nruns; p.pos = __popcll(m & below); p.ntok = __popcll(m); }
+                rem &= ~m; ++p.nruns;
             }
         }
+    return p;
+}
+__device__ __forceinline__ void write_header(RunHdr& R, const int64_t (&f)[TBL_W], int mode, int level, int ntok)      // all but the slots
+{
+    const int o = mode == 0 ? 1 : 5;
+    R.P.base = (gp_u4)f[o]; R.P.res = (gp_u8)f[o + 1]; R.P.dw = (gp_u32)f[o + 2]; R.P.flags = (gp_u64)f[o + 3];
+    R.P.var = (gp_u8)f[12 + mode]; R.P.code = (int)f[10 + mode]; R.P.bcode = (int)((f[19] >> (8 * mode)) & 0xFF);
+    R.signs = (const _Float16*)f[9];
+    R.level = level;
+    R.had = f[18] == 512 ? 512 : 128;
+    R.lr = (const _Float16*)f[14]; R.lr4 = (const _Float16*)f[15]; R.rg = (int)f[16]; R.rd = (int)f[17];
+    R.ntok = ntok;
+}
+__device__ __forceinline__ void route(const MoeArgs& a, RouteWs* W, int lane)
+{
+    const Pick p = load_pick(a, lane);
+    const int64_t (&f)[TBL_W] = p.f;
+    const int level = p.level;
+    if (a.hits && p.inrange && rw_at(a, lane) != 0.f)
+        __hip_atomic_fetch_add(a.hits + p.e, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    const Place at = number_runs(a, p.e, p.ok, level, lane);
+    const int my_run = at.run, my_pos = at.pos;
     // the headers, after the numbering: every lane holds its own pick's row, so the first lanes of all runs write their runs'
     // headers side by side (inside the loop above the same stores would be issued once per run, one lane at a time)
     if (my_run >= 0)
@@ -225,25 +252,26 @@ __device__ __forceinline__ void route(const MoeArgs& a, RouteWs* W, int lane)
         if (my_pos == 0)
         {
 #pragma unroll
-            for (int mode = 0; mode < 2; ++mode)
-            {
-                RunHdr& R = W->run[mode][my_run];
-                const int o = mode == 0 ? 1 : 5;
-                R.P.base = (gp_u4)f[o]; R.P.res = (gp_u8)f[o + 1]; R.P.dw = (gp_u32)f[o + 2]; R.P.flags = (gp_u64)f[o + 3];
-                R.P.var = (gp_u8)f[12 + mode]; R.P.code = (int)f[10 + mode]; R.P.bcode = (int)((f[19] >> (8 * mode)) & 0xFF);
-                R.signs = (const _Float16*)f[9];
-                R.level = level;
-                R.had = f[18] == 512 ? 512 : 128;
-                R.lr = (const _Float16*)f[14]; R.lr4 = (const _Float16*)f[15]; R.rg = (int)f[16]; R.rd = (int)f[17];
-                R.ntok = my_ntok;
-            }
+            for (int mode = 0; mode < 2; ++mode) write_header(W->run[mode][my_run], f, mode, level, at.ntok);
         }
     }
     PickInfo& K = W->picks;
-    K.w[lane] = ok ? rw_at(a, lane) : 0.f; K.signs[lane] = (const _Float16*)f[9];
+    K.w[lane] = p.ok ? rw_at(a, lane) : 0.f; K.signs[lane] = (const _Float16*)f[9];
     K.lr[lane] = (const _Float16*)f[14]; K.lr4[lane] = (const _Float16*)f[15];
     K.rg[lane] = (unsigned char)f[16]; K.rd[lane] = (unsigned char)f[17]; K.lv[lane] = (unsigned char)level;
-    if (lane == 0) W->nruns = r;
+    if (lane == 0) W->nruns = at.nruns;
+}
+// run z of the call and the number of runs, found by one wavefront of the workgroup itself (the gate|up launch of a call without a routing
+// launch): the header that route() writes, in LDS
+struct OwnRun { RunHdr run; int nruns; };
+__device__ __forceinline__ void own_run(const MoeArgs& a, int z, int lane, OwnRun* W)
+{
+    const Pick p = load_pick(a, lane);
+    const Place at = number_runs(a, p.e, p.ok, p.level, lane);
+    if (lane == 0) W->nruns = at.nruns;
+    if (at.run != z) return;
+    W->run.slot[at.pos] = (unsigned char)lane;
+    if (at.pos == 0) write_header(W->run, p.f, 0, p.level, at.ntok);
 }
 
 // The mailbox of a layer call (reference nq_mailbox, sm120/nqmoe.cu:908-923, a launch of its own there), in two halves that
@@ -280,7 +308,27 @@ __device__ __forceinline__ void publish_applied(const int32_t* applied, int32_t*
         __hip_atomic_store(applied_host + e, applied[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// First launch of every layer call. Workgroup 0 does the routing: run headers for both projection launches, which then read one
+__device__ __forceinline__ void call_salience(const MoeArgs& a)  // by a workgroup of 256 threads
+{
+    __shared__ SalShared S;
+    const SalArgs sa{a.x, a.H, a.rw, a.sel, a.B, a.H, a.topk, a.E, a.x_dtype, a.rw_dtype, a.sel_dtype, a.sal_rsf, a.sal_acc, a.sal_host};
+    salience<4>(sa, &S);
+}
+// fp16(Hadamard-128(x[token] * su)) of a chunk of 128 columns, eight of them per lane (place L8 of 16), in B-operand order
+__device__ __forceinline__ uint4 rotate8(const MoeArgs& a, int token, const _Float16* su, int chunk, int L8, const WhtSigns& ws)
+{
+    const int col = chunk * 128 + 32 * (L8 >> 2) + 2 * (L8 & 3);
+    half2_t xv[4], sv[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) { xv[i] = x2_at(a, (size_t)token * a.H + col + 8 * i); sv[i] = *(const half2_t*)(su + col + 8 * i); }
+    float v[8];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) { v[2 * i] = (float)xv[i].x * (float)sv[i].x; v[2 * i + 1] = (float)xv[i].y * (float)sv[i].y; }
+    wht8_bop_sums(v, ws);
+    return bop_block_scaled(v, ws.scale);
+}
+
+// First launch of a layer call, except where the gate|up launch does its work (launch_moe). Workgroup 0 does the routing: run headers for both projection launches, which then read one
 // header each instead of repeating the dependent loads sel -> table row in every one of their ~1800 workgroups, the per-pick
 // data of the combine, the hits export; with a mailbox in the call its other three wavefronts publish what earlier calls applied
 // (publish_applied). Nothing here reads seq or stage and nothing writes the table. With salience in the call workgroup 1 exports
@@ -296,13 +344,7 @@ __global__ void __launch_bounds__(256) nq_prep_k(MoeArgs a)
     __shared__ PrepRows Q;
     const int lane = threadIdx.x & 63;
     const int extra = a.sal_acc ? 2 : 1;                         // workgroup 0 routes; 1 exports the salience of a call that asks for it
-    if (a.sal_acc && blockIdx.x == 1)
-    {
-        __shared__ SalShared S;
-        const SalArgs sa{a.x, a.H, a.rw, a.sel, a.B, a.H, a.topk, a.E, a.x_dtype, a.rw_dtype, a.sel_dtype, a.sal_rsf, a.sal_acc, a.sal_host};
-        salience<4>(sa, &S);
-        return;
-    }
+    if (a.sal_acc && blockIdx.x == 1) { call_salience(a); return; }
     if (blockIdx.x == 0)
     {
         if (threadIdx.x < 64) route(a, a.route, lane);
@@ -610,7 +652,9 @@ __device__ __forceinline__ void finish_dn_all(const MoeArgs& a, const PickInfo& 
 // not have to pay for. Four wavefronts per SIMD is the measured optimum for the gate|up launch (three: +4 us per layer; five:
 // +1.5 us), so the register allocator is told to aim at exactly that. The common down launch gains from five (90 registers): its
 // 1536 workgroups then need 1.2 rounds instead of 1.5 (-0.4 us per layer at one token, -2.5 us at four).
-template <int MODE, bool ANYROW>
+// OWN (gate|up of the common rows only): no routing launch comes before, see launch_moe; the last plane of blocks does that launch's other
+// work. A kernel of its own: carried along in the other one, unused, it cost 0.5 to 1.5 % of a call.
+template <int MODE, bool ANYROW, bool OWN = false>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == 1 && !ANYROW ? 5 : 4, MODE == 1 && !ANYROW ? 5 : 4)))
 nq_gemv_k(MoeArgs a, int NC)
 {
@@ -629,17 +673,41 @@ nq_gemv_k(MoeArgs a, int NC)
         if (blockIdx.x == 0 && blockIdx.y == 0) mailbox_apply(a.mb_table, a.mb_stage, a.mb_seq, a.mb_applied, a.E);
         return;
     }
+    if constexpr (OWN) if (blockIdx.z == gridDim.z - 1)
+    {   // the extra plane of blocks does the routing launch's other work: what the down launch reads, the publication, the salience
+        const int id = blockIdx.x + gridDim.x * blockIdx.y;
+        if (id == 0)
+        {
+            if (threadIdx.x < 64) route(a, a.route, lane);
+            else if (a.mb_table && a.mb_applied_host) publish_applied(a.mb_applied, a.mb_applied_host, a.E, threadIdx.x - 64, 192);
+            if (threadIdx.x == 0) a.route->ny_gu = gridDim.y;
+        }
+        else if (id == 1 && a.sal_acc) call_salience(a);
+        return;
+    }
     // the run's header, written by nq_prep_k: block-uniform, read through the scalar cache (constant address space)
     typedef const __attribute__((address_space(4))) RouteWs* cws_t;
     const cws_t W = (cws_t)a.route;
     struct RawHdr { uint32_t w[sizeof(RunHdr) / 4]; } raw;       // requested together with nruns: one round trip, not two
+    int nruns, ny_gu = 0;
+    if constexpr (OWN)
+    {
+        __shared__ OwnRun ow;
+        if (warp == 0) own_run(a, blockIdx.z, lane, &ow);
+        __syncthreads();
+        const uint32_t v = ((const uint32_t*)&ow)[lane < (int)sizeof(OwnRun) / 4 ? lane : 0];      // a word per lane, then into scalar registers
+#pragma unroll
+        for (int i = 0; i < (int)(sizeof(RunHdr) / 4); ++i) raw.w[i] = __builtin_amdgcn_readlane(v, i);
+        nruns = __builtin_amdgcn_readlane(v, sizeof(RunHdr) / 4);
+    }
+    else
     {
         const __attribute__((address_space(4))) uint32_t* src = (const __attribute__((address_space(4))) uint32_t*)&a.route->run[MODE][blockIdx.z];
 #pragma unroll
         for (int i = 0; i < (int)(sizeof(RunHdr) / 4); ++i) raw.w[i] = src[i];
+        nruns = W->nruns;
+        ny_gu = W->ny_gu;                                        // MODE 1: how many k-slices the gate|up launch that filled part_gu wrote
     }
-    const int nruns = W->nruns;
-    const int ny_gu = W->ny_gu;                                  // MODE 1: how many k-slices the gate|up launch that filled part_gu wrote
     const int N = MODE == 0 ? 2 * a.I : a.H, K = MODE == 0 ? a.H : a.I, C = K / 128;
     if (MODE == 1 && nruns == 0 && blockIdx.z == 0 && blockIdx.y == 0)
     {   // no active pick at all: nobody will arrive last, so the first plane of blocks writes the zero output
@@ -649,7 +717,7 @@ nq_gemv_k(MoeArgs a, int NC)
     if ((int)blockIdx.z >= nruns) return;                        // block-uniform
     const RunHdr R = __builtin_bit_cast(RunHdr, raw);
     const int NY = C / NC;
-    if (MODE == 0 && threadIdx.x == 0 && blockIdx.x + blockIdx.y + blockIdx.z == 0) a.route->ny_gu = NY;   // for the down launch's fused staging
+    if (MODE == 0 && !OWN && threadIdx.x == 0 && blockIdx.x + blockIdx.y + blockIdx.z == 0) a.route->ny_gu = NY;   // for the down launch's fused staging
     const int ntok = R.ntok, chunk0 = blockIdx.y * NC, k0 = chunk0 * 128;
     const int rowstride = NC * 256 + 16;                         // bytes per staged token (+16: spread tokens over banks)
     char* zero = smem + ntok * rowstride;                        // 256 zero bytes after the token rows
@@ -674,11 +742,24 @@ nq_gemv_k(MoeArgs a, int NC)
     // ---- stage the run's tokens for this k-slice in B-operand order
     if constexpr (MODE == 0)
     {
-        // rotated by nq_prep_k, already in B-operand order: 16 bytes per thread and step
-        const bool up = (int)(blockIdx.x * SB * 32) >= a.I;      // gate rows were rotated with su_g, up rows with su_u
-        const _Float16* xr = a.xrot + (up ? a.H : 0) + k0;
-        for (int i = threadIdx.x; i < ntok * NC * 16; i += blockDim.x)
+        const bool up = (int)(blockIdx.x * SB * 32) >= a.I;      // gate rows are rotated with su_g, up rows with su_u
+        _Float16* xr = a.xrot + (up ? a.H : 0) + k0;
+        if constexpr (OWN)
+        {   // (token, chunk) tasks, four per wavefront at a time; the first row block of either kind leaves its rows where nq_prep_k would
+            const WhtSigns ws = wht_signs(lane);
+            const int L8 = wht_place(lane), tasks = ntok * NC;
+            const bool keep = blockIdx.x * SB * 32 == (up ? a.I : 0);
+            for (int q0 = 4 * warp; q0 < tasks; q0 += 4 * SB)
+            {
+                const int q = min(q0 + (lane >> 4), tasks - 1), j = q / NC, c = q - j * NC, pick = R.slot_of(j);       // lanes beyond the last task repeat it
+                const uint4 b = rotate8(a, pick / a.topk, signs + (up ? 2 * a.H + 3 * a.I : 0), chunk0 + c, L8, ws);
+                *(uint4*)(smem + j * rowstride + c * 256 + 16 * L8) = b;
+                if (keep) *(uint4*)(xr + (size_t)pick * 2 * a.H + c * 128 + 8 * L8) = b;
+            }
+        }
+        else for (int i = threadIdx.x; i < ntok * NC * 16; i += blockDim.x)
         {
+            // rotated by nq_prep_k, already in B-operand order: 16 bytes per thread and step
             const int j = i / (NC * 16), r = i - j * NC * 16;
             *(u32x4*)(smem + j * rowstride + r * 16) = *(const u32x4*)(xr + (size_t)R.slot_of(j) * 2 * a.H + r * 8);
         }
@@ -809,13 +890,21 @@ __global__ void nq_mailbox_k(int64_t* table, const int64_t* stage, const int32_t
     if (applied_host) __hip_atomic_store(applied_host + e, ap, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// Which calls do without the routing launch: both projections in the call, rows of the common kind, and a gate|up launch of at most two
+// workgroups on each of 256 CUs. Every one of them then repeats the routing (about 2 us, three dependent reads) and rotates
+// its own columns, beside one another, in place of a launch of 3.4 to 4.9 us before them. us a call with / without the routing launch: 256 x 128,
+// 1 token 15.0 / 12.8; 512 x 256, 2 tokens 15.6 / 14.3; 2048 x 1024, 3 picks 18.0 / 16.7; 6144 x 2048, 4 picks 41.7 / 40.3. With four on each (1024)
+// 2048 x 1024, 8 picks 24.2 / 23.4, but 6144 x 2048, 8 picks 58.0 / 56.2 to 58.9 from one process to the next; beyond that a second round
+// pays for it again: 2048 x 1024, 6 picks (1536) 22.9 / 24.6, 896 x 512, 8 tokens (3584) 45.6 / 63.9.
+constexpr int OWN_ROUTE_WGS = 512;
 int launch_moe(const MoeArgs& a, const int* cfg_gu, const int* cfg_dn, int which, hipStream_t st)
 {
     const int S = a.B * a.topk;
     const bool reuse = (which & 4) != 0;                          // the routing launch of an earlier call left route_ws / xrot as this call needs them
     const bool defer = (which & 8) != 0;                          // two-call form of the one-call arithmetic: h is formed by the down launch
     which &= 3;
-    if (!reuse)
+    const bool own = which == 3 && !reuse && a.common_rows == 1 && cfg_gu[1] == 4 && (2 * a.I / 128) * (a.H / 128 / (cfg_gu[0] * cfg_gu[2])) * S <= OWN_ROUTE_WGS;
+    if (!reuse && !own)
     {
         const int ntask = S * 2 * (a.H / 128);                   // upper bound: every pick active
         nq_prep_k<<<std::min((ntask + 3) / 4, 1023) + (a.sal_acc ? 2 : 1), 256, 0, st>>>(a);       // one workgroup per four rotation tasks, plus the one that routes
@@ -836,13 +925,14 @@ int launch_moe(const MoeArgs& a, const int* cfg_gu, const int* cfg_dn, int which
         MoeArgs b = a;
         b.fuse = which == 3 || defer;                             // both launches belong to this call (or the caller says the other one follows)
         b.mb_apply = a.mb_table != nullptr && mode == last_mode;  // the call's last projection launch carries the mailbox block
-        auto kern = mode == 0 ? (any ? nq_gemv_k<0, true> : nq_gemv_k<0, false>) : (any ? nq_gemv_k<1, true> : nq_gemv_k<1, false>);
+        const bool self = own && mode == 0;
+        auto kern = self ? nq_gemv_k<0, false, true> : mode == 0 ? (any ? nq_gemv_k<0, true> : nq_gemv_k<0, false>) : (any ? nq_gemv_k<1, true> : nq_gemv_k<1, false>);
         if (shm > 48 * 1024)
         {
             hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
             if (e != hipSuccess) return set_error("moe_forward: LDS %d bytes: %s", shm, hipGetErrorString(e));
         }
-        kern<<<dim3(NX, NY, S + (b.mb_apply ? 1 : 0)), 64 * SB, shm, st>>>(b, NC);
+        kern<<<dim3(NX, NY, S + (b.mb_apply || self ? 1 : 0)), 64 * SB, shm, st>>>(b, NC);
         NQ_LAUNCH_CHECK("moe_forward");
     }
     return 0;

@@ -155,11 +155,15 @@ template <int D> __device__ __forceinline__ void wht_inside(float* v)
         if (!(i & D)) { const float a = v[i], b = v[i + D]; v[i] = a + b; v[i + D] = a - b; }
 }
 // place L = 4 mm + kg of the chunk; v[j + 2 a + 4 b] = column 32 mm + 2 kg + j + 8 a + 16 b
-__device__ __forceinline__ void wht8_bop(float* v, const WhtSigns& w)
+__device__ __forceinline__ void wht8_bop_sums(float* v, const WhtSigns& w)       // still to be multiplied by w.scale
 {
     wht_inside<1>(v); wht_lanes1(v, w.s0); wht_lanes2(v, w.s1);        // columns apart by 1, 2, 4
     wht_inside<2>(v); wht_inside<4>(v);                                          // 8, 16
     wht_lanes7(v, w.s2); wht_lanes8(v, w.s3);                        // 32, 64
+}
+__device__ __forceinline__ void wht8_bop(float* v, const WhtSigns& w)
+{
+    wht8_bop_sums(v, w);
 #pragma unroll
     for (int i = 0; i < 8; ++i) v[i] *= w.scale;
 }
@@ -180,6 +184,18 @@ __device__ __forceinline__ uint32_t pack_f16(float lo, float hi)
 __device__ __forceinline__ uint4 bop_block(const float* v)
 {
     return make_uint4(pack_f16(v[0], v[4]), pack_f16(v[1], v[5]), pack_f16(v[2], v[6]), pack_f16(v[3], v[7]));
+}
+// the same of scale * v, each product rounded once
+__device__ __forceinline__ uint4 bop_block_scaled(const float* v, float scale)
+{
+    uint32_t d[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+    {
+        asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(d[i]) : "v"(v[i]), "v"(scale));
+        asm("v_fma_mixhi_f16 %0, %1, %2, 0" : "+v"(d[i]) : "v"(v[i + 4]), "v"(scale));
+    }
+    return make_uint4(d[0], d[1], d[2], d[3]);
 }
 // the same from wht8_row's arrangement: two exchanges within the four lanes that hold columns 32 mm .. 32 mm + 31 (places 4 mm + q,
 // q = bit 3 of the column + 2 * bit 4): first with the lane 16 columns on, which makes the pairs, then with the one 8 columns on.

@@ -12,7 +12,7 @@ import numpy as np
 import pytest
 import torch
 
-from nestquant_amd import _lib, format as F, moe as M, routing as RT
+from nestquant_amd import _lib, format as F, moe as M, routing as RT, salience
 from oracle import nq_oracle as O
 from tests.util import oracle_plane, rel_err
 
@@ -688,3 +688,51 @@ def test_arrival_counters_side_by_side_or_apart(H, I, B, topk):
             assert torch.equal(L(x, sel, rw), want), n
         assert not L.cnt_d.any() and bool((guarded[n:] == -7).all())
     assert not wide.any()
+
+
+@pytest.mark.parametrize("H,I,B,topk,force", [(128, 128, 1, 1, 0), (256, 128, 8, 8, 0), (640, 256, 3, 4, 0), (1536, 384, 1, 8, 2), (2048, 1024, 1, 8, 0), (512, 1024, 4, 8, 0), (896, 128, 5, 5, 0)])
+def test_calls_without_a_routing_launch(H, I, B, topk, force):
+    """a call of few gate|up workgroups (up to 512, the last but one shape just there) routes and rotates in that launch: bitwise the two-call form, which
+    has a routing launch, the same routing and rotated rows left behind (which bit 2 works from them), hits and salience as there; with an expert
+    named twice by a token, weights of zero, ids outside the table, an expert at level 0, and a call with no active pick"""
+    E = 10
+    ex = to_dev(experts_on_gpu(H, I, E, 300, nested_ids=(2, 5)))
+    L = M.MoELayer(E, H, I, Bmax=8, topk=topk)
+    for e in range(E):
+        L.set(e, ex[e], 0 if e == 7 else 4 if e == 2 else 3 if e == 5 else 2)
+    rng = np.random.default_rng(H + I + B)
+    x = torch.from_numpy((rng.standard_normal((B, H)) * 0.5).astype(np.float32)).to(DEV).bfloat16()
+    sel = rng.integers(-1, E + 1, (B, topk)).astype(np.int32)
+    sel[0, -1] = sel[0, 0] = 2
+    rw = rng.uniform(0.1, 1.0, (B, topk)).astype(np.float32)
+    if topk > 2:
+        rw[B // 2, 1] = 0.0
+    sel, rw = torch.from_numpy(sel).to(DEV), torch.from_numpy(rw).to(DEV)
+    cg, cd = [1, 4, H // 128], [1, 4, 1]
+    assert 2 * I // 128 * B * topk <= 512
+    hits = torch.zeros(E, dtype=torch.int32, device=DEV)
+
+    def both(sel, rw):
+        L.xrot.fill_(-3); L.route.fill_(0); hits.zero_()
+        L.hits_ptr = hits.data_ptr()
+        y = L(x, sel, rw, cfg_gu=cg, cfg_dn=cd, force_level=force).clone()
+        got = L.xrot.clone(), L.route.clone(), hits.clone()
+        L.hits_ptr = 0
+        assert torch.equal(y, L(x, sel, rw, which=7, cfg_gu=cg, cfg_dn=cd, force_level=force))
+        L.xrot.fill_(-3); L.route.fill_(0); hits.zero_()
+        L.hits_ptr = hits.data_ptr()
+        L(x, sel, rw, which=1 | 8, cfg_gu=cg, cfg_dn=cd, force_level=force)
+        L.hits_ptr = 0
+        assert torch.equal(y, L(x, sel, rw, which=2 | 4 | 8, cfg_gu=cg, cfg_dn=cd, force_level=force))
+        assert torch.equal(got[0], L.xrot) and torch.equal(got[2], hits)
+        at = 0 if rw.any() else 8                                 # no run: nobody records the number of k-slices
+        assert torch.equal(got[1][at:], L.route[at:])
+        assert not L.cnt_gu.any() and not L.cnt_d.any()
+        return y
+    assert both(sel, rw).abs().max() > 0
+    assert not both(sel, torch.zeros_like(rw)).any()
+    sal = [salience.Salience(E, dev=DEV) for _ in range(2)]
+    L(x, sel, rw, cfg_gu=cg, cfg_dn=cd, sal=sal[0])
+    L(x, sel, rw, which=1 | 8, cfg_gu=cg, cfg_dn=cd, sal=sal[1])
+    torch.cuda.synchronize()
+    assert torch.equal(sal[0].acc, sal[1].acc)
