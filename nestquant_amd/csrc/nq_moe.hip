@@ -1,5 +1,5 @@
 // Decode-path MoE layer for 1..8 tokens (reference sm120/nqmoe.cu:375-449 route, :493-771 do_item, :858-907 moe_forward,
-// :908-929 mailbox). Three launches on one stream, every routing / level / pointer decision read on the device:
+// :908-929 mailbox). Three launches on one stream (two for calls of few workgroups, see launch_moe), every routing / level / pointer decision read on the device:
 //
 //   nq_prep_k        routing once per call (picks -> runs of distinct experts, their table rows -> run headers in RouteWs) and
 //                 the rotation of the activations of every active pick (x * su -> Hadamard-128 -> fp16, B-operand order).
