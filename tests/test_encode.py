@@ -210,6 +210,80 @@ def test_block_ldl():
     assert all(float(torch.linalg.eigvalsh(D[i]).min()) > 0 for i in range(2))
 
 
+def _two_devices(monkeypatch):
+    """stand-ins for the streams of two devices of which cuda:0 is current -> (current stream by device, what ran: (what, stream, ..))"""
+    import contextlib
+    now, current, ran = [0], {}, []
+
+    class Stream:
+        def __init__(s, dev=None):
+            s.dev = now[0] if dev is None else torch.device(dev).index
+
+        def wait_event(s, e):
+            ran.append(("waits", s, e.at))
+
+        def wait_stream(s, o):
+            ran.append(("waits", s, o))
+
+        def record_event(s, e=None):
+            e = e or Event()
+            e.record(s)
+            return e
+
+    class Event:
+        at = None
+
+        def record(s, stream=None):
+            s.at = stream or current[now[0]]
+            ran.append(("event", s.at))
+
+        def synchronize(s):
+            ran.append(("waits", "host", s.at))
+
+    @contextlib.contextmanager
+    def device(d):
+        old, now[0] = now[0], torch.device(d).index
+        yield
+        now[0] = old
+
+    @contextlib.contextmanager
+    def stream(s):
+        old, was = now[0], current[s.dev]
+        now[0], current[s.dev] = s.dev, s
+        yield
+        now[0], current[s.dev] = old, was
+    current.update({i: Stream(f"cuda:{i}") for i in (0, 1)})
+    empty = torch.empty
+    for name, f in (("Stream", Stream), ("Event", Event), ("device", device), ("stream", stream),
+                    ("current_stream", lambda d=None: current[now[0] if d is None else torch.device(d).index])):
+        monkeypatch.setattr(torch.cuda, name, f)
+    monkeypatch.setattr(torch, "empty", lambda *a, pin_memory=False, **k: pin_memory and ran.append(("pinned",)) or empty(*a, **k))
+    monkeypatch.setattr(torch.Tensor, "pin_memory", lambda t: ran.append(("pinned",)) or t)
+    monkeypatch.setattr(torch.Tensor, "to", lambda t, d, non_blocking=False: ran.append(("upload", current[now[0]])) or t)
+    monkeypatch.setattr(torch.Tensor, "record_stream", lambda t, s: ran.append(("used", s)))
+    return dict(current), ran
+
+
+class _OnSecondDevice(torch.Tensor):
+    is_cuda, device = True, torch.device("cuda", 1)
+
+
+def test_factorisation_waits_for_the_matrix_on_its_own_device(monkeypatch):
+    """the deferred block LDL of a matrix on cuda:1 with cuda:0 current: what the host waits for is recorded behind the work on the matrix,
+    on the stream of its device, and the factors come back there"""
+    X = torch.randn(512, 256, generator=torch.Generator().manual_seed(4))
+    H = (X.T @ X / 512).double()
+    L, D = EN.block_ldl(H)
+    streams, ran = _two_devices(monkeypatch)
+    later = EN._block_ldl_later(H.as_subclass(_OnSecondDevice))
+    got = later()
+    assert torch.equal(got[0], L) and torch.equal(got[1], D)
+    events = [e for e in ran if e[0] == "event"]
+    assert events and all(s is streams[1] for _, s in events)
+    assert any(e[0] == "waits" and e[2] is streams[1] for e in ran)
+    assert [s.dev for k, *r in ran if k == "upload" for s in r] == [1, 1]
+
+
 def test_ldlq_fit_feeds_errors_forward_and_lowers_the_output_error():
     """activations with a few strong directions shared by both 128-column chunks. Pinned: (1) the LDLQ identity
     tr(E H' E^T) = sum over chunks of tr(eta D eta^T), eta the chunk's own fitting error against its fed-forward target --
