@@ -270,7 +270,7 @@ class _OnSecondDevice(torch.Tensor):
 
 def test_factorisation_waits_for_the_matrix_on_its_own_device(monkeypatch):
     """the deferred block LDL of a matrix on cuda:1 with cuda:0 current: what the host waits for is recorded behind the work on the matrix,
-    on the stream of its device, and the factors come back there"""
+    on the stream of its device, and the factors come back there. Nothing is page-locked: torch would keep that memory for good"""
     X = torch.randn(512, 256, generator=torch.Generator().manual_seed(4))
     H = (X.T @ X / 512).double()
     L, D = EN.block_ldl(H)
@@ -282,6 +282,8 @@ def test_factorisation_waits_for_the_matrix_on_its_own_device(monkeypatch):
     assert events and all(s is streams[1] for _, s in events)
     assert any(e[0] == "waits" and e[2] is streams[1] for e in ran)
     assert [s.dev for k, *r in ran if k == "upload" for s in r] == [1, 1]
+    assert ("pinned",) not in ran
+    assert [s for k, *r in ran if k == "used" for s in r] == [streams[1]] * 2          # the side stream's memory, used on the caller's
 
 
 def test_ldlq_fit_feeds_errors_forward_and_lowers_the_output_error():
