@@ -360,9 +360,9 @@ __global__ void __launch_bounds__(256) nq_prep_k(MoeArgs a)
         const _Float16* su = Q.signs[q] + (up ? 2 * a.H + 3 * a.I : 0);
         const half2_t xv = x2_at(a, (size_t)(pick / a.topk) * a.H + kk), sv = *(const half2_t*)(su + kk);
         float v0 = (float)xv.x * (float)sv.x, v1 = (float)xv.y * (float)sv.y;
-        wht128(v0, v1, lane);
+        wht128_sums(v0, v1, lane);
         _Float16* dst = a.xrot + ((size_t)pick * 2 + up) * a.H + c * 128;
-        dst[bop_index(2 * lane)] = (_Float16)v0; dst[bop_index(2 * lane + 1)] = (_Float16)v1;
+        dst[bop_index(2 * lane)] = f16_scaled(v0, WHT128_SCALE); dst[bop_index(2 * lane + 1)] = f16_scaled(v1, WHT128_SCALE);
     }
 }
 
@@ -1049,10 +1049,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))
         float v[8];
 #pragma unroll
         for (int i = 0; i < 4; ++i) { v[2 * i] = (float)xv[i].x * (float)sv[i].x; v[2 * i + 1] = (float)xv[i].y * (float)sv[i].y; }
-        wht8_bop(v, ws);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) asm volatile("" : "+v"(v[i]));                // scaled in fp32, then rounded to fp16, as nq_prep_k does (see finish_gu)
-        *(uint4*)(smem + j * rowstride + c * 256 + 16 * L8) = bop_block(v);
+        wht8_bop_sums(v, ws);
+        *(uint4*)(smem + j * rowstride + c * 256 + 16 * L8) = bop_block_scaled(v, ws.scale);      // one rounding, as nq_prep_k: the same bits
     }
     if (threadIdx.x < 64) ((uint32_t*)zero)[threadIdx.x] = 0u;
     __syncthreads();

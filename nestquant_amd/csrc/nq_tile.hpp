@@ -97,7 +97,8 @@ __device__ __forceinline__ void swap_halves32(float v, float& lo, float& hi)
     lo = v; hi = v;
     asm volatile("s_nop 3\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 3" : "+v"(lo), "+v"(hi));
 }
-__device__ __forceinline__ void wht128(float& a, float& b, int lane)
+constexpr float WHT128_SCALE = 0.08838834764f;                   // 1 / sqrt(128)
+__device__ __forceinline__ void wht128_sums(float& a, float& b, int lane)        // still to be multiplied by WHT128_SCALE
 {
     const float s = a + b, d = a - b; a = s; b = d;
     const uint32_t l = (uint32_t)lane;
@@ -113,7 +114,11 @@ __device__ __forceinline__ void wht128(float& a, float& b, int lane)
     swap_rows16(b, lo, hi); b = __builtin_fmaf(hi, s16, lo);
     swap_halves32(a, lo, hi); a = __builtin_fmaf(hi, s32, lo);
     swap_halves32(b, lo, hi); b = __builtin_fmaf(hi, s32, lo);
-    a *= 0.08838834764f; b *= 0.08838834764f;
+}
+__device__ __forceinline__ void wht128(float& a, float& b, int lane)
+{
+    wht128_sums(a, b, lane);
+    a *= WHT128_SCALE; b *= WHT128_SCALE;
 }
 
 // ---- Hadamard-128 on sixteen lanes: eight elements per lane, four chunks per wavefront ---------------------------------
@@ -129,7 +134,7 @@ __device__ __forceinline__ WhtSigns wht_signs(int lane)
 {
     const int L = wht_place(lane);
     const float s0 = (L & 1) ? -1.f : 1.f, s1 = (L & 2) ? -1.f : 1.f, s2 = (L & 4) ? -1.f : 1.f, s3 = (L & 8) ? -1.f : 1.f;
-    return WhtSigns{s0, s1, s2, s3, 0.08838834764f * s0 * s1 * s2 * s3};
+    return WhtSigns{s0, s1, s2, s3, WHT128_SCALE * s0 * s1 * s2 * s3};
 }
 // v[i] = v[i] + s * (v[i] of the partner lane). Asm, because the compiler puts the select into a move of its own; a DPP read needs two
 // wait states after the write of its register, which it cannot see, so they are written out.
@@ -185,7 +190,15 @@ __device__ __forceinline__ uint4 bop_block(const float* v)
 {
     return make_uint4(pack_f16(v[0], v[4]), pack_f16(v[1], v[5]), pack_f16(v[2], v[6]), pack_f16(v[3], v[7]));
 }
-// the same of scale * v, each product rounded once
+// fp16 of scale * v, rounded once. Asm, because the compiler merges a multiplication into a conversion at some call sites and not at
+// others, and the rotations of one activation must give the same bits in every launch that makes them.
+__device__ __forceinline__ _Float16 f16_scaled(float v, float scale)
+{
+    uint32_t d;
+    asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(d) : "v"(v), "v"(scale));
+    return __builtin_bit_cast(_Float16, (uint16_t)d);
+}
+// the block of scale * v, likewise
 __device__ __forceinline__ uint4 bop_block_scaled(const float* v, float scale)
 {
     uint32_t d[4];

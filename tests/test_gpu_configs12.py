@@ -303,8 +303,8 @@ def test_projection_captured_before_its_first_eager_call():
 ])
 def test_projection_launch_equals_a_layer_call_of_one_run(H, I, B, level, cfg, dt, G):
     """the one-launch projection against the layer call and slice sum that it stands for (which it still is where the picks are counted):
-    the same products, with at most a few activations rounded to the other fp16 neighbour (2^-11 of one of H terms each); bitwise
-    repeatable, counters left at zero, level 0 zero, a foreign row NaN"""
+    the same roundings, products and sums in the same order, so the same bits; bitwise repeatable, counters left at zero, level 0 zero,
+    a foreign row NaN"""
     ex = F.Expert(H, I, seed=3, dev="cpu", nested=True)
     ex.gu.to(DEV); ex.dn.to(DEV); ex.signs = ex.signs.to(DEV)
     ex.gu.slot = ex.gu.nested_plane(); ex.dn.slot = ex.dn.nested_plane()
@@ -318,7 +318,7 @@ def test_projection_launch_equals_a_layer_call_of_one_run(H, I, B, level, cfg, d
     want = M.proj_gemv(L, x, 1, cfg)
     L.hits_ptr = 0
     assert hits.tolist() == [0, B, 0]
-    assert rel_err(got.cpu().numpy(), want.cpu().numpy()) < 4 * 2.0 ** -11 / H ** 0.5
+    assert torch.equal(got, want)
     assert not M.proj_gemv(L, x, 0, cfg).any()                    # level 0
     L.table[2].copy_(L.table[1]); L.table[2, 19] = 1              # a base plane of another window code, written past the layer
     assert M.proj_gemv(L, x, 2, cfg).isnan().all()
