@@ -61,15 +61,16 @@ int nq_pf_decode(const int64_t* table, const int32_t* experts, int G, void* Wgu_
  * for gate|up); the 4th entry
  * (persistent mode) must be 0. Workspaces: acc_gu / acc_d hold k-slice partial sums (plain stores, no float atomics):
  * acc_gu >= (H/128/(cpw*nst)) * B*topk * 2I floats, acc_d >= (I/128/(cpw*nst)) * B*topk * H floats, h >= B*topk * I
- * halfs; cnt_gu >= B*topk * I/128 and cnt_d >= H/128 int32 arrival counters (cnt_d better NQ_CNT_STEP * H/128: with that capacity they are
- * NQ_CNT_STEP ints apart, which the last workgroups of a short launch wait less for), zero on entry and zero again on exit (the
- * reference's workspace contract, sm120/nqmoe.cu:855-857). Picks with rw == 0, level <= 0 or an expert id outside
+ * halfs; cnt_gu >= B*topk * I/128 and cnt_d >= H/128 int32 arrival counters (with which bit 4 NQ_CNT_STEP * H/128), zero on entry
+ * and zero again on exit (the reference's workspace contract, sm120/nqmoe.cu:855-857); ints beyond these are not touched. Picks with rw == 0, level <= 0 or an expert id outside
  * [0, E) contribute nothing. which: bit 0 = gate|up launch, bit 1 = down launch; bit 2 = skip the call's first launch (routing
  * and rotation of the activations) because route_ws and xrot still hold what an earlier call with the same x, sel, rw and table
  * rows left there (what a benchmark of one projection launch alone uses); bit 3 = the two launches come as two calls but with the
  * arithmetic of one: the gate|up call (which = 1 | 8) leaves h to the down call (which = 2 | 4 | 8), which forms it from the gate|up
- * partial sums exactly as a which = 3 call does (same bits). Calls that share a routing (bits 2 / 3) must agree in B, topk, x, sel,
- * rw and cfg_gu's sb; the number of gate|up k-slices is taken from what the gate|up launch recorded in route_ws. hits: optional int32[E] pick counters
+ * partial sums exactly as a which = 3 call does (same bits); bit 4 (with bit 1) = the counters of cnt_d are NQ_CNT_STEP ints apart, all
+ * NQ_CNT_STEP * H/128 of them zero on entry and on exit, which the last workgroups of a short down launch wait less for (same bits).
+ * Calls that share a routing (bits 2 / 3) must agree in B, topk, x, sel, rw and cfg_gu's sb; the number of gate|up k-slices is taken
+ * from what the gate|up launch recorded in route_ws. hits: optional int32[E] pick counters
  * (device or host-mapped memory), incremented once per pick with rw != 0 (reference :784-787). */
 /* Element types of the caller's tensors. The casts the reference's caller launches around the call (x.half(), ids.long(),
  * w.half(), out.to(x.dtype): sm120/serve/nq_vllm.py:522,560,573; fusing them is the open item of
@@ -159,7 +160,7 @@ typedef struct NqMoeArgs
     int32_t reserved_;
 } NqMoeArgs;
 #define NQ_ROUTE_WS_BYTES 32768
-#define NQ_CNT_STEP 64            /* ints between two arrival counters where the workspace has room for it: 256 bytes */
+#define NQ_CNT_STEP 64            /* ints between two arrival counters that stand apart: 256 bytes */
 int nq_moe_forward(const NqMoeArgs* args, void* stream);
 
 /* nq_moe_forward for callers that cannot allocate device memory or keep workspaces of their own (code under HIP graph
@@ -273,7 +274,8 @@ int nq_sum_slices(const float* part, int ny, int64_t n, float* out, void* stream
 /* One expert's gate|up projection alone, in one launch: out [B][2I] fp32 = W_gu . fp16(Hadamard-128(x * su)) for x [B][H] (B <= 8), gate rows
  * rotated with su_g, up rows with su_u; row = the expert's table row (device). k-slices of `chunks` 128-column chunks (a divisor of H / 128, at
  * most 48), sb = 1, 2 or 4 wavefronts per block. part: (H / 128 / chunks) * B * 2I floats, not initialised, holds the k-slice partial sums
- * [slice][B][2I] afterwards (with one slice untouched); cnt: 2I / 128 counters (better NQ_CNT_STEP times as many, see nq_moe_forward), zero on entry and exit. Rows of the common kind only (base
+ * [slice][B][2I] afterwards (with one slice untouched); cnt: 2I / 128 counters, all cnt_elems ints zero on entry and on exit (from
+ * NQ_CNT_STEP times as many on the counters are that far apart). Rows of the common kind only (base
  * window code 0, no mask-mode flags): another kind comes out NaN, level 0 zero. */
 int nq_proj(const void* x, int x_dtype, int B, const int64_t* row, int H, int I, int G, int chunks, int sb, float* part, int64_t part_elems,
             int32_t* cnt, int64_t cnt_elems, float* out, void* stream);

@@ -208,7 +208,7 @@ int main(int argc, char** argv)
     a.x = x; a.rw = rw; a.table = d_table; a.out = out; a.acc_gu = acc_gu; a.h = h; a.acc_d = acc_d; a.cnt_gu = cnt_gu; a.cnt_d = cnt_d;
     a.acc_gu_elems = (int64_t)ny_gu * S * 2 * I; a.acc_d_elems = (int64_t)ny_dn * S * H; a.h_elems = (int64_t)S * I; a.out_elems = (int64_t)B * H;
     a.cnt_gu_elems = (int64_t)S * (I / 128); a.cnt_d_elems = (int64_t)(H / 128) * NQ_CNT_STEP; a.cnt_h = cnt_h; a.cnt_h_elems = (int64_t)S * (I / 128); a.zd = zd; a.zd_elems = (int64_t)S * (I / 128) * 4; a.route_ws = route_ws; a.route_ws_bytes = NQ_ROUTE_WS_BYTES; a.xrot = xrot; a.xrot_elems = (int64_t)S * 2 * H; a.common_rows = 1;   /* every row here has the K=2 base and a dense residual plane */
-    a.B = B; a.topk = topk; a.E = E; a.H = H; a.I = I; a.which = 3; a.hoist_value_map = hoist;
+    a.B = B; a.topk = topk; a.E = E; a.H = H; a.I = I; a.which = 3 | 16; a.hoist_value_map = hoist;
     memcpy(a.cfg_gu, cfg_gu, sizeof cfg_gu); memcpy(a.cfg_dn, cfg_dn, sizeof cfg_dn);
     hipEvent_t e0, e1; HIPCHK(hipEventCreate(&e0)); HIPCHK(hipEventCreate(&e1));
     a.sel = sel; NQCHK(nq_moe_forward(&a, nullptr)); HIPCHK(hipDeviceSynchronize());            // warm-up

@@ -108,15 +108,16 @@ extern "C" int nq_sal(const void* x, int x_dtype, int64_t x_row_stride, const vo
     return launch_sal(x, x_dtype, x_row_stride, w, w_dtype, ids, ids_dtype, T, H, K, E, (float)rsf, acc, host, (hipStream_t)stream);
 }
 
-// checks shared by the two decode entry points; own_ws: the caller brings the workspaces (nq_moe_forward), else they are
-// carved from the library's built-in scratch (nq_moe_forward_static) and the workspace fields of *p are not looked at
-// Ints between two arrival counters of a launch: NQ_CNT_STEP if the workspace has room for it. Every workgroup of a launch adds to one counter,
-// and additions to one line of memory follow one another at about 9 ns each, whichever counter they are for: in the down launch of
-// 2048 x 1024, 6 picks, 768 of them in two microseconds, the last was through 7 us later. us a call, side by side and apart: that one 30.2 ->
-// 23.4; 2048 x 1024, 4 tokens 51.2 -> 42.0; 896 x 512, 8 tokens 56.3 -> 44.3; 1024 x 384, 4 tokens 27.9 -> 24.6; 6144 x 2048, one to eight
-// tokens the same (spread over 20 us and more). 64, 128, 256, 1024 or 4096 bytes apart: the same; 32 a third of the way back.
+// Ints between two arrival counters of nq_proj: NQ_CNT_STEP if the workspace, zero as a whole, has room for it. Every workgroup of a launch adds to
+// one counter, and additions to one line of memory follow one another at about 9 ns each, whichever counter they are for. The layer call's down
+// launch spaces its counters where the caller says that the workspace is laid out so (which bit 4): in 2048 x 1024, 6 picks, 768 additions
+// in two microseconds, the last was through 7 us later. us a call, side by side and apart: that one 30.2 -> 23.4; 2048 x 1024, 4 tokens 51.2 ->
+// 42.0; 896 x 512, 8 tokens 56.3 -> 44.3; 1024 x 384, 4 tokens 27.9 -> 24.6; 6144 x 2048, one to eight tokens the same (spread over 20 us
+// and more). 64, 128, 256, 1024 or 4096 bytes apart: the same; 32 a third of the way back.
 static int counter_step(int64_t elems, int64_t n) { return elems >= n * NQ_CNT_STEP ? NQ_CNT_STEP : 1; }
 
+// checks shared by the two decode entry points; own_ws: the caller brings the workspaces (nq_moe_forward), else they are
+// carved from the library's built-in scratch (nq_moe_forward_static) and the workspace fields of *p are not looked at
 static int moe_args(const char* who, const NqMoeArgs* p, bool own_ws, MoeArgs& a)
 {
     NQ_REQUIRE(p, "%s: null args", who);
@@ -125,7 +126,7 @@ static int moe_args(const char* who, const NqMoeArgs* p, bool own_ws, MoeArgs& a
     NQ_REQUIRE(p->B >= 1 && p->B <= 8 && p->topk >= 1 && p->B * p->topk <= 64, "%s: B=%d topk=%d (B <= 8, B*topk <= 64)", who, p->B, p->topk);
     NQ_REQUIRE(p->E >= 1, "%s: E=%d", who, p->E);
     NQ_REQUIRE(shape_ok(p->H, p->I), "%s: H=%d I=%d must be positive multiples of 128", who, p->H, p->I);
-    NQ_REQUIRE((p->which & ~15) == 0, "%s: which=%d", who, p->which);
+    NQ_REQUIRE((p->which & ~31) == 0 && (p->which & 18) != 16, "%s: which=%d", who, p->which);       // bit 4 says something about the down launch
     NQ_REQUIRE(!(p->which & 4) || own_ws, "%s: which bit 2 (routing of an earlier call) needs the caller's route_ws / xrot", who);
     NQ_REQUIRE(p->force_level == 0 || p->force_level == 2 || p->force_level == 3 || p->force_level == 4, "%s: force_level=%d", who, p->force_level);
     NQ_REQUIRE(p->x_dtype >= 0 && p->x_dtype <= 2 && p->rw_dtype >= 0 && p->rw_dtype <= 2 && p->sel_dtype >= 0 && p->sel_dtype <= 1 && p->out_dtype >= 0 && p->out_dtype <= 2,
@@ -133,6 +134,7 @@ static int moe_args(const char* who, const NqMoeArgs* p, bool own_ws, MoeArgs& a
     NQ_REQUIRE(aligned16(p->x) && aligned16(p->out), "%s: x and out must be 16-byte aligned", who);
     NQ_REQUIRE(!own_ws || (aligned16(p->acc_gu) && aligned16(p->acc_d) && aligned16(p->h)), "%s: acc_gu, acc_d and h must be 16-byte aligned", who);
     const int64_t S = (int64_t)p->B * p->topk;
+    const int cnt_step = (p->which & 16) ? NQ_CNT_STEP : 1;
     for (int mode = 0; mode < 2; ++mode)
     {
         const int32_t* cf = mode == 0 ? p->cfg_gu : p->cfg_dn;
@@ -153,11 +155,11 @@ static int moe_args(const char* who, const NqMoeArgs* p, bool own_ws, MoeArgs& a
     if (own_ws)
     {
         NQ_REQUIRE(p->h_elems >= S * p->I, "workspace too small: h");
-        NQ_REQUIRE(p->cnt_gu_elems >= S * (p->I / 128) && p->cnt_d_elems >= p->H / 128, "workspace too small: cnt_gu or cnt_d");
+        NQ_REQUIRE(p->cnt_gu_elems >= S * (p->I / 128) && p->cnt_d_elems >= (int64_t)p->H / 128 * cnt_step, "workspace too small: cnt_gu or cnt_d");
         NQ_REQUIRE(p->cnt_h && p->cnt_h_elems >= S * (p->I / 128), "workspace too small: cnt_h");
         NQ_REQUIRE(p->zd && p->zd_elems >= S * (p->I / 128) * 4, "workspace too small: zd");
         a.part_gu = (float*)p->acc_gu; a.h = (_Float16*)p->h; a.part_d = (float*)p->acc_d;
-        a.cnt_gu = p->cnt_gu; a.cnt_d = p->cnt_d; a.cnt_d_step = counter_step(p->cnt_d_elems, p->H / 128); a.cnt_h = p->cnt_h; a.zd = (float*)p->zd;
+        a.cnt_gu = p->cnt_gu; a.cnt_d = p->cnt_d; a.cnt_d_step = cnt_step; a.cnt_h = p->cnt_h; a.zd = (float*)p->zd;
         NQ_REQUIRE(p->route_ws && p->route_ws_bytes >= NQ_ROUTE_WS_BYTES && ((uintptr_t)p->route_ws & 63) == 0,
                    "workspace too small: route_ws needs %d bytes, 64-byte aligned", NQ_ROUTE_WS_BYTES);
         a.route = (RouteWs*)p->route_ws;

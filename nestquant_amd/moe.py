@@ -292,6 +292,8 @@ class MoELayer:
                                     and sal.acc.numel() >= tb.shape[0] <= sal.host.numel() and rw.numel() == sel.numel()):
             raise RuntimeError("salience: acc and its host mirror must be contiguous float64 with an entry per expert, rw one weight per pick")
         sl = (0, 0, 0, 0.0) if sal is None else (1, sal.acc.data_ptr(), sal.host.data_ptr(), sal.rsf)
+        if which & 2 and s.cnt_d.numel() >= _lib.CNT_STEP * x.shape[1] // 128:       # room for the down launch's counters to stand apart
+            which |= 16
         raw = _lib.PACK_MOE_ARGS(
             x.data_ptr(), sel.data_ptr(), rw.data_ptr(), tb.data_ptr(), out.data_ptr(), s.acc_gu.data_ptr(), s.h.data_ptr(), s.acc_d.data_ptr(),
             s.cnt_gu.data_ptr(), s.cnt_d.data_ptr(), s.hits_ptr or 0,

@@ -131,6 +131,25 @@ def test_argument_checks_run_before_any_device_work():
     assert L.nq_mailbox(None, base, base, base, None, 4, None) != 0 and "null" in err()
 
 
+def test_counters_apart_are_asked_for_and_checked():
+    """which bit 4 needs NQ_CNT_STEP * H / 128 counters and the down launch; without it H / 128 are enough, and no capacity changes what they mean"""
+    L = _lib.lib()
+    err = lambda: L.nq_last_error().decode()
+    buf = (C.c_char * 4096)()
+    base = C.addressof(buf)
+    base += (-base) % 64
+    a = _lib.NqMoeArgs()
+    for f in ("x", "sel", "rw", "table", "out", "acc_gu", "h", "acc_d", "cnt_gu", "cnt_d", "cnt_h", "zd"):
+        setattr(a, f, base)
+    a.B, a.topk, a.E, a.H, a.I = 1, 8, 256, 6144, 2048
+    a.cfg_gu = (C.c_int32 * 4)(1, 4, 12, 0); a.cfg_dn = (C.c_int32 * 4)(1, 4, 4, 0)
+    a.acc_gu_elems = a.acc_d_elems = a.h_elems = a.out_elems = a.cnt_gu_elems = a.cnt_h_elems = a.zd_elems = 1 << 40
+    for which, elems, want in ((3, 47, "cnt_d"), (3, 48, "route_ws"), (3 | 16, 48 * _lib.CNT_STEP - 1, "cnt_d"), (3 | 16, 48 * _lib.CNT_STEP, "route_ws"),
+                               (2 | 16, 48 * _lib.CNT_STEP, "route_ws"), (16, 1 << 40, "which=16"), (1 | 16, 1 << 40, "which=17"), (32, 1 << 40, "which=32")):
+        a.which, a.cnt_d_elems = which, elems
+        assert L.nq_moe_forward(C.byref(a), None) != 0 and want in err(), (which, elems, err())
+
+
 def test_stream_engine_refuses_bad_arguments_before_touching_the_gpu(tmp_path):
     """the checks of the reference's Engine constructor (streaming/nqstream.cu:76,77,81): record size a multiple of 4 KiB,
     at least as many host entries as reads in flight, the record file must exist"""

@@ -690,6 +690,44 @@ def test_arrival_counters_side_by_side_or_apart(H, I, B, topk):
     assert not wide.any()
 
 
+@pytest.mark.parametrize("H,I,B,topk", [(128, 128, 1, 1), (384, 256, 3, 4), (2048, 128, 8, 8)])
+def test_a_longer_counter_workspace_needs_only_its_contract_zero(H, I, B, topk):
+    """a C caller that gives cnt_d more room than H / 128 and clears those alone, as the contract without which bit 4 says: the right
+    output, and nothing beyond them touched; with the bit the room is checked"""
+    import ctypes as C
+    E = 8
+    ex = to_dev(experts_on_gpu(H, I, E, 41, nested_ids=(2,)))
+    L = M.MoELayer(E, H, I, Bmax=8, topk=topk)
+    for e in range(E):
+        L.set(e, ex[e], 4 if e == 2 else 2)
+    rng = np.random.default_rng(H + B)
+    x = torch.from_numpy((rng.standard_normal((B, H)) * 0.5).astype(np.float16)).to(DEV)
+    sel = torch.from_numpy(np.stack([rng.permutation(E)[:topk] for _ in range(B)])).to(DEV)
+    rw = torch.from_numpy(rng.uniform(0.1, 1.0, (B, topk)).astype(np.float16)).to(DEV)
+    want = L(x, sel, rw).clone()
+    cg, cd = L.cfg_for(B)
+    n = H // 128
+    cnt = torch.full((_lib.CNT_STEP * n + 5,), 1 << 20, dtype=torch.int32, device=DEV)
+    cnt[:n] = 0
+    out = torch.full((B, H), float("nan"), device=DEV)
+    a = _lib.NqMoeArgs()
+    for f, t in (("x", x), ("sel", sel), ("rw", rw), ("table", L.table), ("out", out), ("acc_gu", L.acc_gu), ("h", L.h), ("acc_d", L.acc_d), ("cnt_gu", L.cnt_gu),
+                 ("cnt_d", cnt), ("cnt_h", L.cnt_h), ("zd", L.zd), ("route_ws", L.route), ("xrot", L.xrot)):
+        setattr(a, f, t.data_ptr())
+        size = f + ("_bytes" if f == "route_ws" else "_elems")
+        if hasattr(a, size):
+            setattr(a, size, t.numel())
+    a.B, a.topk, a.E, a.H, a.I, a.common_rows, a.which = B, topk, E, H, I, 1, 3
+    a.cfg_gu = (C.c_int32 * 4)(*cg, 0); a.cfg_dn = (C.c_int32 * 4)(*cd, 0)
+    for _ in range(2):
+        out.fill_(float("nan"))
+        _lib.check(_lib.lib().nq_moe_forward(C.byref(a), _lib.stream_ptr()))
+        assert torch.equal(out, want)
+    assert not cnt[:n].any() and bool((cnt[n:] == 1 << 20).all())
+    a.which, a.cnt_d_elems = 3 | 16, _lib.CNT_STEP * n - 1
+    assert _lib.lib().nq_moe_forward(C.byref(a), _lib.stream_ptr()) != 0 and b"cnt_d" in _lib.lib().nq_last_error()
+
+
 @pytest.mark.parametrize("H,I,B,topk,force", [(128, 128, 1, 1, 0), (256, 128, 8, 8, 0), (640, 256, 3, 4, 0), (1536, 384, 1, 8, 2), (2048, 1024, 1, 8, 0), (512, 1024, 4, 8, 0), (896, 128, 5, 5, 0)])
 def test_calls_without_a_routing_launch(H, I, B, topk, force):
     """a call of few gate|up workgroups (up to 512, the last but one shape just there) routes and rotates in that launch: bitwise the two-call form, which
