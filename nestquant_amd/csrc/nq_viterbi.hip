@@ -237,19 +237,28 @@ __global__ void __launch_bounds__(VT) nq_viterbi_k(VitArgs a)
 int launch_viterbi(const float* w, int T, int L, int K, const float* lut, int64_t* st, uint32_t* back, int slots, int rev, hipStream_t s)
 {
     const int shm = 2 * 16384 * 4;
-    // Rings that leave more than half of the last round's workgroups idle are searched pass by pass, in launches of `slots` passes (all first ones,
-    // then all second ones: T > slots, so the two of a ring are in different launches): halves of a round are then filled. us for 320 / 384 rings
-    // of 256 steps on 256 CUs: K = 2 1480 / 1560 -> 1265 / 1380, K = 1 1874 / 1872 -> 1523 / 1590. Elsewhere both take as many rounds.
-    const bool halves = T > slots && (2 * (int64_t)T + slots - 1) / slots < 2 * (((int64_t)T + slots - 1) / slots);
-    auto kern = halves ? (K == 2 ? nq_viterbi_k<2, true> : nq_viterbi_k<1, true>) : (K == 2 ? nq_viterbi_k<2, false> : nq_viterbi_k<1, false>);
-    const hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
-    if (e != hipSuccess) return set_error("nq_viterbi: LDS %d bytes: %s", shm, hipGetErrorString(e));
-    const int64_t units = halves ? 2 * (int64_t)T : T;
-    for (int64_t from = 0; from < units; from += halves ? slots : units)
-    {
-        const int64_t to = halves && from + slots < units ? from + slots : units;
-        kern<<<(int)(to - from < slots ? to - from : slots), VT, shm, s>>>(VitArgs{w, lut, st, back, T, L, rev, (int)from, (int)to});
+    // Where the last round would leave at least half of the workgroups idle, its rings and those of the round before are searched pass by pass, in
+    // three launches of at most `slots` passes (all first ones, then all second ones: more than `slots` rings, so the two of a ring are in different
+    // launches): three halves of a round in place of two rounds. us for 320 / 384 rings of 256 steps on 256 CUs: K = 2 1480 / 1560 -> 1265 /
+    // 1380, K = 1 1874 / 1872 -> 1523 / 1590. The rounds before them are whole rings in one launch, whose workgroups need not wait for the slowest of
+    // each round. ms for 2688 / 10304 / 24640 rings, all whole, all passes in launches of their own, and so: K = 2 7.54 / 28.3 / 66.8, 7.45 / 28.7 /
+    // 68.4, 7.32 / 28.2 / 66.8; K = 1 9.95 / 37.0 / 87.7, 9.88 / 38.0 / 90.4, 9.60 / 36.7 / 87.5.
+    const int rest = T % slots;
+    const int whole = T > slots && rest > 0 && 2 * (int64_t)rest <= slots ? T - rest - slots : T;
+    auto launch = [&](auto kern, int grid, const VitArgs& A) {
+        const hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
+        if (e != hipSuccess) return set_error("nq_viterbi: LDS %d bytes: %s", shm, hipGetErrorString(e));
+        kern<<<grid, VT, shm, s>>>(A);
         NQ_LAUNCH_CHECK("nq_viterbi");
+        return 0;
+    };
+    if (whole > 0)
+        if (int rc = launch(K == 2 ? nq_viterbi_k<2, false> : nq_viterbi_k<1, false>, whole < slots ? whole : slots, VitArgs{w, lut, st, back, whole, L, rev, 0, 0})) return rc;
+    const int n = T - whole;
+    for (int from = 0; from < 2 * n; from += slots)
+    {
+        const int to = 2 * n - from < slots ? 2 * n : from + slots;
+        if (int rc = launch(K == 2 ? nq_viterbi_k<2, true> : nq_viterbi_k<1, true>, to - from, VitArgs{w + (size_t)whole * L, lut, st + (size_t)whole * L, back, n, L, rev, from, to})) return rc;
     }
     return 0;
 }

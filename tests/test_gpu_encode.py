@@ -24,9 +24,9 @@ def test_viterbi_search_equals_the_torch_form(T, L, K):
 
 
 @pytest.mark.parametrize("K", [1, 2])
-@pytest.mark.parametrize("T,slots,L,position", [(3, 2, 40, False), (4, 3, 9, True), (5, 2, 1, False), (6, 5, 2, True), (7, 3, 33, True), (9, 4, 17, False)])
+@pytest.mark.parametrize("T,slots,L,position", [(3, 2, 40, False), (4, 3, 9, True), (5, 2, 1, False), (6, 5, 2, True), (7, 3, 33, True), (9, 4, 17, False), (22, 4, 5, True)])
 def test_viterbi_search_pass_by_pass(T, slots, L, position, K):
-    """more rings than the scratch holds at a time, with a last round that is at most half full: passes instead of rings, the same
+    """more rings than the scratch holds at a time, with a last round that is at most half full: its rings and those before by passes, the same
     states as with a scratch for all of them (whole rings)"""
     g = torch.Generator().manual_seed(T + L)
     w, lut = (torch.randn(T, L, generator=g) * 1.3).cuda(), EN.codebook().cuda()
