@@ -268,9 +268,11 @@ class _OnSecondDevice(torch.Tensor):
     is_cuda, device = True, torch.device("cuda", 1)
 
 
-def test_factorisation_waits_for_the_matrix_on_its_own_device(monkeypatch):
+@pytest.mark.parametrize("ahead", [255, 256])
+def test_factorisation_waits_for_the_matrix_on_its_own_device(monkeypatch, ahead):
     """the deferred block LDL of a matrix on cuda:1 with cuda:0 current: what the host waits for is recorded behind the work on the matrix,
-    on the stream of its device, and the factors come back there. Nothing is page-locked: torch would keep that memory for good"""
+    on the stream of its device, and the factors come back there. Page-locked memory, which torch keeps for good, holds a small matrix at most"""
+    monkeypatch.setattr(EN, "LDL_AHEAD", ahead)
     X = torch.randn(512, 256, generator=torch.Generator().manual_seed(4))
     H = (X.T @ X / 512).double()
     L, D = EN.block_ldl(H)
@@ -282,7 +284,7 @@ def test_factorisation_waits_for_the_matrix_on_its_own_device(monkeypatch):
     assert events and all(s is streams[1] for _, s in events)
     assert any(e[0] == "waits" and e[2] is streams[1] for e in ran)
     assert [s.dev for k, *r in ran if k == "upload" for s in r] == [1, 1]
-    assert ("pinned",) not in ran
+    assert ran.count(("pinned",)) == (ahead == 256)
     assert [s for k, *r in ran if k == "used" for s in r] == [streams[1]] * 2          # the side stream's memory, used on the caller's
 
 
