@@ -31,7 +31,8 @@ const char* nq_last_error(void);
  * {gate|up, down}; replaces rk_codes() / bk_codes() (reference sm120/nqmoe.cu:938-940, sm120/moe.py:246-252). */
 int nq_codes(uint32_t out[4]);
 
-/* Occupancy of a decode kernel (mode 0 = gate|up, 1 = down; any_rows as NqMoeArgs.common_rows != 1) launched with sb
+/* Occupancy of a projection kernel of a layer call that has a routing launch (mode 0 = gate|up, 1 = down; any_rows as NqMoeArgs.common_rows
+ * != 1; the gate|up kernel of small calls that routes itself and nq_proj's kernel are built for the same bounds and are not asked about) launched with sb
  * wavefronts per workgroup and shm bytes of dynamic LDS: out[0] = resident workgroups per CU, out[1] = registers per lane,
  * out[2] = spill bytes per lane. Replaces occ(mode, G, cpw, sb, shm) (reference sm120/nqmoe.cu:930-937, which packs the
  * three figures into one integer; G and cpw select no separate kernel here). Needs a GPU. */

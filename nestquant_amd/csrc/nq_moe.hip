@@ -591,8 +591,8 @@ __device__ __forceinline__ void finish_dn(const MoeArgs& a, const PickInfo& R, c
 
 // Several tokens: all at once (red: B * SB * 128 floats), N picks of a wavefront in flight with their scales, one barrier. Token by token as
 // above, with two barriers each, the last workgroup's tail grew with the tokens: us a call, before and now: 512 x 256, 2 tokens 16.9 -> 15.6;
-// 1024 x 384, 4 tokens 29.8 -> 28.3; 4736 x 1152, 3 tokens 72.9 -> 70.9; 2048 x 1024, 4 tokens 52.8 -> 51.8, 8 tokens 83.2 -> 80.0; 6144 x 2048, 4
-// tokens 204.0 -> 202.4. For one token the walk over tokens costs more than it gives (30.7 against 30.5 at 2048 x 1024); N = 2 where
+// 1024 x 384, 4 tokens 29.8 -> 28.3; 4736 x 1152, 3 tokens 72.9 -> 70.9; 2048 x 1024, 4 tokens 52.8 -> 51.8, 8 tokens 83.2 -> 80.0; 6144 x 2048
+// the same within the noise. For one token the walk over tokens costs more than it gives (30.7 against 30.5 at 2048 x 1024); N = 2 where
 // that is all a wavefront has (four reads' worth of dummies cost 1 us at 512 x 256), else 4.
 template <int N>
 __device__ __forceinline__ void finish_dn_all(const MoeArgs& a, const PickInfo& R, const PickLanes& P, int grp, int NY, int warp, int SB, int lane, float* red)
@@ -896,6 +896,8 @@ __global__ void nq_mailbox_k(int64_t* table, const int64_t* stage, const int32_t
 // 1 token 15.0 / 12.8; 512 x 256, 2 tokens 15.6 / 14.3; 2048 x 1024, 3 picks 18.0 / 16.7; 6144 x 2048, 4 picks 41.7 / 40.3. With four on each (1024)
 // 2048 x 1024, 8 picks 24.2 / 23.4, but 6144 x 2048, 8 picks 58.0 / 56.2 to 58.9 from one process to the next; beyond that a second round
 // pays for it again: 2048 x 1024, 6 picks (1536) 22.9 / 24.6, 896 x 512, 8 tokens (3584) 45.6 / 63.9.
+// With a layer and inputs met for the first time, nothing of them in any cache, the heads cost more and the gain is smaller. us of the two
+// projection kernels, and of the routing launch before them: 512 x 256, 2 tokens 4.4 + 17.4 / 20.1; repeated 3.4 + 14.0 / 14.2.
 constexpr int OWN_ROUTE_WGS = 512;
 int launch_moe(const MoeArgs& a, const int* cfg_gu, const int* cfg_dn, int which, hipStream_t st)
 {

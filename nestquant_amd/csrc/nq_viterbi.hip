@@ -19,7 +19,8 @@
 // the word (9.3 for two candidates) is ahead of the carried mask (9.6) by more than that inside the kernel, of minima of doubles too.
 // Measured, us for 128 / 256 / 512 rings of 256 steps: K = 2 725 / 935 / 1785 (858 / 1019 / 2034 with the carried masks, decisions in steps
 // that nobody walks back over, and a walk that waited for each of its blocks), K = 1 932 / 1050 / 1990 (1084 / 1190 / 2300; its
-// single array costs a second barrier). The walks back are about 40 of them. Without any decisions 640 and 758 (K = 2): keeping
+// single array costs a second barrier). 267 vector instructions per wavefront and step at K = 2, one per 3.0 clocks and SIMD over the
+// whole launch, 288 and 3.9 at K = 1 (313 and 3.1, 320 and 4.0 with the carried masks). The walks back are about 40 of them. Without any decisions 640 and 758 (K = 2): keeping
 // every seventh step's costs instead and finding the decisions anew from them cost more in traffic than that gives.
 #include "nq_decode.hpp"
 #include "nq_host.hpp"

@@ -96,8 +96,8 @@ def rk_codes():
 
 
 def occ(mode, sb, shm, any_rows=False):
-    """(resident workgroups per CU, registers per lane, spill bytes per lane) of the decode kernel `mode` (0 gate|up, 1 down)
-    launched with sb wavefronts per workgroup and shm bytes of dynamic LDS; the reference's M.occ (sm120/nqmoe.cu:930-937)"""
+    """(resident workgroups per CU, registers per lane, spill bytes per lane) of the decode kernel `mode` (0 gate|up, 1 down) of a
+    call with a routing launch, launched with sb wavefronts per workgroup and shm bytes of dynamic LDS; the reference's M.occ (sm120/nqmoe.cu:930-937)"""
     out = (C.c_int * 3)()
     _lib.check(_lib.lib().nq_occ(mode, int(any_rows), sb, shm, out))
     return tuple(out)
@@ -313,7 +313,7 @@ PF_TILES = (16, 32, 64, 128, 256)            # token-tile heights the grouped GE
 # An expert with at least PF_HOT_MIN pair rows in a chunk (more than one 256-row tile) can be decoded once per call into a scratch
 # of decoded weights (at most PF_HOT_SLOTS experts at 6 H I bytes each) instead of once per tile; see nq_pf_wdecode. Off by
 # default (0 slots): a tile then reads 75 MB of fp16 operands from HBM where the decode-fused kernel reads 12.6 MB of codes, and
-# on the 4096-token benchmark the call takes 6.36 ms with 32 slots against 6.29 to 6.36 without (the tiles save 0.7 ms of their own
+# on the 4096-token benchmark the call takes 6.22 ms with 32 slots against 6.06 without (the tiles save 0.6 ms of their own
 # time, the decode launches cost 0.61) plus 2.4 GB of scratch. Same bits either way.
 PF_HOT_MIN, PF_HOT_SLOTS = 257, 0
 
