@@ -227,9 +227,9 @@ int nq_pf_gemm(const int64_t* table, const int32_t* tiles, int ntiles, int bm, i
                const void* A1_f16, float* C, int E, int H, int I, const void* Wop, void* stream);
 
 /* Decode the experts that nq_pf_plan marked hot (hot[e] = their slot, -1 = none; device int32 [E]) once per call: projection
- * `mode` (0 gate|up, 1 down) of each into slot hot[e] of the scratch Wop (slots x 3 * H * I fp16, 16-byte aligned), in the
- * order in which nq_pf_gemm holds weights in registers, so that every tile of such an expert (fourth word of the tile = slot + 1)
- * loads its operands instead of decoding the expert again. Experts at level <= 0, in mask mode or with a base code other than 0
+ * `mode` (0 gate|up, 1 down) of each into slot hot[e] < slots of the scratch Wop (slots x 3 * H * I fp16, 16-byte aligned), as MFMA
+ * operands, so that the 256-row tiles of such an expert (fourth word of the tile = slot + 1) are a product of decoded weights in nq_pf_gemm
+ * instead of decoding the expert again. Experts at level <= 0, in mask mode or with a base code other than 0
  * are left out (their tiles decode in the GEMM as before). Pass the same Wop to nq_pf_gemm; NULL there = every tile decodes.
  * The reference decodes every expert of a group once too, but into dense [2I][H] / [H][I] matrices for a library GEMM
  * (pf_decode, sm120/nqmoe.cu:1013-1080,1247-1257; sm120/moe.py:303-324). */
@@ -262,7 +262,7 @@ int nq_pf_post(const float* y, const int32_t* pos, const int64_t* sel, const voi
  * the remainder goes to index e of the list of the smallest height that holds it; every other entry gets expert -1, which
  * nq_pf_gemm skips. Launch nq_pf_gemm on list k with ntiles = E (k < 4) or cap (k = 4). hot (device int32 [E], may be NULL):
  * experts with at least hot_min rows in the chunk get a slot 0 .. hot_cap - 1 of the decoded-weight scratch, in expert order as
- * far as the slots reach: hot[e] = slot or -1, and the fourth word of each of their tiles = slot + 1 (0 otherwise); see
+ * far as the slots reach: hot[e] = slot or -1, and the fourth word of each of their tiles in list 4 = slot + 1 (0 otherwise); see
  * nq_pf_wdecode. Replaces the host loop over the
  * expert counts of the reference's prefill (sm120/moe.py:296-302) and the host synchronisation that feeds it. */
 int nq_pf_plan(const int32_t* counts, int E, int row_lo, int nrows, int32_t* tiles, int cap, int32_t* hot, int hot_min, int hot_cap,
@@ -305,10 +305,14 @@ typedef struct NqPfArgs
     int32_t T, topk, E, H, I;
     int32_t rows;                  /* pair rows the scratch holds; more pairs are worked through in chunks (out must then be fp32) */
     int32_t x_dtype, sel_dtype, rw_dtype, out_dtype;   /* as in NqMoeArgs */
-    int32_t variants;              /* 1: every row has base code 0 and no mask-mode flags (others come out NaN); 3: unknown */
+    int32_t variants;              /* 1: every row has base code 0 and no mask-mode flags (others come out NaN); 3: unknown; | 4: decoded weights only
+                                    * for experts above level 2 and where their tiles fill the GPU (with nq_pf_wide_slots) */
     int32_t hot_min, wop_slots;
 } NqPfArgs;
 int nq_pf_step(const NqPfArgs* args, void* stream);
+/* Slots of decoded weights that a step of these sizes is worth giving (0: none), side = with side streams; *hot_min = the rows from which
+ * an expert should take one. */
+int nq_pf_wide_slots(int T, int topk, int rows, int E, int H, int I, int side, int32_t* hot_min);
 int64_t nq_pf_meta_bytes(int T, int topk, int rows, int E);   /* -1: arguments out of range */
 
 /* hits[e] += counts[e] (hits may be host-mapped). Replaces pf_hits (reference sm120/nqmoe.cu:1241-1245,1288-1293). */

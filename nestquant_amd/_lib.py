@@ -76,6 +76,7 @@ SIGNATURES = {
     "nq_proj": (C.c_int, [_vp, _i, _i, _vp, _i, _i, _i, _i, _i, _vp, C.c_int64, _vp, C.c_int64, _vp, _vp]),
     "nq_sum_slices": (C.c_int, [_vp, _i, C.c_int64, _vp, _vp]),
     "nq_pf_step": (C.c_int, [C.POINTER(NqPfArgs), _vp]),
+    "nq_pf_wide_slots": (C.c_int, [_i, _i, _i, _i, _i, _i, _i, _i32p]),
     "nq_pf_meta_bytes": (C.c_int64, [_i, _i, _i, _i]),
     "nq_pf_hits": (C.c_int, [_i32p, _i32p, _i, _vp]),
     "nq_viterbi": (C.c_int, [_vp, _i, _i, _i, _vp, _vp, _vp, C.c_int64, _i, _vp]),

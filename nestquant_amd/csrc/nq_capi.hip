@@ -244,7 +244,9 @@ extern "C" int nq_pf_gemm(const int64_t* table, const int32_t* tiles, int ntiles
     NQ_REQUIRE(E >= 1 && shape_ok(H, I), "nq_pf_gemm: E=%d H=%d I=%d (H, I positive multiples of 128)", E, H, I);
     NQ_REQUIRE(aligned16(A0) && aligned16(A1) && aligned16(C) && aligned16(tiles), "nq_pf_gemm: tiles, activations and C must be 16-byte aligned");
     NQ_REQUIRE(aligned16(Wop), "nq_pf_gemm: the decoded-weight scratch must be 16-byte aligned");
-    return launch_pf_gemm(table, tiles, ntiles, bm, mode, A0, A1, C, E, H, I, Wop, (hipStream_t)stream);
+    const bool wide = Wop && bm == 256;
+    if (int rc = launch_pf_gemm(table, tiles, ntiles, bm, mode, A0, A1, C, E, H, I, wide, (hipStream_t)stream)) return rc;
+    return wide && !(mode & 2) ? launch_pf_wide(table, tiles, ntiles, mode, A0, A1, C, E, H, I, Wop, (hipStream_t)stream) : 0;
 }
 
 extern "C" int nq_pf_mid(const float* acc_gu, const int32_t* pe, int np, const int64_t* table, void* h, const float* zg, float* zd,
@@ -284,10 +286,10 @@ extern "C" int nq_pf_post(const float* y, const int32_t* pos, const int64_t* sel
 extern "C" int nq_pf_wdecode(const int64_t* table, const int32_t* hot, int E, int mode, void* Wop, int64_t wop_bytes, int slots, int H, int I, void* stream)
 {
     NQ_REQUIRE(table && hot && Wop, "nq_pf_wdecode: null pointer");
-    NQ_REQUIRE(E >= 1 && E <= 65535 && (mode == 0 || mode == 1) && slots >= 1, "nq_pf_wdecode: E=%d (1..65535) mode=%d slots=%d", E, mode, slots);
+    NQ_REQUIRE(E >= 1 && E <= 65535 && (mode == 0 || mode == 1) && slots >= 1 && slots <= 65535, "nq_pf_wdecode: E=%d (1..65535) mode=%d slots=%d", E, mode, slots);
     NQ_REQUIRE(shape_ok(H, I), "nq_pf_wdecode: H=%d I=%d (positive multiples of 128)", H, I);
     NQ_REQUIRE(aligned16(Wop) && wop_bytes >= (int64_t)slots * 3 * H * I * 2, "nq_pf_wdecode: the scratch needs %d slots of 3 * H * I halfs, 16-byte aligned", slots);
-    return launch_pf_wdecode(table, hot, E, mode, Wop, H, I, (hipStream_t)stream);
+    return launch_pf_wdecode(table, hot, E, nullptr, mode, Wop, slots, H, I, (hipStream_t)stream);
 }
 
 extern "C" int nq_pf_plan(const int32_t* counts, int E, int row_lo, int nrows, int32_t* tiles, int cap, int32_t* hot, int hot_min, int hot_cap, void* stream)
@@ -297,7 +299,7 @@ extern "C" int nq_pf_plan(const int32_t* counts, int E, int row_lo, int nrows, i
     NQ_REQUIRE(aligned16(tiles), "nq_pf_plan: tiles must be 16-byte aligned");
     NQ_REQUIRE(cap >= E + nrows / 256 + 1, "nq_pf_plan: cap=%d, need at least E + nrows / 256 + 1 = %d", cap, E + nrows / 256 + 1);
     NQ_REQUIRE(!hot || (hot_min >= 1 && hot_cap >= 1), "nq_pf_plan: hot_min=%d hot_cap=%d (both at least 1 with a hot list)", hot_min, hot_cap);
-    return launch_pf_plan(counts, E, row_lo, nrows, tiles, cap, hot, hot_min, hot_cap, (hipStream_t)stream);
+    return launch_pf_plan(counts, E, row_lo, nrows, tiles, cap, hot, hot_min, hot_cap, nullptr, 0, nullptr, (hipStream_t)stream);
 }
 
 extern "C" int nq_pf_hits(const int32_t* counts, int32_t* hits, int E, void* stream)
@@ -324,6 +326,12 @@ extern "C" int64_t nq_pf_meta_bytes(int T, int topk, int rows, int E)
     return pf_meta_bytes(T * topk, rows < T * topk ? rows : T * topk, E);
 }
 
+extern "C" int nq_pf_wide_slots(int T, int topk, int rows, int E, int H, int I, int side, int32_t* hot_min)
+{
+    if (T < 0 || topk < 1 || rows < 1 || E < 1 || !shape_ok(H, I) || (int64_t)T * topk > INT32_MAX || !hot_min) return 0;
+    return pf_wide_slots(T, T * topk, rows < T * topk ? rows : T * topk, E, H, I, side != 0, hot_min);
+}
+
 extern "C" int nq_pf_step(const NqPfArgs* p, void* stream)
 {
     NQ_REQUIRE(p, "nq_pf_step: null args");
@@ -334,7 +342,7 @@ extern "C" int nq_pf_step(const NqPfArgs* p, void* stream)
     NQ_REQUIRE(a.E >= 1 && a.E <= 4096 && shape_ok(a.H, a.I), "nq_pf_step: E=%d (1..4096) H=%d I=%d (positive multiples of 128)", a.E, a.H, a.I);
     NQ_REQUIRE(a.x_dtype >= 0 && a.x_dtype <= 2 && a.rw_dtype >= 0 && a.rw_dtype <= 2 && a.sel_dtype >= 0 && a.sel_dtype <= 1 && a.out_dtype >= 0 && a.out_dtype <= 2,
                "nq_pf_step: dtype codes x=%d sel=%d rw=%d out=%d", a.x_dtype, a.sel_dtype, a.rw_dtype, a.out_dtype);
-    NQ_REQUIRE(a.variants >= 1 && a.variants <= 3, "nq_pf_step: variants=%d (1 common rows, 2 rare rows, 3 both)", a.variants);
+    NQ_REQUIRE((a.variants & ~4) >= 1 && (a.variants & ~4) <= 3, "nq_pf_step: variants=%d (1 common rows, 2 rare rows, 3 both; 4 beside them: decoded weights where they pay)", a.variants);
     NQ_REQUIRE(aligned16(a.x) && aligned16(a.out) && aligned16(a.meta) && aligned16(a.xg) && aligned16(a.xu) && aligned16(a.acc) && aligned16(a.h) && aligned16(a.y) && aligned16(a.wop),
                "nq_pf_step: buffers must be 16-byte aligned");
     NQ_REQUIRE(a.rows >= 1 && (a.out_dtype == 0 || a.rows >= (int64_t)a.T * a.topk), "nq_pf_step: rows=%d; a result of another type than fp32 needs all %d pairs in one chunk", a.rows, a.T * a.topk);

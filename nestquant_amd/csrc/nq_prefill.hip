@@ -10,6 +10,7 @@
 //                 decodes two strips of the expert's records into MFMA A operands, then runs TG x 8 MFMAs
 //                 (v_mfma_f32_16x16x32_f16, fp32 accumulate) over the staged tokens. Level from the live table row.
 //   nq_pf_short_k the same for all tiles of up to 64 rows in one launch
+//   nq_pf_wdecode_k, nq_pf_wide_k   weights of experts with many rows decoded once into a scratch, and their tiles
 //   nq_pf_mid_k   Hadamard * sv, SwiGLU, * su_d, Hadamard -> h fp16 (B-operand order)               (reference nq_pf_mid)
 //   nq_pf_post_k  out[token] += sum over its picks of rw * sv_o (.) Hadamard(y): gathered per token, no atomics  (reference nq_pf_post)
 //   nq_pf_hits_k  hits[e] += counts[e]                                                            (reference nq_pf_hits)
@@ -349,52 +350,76 @@ __device__ __forceinline__ void block_scan(int* a, int n)
 }
 
 // hot (may be null): experts with at least hot_min rows in the chunk get a slot 0 .. hot_cap - 1 of the decoded-weight scratch (in
-// expert order, as far as the slots reach), written to hot[e] (-1: none) and, plus one, into the fourth word of their tiles.
+// expert order, as far as the slots reach), written to hot[e] (-1: none) and, plus one, into the fourth word of their tiles in list 4 (a
+// remainder of up to 128 rows is decoded inside its GEMM: as dear as a whole unit of nq_pf_wide_k). wide (may be null): those tiles
+// once more without gaps from wide + 4 on, their number in wide[0].
 __global__ void __launch_bounds__(256) nq_pf_plan_k(const int32_t* __restrict__ counts, int E, int row_lo, int nrows, int32_t* tiles, int cap,
-                                                    int32_t* hot, int hot_min, int hot_cap)
+                                                    int32_t* hot, int hot_min, int hot_cap, int32_t* wide, int wide_min, const int64_t* __restrict__ table)
 {
     extern __shared__ int plan_sh[];
-    int *incl = plan_sh, *tmp = plan_sh + E, *full = plan_sh + 2 * E, *hrank = plan_sh + 3 * E;
+    int *incl = plan_sh, *fincl = plan_sh + E, *wincl = plan_sh + 2 * E, *hrank = plan_sh + 3 * E;
     for (int e = threadIdx.x; e < E; e += blockDim.x) incl[e] = counts[e] > 0 ? counts[e] : 0;
     __syncthreads();
     block_scan(incl, E);
     const int row_hi = row_lo + nrows;
-    for (int e = threadIdx.x; e < E; e += blockDim.x)
-    {
+    auto rows_of = [&](int e, int& r0) {                         // of expert e in the chunk, the first of them at r0
         const int c = counts[e] > 0 ? counts[e] : 0, start = incl[e] - c;
         const int u = start > row_lo ? start : row_lo, v = start + c < row_hi ? start + c : row_hi;
-        const int n = v > u ? v - u : 0;
-        full[e] = n / 256;
-        hrank[e] = hot != nullptr && n >= hot_min ? 1 : 0;
+        r0 = u - row_lo;
+        return v > u ? v - u : 0;
+    };
+    auto is_hot = [&](int e, int n) { return hot != nullptr && n >= hot_min && (table == nullptr || table[(size_t)e * TBL_W] > 2); };
+    for (int e = threadIdx.x; e < E; e += blockDim.x)
+    {
+        int r0;
+        const int n = rows_of(e, r0);
+        fincl[e] = n / 256;
+        hrank[e] = is_hot(e, n);
     }
     __syncthreads();
-    block_scan(hrank, E);                                   // inclusive: hot experts up to and including e
-    int* fincl = tmp;                                            // inclusive scan of the full-tile counts
-    for (int e = threadIdx.x; e < E; e += blockDim.x) fincl[e] = full[e];
-    __syncthreads();
-    block_scan(fincl, E);
-    int4* T4 = (int4*)tiles;
+    block_scan(hrank, E);                                        // inclusive: hot experts up to and including e
+    block_scan(fincl, E);                                        // full tiles, likewise
+    auto slot1_of = [&](int e, int n) { return is_hot(e, n) && hrank[e] <= hot_cap ? hrank[e] : 0; };        // scratch slot + 1
+    if (wide)
+    {
+        for (int e = threadIdx.x; e < E; e += blockDim.x)
+        {
+            int r0;
+            const int n = rows_of(e, r0);
+            wincl[e] = slot1_of(e, n) ? n / 256 + (n % 256 > 128) : 0;
+        }
+        __syncthreads();
+        block_scan(wincl, E);
+        if (wincl[E - 1] < wide_min) hot_cap = 0;                // too few to fill the GPU: nobody takes a slot
+        if (threadIdx.x == 0) wide[0] = hot_cap ? wincl[E - 1] : 0;
+    }
+    int4 *T4 = (int4*)tiles, *W4 = (int4*)wide + 1;
     for (int e = threadIdx.x; e < E; e += blockDim.x)
     {
-        const int c = counts[e] > 0 ? counts[e] : 0, start = incl[e] - c;
-        const int u = start > row_lo ? start : row_lo, v = start + c < row_hi ? start + c : row_hi;
-        const int n = v > u ? v - u : 0, r0 = u - row_lo, nf = n / 256, rem = n % 256;
+        int r0;
+        const int n = rows_of(e, r0), nf = n / 256, rem = n % 256;
         const int k = rem == 0 ? -1 : rem <= 16 ? 0 : rem <= 32 ? 1 : rem <= 64 ? 2 : rem <= 128 ? 3 : 4;
-        const bool is_hot = hot != nullptr && n >= hot_min && hrank[e] <= hot_cap;
-        const int slot1 = is_hot ? hrank[e] : 0;                 // scratch slot + 1
+        const int slot1 = slot1_of(e, n);
         if (hot != nullptr) hot[e] = slot1 - 1;
+        const int4 last = make_int4(e, r0 + 256 * nf, rem, k == 4 ? slot1 : 0);
 #pragma unroll
-        for (int q = 0; q < 5; ++q) T4[(size_t)q * cap + e] = q == k ? make_int4(e, r0 + 256 * nf, rem, slot1) : make_int4(-1, 0, 0, 0);
-        const int base = E + fincl[e] - nf;
-        for (int j = 0; j < nf; ++j) T4[(size_t)4 * cap + base + j] = make_int4(e, r0 + 256 * j, 256, slot1);
+        for (int q = 0; q < 5; ++q) T4[(size_t)q * cap + e] = q == k ? last : make_int4(-1, 0, 0, 0);
+        const int base = E + fincl[e] - nf, wbase = wide && slot1 ? wincl[e] - nf - (k == 4) : 0;
+        for (int j = 0; j < nf; ++j)
+        {
+            const int4 t = make_int4(e, r0 + 256 * j, 256, slot1);
+            T4[(size_t)4 * cap + base + j] = t;
+            if (wide && slot1) W4[wbase + j] = t;
+        }
+        if (wide && slot1 && k == 4) W4[wbase + nf] = last;
     }
     const int total = E + fincl[E - 1];
     for (int i = total + threadIdx.x; i < cap; i += blockDim.x) T4[(size_t)4 * cap + i] = make_int4(-1, 0, 0, 0);
 }
 
-int launch_pf_plan(const int32_t* counts, int E, int row_lo, int nrows, int32_t* tiles, int cap, int32_t* hot, int hot_min, int hot_cap, hipStream_t st)
+int launch_pf_plan(const int32_t* counts, int E, int row_lo, int nrows, int32_t* tiles, int cap, int32_t* hot, int hot_min, int hot_cap, int32_t* wide, int wide_min, const int64_t* table, hipStream_t st)
 {
-    nq_pf_plan_k<<<1, 256, 4 * E * sizeof(int), st>>>(counts, E, row_lo, nrows, tiles, cap, hot, hot_min, hot_cap);
+    nq_pf_plan_k<<<1, 256, 4 * E * sizeof(int), st>>>(counts, E, row_lo, nrows, tiles, cap, hot, hot_min, hot_cap, wide, wide_min, table);
     NQ_LAUNCH_CHECK("nq_pf_plan");
     return 0;
 }
@@ -405,14 +430,13 @@ struct PfGemm
     const _Float16* A0; const _Float16* A1;         // activations in B-operand order: A0 for weight rows < I (or all rows of down), A1 above
     float* C; int mode, E, H, I;
     int solo;                                       // the other kernel variant will not be launched on these tiles: a tile that is its kind comes out NaN
-    const u32x4* Wop;                               // decoded weights of hot experts in A-operand order (nq_pf_wdecode_k), or null
+    int wide;                                       // tiles of experts with decoded weights (fourth word > 0) are nq_pf_wide_k's
 };
 
 // ---- decoded-weight scratch of hot experts --------------------------------------------------------------------------------
 // An expert with many pair rows is cut into several 256-row tiles, and every tile's workgroups would decode the expert again.
-// Such experts are decoded once per call instead, into fp16 scratch laid out exactly as the grouped GEMM holds weights in
-// registers: for strip pair sp (32 weight rows), chunk c, MFMA (mm, rho) one 1 KB block of 64 lanes x 16 bytes, the A operand of
-// that MFMA. A tile of a hot expert then loads its operands (coalesced, 16 bytes per lane) where the others decode.
+// Such experts are decoded once per call instead, into fp16 scratch laid out as MFMA A operands: for strip pair sp (32 weight rows),
+// chunk c, MFMA (mm, rho) one 1 KB block of 64 lanes x 16 bytes. nq_pf_wide_k multiplies them.
 // Slot k of the scratch holds gate|up ([2I / 32][H / 128][8] blocks) followed by down ([H / 32][I / 128][8] blocks).
 __device__ __forceinline__ size_t wop_base(int slot, int mode, int H, int I)
 {   // in 16-byte units
@@ -420,27 +444,27 @@ __device__ __forceinline__ size_t wop_base(int slot, int mode, int H, int I)
     return (size_t)slot * (gu + dn) + (mode ? gu : 0);
 }
 
+// chunks c0 .. c1 - 1 of one strip pair; dst: the strip pair's blocks
 template <bool RES, int CODE>
-__device__ __forceinline__ void wdecode_chunks(const Planes& P, const LaneCtx& L, int C, u32x4* dst, int lane)
+__device__ __forceinline__ void wdecode_chunks(const Planes& P, const LaneCtx& L, int c0, int c1, u32x4* dst, int lane)
 {
     constexpr int NW = RES ? Rec<CODE>::NW : 1;
-    u32x4 nb = load_base<0>(P, L.rec0, L.nrec);
+    u32x4 nb;
     uint32_t nr[NW + 2] = {0}, ndw = 0, nvar = 0;
-    if constexpr (RES) { load_record<CODE>(nr, P.res, L.rec0, L.nrec); ndw = at_offset<uint32_t>((gp_u8)P.dw, L.unit0 * 4u); }
-    if (P.var) nvar = at_offset<uint8_t>(P.var, L.unit0);
-    for (int c = 0; c < C; ++c)
+    auto request = [&](int c) {
+        nb = load_base<0>(P, L.rec0 + (uint32_t)c * 32, L.nrec);
+        if constexpr (RES) { load_record<CODE>(nr, P.res, L.rec0 + (uint32_t)c * 32, L.nrec); ndw = at_offset<uint32_t>((gp_u8)P.dw, (L.unit0 + c) * 4u); }
+        if (P.var) nvar = at_offset<uint8_t>(P.var, L.unit0 + c);
+    };
+    request(c0);
+    for (int c = c0; c < c1; ++c)
     {
         uint32_t wb[6], wr[NW + 2];
         wb[0] = nb.x; wb[1] = nb.y; wb[2] = nb.z; wb[3] = nb.w;
 #pragma unroll
         for (int i = 0; i < NW; ++i) wr[i] = nr[i];
         const uint32_t dw = ndw, var = nvar;
-        if (c + 1 < C)
-        {
-            nb = load_base<0>(P, L.rec0 + (uint32_t)(c + 1) * 32, L.nrec);
-            if constexpr (RES) { load_record<CODE>(nr, P.res, L.rec0 + (uint32_t)(c + 1) * 32, L.nrec); ndw = at_offset<uint32_t>((gp_u8)P.dw, (L.unit0 + c + 1) * 4u); }
-            if (P.var) nvar = at_offset<uint8_t>(P.var, L.unit0 + c + 1);
-        }
+        if (c + 1 < c1) request(c + 1);
         ext_base<0>(wb, __shfl(wb[0], L.src));
         const uint32_t sgm = ((var >> L.g) & 1u) * 0x80008000u;
         FoldK k;
@@ -455,12 +479,23 @@ __device__ __forceinline__ void wdecode_chunks(const Planes& P, const LaneCtx& L
     }
 }
 
-// grid (N / 128, E), block 256: block (x, e) decodes 128 weight rows of expert e if it has a scratch slot (hot[e] >= 0) and its
-// row is of the common kind (K = 2 base plane, no mask-mode flags; others keep decoding inside the GEMM, whatever hot[] says)
-__global__ void __launch_bounds__(256) nq_pf_wdecode_k(const int64_t* table, const int32_t* hot, int mode, u32x4* Wop, int H, int I)
+// grid (N / 128, k-slices, slots), block 256: 128 weight rows x WDEC_CHUNKS chunks of the expert with scratch slot blockIdx.z, if its row is
+// of the common kind (K = 2 base plane, no mask-mode flags; others keep decoding inside the GEMM, whatever hot[] says). Bound by its writes:
+// 16 experts' down projections 89 us = 4.5 TB/s (a whole row of chunks per wavefront: 126 us, too few in flight); gate|up beside other launches 3.5 TB/s.
+// tiles (may be null): the number of tiles of decoded weights.
+constexpr int WDEC_CHUNKS = 8;
+__global__ void __launch_bounds__(256) nq_pf_wdecode_k(const int64_t* table, const int32_t* hot, int E, const int32_t* tiles, int mode, u32x4* Wop, int H, int I)
 {
-    const int e = blockIdx.y, slot = hot[e];
-    if (slot < 0) return;
+    const int slot = blockIdx.z;
+    if (tiles && *tiles == 0) return;                            // no tile of decoded weights
+    int e = -1;
+    for (int i0 = 0; i0 < E && e < 0; i0 += 64)                  // every wavefront looks for itself
+    {
+        const int i = i0 + (threadIdx.x & 63);
+        const unsigned long long m = __ballot(i < E && hot[i] == slot);
+        if (m) e = i0 + __ffsll((long long)m) - 1;
+    }
+    if (e < 0) return;
     const int64_t* ent = table + (size_t)e * TBL_W;
     const int lv = (int)ent[0];
     if (lv <= 0) return;
@@ -468,6 +503,7 @@ __global__ void __launch_bounds__(256) nq_pf_wdecode_k(const int64_t* table, con
     if (P.bcode != 0 || P.flags != nullptr) return;
     const int lane = threadIdx.x & 63, warp = threadIdx.x >> 6;
     const int N = mode == 0 ? 2 * I : H, K = mode == 0 ? H : I, C = K / 128;
+    const int c0 = blockIdx.y * WDEC_CHUNKS, c1 = min(C, c0 + WDEC_CHUNKS);
     const int sp = blockIdx.x * 4 + warp, t4 = lane >> 4, ss = (lane >> 3) & 1, g = lane & 7;
     LaneCtx L;
     L.unit0 = (uint32_t)(2 * sp + ss) * C; L.rec0 = L.unit0 * 32 + 4 * g + t4;
@@ -475,18 +511,147 @@ __global__ void __launch_bounds__(256) nq_pf_wdecode_k(const int64_t* table, con
     L.src = (lane + 16) & 63; L.g = g; L.xs = nullptr; L.xstep = 0;
     L.strip = (uint32_t)(2 * sp + ss); L.nstrips = (size_t)(N / 16); L.chunk0 = 0;
     u32x4* dst = Wop + wop_base(slot, mode, H, I) + (size_t)sp * C * 8 * 64;
-    if (lv == 2) wdecode_chunks<false, 0>(P, L, C, dst, lane);
-    else dispatch_code(P.code, [&](auto tag) { wdecode_chunks<true, decltype(tag)::value>(P, L, C, dst, lane); });
+    if (lv == 2) wdecode_chunks<false, 0>(P, L, c0, c1, dst, lane);
+    else dispatch_code(P.code, [&](auto tag) { wdecode_chunks<true, decltype(tag)::value>(P, L, c0, c1, dst, lane); });
 }
 
-int launch_pf_wdecode(const int64_t* table, const int32_t* hot, int E, int mode, void* Wop, int H, int I, hipStream_t st)
+int launch_pf_wdecode(const int64_t* table, const int32_t* hot, int E, const int32_t* tiles, int mode, void* Wop, int slots, int H, int I, hipStream_t st)
 {
-    const int N = mode == 0 ? 2 * I : H;
-    nq_pf_wdecode_k<<<dim3(N / 128, E), 256, 0, st>>>(table, hot, mode, (u32x4*)Wop, H, I);
+    const int N = mode == 0 ? 2 * I : H, C = (mode == 0 ? H : I) / 128;
+    nq_pf_wdecode_k<<<dim3(N / 128, (C + WDEC_CHUNKS - 1) / WDEC_CHUNKS, slots), 256, 0, st>>>(table, hot, E, tiles, mode, (u32x4*)Wop, H, I);
     NQ_LAUNCH_CHECK("nq_pf_wdecode");
     return 0;
 }
 
+// ---- grouped GEMM over decoded weights --------------------------------------------------------------------------------------
+struct PfWide
+{
+    const int64_t* table; const int32_t* tiles; const int32_t* count;      // count: tiles in the list, or null: `ntiles`
+    const _Float16* A0; const _Float16* A1; float* C; const u32x4* Wop; int mode, E, H, I, ntiles;
+};
+constexpr int WIDE_GRID = 512;                                  // workgroups, one per CU at a time; most steps have fewer units than they might
+constexpr int WIDE_STAGES = 4, WIDE_GROUP = 4;                   // stages of 32 columns in LDS; tiles that share column blocks at a time
+constexpr uint32_t WIDE_HALF = 16384, WIDE_STAGE = 2 * WIDE_HALF; // LDS bytes of a stage: weights, then tokens
+
+// 64 lanes x 16 bytes from base + off to LDS from `at` on (twice: and the next 1 KB of both). The offset of an instruction counts on both
+// sides. Asm, because the compiler would wait for these loads before every LDS read that it cannot tell apart from them.
+__device__ __forceinline__ void to_lds(const void* base, uint32_t off, uint32_t at)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(at), "v"(off), "s"(base) : "memory", "m0");
+}
+__device__ __forceinline__ void to_lds2(const void* base, uint32_t off, uint32_t at)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\tglobal_load_lds_dwordx4 %1, %2 offset:1024" :: "s"(at), "v"(off), "s"(base) : "memory", "m0");
+}
+__device__ __forceinline__ half8_t from_lds(uint32_t at) { return *(const __attribute__((address_space(3))) half8_t*)(uintptr_t)at; }
+// slot of a token row's four 16-byte columns of a stage: q ^ wide_swizzle(row), without bank conflicts for the operand reads
+__device__ __forceinline__ int wide_swizzle(int row) { return ((row >> 2) & 1) * 2 ^ ((row >> 3) & 1) * 3; }
+
+__device__ __forceinline__ void wide_unit(const PfWide& a, int unit, int nt, int ncol, int nb, char* smem)
+{
+    const int grp = unit / (WIDE_GROUP * ncol), in = unit - grp * WIDE_GROUP * ncol, gt = min(WIDE_GROUP, nt - WIDE_GROUP * grp);
+    const int bx = in / gt, t = WIDE_GROUP * grp + in % gt;
+    const int e = a.tiles[4 * t], row0 = a.tiles[4 * t + 1], nrows = a.tiles[4 * t + 2], slot = a.tiles[4 * t + 3] - 1;
+    if (e < 0 || e >= a.E || nrows <= 0 || slot < 0) return;
+    const int64_t* ent = a.table + (size_t)e * TBL_W;
+    if ((int)ent[0] <= 0) return;
+    const Planes P = planes_of(ent, a.mode);
+    if (P.bcode != 0 || P.flags != nullptr) return;              // decoded inside nq_pf_gemm_k
+    const int N = a.mode == 0 ? 2 * a.I : a.H, K = a.mode == 0 ? a.H : a.I, S = K / 32;
+    const bool upper = a.mode == 0 && bx >= nb;                  // the up half has activations of its own
+    const int w0 = a.mode == 0 ? (upper ? a.I + 256 * (bx - nb) : 256 * bx) : 256 * bx;
+    const int mrows = min(256, (a.mode == 0 ? (upper ? 2 * a.I : a.I) : a.H) - w0);       // 128 or 256
+    const int lane = threadIdx.x & 63, warp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t4 = lane >> 4, n = lane & 15;
+    const int wm = warp & 1, wn = warp >> 1;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
+    // wavefront w brings strip pair w (beyond the block: the last one again) and pair rows 32 w .. 32 w + 31 (beyond the tile: its last row again)
+    const char* wsrc = (const char*)(a.Wop + wop_base(slot, a.mode, a.H, a.I)) + (size_t)(w0 / 32 + min(warp, mrows / 32 - 1)) * S * 2048;
+    const char* tsrc = (const char*)((upper ? a.A1 : a.A0) + (size_t)row0 * K);
+    const uint32_t woff = lane * 16;
+    uint32_t toff[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+        toff[q] = (uint32_t)min(32 * warp + 16 * q + (lane >> 2), nrows - 1) * K * 2 + (uint32_t)(((lane & 3) ^ wide_swizzle(lane >> 2)) * 16);
+    auto fetch = [&](int s, uint32_t stage) {                    // stages beyond the last repeat it, so that every wait below counts the same loads
+        s = s < S ? s : S - 1;
+        to_lds2(wsrc + (size_t)s * 2048, woff, stage + warp * 2048);
+#pragma unroll
+        for (int q = 0; q < 2; ++q) to_lds(tsrc + (size_t)s * 64, toff[q], stage + WIDE_HALF + warp * 2048 + q * 1024);
+    };
+    float4_t acc[8][4];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
+    const uint32_t aoff = wm * 8192 + lane * 16, boff = WIDE_HALF + (64 * wn + n) * 64 + ((t4 ^ wide_swizzle(n)) << 4);
+#pragma unroll
+    for (int s = 0; s < WIDE_STAGES - 1; ++s) fetch(s, lds0 + s * WIDE_STAGE);
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" :: "n"(4 * (WIDE_STAGES - 2)) : "memory");
+    if (warp >= 4) asm volatile("s_barrier" ::: "memory");       // half a stage behind from here on; wavefronts 0 .. 3 make up for it at the end
+    uint32_t cur = lds0, prev = lds0 + (WIDE_STAGES - 1) * WIDE_STAGE;
+    for (int s = 0; s < S; ++s)
+    {
+        half8_t A[8], B[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) B[j] = from_lds(cur + boff + j * 1024);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) A[i] = from_lds(cur + aoff + i * 1024);
+        fetch(s + WIDE_STAGES - 1, prev);                        // everybody has read stage s - 1
+        // this wavefront's share of stage s + 1 has landed, and its operands of stage s are in registers
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(4 * (WIDE_STAGES - 2)) : "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[i], B[j], acc[i][j], 0, 0, 0);
+        __builtin_amdgcn_s_setprio(0);
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_barrier" ::: "memory");
+        prev = cur;
+        cur = cur + WIDE_STAGE == lds0 + WIDE_STAGES * WIDE_STAGE ? lds0 : cur + WIDE_STAGE;
+    }
+    if (warp < 4) asm volatile("s_barrier" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");  // the repeated loads have landed: LDS is free for the next unit, or for somebody else
+    if (128 * wm >= mrows) return;
+    // lane (t4, n) holds, for pair row 16 j + n, weight rows 32 (i / 2) + 8 (i & 1) + 16 (t4 >> 1) + 4 (t4 & 1) + 0 .. 3
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+    {
+        const int tok = 64 * wn + 16 * j + n;
+        if (tok >= nrows) continue;
+        float* c = a.C + (size_t)(row0 + tok) * N + w0 + 128 * wm + 16 * (t4 >> 1) + 4 * (t4 & 1);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) *(float4_t*)(c + 32 * (i >> 1) + 8 * (i & 1)) = acc[i][j];
+    }
+}
+// The tiles of experts whose weights nq_pf_wdecode_k has laid out. A unit = 256 weight rows x a tile of at most 256 pair rows, one workgroup of
+// eight wavefronts, each 128 weight rows x 64 pair rows (128 accumulators). Both operands pass through LDS in stages of 32 columns (one MFMA deep),
+// requested three stages ahead. Wavefronts w and w + 4 share a SIMD and work half a stage apart: one multiplies while the other reads its
+// operands and requests the next stage, so the matrix pipe always has a wavefront with its operands at hand (without that, all eight reading ahead
+// in step: 126 instead of 110 us for 64 units of 6144 columns on an otherwise idle GPU). Products and their order are those of the decode-fused
+// tiles, so are the bits. With all CUs at work it is bound by the power limit: 16 experts of 2048 rows, 6144 x 2048, gate|up 1.54 ms and down 0.88 =
+// 1070 / 940 TFLOP/s at 1.4 GHz, whatever the order of products, the number of stages or of wavefronts, as 32 x 32 products 6 % slower (the same
+// bits); 18.9 us per 256 rows, where a decode-fused tile takes 29.5 at level 4 and 23 at level 2. Its weights have to be decoded first: 17 us an expert.
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) nq_pf_wide_k(PfWide a)
+{
+    extern __shared__ __align__(16) char smem[];
+    const int nb = (a.I + 255) / 256, ncol = a.mode == 0 ? 2 * nb : (a.H + 255) / 256;
+    // An XCD works through a run of neighbouring units: WIDE_GROUP tiles by one column block after the other
+    const int nt = a.count ? *a.count : a.ntiles, units = nt * ncol, per = (units + 7) / 8, first = (int)(blockIdx.x & 7) * per;
+    for (int unit = first + (int)(blockIdx.x >> 3); unit < min(units, first + per); unit += (int)gridDim.x >> 3)
+        wide_unit(a, unit, nt, ncol, nb, smem);
+}
+
+static int launch_wide(const PfWide& a, int most, hipStream_t st)
+{
+    const int shm = WIDE_STAGES * WIDE_STAGE, ncol = a.mode == 0 ? 2 * ((a.I + 255) / 256) : (a.H + 255) / 256;
+    const hipError_t e = hipFuncSetAttribute((const void*)nq_pf_wide_k, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
+    if (e != hipSuccess) return set_error("nq_pf_wide: LDS %d bytes: %s", shm, hipGetErrorString(e));
+    nq_pf_wide_k<<<(int)std::min<int64_t>(WIDE_GRID, ((int64_t)most * ncol + 7) / 8 * 8), 512, shm, st>>>(a);
+    NQ_LAUNCH_CHECK("nq_pf_wide");
+    return 0;
+}
 
 // The MFMA phase of one chunk: TG x 8 MFMAs, tokens 16 tg + n as the N dimension (row groups beyond the tile multiply stale
 // LDS rows whose results are never stored). Two row groups are interleaved so that four different accumulators separate an
@@ -548,38 +713,6 @@ __device__ __forceinline__ void pf_stage_tokens(const _Float16* A, int K, int ro
         uint32_t off = lane_off + (uint32_t)u * ustep;
         off = 16 * u + srow < nrows ? off : last_off;
         __builtin_amdgcn_global_load_lds((gvp)(base + off), (lvp)(smem + (16 * u + 4 * warp) * PF_ROW), 16, 0, 0);
-    }
-}
-
-// body for a tile of a hot expert: the A operands of this wavefront's two strips come from the decoded-weight scratch
-// (w: this strip pair's blocks, [C][8][64] x 16 bytes), one chunk ahead of the MFMAs that use them
-template <int TG>
-__device__ __forceinline__ void pf_chunks_pre(const u32x4* w, int C, const _Float16* A, int K, int row0, int nrows, char* smem, float4_t (*acc)[2])
-{
-    const int lane = threadIdx.x & 63, warp = threadIdx.x >> 6, t4 = lane >> 4, n = lane & 15;
-    const int srow = 4 * warp + t4;
-    const uint32_t scol = (uint32_t)((n ^ srow) * 16);
-    uint32_t boff[4];
-#pragma unroll
-    for (int mm = 0; mm < 4; ++mm) boff[mm] = (uint32_t)(n * PF_ROW + (((4 * mm + t4) ^ n) << 4));
-    u32x4 nx[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) nx[i] = w[(size_t)i * 64 + lane];
-    for (int c = 0; c < C; ++c)
-    {
-        pf_stage_tokens<TG>(A, K, row0, nrows, c, smem, warp, srow, scol);
-        half8_t aop[4][2];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) aop[i >> 1][i & 1] = __builtin_bit_cast(half8_t, nx[i]);
-        if (c + 1 < C)
-        {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) nx[i] = w[((size_t)(c + 1) * 8 + i) * 64 + lane];
-        }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");         // the tokens have landed (and the next chunk's operands, requested with them)
-        __syncthreads();
-        pf_mfmas<TG>(aop, smem, boff, acc);
-        __syncthreads();
     }
 }
 
@@ -698,6 +831,7 @@ __device__ __forceinline__ void pf_tile(const PfGemm& a, int bx, int e, int row0
     const _Float16* A = (a.mode == 0 && bx * 128 >= a.I) ? a.A1 : a.A0;
     const int t4 = lane >> 4, ss = (lane >> 3) & 1, g = lane & 7, n = lane & 15;
     const Planes P = planes_of(ent, a.mode);
+    if (!MASKED && a.wide && slot >= 0 && P.bcode == 0 && P.flags == nullptr) return;        // block-uniform: nq_pf_wide_k's tile
     if (((P.flags != nullptr && lv == 4) || P.bcode != 0) != MASKED)              // block-uniform: the other variant's tile
     {
         if (a.solo)
@@ -718,10 +852,7 @@ __device__ __forceinline__ void pf_tile(const PfGemm& a, int bx, int e, int row0
     for (int tg = 0; tg < TG; ++tg) { acc[tg][0] = float4_t{0.f, 0.f, 0.f, 0.f}; acc[tg][1] = float4_t{0.f, 0.f, 0.f, 0.f}; }
     if constexpr (!MASKED)
     {
-        // a hot expert (several tiles): its weights were decoded once into the scratch by nq_pf_wdecode_k (block-uniform)
-        const bool pre = a.Wop != nullptr && slot >= 0 && P.flags == nullptr;
-        if (pre) pf_chunks_pre<TG>(a.Wop + wop_base(slot, a.mode, a.H, a.I) + (size_t)sp * C * 8 * 64, C, A, K, row0, nrows, smem, acc);
-        else if (lv == 2) pf_chunks<TG, false, 0, false>(P, L, C, A, K, row0, nrows, smem, acc);
+        if (lv == 2) pf_chunks<TG, false, 0, false>(P, L, C, A, K, row0, nrows, smem, acc);
         else dispatch_code(P.code, [&](auto tag) { pf_chunks<TG, true, decltype(tag)::value, false>(P, L, C, A, K, row0, nrows, smem, acc); });
     }
     else
@@ -938,10 +1069,10 @@ static int launch_gemm_tg(const PfGemm& a, int ntiles, int N, hipStream_t st)
 }
 
 int launch_pf_gemm(const int64_t* table, const int32_t* tiles, int ntiles, int bm, int mode, const void* A0, const void* A1, float* C,
-                   int E, int H, int I, const void* Wop, hipStream_t st)
+                   int E, int H, int I, int wide, hipStream_t st)
 {
     if (!ntiles) return 0;
-    PfGemm a{table, tiles, (const _Float16*)A0, (const _Float16*)A1, C, mode & 1, E, H, I, (mode & 4) != 0, (const u32x4*)Wop};
+    PfGemm a{table, tiles, (const _Float16*)A0, (const _Float16*)A1, C, mode & 1, E, H, I, (mode & 4) != 0, wide};
     const int N = (mode & 1) == 0 ? 2 * I : H;
     const bool masked = (mode & 2) != 0;
     switch (bm)
@@ -955,9 +1086,15 @@ int launch_pf_gemm(const int64_t* table, const int32_t* tiles, int ntiles, int b
     return set_error("nq_pf_gemm: tile height %d not in {16, 32, 64, 128, 256}", bm);
 }
 
+int launch_pf_wide(const int64_t* table, const int32_t* tiles, int ntiles, int mode, const void* A0, const void* A1, float* C, int E, int H, int I, const void* Wop, hipStream_t st)
+{
+    if (!ntiles) return 0;
+    return launch_wide(PfWide{table, tiles, nullptr, (const _Float16*)A0, (const _Float16*)A1, C, (const u32x4*)Wop, mode & 1, E, H, I, ntiles}, ntiles, st);
+}
+
 // ---- a whole step --------------------------------------------------------------------------------------------------------
-// Bytes of the int32 scratch of a step: cnt [E] | pe [P] | pt [P] | pos [P] | hot [E] | tile lists, each on 16 bytes.
-struct PfMeta { int32_t *cnt, *pe, *pt, *pos, *hot, *tiles; int cap, scap; size_t bytes; };
+// Bytes of the int32 scratch of a step: cnt [E] | pe [P] | pt [P] | pos [P] | hot [E] | tile lists | tiles of decoded weights, each on 16 bytes.
+struct PfMeta { int32_t *cnt, *pe, *pt, *pos, *hot, *tiles, *wide; int cap, scap; size_t bytes; };
 static PfMeta pf_meta(void* ws, int P, int R, int E)
 {
     PfMeta m;
@@ -965,7 +1102,7 @@ static PfMeta pf_meta(void* ws, int P, int R, int E)
     auto take = [&](size_t n) { int32_t* p = (int32_t*)((char*)ws + off); off += (n * 4 + 15) & ~(size_t)15; return p; };
     m.cap = E + R / 256 + 1; m.scap = E + P / SHORT_ROWS + 1;
     m.cnt = take(E); m.pe = take(P); m.pt = take(P); m.pos = take(P); m.hot = take(E);
-    m.tiles = take(4 * (size_t)(5 * m.cap > m.scap ? 5 * m.cap : m.scap));
+    m.tiles = take(4 * (size_t)(5 * m.cap > m.scap ? 5 * m.cap : m.scap)); m.wide = take(4 * ((size_t)m.cap + 1));
     m.bytes = off;
     return m;
 }
@@ -983,6 +1120,16 @@ static PfMeta pf_meta(void* ws, int P, int R, int E)
 // 1400 / 1760, 2000 tokens 2498 / 2158 and 2466 / 2478.
 static bool pf_is_short(int64_t P, int E, int H, int I, bool fork) { return P <= 32 * (int64_t)E || P * H * I <= (int64_t)1 << (fork ? 34 : 36); }
 
+// Which experts take decoded weights: at least WIDE_MIN rows (three tiles), above level 2, if their tiles make WIDE_UNITS units of gate|up
+// together (two per CU; the plan counts them). us a step without / from 512 / 768 / 1024 rows on (6144 x 2048, top-8, level 4): 4096 tokens, 256
+// experts, Zipf 5743 / 5679 / 5609 / 5688; 32 experts, evenly 3976 / 3776 / 3735 / 3869; 16 experts, Zipf 3910 / 3459 / 3481 / 3647;
+// 2000 tokens, 16 experts, evenly 1997 / 1830 / 1847 / 2048. At level 2, where a tile's decode is half as long, 16 experts of 2048 rows lose: 3173 / 3281.
+// Fewer units leave CUs idle for the 0.2 ms of one: 1000 tokens, 16 experts, Zipf (a single expert of 993 rows) 1070 / 1173.
+// A block of 128 weight rows costs what one of 256 does: 2304 + 4096 rows, 11 % of them padding in gate|up, 1922 / 1961. Scratch: 2 GB at most.
+constexpr int WIDE_MIN = 768, WIDE_UNITS = 512;
+constexpr int64_t WIDE_BYTES = (int64_t)1 << 31;
+static int wide_tiles(int I) { const int ncol = 2 * ((I + 255) / 256); return (WIDE_UNITS + ncol - 1) / ncol; }
+
 template <bool MASKED>
 static int launch_short(const PfGemm& a, int ntiles, int N, hipStream_t st)
 {
@@ -994,6 +1141,8 @@ static int launch_short(const PfGemm& a, int ntiles, int N, hipStream_t st)
 int launch_pf_step(const NqPfArgs& a, hipStream_t st)
 {
     const int P = a.T * a.topk, R = a.rows < P ? a.rows : P, E = a.E, H = a.H, I = a.I;
+    const int variants = a.variants & 3;
+    const bool advised = a.variants & 4;
     const PfMeta m = pf_meta(a.meta, P, R, E);
     if (m.bytes > (size_t)a.meta_bytes) return set_error("nq_pf_step: meta needs %zu bytes, has %lld", m.bytes, (long long)a.meta_bytes);
     const bool fork = a.side[0] != nullptr, brief = R == P && !a.wop && pf_is_short(P, E, H, I, fork);
@@ -1015,10 +1164,10 @@ int launch_pf_step(const NqPfArgs& a, hipStream_t st)
         if (int rc = launch_pf_pre(a.x, a.x_dtype, m.pt, m.pe, P, a.table, a.xg, a.xu, a.zg, E, H, I, nullptr, 0, 0, st)) return rc;
         for (int mode = 0; mode < 2; ++mode)
         {
-            const PfGemm g{a.table, m.tiles, (const _Float16*)(mode ? a.h : a.xg), (const _Float16*)(mode ? nullptr : a.xu), mode ? y : acc, mode, E, H, I, a.variants == 1, nullptr};
+            const PfGemm g{a.table, m.tiles, (const _Float16*)(mode ? a.h : a.xg), (const _Float16*)(mode ? nullptr : a.xu), mode ? y : acc, mode, E, H, I, variants == 1, 0};
             const int N = mode ? H : 2 * I;
-            if (a.variants & 1) if (int rc = launch_short<false>(g, m.scap, N, st)) return rc;
-            if (a.variants & 2) if (int rc = launch_short<true>(g, m.scap, N, st)) return rc;
+            if (variants & 1) if (int rc = launch_short<false>(g, m.scap, N, st)) return rc;
+            if (variants & 2) if (int rc = launch_short<true>(g, m.scap, N, st)) return rc;
             if (mode == 0) if (int rc = launch_pf_mid(acc, m.pe, P, a.table, a.h, a.zg, a.zd, E, H, I, nullptr, 0, 0, st)) return rc;
         }
         return launch_pf_post(y, m.pos, a.sel, a.sel_dtype, a.rw, a.rw_dtype, a.T, a.topk, 0, P, a.table, a.out, a.out_dtype, 0, a.zd, E, H, I, st);
@@ -1035,9 +1184,8 @@ int launch_pf_step(const NqPfArgs& a, hipStream_t st)
     {
         const int n = P - c < R ? P - c : R;
         const bool wop = a.wop && n >= a.hot_min;
-        if (int rc = launch_pf_plan(m.cnt, E, c, n, m.tiles, m.cap, wop ? m.hot : nullptr, a.hot_min, a.wop_slots, st)) return rc;
-        for (int mode = 0; wop && mode < 2; ++mode)
-            if (int rc = launch_pf_wdecode(a.table, m.hot, E, mode, a.wop, H, I, st)) return rc;
+        if (int rc = launch_pf_plan(m.cnt, E, c, n, m.tiles, m.cap, wop ? m.hot : nullptr, a.hot_min, a.wop_slots, wop ? m.wide : nullptr, advised ? wide_tiles(I) : 0, advised ? a.table : nullptr, st)) return rc;
+        const int most = std::min(m.cap, n / 256 + a.wop_slots / 2 + 1);       // tiles of decoded weights: an expert of r rows has (r + 127) / 256
         if (fork) if (int rc = hip_ok(hipEventRecord((hipEvent_t)a.events[0], st))) return rc;
         for (int i = 1; fork && i < 4; ++i) if (int rc = hip_ok(hipStreamWaitEvent(streams[i], (hipEvent_t)a.events[0], 0))) return rc;
         const int32_t *pts = m.pt + c, *pes = m.pe + c;
@@ -1045,9 +1193,13 @@ int launch_pf_step(const NqPfArgs& a, hipStream_t st)
         auto gemms = [&](int mode) {
             for (int k = 4; k >= 0; --k)
                 for (int v = 0; v < 2; ++v)
-                    if (a.variants >> v & 1)
-                        if (int rc = launch_pf_gemm(a.table, m.tiles + (size_t)k * m.cap * 4, k < 4 ? E : m.cap, 16 << k, mode | 2 * v | (a.variants == 1 ? 4 : 0), mode ? a.h : a.xg,
-                                                    mode ? nullptr : a.xu, mode ? y : acc, E, H, I, wop ? a.wop : nullptr, streams[stream_of[k]])) return rc;
+                    if (variants >> v & 1)
+                        if (int rc = launch_pf_gemm(a.table, m.tiles + (size_t)k * m.cap * 4, k < 4 ? E : m.cap, 16 << k, mode | 2 * v | (variants == 1 ? 4 : 0), mode ? a.h : a.xg,
+                                                    mode ? nullptr : a.xu, mode ? y : acc, E, H, I, wop, streams[stream_of[k]])) return rc;
+            if (wop) if (int rc = launch_pf_wdecode(a.table, m.hot, E, m.wide, mode, a.wop, a.wop_slots, H, I, st)) return rc;
+            if (wop)
+                if (int rc = launch_wide(PfWide{a.table, m.wide + 4, m.wide, (const _Float16*)(mode ? a.h : a.xg), (const _Float16*)(mode ? nullptr : a.xu), mode ? y : acc, (const u32x4*)a.wop,
+                                                mode, E, H, I, 0}, most, st)) return rc;
             return 0;
         };
         auto chains = [&]() {
@@ -1068,6 +1220,14 @@ int launch_pf_step(const NqPfArgs& a, hipStream_t st)
         if (int rc = launch_pf_post(y, m.pos, a.sel, a.sel_dtype, a.rw, a.rw_dtype, a.T, a.topk, c, n, a.table, a.out, a.out_dtype, c != 0, a.zd, E, H, I, st)) return rc;
     }
     return 0;
+}
+
+int pf_wide_slots(int T, int P, int R, int E, int H, int I, bool fork, int* hot_min)
+{
+    *hot_min = WIDE_MIN;
+    const int64_t real = (int64_t)3 * H * I, padded = (int64_t)512 * ((I + 255) / 256) * H + (int64_t)256 * ((H + 255) / 256) * I;
+    if (T < WIDE_MIN || R / 256 < wide_tiles(I) || 20 * padded > 21 * real || (R == P && pf_is_short(P, E, H, I, fork))) return 0;
+    return (int)std::min<int64_t>(std::min(E, R / WIDE_MIN), WIDE_BYTES / ((int64_t)6 * H * I));
 }
 
 int64_t pf_meta_bytes(int P, int R, int E) { return (int64_t)pf_meta(nullptr, P, R, E).bytes; }

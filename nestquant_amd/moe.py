@@ -310,11 +310,9 @@ class MoELayer:
 
 
 PF_TILES = (16, 32, 64, 128, 256)            # token-tile heights the grouped GEMM is compiled for
-# An expert with at least PF_HOT_MIN pair rows in a chunk (more than one 256-row tile) can be decoded once per call into a scratch
-# of decoded weights (at most PF_HOT_SLOTS experts at 6 H I bytes each) instead of once per tile; see nq_pf_wdecode. Off by
-# default (0 slots): a tile then reads 75 MB of fp16 operands from HBM where the decode-fused kernel reads 12.6 MB of codes, and
-# on the 4096-token benchmark the call takes 6.22 ms with 32 slots against 6.06 without (the tiles save 0.6 ms of their own
-# time, the decode launches cost 0.61) plus 2.4 GB of scratch. Same bits either way.
+# Experts with many pair rows can be decoded once per call into a scratch of decoded weights (6 H I bytes each), whose tiles a GEMM of
+# their own multiplies, instead of once per tile; see nq_pf_wdecode. Same bits either way. With PF_HOT_SLOTS = 0 the library says for which
+# steps and experts (nq_pf_wide_slots); > 0: every expert of at least PF_HOT_MIN rows, at most this many; < 0: none.
 PF_HOT_MIN, PF_HOT_SLOTS = 257, 0
 
 
@@ -346,7 +344,7 @@ def pf_scratch(dev, H, I, R, G=0):
     [R, H], the low-rank plane's zg | zd fp32 [R, 4], and wop: decoded weights of up to PF_HOT_SLOTS hot experts (None without).
     A set belongs to whoever asks for it, and every step takes one of its own from torch's allocator: what another layer, stream
     or thread has in flight, or a captured graph holds, is never shared. Unlike the reference (sm120/moe.py:262-274), which
-    keeps one set per device and decodes every expert of a group into it, only experts with more than one tile go through
+    keeps one set per device and decodes every expert of a group into it, only experts with several tiles go through
     decoded weights; the others are decoded in registers inside the grouped GEMM."""
     f16, f32 = torch.float16, torch.float32
     off, size = _pf_offsets(H, I, R)
@@ -404,28 +402,38 @@ def _pf_step(s, x, sel, rw, out, R=None, table=None):
     if nb < 0:
         raise RuntimeError(Lb.nq_last_error().decode())
     # decoded-weight scratch: rows of the common kind only (the variant kernel of the others decodes in the GEMM)
-    slots = _pf_slots(R) if P >= PF_HOT_MIN and not s.rare_rows and table is None else 0
     off, size = _pf_offsets(H, I, R)
     meta_at, wop_at = size, size + -(-nb // 256) * 256
-    # one block per call, the step's own: it goes back to the allocator in the order of the caller's stream, which the side streams join
-    block = torch.empty(wop_at + slots * 6 * H * I, dtype=torch.uint8, device=dev)
     stream = _lib.stream_ptr()
     # a step that is being captured stays on its stream: streams of torch's pool may coincide with one that somebody is using
     held = None if torch.cuda.is_current_stream_capturing() else _pf_side(dev, stream)
+    slots, hot_min, advised = 0, C.c_int32(PF_HOT_MIN), PF_HOT_SLOTS == 0
+    if not s.rare_rows and table is None:            # rows of the common kind only: the variant kernel of the others decodes in the GEMM
+        if advised:
+            slots = Lb.nq_pf_wide_slots(T, k, R, E, H, I, held is not None, C.byref(hot_min))
+        elif P >= PF_HOT_MIN:
+            slots = _pf_slots(R)
+    # one block per call, the step's own: it goes back to the allocator in the order of the caller's stream, which the side streams join
+    try:
+        block = torch.empty(wop_at + slots * 6 * H * I, dtype=torch.uint8, device=dev)
+    except torch.OutOfMemoryError:
+        if slots == 0:
+            raise
+        slots, block = 0, torch.empty(wop_at, dtype=torch.uint8, device=dev)
     whole = out if out.dtype == torch.float32 or R == P else torch.empty(T, H, dtype=torch.float32, device=dev)   # chunks add up in fp32
     a, at = _lib.NqPfArgs(), block.data_ptr()
     a.x, a.sel, a.rw, a.table, a.out, a.hits = x.data_ptr(), sel.data_ptr(), rw.data_ptr(), tb.data_ptr(), whole.data_ptr(), s.hits_ptr or None
     a.meta, a.meta_bytes = at + meta_at, nb
     a.xg, a.xu, a.acc, a.h, a.y, a.zg, a.zd = (at + o for o in off)
     if slots:
-        a.wop, a.wop_bytes, a.wop_slots, a.hot_min = at + wop_at, slots * 6 * H * I, slots, PF_HOT_MIN
+        a.wop, a.wop_bytes, a.wop_slots, a.hot_min = at + wop_at, slots * 6 * H * I, slots, hot_min.value
     if held is not None:
         a.side, a.events = held[2], held[3]
     a.T, a.topk, a.E, a.H, a.I, a.rows = T, k, E, H, I, R
     a.x_dtype, a.sel_dtype, a.rw_dtype, a.out_dtype = _DT_IN[x.dtype], _DT_SEL[sel.dtype], _DT_IN[rw.dtype], _DT_OUT[whole.dtype]
     # mask mode / other base codes run in their own kernel variant; a caller's own table may hold such rows, so it gets both, and
     # a lone variant is told so: should it meet a row of the other kind after all, the result is NaN, not stale scratch
-    a.variants = 3 if (s.rare_rows or table is not None) else 1
+    a.variants = (3 if (s.rare_rows or table is not None) else 1) | (4 if advised else 0)
     _lib.check(Lb.nq_pf_step(C.byref(a), stream))
     return out if whole is out else out.copy_(whole)
 

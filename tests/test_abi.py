@@ -131,6 +131,28 @@ def test_argument_checks_run_before_any_device_work():
     assert L.nq_mailbox(None, base, base, base, None, 4, None) != 0 and "null" in err()
 
 
+def test_which_steps_are_given_decoded_weights():
+    """nq_pf_wide_slots: none for steps of short tiles, of few tokens, of too few tiles to fill the GPU, of shapes that would be padded; no
+    more than 2 GB; nothing for sizes that a step refuses"""
+    L = _lib.lib()
+    m = C.c_int32(0)
+
+    def slots(T, topk, E, H, I, rows=32768, side=1):
+        return L.nq_pf_wide_slots(T, topk, rows, E, H, I, side, C.byref(m))
+    assert slots(4096, 8, 256, 6144, 2048) == 2**31 // (6 * 6144 * 2048) and m.value == 768
+    assert slots(1100, 8, 8, 2048, 2048) == 8
+    assert slots(1024, 8, 8, 2048, 2048) == 8 and slots(1023, 8, 8, 2048, 2048) == 0          # 32 tiles of 256 rows
+    assert slots(767, 64, 8, 6144, 2048) == 0
+    assert slots(1000, 8, 256, 6144, 2048) == 0                  # at most 32 rows per expert on average
+    assert slots(4096, 8, 16, 1024, 512) == 0                    # little work
+    assert slots(4096, 8, 16, 2048, 512, side=0) == 0 and slots(4096, 8, 16, 2048, 512) == 16      # without side streams short tiles go further
+    assert slots(4096, 8, 64, 4096, 1152) == 0 and slots(4096, 8, 64, 4096, 1024) > 0
+    assert slots(4096, 8, 256, 6144, 2048, rows=4096) == 0       # chunks of few rows
+    for bad in ((-1, 8, 16, 2048, 1024), (4096, 0, 16, 2048, 1024), (4096, 8, 0, 2048, 1024), (4096, 8, 16, 2000, 1024), (4096, 8, 16, 2048, 0)):
+        assert slots(*bad) == 0
+    assert L.nq_pf_wide_slots(4096, 8, 32768, 256, 6144, 2048, 1, None) == 0
+
+
 def test_counters_apart_are_asked_for_and_checked():
     """which bit 4 needs NQ_CNT_STEP * H / 128 counters and the down launch; without it H / 128 are enough, and no capacity changes what they mean"""
     L = _lib.lib()

@@ -120,6 +120,59 @@ def test_hot_expert_scratch_gives_the_same_bits():
     assert rel_err(y0.cpu().numpy(), ys.cpu().numpy()) < 5e-5
 
 
+@pytest.mark.parametrize("H,I", [(128, 128), (384, 256), (256, 640), (1024, 512)])        # one chunk; blocks of 128 weight rows; K = 128 .. 1024
+def test_tiles_of_decoded_weights_give_the_bits_of_decode_fused_tiles(H, I):
+    """nq_pf_wdecode_k and nq_pf_wide_k at the edges of their tiles: one row more than a remainder that decodes in its GEMM, full tiles, a
+    row beyond, several tiles; every level, window codes of several record lengths, sign planes; and the same in chunks of pair rows"""
+    rows = [129, 255, 256, 257, 385, 512, 130, 700, 0, 1]
+    rk = [(0, 0), (3, 7), (6, 9), (8, 3), (0, 0), (1, 2), (4, 5), (0, 0), (7, 6), (0, 0)]
+    ex = to_dev(experts_on_gpu(H, I, len(rows), 77, nested_ids=(4, 7, 9), rk=rk, var_ids=(1, 4)))
+    L = M.MoELayer(len(rows), H, I, Bmax=8, topk=1)
+    for e, lv in enumerate([4, 4, 4, 4, 3, 2, 4, 4, 2, 4]):
+        L.set(e, ex[e], lv)
+    g = torch.Generator().manual_seed(78)
+    sel = torch.repeat_interleave(torch.arange(len(rows)), torch.tensor(rows))[torch.randperm(sum(rows), generator=g)].view(-1, 1).to(DEV)
+    rw = (torch.rand(sel.shape, generator=g) + 0.1).half().to(DEV)
+    x = (torch.randn(sel.shape[0], H, generator=g) * 0.05).half().to(DEV)
+    try:
+        M.PF_HOT_SLOTS = -1
+        want = L.prefill(x, sel, rw)
+        for M.PF_HOT_SLOTS, hot_min in ((10, 1), (3, 200)):
+            hot, M.PF_HOT_MIN = M.PF_HOT_MIN, hot_min
+            got = [L.prefill(x, sel, rw, R=R) for R in (None, 600)]
+            M.PF_HOT_MIN = hot
+            torch.cuda.synchronize()
+            assert all(torch.equal(want, y) for y in got), (M.PF_HOT_SLOTS, hot_min)
+    finally:
+        M.PF_HOT_SLOTS, M.PF_HOT_MIN = 0, 257
+    assert want.isfinite().all()
+
+
+def test_a_step_takes_decoded_weights_where_they_pay():
+    """the rule's first step (eight experts of 1100 rows: 32 tiles of a shape whose units are then 512): equal bits with all experts above
+    level 2, and with one below, which leaves too few tiles"""
+    H = I = 2048
+    E, T = 8, 1100
+    assert M._lib.lib().nq_pf_wide_slots(T, 8, 8 * T, E, H, I, 1, M.C.byref(M.C.c_int32())) == E
+    ex = to_dev(experts_on_gpu(H, I, 4, 79, nested_ids=(1, 3)))
+    L = M.MoELayer(E, H, I, Bmax=8, topk=8)
+    g = torch.Generator().manual_seed(80)
+    sel = torch.stack([torch.randperm(E, generator=g) for _ in range(T)]).to(DEV)
+    rw = torch.softmax(torch.randn(T, 8, generator=g), -1).half().to(DEV)
+    x = (torch.randn(T, H, generator=g) * 0.05).half().to(DEV)
+    for levels in ([4, 4, 4, 3, 4, 4, 4, 3], [4, 4, 4, 3, 2, 4, 4, 3]):
+        for e in range(E):
+            L.set(e, ex[e % 4], levels[e])
+        got = L.prefill(x, sel, rw)
+        try:
+            M.PF_HOT_SLOTS = -1
+            want = L.prefill(x, sel, rw)
+        finally:
+            M.PF_HOT_SLOTS = 0
+        torch.cuda.synchronize()
+        assert torch.equal(got, want) and got.isfinite().all()
+
+
 def test_prefill_argument_errors_and_empty():
     L = M.MoELayer(4, 256, 256, Bmax=2, topk=2)
     tb = L.table
