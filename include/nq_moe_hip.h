@@ -330,6 +330,29 @@ int nq_viterbi(const float* w, int T, int L, int K, const float* lut, int64_t* s
  * values lut[spread(a) | spread(b) << 1]; a int64 [T][L]: P3's windows (low eight bits used), b int64 [T][L]: P4's windows. */
 int nq_viterbi_p4(const float* w, const int64_t* a, int T, int L, const float* lut, int64_t* b, int position_order, void* stream);
 
+/* Encoder: what an encode does around its searches (reference nq_encode.py:135-183,206-339). W fp32 [N][K], N and K multiples of 128; units of 16 x 128 by strips,
+ * in ring position order 8 x 256; a column chunk is 128 columns, unit s of it strip s.
+ * nq_enc_prepare: signs int64 [K + N] (0: -1, else +1) -> su fp16 [K], sv fp16 [N] (signed rms per input channel, then per output channel),
+ * target fp32 [N][K] = B (W / su / sv) B with B the 128-blocked orthonormal Hadamard; rings (may be NULL): the same in ring order, fp32
+ * [units][8][256], and with `negated` once more, negated, behind it. ws: K doubles.
+ * nq_enc_hessian: out [K][K] = B D(su) H D(su) B, fp64.
+ * nq_enc_inverse: out [128][128] = inverse of the symmetric positive definite A (rows lda apart); a pivot (of its LDL^T) that is not positive sets *bad,
+ * if it is zero, to order0 + the pivot's number, from one.
+ * nq_enc_targets: T fp64 [levels][N][128] = the chunk of W + fed (same layout, may be NULL); rings: of T alone (levels = 1), or of (1 - lam) T_0 + lam T_1,
+ * with `negated` the same negated, then of T_1 (levels = 2), each N * 128 floats.
+ * nq_enc_base: states int64 of the units' rings, with var also of the negated ones behind them: the orientation of the smaller squared error (the first of
+ * equals) -> own int64 [units][8][256], sign fp32 [units][8]. With W (units = strips of chunk `chunk`; T its targets [16 units][128]) also st_all, sign_all (of all units,
+ * by strip and chunk) and, fp64 [16 units][K] at the chunk's columns, err = W - value and eta = T - value.
+ * nq_enc_feed: states, values Q (ring order) and block words of the chunk's strips to their place among all units, err and eta likewise. */
+int nq_enc_prepare(const float* W, int N, int K, const int64_t* signs, double* ws, void* su_f16, void* sv_f16, float* target, float* rings, int negated, void* stream);
+int nq_enc_hessian(const double* H, int K, const void* su_f16, double* out, void* stream);
+int nq_enc_inverse(const double* A, int lda, double* out, int32_t* bad, int order0, void* stream);
+int nq_enc_targets(const float* W, int N, int K, int chunk, const double* fed, int levels, double lam, double* T, float* rings, int negated, void* stream);
+int nq_enc_base(const int64_t* states, int units, int var, const float* rings, const float* lut, const float* W, const double* T, int K, int chunk, int64_t* own, float* sign,
+                int64_t* st_all, float* sign_all, double* err, double* eta, void* stream);
+int nq_enc_feed(const int64_t* states, const float* Q, const int64_t* Mb, const int64_t* N, const float* W, const double* T, int rows, int K, int chunk, int64_t* st_all,
+                float* Q_all, int64_t* Mb_all, int64_t* N_all, double* err, double* eta, void* stream);
+
 /* Encoder: one refinement stage on a frozen base plane, units of 16 x 128 weights as 8 rings of 256 in ring position order
  * (reference nq_encode.py:186-198,286-316). target fp32 [U][8][256]; sign fp32 [U][8] (+-1 per ring, NULL = +1); st_base, st_res int64
  * [U][8][256] states; lut fp32 [65536] codebook.

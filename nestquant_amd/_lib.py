@@ -81,6 +81,12 @@ SIGNATURES = {
     "nq_pf_hits": (C.c_int, [_i32p, _i32p, _i, _vp]),
     "nq_viterbi": (C.c_int, [_vp, _i, _i, _i, _vp, _vp, _vp, C.c_int64, _i, _vp]),
     "nq_viterbi_p4": (C.c_int, [_vp, _vp, _i, _i, _vp, _vp, _i, _vp]),
+    "nq_enc_prepare": (C.c_int, [_vp, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _vp]),
+    "nq_enc_hessian": (C.c_int, [_vp, _i, _vp, _vp, _vp]),
+    "nq_enc_inverse": (C.c_int, [_vp, _i, _vp, _vp, _i, _vp]),
+    "nq_enc_targets": (C.c_int, [_vp, _i, _i, _i, _vp, _i, C.c_double, _vp, _vp, _i, _vp]),
+    "nq_enc_base": (C.c_int, [_vp, _i, _i, _vp, _vp, _vp, _vp, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "nq_enc_feed": (C.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "nq_fit_residual": (C.c_int, [_vp, _vp, _vp, _vp, C.c_double, _i, _vp, _vp]),
     "nq_fit_words": (C.c_int, [_vp, _vp, _vp, _vp, _vp, _i, _vp, C.c_int64, _vp, C.c_int64, _vp, C.c_int64, _vp, _vp, _vp, _vp, _vp]),
     "nq_fit_pack": (C.c_int, [_vp, _i, _vp, _vp, _vp, _vp, _vp, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp]),

@@ -385,6 +385,52 @@ extern "C" int nq_fit_pack(const int64_t* states, int K, const float* values, co
     return launch_fit_pack(states, K, values, sign, lut, Mb, N, strips * chunks, chunks, words, dw, var, Q, bad, (hipStream_t)stream);
 }
 
+static bool enc_shape_ok(int N, int K) { return N >= 128 && N % 128 == 0 && K >= 128 && K % 128 == 0 && N <= (1 << 23); }
+
+extern "C" int nq_enc_prepare(const float* W, int N, int K, const int64_t* signs, double* ws, void* su, void* sv, float* target, float* rings, int negated, void* stream)
+{
+    NQ_REQUIRE(enc_shape_ok(N, K), "nq_enc_prepare: N=%d K=%d (positive multiples of 128)", N, K);
+    NQ_REQUIRE(W && signs && ws && su && sv && target, "nq_enc_prepare: null pointer");
+    return launch_enc_prepare(W, N, K, signs, ws, su, sv, target, rings, negated, (hipStream_t)stream);
+}
+
+extern "C" int nq_enc_hessian(const double* H, int K, const void* su, double* out, void* stream)
+{
+    NQ_REQUIRE(enc_shape_ok(K, K), "nq_enc_hessian: K=%d (a positive multiple of 128)", K);
+    NQ_REQUIRE(H && su && out, "nq_enc_hessian: null pointer");
+    return launch_enc_hessian(H, K, su, out, (hipStream_t)stream);
+}
+
+extern "C" int nq_enc_inverse(const double* A, int lda, double* out, int32_t* bad, int order0, void* stream)
+{
+    NQ_REQUIRE(A && out && bad && lda >= 128 && order0 >= 0, "nq_enc_inverse: null pointer, lda=%d (at least 128) or order0=%d", lda, order0);
+    return launch_enc_inverse(A, lda, out, bad, order0, (hipStream_t)stream);
+}
+
+extern "C" int nq_enc_targets(const float* W, int N, int K, int chunk, const double* fed, int levels, double lam, double* T, float* rings, int negated, void* stream)
+{
+    NQ_REQUIRE(enc_shape_ok(N, K) && chunk >= 0 && chunk < K / 128 && (levels == 1 || levels == 2), "nq_enc_targets: N=%d K=%d chunk=%d levels=%d (1 or 2)", N, K, chunk, levels);
+    NQ_REQUIRE(W && T && rings && (levels == 2 || !negated), "nq_enc_targets: null pointer, or one level negated");
+    return launch_enc_targets(W, N, K, chunk * 128, fed, levels, lam, levels == 2, T, rings, negated, (hipStream_t)stream);
+}
+
+extern "C" int nq_enc_base(const int64_t* states, int units, int var, const float* rings, const float* lut, const float* W, const double* T, int K, int chunk, int64_t* own, float* sign,
+                           int64_t* st_all, float* sign_all, double* err, double* eta, void* stream)
+{
+    NQ_REQUIRE(units >= 0 && units <= (1 << 24) && K >= 128 && K % 128 == 0 && chunk >= 0 && chunk < K / 128, "nq_enc_base: units=%d K=%d chunk=%d", units, K, chunk);
+    if (units == 0) return 0;
+    NQ_REQUIRE(states && rings && lut && own && sign && (!W || (T && st_all && sign_all && err && eta)), "nq_enc_base: null pointer");
+    return launch_enc_base(states, units * 16, var, rings, lut, W, T, K, chunk, own, sign, st_all, sign_all, err, eta, (hipStream_t)stream);
+}
+
+extern "C" int nq_enc_feed(const int64_t* states, const float* Q, const int64_t* Mb, const int64_t* N, const float* W, const double* T, int rows, int K, int chunk, int64_t* st_all,
+                           float* Q_all, int64_t* Mb_all, int64_t* N_all, double* err, double* eta, void* stream)
+{
+    NQ_REQUIRE(enc_shape_ok(rows, K) && chunk >= 0 && chunk < K / 128, "nq_enc_feed: rows=%d K=%d chunk=%d", rows, K, chunk);
+    NQ_REQUIRE(states && Q && Mb && N && W && T && st_all && Q_all && Mb_all && N_all && err && eta, "nq_enc_feed: null pointer");
+    return launch_enc_feed(states, Q, Mb, N, W, T, rows, K, chunk, st_all, Q_all, Mb_all, N_all, err, eta, (hipStream_t)stream);
+}
+
 extern "C" int nq_viterbi_p4(const float* w, const int64_t* a, int T, int L, const float* lut, int64_t* b, int position_order, void* stream)
 {
     NQ_REQUIRE(T >= 0 && L >= 1 && L <= 256, "nq_viterbi_p4: T=%d L=%d (1..256)", T, L);

@@ -80,6 +80,14 @@ int launch_fit_words(const float* target, const float* sign, const int64_t* st_b
                      const double* Do, int64_t do_step, void* ws, float* Q, int64_t* Mb, int64_t* N, double* delta, hipStream_t st);
 int launch_fit_pack(const int64_t* st, int K, const float* values, const float* sign, const float* lut, const int64_t* Mb, const int64_t* N, int U, int C,
                     int32_t* words, int32_t* dw, uint8_t* var, float* Q, int32_t* bad, hipStream_t s);
+int launch_enc_prepare(const float* W, int N, int K, const int64_t* sgn, double* c, void* su, void* sv, float* target, float* rings, int negated, hipStream_t st);
+int launch_enc_hessian(const double* H, int K, const void* su, double* out, hipStream_t st);
+int launch_enc_inverse(const double* A, int lda, double* out, int32_t* bad, int order0, hipStream_t st);
+int launch_enc_targets(const float* W, int N, int K, int col0, const double* fed, int levels, double lam, int mix, double* T, float* rings, int negated, hipStream_t st);
+int launch_enc_base(const int64_t* st, int N, int var, const float* rings, const float* lut, const float* W, const double* T0, int K, int chunk, int64_t* own, float* sign,
+                    int64_t* st_all, float* sign_all, double* err, double* eta, hipStream_t s);
+int launch_enc_feed(const int64_t* st, const float* Q, const int64_t* Mb, const int64_t* Nw, const float* W, const double* T0, int N, int K, int chunk, int64_t* st_all, float* Q_all,
+                    int64_t* Mb_all, int64_t* N_all, double* err, double* eta, hipStream_t s);
 int launch_viterbi_p4(const float* w, const int64_t* a, int T, int L, const float* lut, int64_t* b, int rev, hipStream_t s);
 int launch_viterbi(const float* w, int T, int L, int K, const float* lut, int64_t* st, uint32_t* back, int slots, int rev, hipStream_t s);
 

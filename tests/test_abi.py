@@ -131,6 +131,22 @@ def test_argument_checks_run_before_any_device_work():
     assert L.nq_mailbox(None, base, base, base, None, 4, None) != 0 and "null" in err()
 
 
+def test_encoder_entry_points_refuse_bad_arguments():
+    """shapes, chunks and pointers that the kernels index without looking"""
+    L = _lib.lib()
+    err = lambda: L.nq_last_error().decode()
+    b = 64
+    assert L.nq_enc_prepare(b, 100, 128, b, b, b, b, b, None, 0, None) != 0 and "multiples of 128" in err()
+    assert L.nq_enc_prepare(b, 128, 128, None, b, b, b, b, None, 0, None) != 0 and "null" in err()
+    assert L.nq_enc_hessian(b, 64, b, b, None) != 0 and "multiple of 128" in err()
+    assert L.nq_enc_inverse(b, 127, b, b, 0, None) != 0 and "lda" in err()
+    assert L.nq_enc_targets(b, 128, 256, 2, None, 2, 0.3, b, b, 0, None) != 0 and "chunk" in err()
+    assert L.nq_enc_targets(b, 128, 256, 0, None, 1, 0.3, b, b, 1, None) != 0 and "negated" in err()
+    assert L.nq_enc_base(b, 4, 1, b, b, b, None, 128, 0, b, b, b, b, b, b, None) != 0 and "null" in err()
+    assert L.nq_enc_base(b, 0, 1, None, None, None, None, 128, 0, None, None, None, None, None, None, None) == 0
+    assert L.nq_enc_feed(b, b, b, b, b, b, 128, 256, -1, b, b, b, b, b, b, None) != 0 and "chunk" in err()
+
+
 def test_which_steps_are_given_decoded_weights():
     """nq_pf_wide_slots: none for steps of short tiles, of few tokens, of too few tiles to fill the GPU, of shapes that would be padded; no
     more than 2 GB; nothing for sizes that a step refuses"""

@@ -234,3 +234,89 @@ def test_planes_are_packed_as_in_torch(N, K, signed, nested):
         for args in ((s, f, sign), (s.cuda(), dev(f), put(sign))):
             with pytest.raises(AssertionError, match="tail-biting"):
                 EN.pack_planes({}, N, K, *args)
+
+
+@pytest.mark.parametrize("N,K", [(128, 128), (256, 384), (384, 128)])
+def test_prepared_weights_equal_the_torch_form(N, K):
+    """scales, signs, rotated targets and their ring order; 16-bit and strided weights, a channel of zeros, values that are not finite. The torch form is what a
+    float64 weight takes; sums in another order leave 1e-16, which a rounding to fp16 or fp32 shows once in 1e8"""
+    g = torch.Generator().manual_seed(N + K)
+    W = torch.randn(N, K, generator=g).cuda()
+    dead, wild = W.clone(), W.clone()
+    dead[:, 5] = 0; dead[7] = 0
+    wild[3, 9] = float("inf"); wild[100, 100] = float("nan")
+    for w in (W, W.half(), W.bfloat16(), torch.randn(K, N, generator=g).cuda().t(), dead, wild):
+        got, want = EN.prepare(w, 11), EN.prepare(w.double(), 11)
+        for a, b in zip(got, want):
+            assert a.dtype == b.dtype and torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(), b.nan_to_num()), w.dtype
+        for n in (1, 2):
+            rings = EN._prepare_gpu(w, 11, n)[3].nan_to_num()
+            assert torch.equal(rings[: N * K // 256], EN.to_rings(got[2]).nan_to_num()) and (n == 1 or torch.equal(rings[N * K // 256:], EN.to_rings(-got[2]).nan_to_num()))
+
+
+def test_orientation_of_rings_equals_the_torch_form():
+    """each ring fitted as it is and negated: the better of the two, the first where they are equal (a ring of zeros, whose two searches give one path)"""
+    g = torch.Generator().manual_seed(12)
+    rings = torch.randn(24, 256, generator=g).cuda()
+    rings[3] = 0
+    got, sign = EN.base_rings(rings, var=True)
+    lut = EN.codebook("cuda")
+    st = EN.viterbi_rings(torch.cat([rings, -rings]))
+    e = (lut[st] - torch.cat([rings, -rings])).double().square().sum(1)
+    neg = e[24:] < e[:24]
+    assert 0 < int(neg.sum()) < 24 and torch.equal(sign[:, 0], 1.0 - 2.0 * neg.float()) and sign.shape == (24, 1)
+    assert torch.equal(got, torch.where(neg[:, None], st[24:], st[:24]))
+
+
+@pytest.mark.parametrize("m", [1, 2, 5])
+def test_block_factors_on_the_gpu(m):
+    """L D L^T is the matrix, as far as 64 bits hold it; a matrix that is not positive definite is reported with the order of its first minor that is not"""
+    g = torch.Generator().manual_seed(m)
+    n = 128 * m
+    X = torch.randn(2 * n, n, generator=g, dtype=torch.float64) * (1 + torch.arange(n)) ** -0.5
+    H = (X.T @ X / n).cuda()
+
+    def factors(H):
+        D, Lc = torch.empty(m, 128, 128, dtype=torch.float64, device="cuda"), [torch.empty(n - 128 * (i + 1), 128, dtype=torch.float64, device="cuda") for i in range(m - 1)]
+        bad = torch.zeros(1, dtype=torch.int32, device="cuda")
+        EN._block_ldl_gpu(H, D, Lc, bad)
+        L = torch.eye(n, dtype=torch.float64, device="cuda")
+        for i, c in enumerate(Lc):
+            L[128 * (i + 1):, 128 * i: 128 * (i + 1)] = c
+        return L, D, int(bad)
+    before = H.clone()
+    L, D, bad = factors(H)
+    L0, D0 = EN.block_ldl(H)
+    assert bad == 0 and torch.equal(H, before)
+    assert float((L @ torch.block_diag(*D) @ L.T - H).norm() / H.norm()) < 4e-15
+    assert float((D - D0).norm() / D0.norm()) < 1e-13 and float((L - L0).norm() / L0.norm()) < 1e-12
+    for at in (0, n // 2 + 3, n - 1):
+        B = H.clone()
+        B[at, at] = -1.0
+        assert factors(B)[2] == int(torch.linalg.cholesky_ex(B.cpu()).info) == at + 1
+    assert factors(H * float("nan"))[2] == 1
+
+
+@pytest.mark.parametrize("N,K,var", [(128, 128, True), (128, 384, False), (256, 256, True)])
+def test_hessian_aware_fit_equals_the_torch_form(N, K, var):
+    """encode_ldlq with its glue in kernels and level 3 at its own pace against the torch form (which a float64 weight takes): the same bytes, errors to
+    the rounding of other sums; a metric that is not positive definite raises as there"""
+    g = torch.Generator().manual_seed(N + K)
+    W = torch.randn(N, K, generator=g).cuda()
+    X = torch.randn(4 * K, K, generator=g) * (1 + torch.arange(K)) ** -0.25
+    H = (X.T @ X / (4 * K)).cuda()
+    got, want = EN.encode_ldlq(W, H, seed=5, var=var), EN.encode_ldlq(W.double(), H, seed=5, var=var)
+    assert got.keys() == want.keys()
+    for k, w in want.items():
+        if k == "proxy":
+            assert all(abs(got[k][l] - w[l]) < 1e-12 * w[l] for l in (2, 3, 4))
+        elif k == "eta":
+            assert all(float((got[k][l] - w[l]).abs().max()) < 1e-12 for l in (2, 3, 4))
+        elif k in ("Hr", "D"):
+            assert got[k].shape == w.shape and float((got[k] - w).norm() / w.norm()) < 1e-13
+        else:
+            assert (w is None and got[k] is None) or (got[k].dtype == w.dtype and torch.equal(got[k], w)), k
+    for bad in (-H, H * float("nan")):
+        for w in (W, W.double()):
+            with pytest.raises(torch.linalg.LinAlgError):
+                EN.encode_ldlq(w, bad)
