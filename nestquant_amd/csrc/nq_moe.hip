@@ -732,6 +732,7 @@ nq_gemv_k(MoeArgs a, int NC)
     L.nrec = (size_t)(N / 16) * C * 32;
     L.src = a.G == 2 ? lane ^ 16 : (lane + 16) & 63;             // next record of the ring: rings of four lanes, or of two
     L.g = g; L.strip = (uint32_t)strip; L.nstrips = (size_t)(N / 16); L.chunk0 = chunk0;
+    L.half0 = (uint32_t)(2 * (blockIdx.x * SB + warp) + (lane >> 5)) * C + chunk0;
     L.xs = (n < ntok ? smem + n * rowstride : zero) + t4 * 16; L.xstep = n < ntok ? 256 : 0;
     // block-uniform: a row the common kernel has no loop for (its plane is not read: the records have another size or order)
     const bool foreign = !ANYROW && (P.bcode != 0 || (P.flags != nullptr && R.level != 2));
@@ -1035,6 +1036,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))
     L.nrec = (size_t)(N / 16) * C * 32;
     L.src = a.G == 2 ? lane ^ 16 : (lane + 16) & 63;
     L.g = g; L.strip = (uint32_t)strip; L.nstrips = (size_t)(N / 16); L.chunk0 = chunk0;
+    L.half0 = (uint32_t)(2 * (blockIdx.x * SB + warp) + (lane >> 5)) * C + chunk0;
     char* zero = smem + a.B * rowstride;
     L.xs = (n < a.B ? smem + n * rowstride : zero) + t4 * 16; L.xstep = n < a.B ? 256 : 0;
     u32x4 nb0 = {0u, 0u, 0u, 0u};

@@ -509,7 +509,7 @@ __global__ void __launch_bounds__(256) nq_pf_wdecode_k(const int64_t* table, con
     L.unit0 = (uint32_t)(2 * sp + ss) * C; L.rec0 = L.unit0 * 32 + 4 * g + t4;
     L.nrec = (size_t)(N / 16) * C * 32;
     L.src = (lane + 16) & 63; L.g = g; L.xs = nullptr; L.xstep = 0;
-    L.strip = (uint32_t)(2 * sp + ss); L.nstrips = (size_t)(N / 16); L.chunk0 = 0;
+    L.strip = (uint32_t)(2 * sp + ss); L.nstrips = (size_t)(N / 16); L.chunk0 = 0; L.half0 = (uint32_t)(2 * sp + (lane >> 5)) * C;
     u32x4* dst = Wop + wop_base(slot, mode, H, I) + (size_t)sp * C * 8 * 64;
     if (lv == 2) wdecode_chunks<false, 0>(P, L, c0, c1, dst, lane);
     else dispatch_code(P.code, [&](auto tag) { wdecode_chunks<true, decltype(tag)::value>(P, L, c0, c1, dst, lane); });
@@ -723,13 +723,15 @@ __device__ __forceinline__ void pf_chunks(const Planes& P, const LaneCtx& L, int
 {
     constexpr int NW = RES ? Rec<CODE>::NW : 1;
     u32x4 nb = load_base<BK>(P, L.rec0, L.nrec);
-    uint32_t nr[NW + 2] = {0}, ndw = 0, nvar = 0;
+    uint32_t nr[NW + 2] = {0}, nvar = 0;
     constexpr bool masked = RES && MASKED;                       // the kernel variant for experts in mask mode
     // an expert without flags that comes through this variant (base code other than 0) reads as "every chunk refined",
     // for which the compact residual indexing is the dense one
     const uint64_t mflags = masked ? (P.flags ? P.flags[L.strip] : (C >= 64 ? ~0ull : (1ull << C) - 1ull)) : 0ull;
-    if constexpr (RES && !masked) { load_record<CODE>(nr, P.res, L.rec0, L.nrec); ndw = at_offset<uint32_t>((gp_u8)P.dw, L.unit0 * 4u); }
-    if (P.var) nvar = at_offset<uint8_t>(P.var, L.unit0);
+    if constexpr (RES && !masked) load_record<CODE>(nr, P.res, L.rec0, L.nrec);
+    UnitConsts<RES> consts;                                      // mask mode works a chunk's constants out itself
+    if constexpr (!masked) consts.start(P, L, C);
+    else if (P.var) nvar = at_offset<uint8_t>(P.var, L.unit0);
     const int lane = threadIdx.x & 63, warp = threadIdx.x >> 6, t4 = lane >> 4, n = lane & 15;
     // Staging: wavefront w copies rows 16 u + 4 w + (lane >> 4), u = 0 .. TG - 1, of the tile, one 1 KB
     // global -> LDS load per u (64 lanes x 16 bytes land in LDS in lane order, so a load fills 4 rows x 256 bytes). The
@@ -749,7 +751,7 @@ __device__ __forceinline__ void pf_chunks(const Planes& P, const LaneCtx& L, int
         wb[0] = nb.x; wb[1] = nb.y; wb[2] = nb.z; wb[3] = nb.w;
 #pragma unroll
         for (int i = 0; i < NW; ++i) wr[i] = nr[i];
-        uint32_t dw = ndw;
+        uint32_t dw = 0u;
         const uint32_t var = nvar;
         bool on = true;                                          // mask mode: is chunk c refined? (the same for the whole workgroup)
         if constexpr (masked)
@@ -761,11 +763,11 @@ __device__ __forceinline__ void pf_chunks(const Planes& P, const LaneCtx& L, int
         if (c + 1 < C)
         {
             nb = load_base<BK>(P, L.rec0 + (uint32_t)(c + 1) * 32, L.nrec);
-            if constexpr (RES && !masked) { load_record<CODE>(nr, P.res, L.rec0 + (uint32_t)(c + 1) * 32, L.nrec); ndw = at_offset<uint32_t>((gp_u8)P.dw, (L.unit0 + c + 1) * 4u); }
-            if (P.var) nvar = at_offset<uint8_t>(P.var, L.unit0 + c + 1);
+            if constexpr (RES && !masked) load_record<CODE>(nr, P.res, L.rec0 + (uint32_t)(c + 1) * 32, L.nrec);
+            if (masked && P.var) nvar = at_offset<uint8_t>(P.var, L.unit0 + c + 1);
         }
         ext_base<BK>(wb, __shfl(wb[0], L.src));
-        const uint32_t sgm = ((var >> L.g) & 1u) * 0x80008000u;
+        const uint32_t sgm = masked ? ((var >> L.g) & 1u) * 0x80008000u : 0u;
         half8_t aop[4][2];
         if (RES && (!masked || on))
         {
@@ -773,7 +775,8 @@ __device__ __forceinline__ void pf_chunks(const Planes& P, const LaneCtx& L, int
             {
                 prepare_record<CODE>(wr);
                 ext_words<Rec<CODE>::BITS, Rec<CODE>::NW>(wr, __shfl(wr[0], L.src));
-                const FoldK k = consts_fold(dw, sgm);
+                if constexpr (masked) consts.k = consts_fold(dw, sgm); else consts.take(P, L, c, C);
+                const FoldK& k = consts.k;
                 static_for<4>([&](auto mm) {
                     constexpr int MM = decltype(mm)::value;
                     pf_stage_tokens<TG, MM>(A, K, row0, nrows, c, smem, warp, srow, scol);
@@ -784,7 +787,8 @@ __device__ __forceinline__ void pf_chunks(const Planes& P, const LaneCtx& L, int
         }
         else
         {
-            const FoldK k = consts_l2(sgm);
+            if constexpr (masked) consts.k = consts_l2(sgm); else consts.take(P, L, c, C);
+            const FoldK& k = consts.k;
             static_for<4>([&](auto mm) {
                 constexpr int MM = decltype(mm)::value;
                 pf_stage_tokens<TG, MM>(A, K, row0, nrows, c, smem, warp, srow, scol);
@@ -846,7 +850,7 @@ __device__ __forceinline__ void pf_tile(const PfGemm& a, int bx, int e, int row0
     L.unit0 = (uint32_t)(2 * sp + ss) * C; L.rec0 = L.unit0 * 32 + 4 * g + t4;
     L.nrec = (size_t)(N / 16) * C * 32;
     L.src = (lane + 16) & 63; L.g = g; L.xs = nullptr; L.xstep = 0;
-    L.strip = (uint32_t)(2 * sp + ss); L.nstrips = (size_t)(N / 16); L.chunk0 = 0;
+    L.strip = (uint32_t)(2 * sp + ss); L.nstrips = (size_t)(N / 16); L.chunk0 = 0; L.half0 = (uint32_t)(2 * sp + (lane >> 5)) * C;
     float4_t acc[TG][2];
 #pragma unroll
     for (int tg = 0; tg < TG; ++tg) { acc[tg][0] = float4_t{0.f, 0.f, 0.f, 0.f}; acc[tg][1] = float4_t{0.f, 0.f, 0.f, 0.f}; }

@@ -277,6 +277,50 @@ struct LaneCtx
     const char* xs;       // this lane's B-operand base in LDS (bytes), kg folded in
     int xstep;            // bytes per chunk (0 for lanes without a token)
     uint32_t strip; size_t nstrips; int chunk0;   // mask mode: this lane's strip, strips of the projection, first chunk of the k-slice
+    uint32_t half0;       // unit index of strip lane / 32 of the wavefront's two, first chunk (UnitConsts)
+};
+
+// What a chunk's decode needs beside the records, fold constants and ring signs, for 32 chunks of the wavefront's two strips at a time: lane 32 s + i
+// reads the block word and sign byte of strip s, chunk c0 + i, and works out its constants; a chunk's come from there by one
+// lane permute (two at levels 3 / 4). Worked out by every lane in every chunk they were some 25 of the 600 vector instructions of a refined chunk
+// and, with no sign plane, 5 of the 275 of a chunk at level 2, beside one or two loads.
+template <bool RES>
+struct UnitConsts
+{
+    uint32_t word, ac, next_word, next_var;       // block word | sign byte << 16; fold_ac of it; as loaded, 32 chunks on
+    int from;                                     // 4 * the lane that holds this lane's strip, chunk 0
+    FoldK k;
+    __device__ __forceinline__ void request(const Planes& P, const LaneCtx& L, int c, int NC)
+    {
+        const uint32_t unit = L.half0 + (uint32_t)min(c + (int)(threadIdx.x & 31), NC - 1);
+        if constexpr (RES) next_word = at_offset<uint32_t>((gp_u8)P.dw, unit * 4u);
+        if (P.var) next_var = at_offset<uint8_t>(P.var, unit);
+    }
+    __device__ __forceinline__ void start(const Planes& P, const LaneCtx& L, int NC)
+    {
+        word = ac = next_word = next_var = 0u;
+        from = (int)(threadIdx.x & 8u) << 4;
+        k = consts_l2(0u);
+        request(P, L, 0, NC);
+    }
+    // the constants of chunk c, in k
+    __device__ __forceinline__ void take(const Planes& P, const LaneCtx& L, int c, int NC)
+    {
+        if ((RES || P.var) && (c & 31) == 0)
+        {
+            if constexpr (RES) ac = fold_ac(next_word);
+            word = (next_word & 0xFFFFu) | next_var << 16;
+            if (c + 32 < NC) request(P, L, c + 32, NC);
+        }
+        const int lane = from + 4 * (c & 31);
+        if constexpr (RES) k = fold_k((uint32_t)__builtin_amdgcn_ds_bpermute(lane, (int)word), (uint32_t)__builtin_amdgcn_ds_bpermute(lane, (int)ac), 0u);
+        if (P.var)
+        {
+            uint32_t sgm = (((uint32_t)__builtin_amdgcn_ds_bpermute(lane, (int)word) >> (16 + L.g)) & 1u) * 0x80008000u;
+            asm volatile("" : "+v"(sgm));                        // a branch, not a selection that every chunk pays for
+            k.A2 = (RES ? k.A2 : MUL1_A2) ^ sgm; k.C2 = (RES ? k.C2 : MUL1_B2) ^ sgm;
+        }
+    }
 };
 
 // mask mode: chunk by chunk either the folded decode (refined chunks, residual records compact over them) or the level-2
@@ -352,9 +396,10 @@ __device__ __forceinline__ void gemv_chunks(const Planes& P, const LaneCtx& L, i
     if constexpr (RES && MASKOK)
         if (P.flags) { gemv_chunks_masked<CODE, BK>(P, L, NC, acc, nb); return; }     // block-uniform
     constexpr int NW = RES ? Rec<CODE>::NW : 1;
-    uint32_t nr[NW + 2] = {0}, ndw = 0, nvar = 0;
-    if constexpr (RES) { load_record<CODE>(nr, P.res, L.rec0, L.nrec); ndw = at_offset<uint32_t>((gp_u8)P.dw, L.unit0 * 4u); }
-    if (P.var) nvar = at_offset<uint8_t>(P.var, L.unit0);
+    uint32_t nr[NW + 2] = {0};
+    if constexpr (RES) load_record<CODE>(nr, P.res, L.rec0, L.nrec);
+    UnitConsts<RES> consts;
+    consts.start(P, L, NC);
     for (int c = 0; c < NC; ++c)
     {
         progress_priority(c, NC);
@@ -362,23 +407,19 @@ __device__ __forceinline__ void gemv_chunks(const Planes& P, const LaneCtx& L, i
         wb[0] = nb.x; wb[1] = nb.y; wb[2] = nb.z; wb[3] = nb.w;
 #pragma unroll
         for (int i = 0; i < NW; ++i) wr[i] = nr[i];
-        const uint32_t dw = ndw, var = nvar;
         if (c + 1 < NC)                                         // prefetch the next chunk's records
         {
             nb = load_base<BK>(P, L.rec0 + (uint32_t)(c + 1) * 32, L.nrec);
-            if constexpr (RES) { load_record<CODE>(nr, P.res, L.rec0 + (uint32_t)(c + 1) * 32, L.nrec); ndw = at_offset<uint32_t>((gp_u8)P.dw, (L.unit0 + c + 1) * 4u); }
-            if (P.var) nvar = at_offset<uint8_t>(P.var, L.unit0 + c + 1);
+            if constexpr (RES) load_record<CODE>(nr, P.res, L.rec0 + (uint32_t)(c + 1) * 32, L.nrec);
         }
         ext_base<BK>(wb, __shfl(wb[0], L.src));
-        const uint32_t sgm = ((var >> L.g) & 1u) * 0x80008000u;
-        FoldK k;
         if constexpr (RES)
         {
             prepare_record<CODE>(wr);
             ext_words<Rec<CODE>::BITS, Rec<CODE>::NW>(wr, __shfl(wr[0], L.src));
-            k = consts_fold(dw, sgm);
         }
-        else k = consts_l2(sgm);
+        consts.take(P, L, c, NC);
+        const FoldK& k = consts.k;
         const char* xp = L.xs + c * L.xstep;
         if constexpr (RAW && RES)
         {
