@@ -693,26 +693,26 @@ __device__ __forceinline__ void pf_mfmas(const half8_t (*aop)[2], const char* sm
 // PART = 0 .. 3 issues a quarter of the loads (all of them in part 0 when there are fewer than four): the decode-fused body
 // spreads them over its decode, because the texture path takes 16 clocks per 1 KB load and a wavefront that issues sixteen in
 // a row stalls behind its own requests (measured: 1450 clocks per chunk at 256 rows) with the record loads queued after them.
-template <int TG, int PART = -1>
-__device__ __forceinline__ void pf_stage_tokens(const _Float16* A, int K, int row0, int nrows, int c, char* smem, int warp, int srow, uint32_t scol)
+// A load's address is a scalar base (the tile's chunk and row group) and the lane's offset inside the group, one register for all groups; from the
+// group that holds the tile's last row on, that group is read again with an offset that stops there. With a lane offset formed per group (a move, an
+// addition, a selection, a lane read for the LDS address) the tokens of a chunk were up to 18 of 290 vector instructions at 64 rows.
+struct TokenSource { const char* base; uint32_t off, last_off; int last; size_t step; uint32_t lds; };       // last: the row group of the tile's last row
+__device__ __forceinline__ TokenSource token_source(const _Float16* A, int K, int row0, int nrows, const char* smem, int warp, int lane)
 {
-    typedef const __attribute__((address_space(1))) void* gvp;
-    typedef __attribute__((address_space(3))) void* lvp;
-    constexpr int U0 = PART < 0 ? 0 : (TG >= 4 ? PART * (TG / 4) : 0), U1 = PART < 0 ? TG : (TG >= 4 ? U0 + TG / 4 : (PART == 0 ? TG : 0));
-    // uniform base of the tile's chunk (scalar registers) + a 32-bit lane offset inside the tile; the offset passes through an
-    // empty asm so that the addresses of a part are formed when the part is issued, not sixteen of them ahead of the decode
-    const char* base = (const char*)A + ((size_t)row0 * K + c * 128) * 2;
-    uint32_t lane_off = (uint32_t)(srow * K * 2) + scol;
-    asm volatile("" : "+v"(lane_off));
-    const uint32_t ustep = (uint32_t)(16 * K * 2);
-    const uint32_t last_off = (uint32_t)((nrows - 1) * K * 2) + scol;
+    const int srow = 4 * warp + (lane >> 4), last = (nrows - 1) >> 4;            // srow = row & 15 of every row this lane stages
+    const uint32_t scol = (uint32_t)(((lane & 15) ^ srow) * 16);                 // byte offset of the fetched column inside the chunk
+    return TokenSource{(const char*)(A + (size_t)row0 * K), (uint32_t)(srow * K * 2) + scol, (uint32_t)(min(srow, nrows - 1 - 16 * last) * K * 2) + scol, last,
+                       (size_t)K * 32, (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)smem + (uint32_t)__builtin_amdgcn_readfirstlane(4 * warp * PF_ROW)};
+}
+template <int TG, int PART>
+__device__ __forceinline__ void pf_stage_tokens(const TokenSource& t, int c)
+{
+    constexpr int U0 = TG >= 4 ? PART * (TG / 4) : 0, U1 = TG >= 4 ? U0 + TG / 4 : (PART == 0 ? TG : 0);
 #pragma unroll
     for (int u = U0; u < U1; ++u)
     {
-        if constexpr (PART < 0) { if (16 * u >= nrows) break; }  // block-uniform; the spread parts stay free of branches
-        uint32_t off = lane_off + (uint32_t)u * ustep;
-        off = 16 * u + srow < nrows ? off : last_off;
-        __builtin_amdgcn_global_load_lds((gvp)(base + off), (lvp)(smem + (16 * u + 4 * warp) * PF_ROW), 16, 0, 0);
+        const bool whole = TG > 1 && u < t.last;                 // block-uniform
+        to_lds(t.base + (size_t)c * 256 + (whole ? u : t.last) * t.step, whole ? t.off : t.last_off, t.lds + 16 * u * PF_ROW);
     }
 }
 
@@ -733,13 +733,16 @@ __device__ __forceinline__ void pf_chunks(const Planes& P, const LaneCtx& L, int
     if constexpr (!masked) consts.start(P, L, C);
     else if (P.var) nvar = at_offset<uint8_t>(P.var, L.unit0);
     const int lane = threadIdx.x & 63, warp = threadIdx.x >> 6, t4 = lane >> 4, n = lane & 15;
-    // Staging: wavefront w copies rows 16 u + 4 w + (lane >> 4), u = 0 .. TG - 1, of the tile, one 1 KB
-    // global -> LDS load per u (64 lanes x 16 bytes land in LDS in lane order, so a load fills 4 rows x 256 bytes). The
-    // lane picks which 16-byte column of its row it fetches: column (lane & 15) ^ (row & 15) goes to slot lane & 15, and
-    // the MFMA reads undo the XOR, which spreads the 16 tokens of an operand read over all banks without padding.
-    // Rows beyond the tile re-read its last row: their products are never stored.
-    const int srow = 4 * warp + t4;                              // row & 15 of every row this lane stages
-    const uint32_t scol = (uint32_t)((n ^ srow) * 16);           // byte offset of the fetched column inside the chunk
+    const TokenSource tokens = token_source(A, K, row0, nrows, smem, warp, lane);
+    auto stage = [&](auto part, int c) {
+        if constexpr (MASKED && TG == 16)                        // two registers too many: formed anew for every part
+        {
+            int l = lane;
+            asm volatile("" : "+v"(l));
+            pf_stage_tokens<TG, decltype(part)::value>(token_source(A, K, row0, nrows, smem, warp, l), c);
+        }
+        else pf_stage_tokens<TG, decltype(part)::value>(tokens, c);
+    };
     uint32_t boff[4];                                            // B-operand read offsets of this lane for mm = 0..3
 #pragma unroll
     for (int mm = 0; mm < 4; ++mm) boff[mm] = (uint32_t)(n * PF_ROW + (((4 * mm + t4) ^ n) << 4));
@@ -779,7 +782,7 @@ __device__ __forceinline__ void pf_chunks(const Planes& P, const LaneCtx& L, int
                 const FoldK& k = consts.k;
                 static_for<4>([&](auto mm) {
                     constexpr int MM = decltype(mm)::value;
-                    pf_stage_tokens<TG, MM>(A, K, row0, nrows, c, smem, warp, srow, scol);
+                    stage(mm, c);
                     aop[MM][0] = a_operand<RES, CODE, MM, 0, BK>(wb, wr, k);
                     aop[MM][1] = a_operand<RES, CODE, MM, 1, BK>(wb, wr, k);
                 });
@@ -791,7 +794,7 @@ __device__ __forceinline__ void pf_chunks(const Planes& P, const LaneCtx& L, int
             const FoldK& k = consts.k;
             static_for<4>([&](auto mm) {
                 constexpr int MM = decltype(mm)::value;
-                pf_stage_tokens<TG, MM>(A, K, row0, nrows, c, smem, warp, srow, scol);
+                stage(mm, c);
                 aop[MM][0] = a_operand<false, 0, MM, 0, BK>(wb, wr, k);
                 aop[MM][1] = a_operand<false, 0, MM, 1, BK>(wb, wr, k);
             });
