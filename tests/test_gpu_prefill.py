@@ -148,6 +148,37 @@ def test_tiles_of_decoded_weights_give_the_bits_of_decode_fused_tiles(H, I):
     assert want.isfinite().all()
 
 
+@pytest.mark.parametrize("bm,rows", [(64, (33, 48, 49, 64)), (128, (1, 65, 80, 81, 96, 97, 112, 113, 128)), (256, (40, 129, 144, 145, 160, 161, 176, 177, 192, 193, 208, 209, 224, 225, 240, 241, 256))])
+def test_bodies_of_tall_tiles_give_the_bits_of_16_row_tiles(bm, rows):
+    """nq_pf_gemm picks a body by a tile's rows: at the edges of each body the rows come out as in tiles of 16 (which are held against the oracle
+    above), and nothing is written beyond them; levels 2 to 4, mask mode and another base window code"""
+    from nestquant_amd import _lib
+    H, I = 256, 384
+    ex = [F.Expert(H, I, seed=6100 + i, dev="cpu", nm_gu=(1 if i == 3 else None), nm_dn=(2 if i == 3 else None), rk_gu=(0, 3, 7, 6, 9)[i], rk_dn=(0, 9, 3, 8, 0)[i],
+                   nested=i == 1, var=i in (1, 3), bk_gu=int(i == 4), bk_dn=int(i == 4)) for i in range(5)]
+    to_dev(ex)
+    L = M.MoELayer(5, H, I, Bmax=4, topk=1)
+    for e, lv in enumerate([2, 3, 4, 4, 4]):
+        L.set(e, ex[e], lv)
+    g = torch.Generator().manual_seed(bm)
+    A0, A1 = [(torch.randn(300, max(H, I), generator=g) * 0.05).half().to(DEV) for _ in range(2)]
+
+    def run(mode, kind, tiles, height):
+        C = torch.full((300, 2 * I if mode == 0 else H), 7.0, device=DEV)
+        t = torch.tensor(tiles, dtype=torch.int32, device=DEV)
+        _lib.check(_lib.lib().nq_pf_gemm(L.table.data_ptr(), t.data_ptr(), len(tiles), height, mode | kind, A0.data_ptr(), A1.data_ptr(), C.data_ptr(), 5, H, I, None, None))
+        torch.cuda.synchronize()
+        return C
+
+    for n in rows:
+        for e in range(5):
+            for mode in (0, 1):
+                kind = 2 * (e >= 3)
+                want = run(mode, kind, [[e, 8 + r, min(16, n - r), 0] for r in range(0, n, 16)], 16)
+                assert torch.equal(run(mode, kind, [[e, 8, n, 0]], bm), want), (n, e, mode)
+                assert want[8:8 + n].isfinite().all() and bool((want[:8] == 7).all() and (want[8 + n:] == 7).all() and (want[8:8 + n] != 7).any(1).all())
+
+
 def test_a_step_takes_decoded_weights_where_they_pay():
     """the rule's first step (eight experts of 1100 rows: 32 tiles of a shape whose units are then 512): equal bits with all experts above
     level 2, and with one below, which leaves too few tiles"""
