@@ -300,8 +300,8 @@ typedef struct NqPfArgs
     void *acc, *y;                 /* fp32 [rows][2I], [rows][H] */
     float *zg, *zd;                /* fp32 [rows][4] each, or NULL when no expert has a low-rank plane */
     void* wop; int64_t wop_bytes;  /* optional scratch of decoded weights (nq_pf_wdecode) with wop_slots slots for experts of >= hot_min rows */
-    void* side[3];                 /* streams of default priority, or NULL: the step stays on `stream` */
-    void* events[4];               /* events without timing of the same device, with side streams */
+    void* side[3];                 /* streams of default priority (the step forks onto the first two), or NULL: it stays on `stream` */
+    void* events[4];               /* events without timing of the same device (the first three are recorded), with side streams */
     int32_t T, topk, E, H, I;
     int32_t rows;                  /* pair rows the scratch holds; more pairs are worked through in chunks (out must then be fp32) */
     int32_t x_dtype, sel_dtype, rw_dtype, out_dtype;   /* as in NqMoeArgs */

@@ -299,7 +299,7 @@ extern "C" int nq_pf_plan(const int32_t* counts, int E, int row_lo, int nrows, i
     NQ_REQUIRE(aligned16(tiles), "nq_pf_plan: tiles must be 16-byte aligned");
     NQ_REQUIRE(cap >= E + nrows / 256 + 1, "nq_pf_plan: cap=%d, need at least E + nrows / 256 + 1 = %d", cap, E + nrows / 256 + 1);
     NQ_REQUIRE(!hot || (hot_min >= 1 && hot_cap >= 1), "nq_pf_plan: hot_min=%d hot_cap=%d (both at least 1 with a hot list)", hot_min, hot_cap);
-    return launch_pf_plan(counts, E, row_lo, nrows, tiles, cap, hot, hot_min, hot_cap, nullptr, 0, nullptr, (hipStream_t)stream);
+    return launch_pf_plan(counts, E, row_lo, nrows, tiles, cap, hot, hot_min, hot_cap, nullptr, 0, nullptr, nullptr, nullptr, (hipStream_t)stream);
 }
 
 extern "C" int nq_pf_hits(const int32_t* counts, int32_t* hits, int E, void* stream)

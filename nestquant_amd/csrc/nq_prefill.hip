@@ -132,6 +132,13 @@ __global__ void __launch_bounds__(256) nq_pf_mid_k(const float* __restrict__ acc
     const int lane = threadIdx.x & 63, warp = threadIdx.x >> 6, L = wht_place(lane);
     const int p0 = blockIdx.x * rows, nr = min(rows, np - p0), ni = I / 128, nseg = (ni + 3) / 4;
     const WhtSigns ws = wht_signs(lane);
+    __shared__ int held[MID_ROWS];                               // is the row of the heights?
+    if (tiles)
+    {   // looked up side by side: one after the other, as the loop comes to them, every row waited for its own
+        const bool in = (int)threadIdx.x < nr && row_in_heights(tiles, cap, heights, p0 + threadIdx.x, pe[p0 + threadIdx.x], E);
+        if (threadIdx.x < MID_ROWS) held[threadIdx.x] = in;
+        if (!__syncthreads_or(in)) return;
+    }
     if (zd)
     {
         for (int i = threadIdx.x; i < MID_ROWS * 16; i += 256) (&zsh[0][0][0])[i] = 0.f;
@@ -141,7 +148,7 @@ __global__ void __launch_bounds__(256) nq_pf_mid_k(const float* __restrict__ acc
     {
         const int row = t / nseg, p = p0 + row, chunk = (t - row * nseg) * 4 + (lane >> 4);
         const int e = pe[p];
-        if (tiles && !row_in_heights(tiles, cap, heights, p, e, E)) continue;
+        if (tiles && !held[row]) continue;
         const bool mine = chunk < ni, live = e >= 0 && e < E && table[(size_t)e * TBL_W] > 0;
         uint4 b = make_uint4(0, 0, 0, 0);
         if (live)
@@ -216,7 +223,7 @@ __global__ void __launch_bounds__(256) nq_pf_mid_k(const float* __restrict__ acc
     {
         const int p = p0 + i / 4, r = i & 3, e = pe[p];
         if (e < 0 || e >= E || table[(size_t)e * TBL_W] <= 0 || !table[(size_t)e * TBL_W + 14] || table[(size_t)e * TBL_W + 17] <= r) continue;
-        if (tiles && !row_in_heights(tiles, cap, heights, p, e, E)) continue;
+        if (tiles && !held[i / 4]) continue;
         zd[(size_t)p * 4 + r] = zsh[i / 4][0][r] + zsh[i / 4][1][r] + zsh[i / 4][2][r] + zsh[i / 4][3][r];
     }
 }
@@ -349,9 +356,12 @@ __device__ __forceinline__ void block_scan(int* a, int n)
 // hot (may be null): experts with at least hot_min rows in the chunk get a slot 0 .. hot_cap - 1 of the decoded-weight scratch (in
 // expert order, as far as the slots reach), written to hot[e] (-1: none) and, plus one, into the fourth word of their tiles in list 4 (a
 // remainder of up to 128 rows is decoded inside its GEMM: as dear as a whole unit of nq_pf_wide_k). wide (may be null): those tiles
-// once more without gaps from wide + 4 on, their number in wide[0].
+// once more without gaps from wide + 4 on, their number in wide[0]. dense (may be null, with the live table `rows`): the tiles of
+// lists 0 to 2 [E] | of list 3 [E] | of list 4 [cap] once more without gaps, then entries of expert -1: what the GEMMs are launched on, over as many
+// tiles as the rows can make. Experts above level 2, whose decode takes twice as long, come first in the two lists of remainders.
 __global__ void __launch_bounds__(256) nq_pf_plan_k(const int32_t* __restrict__ counts, int E, int row_lo, int nrows, int32_t* tiles, int cap,
-                                                    int32_t* hot, int hot_min, int hot_cap, int32_t* wide, int wide_min, const int64_t* __restrict__ table)
+                                                    int32_t* hot, int hot_min, int hot_cap, int32_t* wide, int wide_min, const int64_t* __restrict__ table,
+                                                    int32_t* dense, const int64_t* __restrict__ rows)
 {
     extern __shared__ int plan_sh[];
     int *incl = plan_sh, *fincl = plan_sh + E, *wincl = plan_sh + 2 * E, *hrank = plan_sh + 3 * E;
@@ -412,11 +422,51 @@ __global__ void __launch_bounds__(256) nq_pf_plan_k(const int32_t* __restrict__ 
     }
     const int total = E + fincl[E - 1];
     for (int i = total + threadIdx.x; i < cap; i += blockDim.x) T4[(size_t)4 * cap + i] = make_int4(-1, 0, 0, 0);
+    if (!dense) return;
+    // the counts per expert in low (above level 2) and high half words (E <= 4096); those of 256 rows in one order
+    auto level_class = [&](int e, int n) {
+        const int64_t lv = n > 0 ? rows[(size_t)e * TBL_W] : 0;
+        return lv > 2 ? 1 : lv > 0 ? 1 << 16 : 0;
+    };
+    __syncthreads();                                             // the ranks have been read
+    for (int e = threadIdx.x; e < E; e += blockDim.x)
+    {
+        int r0;
+        const int n = rows_of(e, r0), rem = n % 256, cls = level_class(e, n);
+        hrank[e] = rem > 0 && rem <= SHORT_ROWS ? cls : 0;
+        wincl[e] = rem > SHORT_ROWS && rem <= 128 ? cls : 0;
+        fincl[e] = cls ? n / 256 + (rem > 128) : 0;
+    }
+    __syncthreads();
+    block_scan(hrank, E);
+    block_scan(wincl, E);
+    block_scan(fincl, E);
+    int4 *D4 = (int4*)dense, *tall = D4 + 2 * E;
+    for (int e = threadIdx.x; e < E; e += blockDim.x)
+    {
+        int r0;
+        const int n = rows_of(e, r0), nf = n / 256, rem = n % 256, cls = level_class(e, n);
+        const int slot1 = hot ? hot[e] + 1 : 0;
+        for (int q = 0; q < 2; ++q)
+        {
+            const int* rank = q ? wincl : hrank;
+            const int above = rank[E - 1] & 0xffff, all = above + (rank[E - 1] >> 16);
+            if (cls && rem > q * SHORT_ROWS && rem <= (q + 1) * SHORT_ROWS)
+                D4[q * E + (cls == 1 ? (rank[e] & 0xffff) - 1 : above + (rank[e] >> 16) - 1)] = make_int4(e, r0 + 256 * nf, rem, 0);
+            if (e >= all) D4[q * E + e] = make_int4(-1, 0, 0, 0);
+        }
+        if (!cls) continue;
+        int at = fincl[e] - nf - (rem > 128);
+        for (int j = 0; j < nf; ++j) tall[at++] = make_int4(e, r0 + 256 * j, 256, slot1);
+        if (rem > 128) tall[at] = make_int4(e, r0 + 256 * nf, rem, slot1);
+    }
+    for (int i = fincl[E - 1] + threadIdx.x; i < cap; i += blockDim.x) tall[i] = make_int4(-1, 0, 0, 0);
 }
 
-int launch_pf_plan(const int32_t* counts, int E, int row_lo, int nrows, int32_t* tiles, int cap, int32_t* hot, int hot_min, int hot_cap, int32_t* wide, int wide_min, const int64_t* table, hipStream_t st)
+int launch_pf_plan(const int32_t* counts, int E, int row_lo, int nrows, int32_t* tiles, int cap, int32_t* hot, int hot_min, int hot_cap, int32_t* wide, int wide_min, const int64_t* table,
+                   int32_t* dense, const int64_t* rows, hipStream_t st)
 {
-    nq_pf_plan_k<<<1, 256, 4 * E * sizeof(int), st>>>(counts, E, row_lo, nrows, tiles, cap, hot, hot_min, hot_cap, wide, wide_min, table);
+    nq_pf_plan_k<<<1, 256, 4 * E * sizeof(int), st>>>(counts, E, row_lo, nrows, tiles, cap, hot, hot_min, hot_cap, wide, wide_min, table, dense, rows);
     NQ_LAUNCH_CHECK("nq_pf_plan");
     return 0;
 }
@@ -802,8 +852,8 @@ int launch_pf_wide(const int64_t* table, const int32_t* tiles, int ntiles, int m
 }
 
 // ---- a whole step --------------------------------------------------------------------------------------------------------
-// Bytes of the int32 scratch of a step: cnt [E] | pe [P] | pt [P] | pos [P] | hot [E] | tile lists | tiles of decoded weights, each on 16 bytes.
-struct PfMeta { int32_t *cnt, *pe, *pt, *pos, *hot, *tiles, *wide; int cap, scap; size_t bytes; };
+// Bytes of the int32 scratch of a step: cnt [E] | pe [P] | pt [P] | pos [P] | hot [E] | tile lists | tiles of decoded weights | tiles without gaps, each on 16 bytes.
+struct PfMeta { int32_t *cnt, *pe, *pt, *pos, *hot, *tiles, *wide, *dense; int cap, scap; size_t bytes; };
 static PfMeta pf_meta(void* ws, int P, int R, int E)
 {
     PfMeta m;
@@ -811,23 +861,28 @@ static PfMeta pf_meta(void* ws, int P, int R, int E)
     auto take = [&](size_t n) { int32_t* p = (int32_t*)((char*)ws + off); off += (n * 4 + 15) & ~(size_t)15; return p; };
     m.cap = E + R / 256 + 1; m.scap = E + P / SHORT_ROWS + 1;
     m.cnt = take(E); m.pe = take(P); m.pt = take(P); m.pos = take(P); m.hot = take(E);
-    m.tiles = take(4 * (size_t)(5 * m.cap > m.scap ? 5 * m.cap : m.scap)); m.wide = take(4 * ((size_t)m.cap + 1));
+    m.tiles = take(4 * (size_t)(5 * m.cap > m.scap ? 5 * m.cap : m.scap)); m.wide = take(4 * ((size_t)m.cap + 1)); m.dense = take(4 * (2 * (size_t)E + m.cap));
     m.bytes = off;
     return m;
 }
 
 // Which steps take the one-launch plan of short tiles. An expert of n rows is decoded n / 64 times there, n / 256 times by the tall
-// tiles, which cost side streams, a launch per height and lower occupancy: about 0.1 ms a step. us short / tall:
-//   few rows per expert, up to 32 on average (E = 256 of 6144 x 2048, top-8, all level 4): even routing of 200 tokens 2301 / 2342, 400
-//   2351 / 2537, 1000 2756 / 2913; Zipf(1.1) popularity 200 1977 / 2126, 400 2470 / 2416, 1000 3173 / 2999, where the popular experts'
-//   further decodes cost up to 6 %. Beyond the line 1400 tokens 3058 / 3271 and 3641 / 3336, 2048 4203 / 3924 and 4437 / 3896.
-//   little work beside the 0.1 ms, rows * H * I <= 2^34 (a decode's price goes with H I): 512 x 256, 16 experts, 1000 tokens
-//   51 / 141; 2048 x 1024, 64 experts, 750 tokens 217 / 277; 6144 x 2048, 8 experts, 93 tokens 146 / 201. At the line 0.84 to 1.02 of
-//   tall over ten shapes, at twice the line 1.06 to 1.27 for all but one.
-// Without side streams the tall tiles' launches follow one another and the line lies at 2^36: 6144 x 2048, 16 experts, 383 tokens 540 / 505
-// and (Zipf) 530 / 917, 1000 tokens, beyond it, 1205 / 1066 and 1204 / 1296; 64 experts 633 / 746 and 741 / 1448, 1338 / 1409 and
-// 1400 / 1760, 2000 tokens 2498 / 2158 and 2466 / 2478.
-static bool pf_is_short(int64_t P, int E, int H, int I, bool fork) { return P <= 32 * (int64_t)E || P * H * I <= (int64_t)1 << (fork ? 34 : 36); }
+// tiles, which cost a launch more to list them, two or three for every one of the other plan, and the events of the side streams. us short / tall:
+//   few rows per expert (E = 256 of 6144 x 2048, top-8): 200 tokens, level 4, evenly 2387 / 2400, Zipf(1.1) popularity 2196 / 2169; 400 tokens
+//   2465 / 2477 and 2579 / 2451; 1000 tokens 2850 / 2865 and 3319 / 2970, of mixed levels 2014 / 2043 and 2313 / 2135. The line is where
+//   popular experts begin to take several short tiles, at 8 rows an expert on average: beyond it up to 1.5 % lost evenly, 4 to 10 gained.
+//   little work beside what the plan costs (a decode's price goes with H I): up to rows * H * I = 2^32 always (1000 tokens, 16 experts of 512 x 256
+//   85 / 115; 50 tokens, 8 of 6144 x 2048 156 / 190), up to 2^34 unless the average expert has more than 96 rows, two tiles (400 tokens, 64 of
+//   2048 x 1024 220 / 250; 170 tokens, 16 of 6144 x 2048, Zipf 288 / 308; 32 370 / 385, 455 / 500; but 130 tokens, 8 330 / 232; 3000 tokens, 64 of 1024 x
+//   512 209 / 187).
+// Without side streams the chains follow one another, and the lines lie at 32 rows an expert and at 2^35: 200 tokens, 64 experts, Zipf 580 / 695, 300
+// 698 / 743; 400 tokens, 256 experts 2546 / 2559, 1000 2323 / 2200 and evenly 2011 / 2030; 170 tokens, 16 experts 300 / 433. Beyond them 383 tokens, 16
+// experts 729 / 690 and evenly 740 / 466; 683, 64 experts 1364 / 1245 and 1462 / 1040.
+static bool pf_is_short(int64_t P, int E, int H, int I, bool fork)
+{
+    const int64_t work = P * H * I;
+    return P <= (fork ? 8 : 32) * (int64_t)E || work <= (int64_t)1 << 32 || (P <= 96 * (int64_t)E && work <= (int64_t)1 << (fork ? 34 : 35));
+}
 
 // Which experts take decoded weights: at least WIDE_MIN rows (three tiles), above level 2, if their tiles make WIDE_UNITS units of gate|up
 // together (two per CU; the plan counts them). us a step without / from 512 / 768 / 1024 rows on (6144 x 2048, top-8, level 4): 4096 tokens, 256
@@ -872,30 +927,40 @@ int launch_pf_step(const NqPfArgs& a, hipStream_t st)
         }
         return launch_pf_post(y, m.pos, a.sel, a.sel_dtype, a.rw, a.rw_dtype, a.T, a.topk, 0, P, a.table, a.out, a.out_dtype, 0, a.zd, E, H, I, st);
     }
-    // Tile heights 256 | 128 | 64, 32, 16 as four chains: the tallest on the caller's stream, the others on side streams between two
+    // Tile heights 256 | 128 | up to 64 as three chains: the tallest on the caller's stream, the others on side streams between two
     // events. A GEMM launch ends with the GPU partly idle while its last workgroups drain; the chains fill each other's tails, and
-    // the memory-bound kernels of one height run under the GEMMs of another.
-    // Without side streams the chains follow one another on the caller's.
-    hipStream_t streams[4] = {st, st, st, st};
-    for (int i = 0; fork && i < 3; ++i) streams[i + 1] = (hipStream_t)a.side[i];
-    static const int stream_of[5] = {3, 3, 2, 1, 0};             // by height 16 << k
+    // the memory-bound kernels of one height run under the GEMMs of another. The tiles of up to 64 rows are one launch over one list.
+    // Without side streams the chains follow one another on the caller's. us a step as four chains over five lists with a place for every expert / as
+    // now: 1000 tokens, 256 experts, level 4, Zipf 2835 / 2760, evenly 2745 / 2665; 4096 tokens of mixed levels 4195 / 4000; 170 tokens, 8 experts
+    // 335 / 261; without side streams 1000 tokens, 16 experts 1353 / 1165, 2000, 64 experts 2793 / 2330. With the tallest on a side stream and
+    // the rest on the caller's 170 tokens, 8 experts took 328.
+    // The activations are prepared for all rows in one launch (a launch per height, each passing over the others' rows, 315 us in place of 261); so is h where nothing runs beside it.
+    constexpr int CHAINS = 3;
+    static const int heights[CHAINS] = {16, 8, 7};               // bit k = height 16 << k
+    hipStream_t streams[CHAINS] = {st, st, st};
+    for (int i = 1; fork && i < CHAINS; ++i) streams[i] = (hipStream_t)a.side[i - 1];
     auto hip_ok = [](hipError_t e) { return e == hipSuccess ? 0 : set_error("nq_pf_step: %s", hipGetErrorString(e)); };
     for (int c = 0; c < P; c += R)
     {
         const int n = P - c < R ? P - c : R;
         const bool wop = a.wop && n >= a.hot_min;
-        if (int rc = launch_pf_plan(m.cnt, E, c, n, m.tiles, m.cap, wop ? m.hot : nullptr, a.hot_min, a.wop_slots, wop ? m.wide : nullptr, advised ? wide_tiles(I) : 0, advised ? a.table : nullptr, st)) return rc;
+        if (int rc = launch_pf_plan(m.cnt, E, c, n, m.tiles, m.cap, wop ? m.hot : nullptr, a.hot_min, a.wop_slots, wop ? m.wide : nullptr, advised ? wide_tiles(I) : 0, advised ? a.table : nullptr,
+                                    m.dense, a.table, st)) return rc;
         const int most = std::min(m.cap, n / 256 + a.wop_slots / 2 + 1);       // tiles of decoded weights: an expert of r rows has (r + 127) / 256
+        if (int rc = launch_pf_pre(a.x, a.x_dtype, m.pt + c, m.pe + c, n, a.table, a.xg, a.xu, a.zg, E, H, I, nullptr, 0, 0, st)) return rc;
         if (fork) if (int rc = hip_ok(hipEventRecord((hipEvent_t)a.events[0], st))) return rc;
-        for (int i = 1; fork && i < 4; ++i) if (int rc = hip_ok(hipStreamWaitEvent(streams[i], (hipEvent_t)a.events[0], 0))) return rc;
-        const int32_t *pts = m.pt + c, *pes = m.pe + c;
-        static const int heights[4] = {16, 8, 4, 3};             // bit k = height 16 << k
+        for (int i = 1; fork && i < CHAINS; ++i) if (int rc = hip_ok(hipStreamWaitEvent(streams[i], (hipEvent_t)a.events[0], 0))) return rc;
         auto gemms = [&](int mode) {
-            for (int k = 4; k >= 0; --k)
-                for (int v = 0; v < 2; ++v)
-                    if (variants >> v & 1)
-                        if (int rc = launch_pf_gemm(a.table, m.tiles + (size_t)k * m.cap * 4, k < 4 ? E : m.cap, 16 << k, mode | 2 * v | (variants == 1 ? 4 : 0), mode ? a.h : a.xg,
-                                                    mode ? nullptr : a.xu, mode ? y : acc, E, H, I, wop, streams[stream_of[k]])) return rc;
+            const int32_t* lists[CHAINS] = {m.dense + 8 * (size_t)E, m.dense + 4 * (size_t)E, m.dense};
+            const int counts[CHAINS] = {n / 129, std::min(E, n / 65), std::min(E, n)};      // the most tiles that n rows make
+            for (int i = 0; i < CHAINS; ++i)
+            {
+                static const int bm[CHAINS] = {256, 128, SHORT_LIST};
+                const PfGemm g{a.table, lists[i], (const _Float16*)(mode ? a.h : a.xg), (const _Float16*)(mode ? nullptr : a.xu), mode ? y : acc, mode, E, H, I, variants == 1, wop};
+                if (!counts[i]) continue;
+                if (variants & 1) if (int rc = launch_tiles<false>(g, bm[i], counts[i], streams[i])) return rc;
+                if (variants & 2) if (int rc = launch_tiles<true>(g, bm[i], counts[i], streams[i])) return rc;
+            }
             if (wop) if (int rc = launch_pf_wdecode(a.table, m.hot, E, m.wide, mode, a.wop, a.wop_slots, H, I, st)) return rc;
             if (wop)
                 if (int rc = launch_wide(PfWide{a.table, m.wide + 4, m.wide, (const _Float16*)(mode ? a.h : a.xg), (const _Float16*)(mode ? nullptr : a.xu), mode ? y : acc, (const u32x4*)a.wop,
@@ -903,15 +968,13 @@ int launch_pf_step(const NqPfArgs& a, hipStream_t st)
             return 0;
         };
         auto chains = [&]() {
-            for (int i = 0; i < 4; ++i)
-                if (int rc = launch_pf_pre(a.x, a.x_dtype, pts, pes, n, a.table, a.xg, a.xu, a.zg, E, H, I, m.tiles, m.cap, heights[i], streams[i])) return rc;
             if (int rc = gemms(0)) return rc;
-            for (int i = 0; i < 4; ++i)
-                if (int rc = launch_pf_mid(acc, pes, n, a.table, a.h, a.zg, a.zd, E, H, I, m.tiles, m.cap, heights[i], streams[i])) return rc;
+            for (int i = 0; i < (fork ? CHAINS : 1); ++i)
+                if (int rc = launch_pf_mid(acc, m.pe + c, n, a.table, a.h, a.zg, a.zd, E, H, I, fork ? m.tiles : nullptr, m.cap, heights[i], streams[i])) return rc;
             return gemms(1);
         };
         const int failed = chains();
-        for (int i = 1; fork && i < 4; ++i)                      // joined in any case: the caller gives the buffers back in its stream's order
+        for (int i = 1; fork && i < CHAINS; ++i)                 // joined in any case: the caller gives the buffers back in its stream's order
         {
             if (int rc = hip_ok(hipEventRecord((hipEvent_t)a.events[i], streams[i]))) return rc;
             if (int rc = hip_ok(hipStreamWaitEvent(st, (hipEvent_t)a.events[i], 0))) return rc;

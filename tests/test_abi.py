@@ -160,8 +160,8 @@ def test_which_steps_are_given_decoded_weights():
     assert slots(1024, 8, 8, 2048, 2048) == 8 and slots(1023, 8, 8, 2048, 2048) == 0          # 32 tiles of 256 rows
     assert slots(767, 64, 8, 6144, 2048) == 0
     assert slots(1000, 8, 256, 6144, 2048) == 0                  # at most 32 rows per expert on average
-    assert slots(4096, 8, 16, 1024, 512) == 0                    # little work
-    assert slots(4096, 8, 16, 2048, 512, side=0) == 0 and slots(4096, 8, 16, 2048, 512) == 16      # without side streams short tiles go further
+    assert slots(4096, 8, 16, 256, 512) == 0                     # little work
+    assert slots(1100, 8, 280, 6144, 2048, side=0) == 0 and slots(1100, 8, 280, 6144, 2048) > 0    # without side streams short tiles go further
     assert slots(4096, 8, 64, 4096, 1152) == 0 and slots(4096, 8, 64, 4096, 1024) > 0
     assert slots(4096, 8, 256, 6144, 2048, rows=4096) == 0       # chunks of few rows
     for bad in ((-1, 8, 16, 2048, 1024), (4096, 0, 16, 2048, 1024), (4096, 8, 0, 2048, 1024), (4096, 8, 16, 2000, 1024), (4096, 8, 16, 2048, 0)):

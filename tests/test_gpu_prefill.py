@@ -383,6 +383,31 @@ def grouped_step_against_slices(H, I, T, E, K, Bmax, xd, wd, sd):
     assert not y[5].any()                                         # all its picks at level 0
 
 
+@pytest.mark.parametrize("R", [None, 500])
+def test_tiles_of_every_list_of_a_tall_step(R):
+    """remainders at the edges of the three lists that the GEMMs are launched on, with and without full tiles before them, at levels 0, 2 and 4 (above
+    2 first), in one pass and in chunks of pair rows that cut experts: equal to the decode kernels, the same bits without side streams"""
+    H, I = 2560, 2304
+    rows = [1, 0, 64, 65, 128, 129, 256, 257, 16, 255, 40, 192, 3]
+    ex = to_dev(experts_on_gpu(H, I, 6, 83, nested_ids=(1, 3)))
+    L = M.MoELayer(len(rows), H, I, Bmax=8, topk=1)
+    for e in range(len(rows)):
+        L.set(e, ex[e % 6], 0 if e == 8 else 4 if ex[e % 6].nested or e in (2, 4, 11) else 2)
+    g = torch.Generator().manual_seed(84)
+    sel = torch.repeat_interleave(torch.arange(len(rows)), torch.tensor(rows))[torch.randperm(sum(rows), generator=g)].view(-1, 1).to(DEV)
+    rw = (torch.rand(sel.shape, generator=g) + 0.1).half().to(DEV)
+    x = (torch.randn(sel.shape[0], H, generator=g) * 0.3).half().to(DEV)
+    got = L.prefill(x, sel, rw, R=R)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        held = L.prefill(x, sel, rw, R=R)
+    graph.replay()
+    want = sliced_decode(L, x, sel, rw)
+    torch.cuda.synchronize()
+    assert torch.equal(got, held)
+    assert rel_err(got.cpu().numpy(), want.cpu().numpy()) < 5e-5 and not got[sel.flatten() == 8].any()
+
+
 @pytest.mark.parametrize("H,I,n", [(128, 128, 1), (640, 384, 37), (2176, 512, 2050), (256, 768, 4100)])
 def test_row_kernels_against_a_float64_hadamard(H, I, n):
     """nq_pf_pre and nq_pf_mid where chunks do not fill a wavefront's four and where a workgroup takes one, two, more rows"""
