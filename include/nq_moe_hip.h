@@ -284,8 +284,8 @@ int nq_proj(const void* x, int x_dtype, int B, const int64_t* row, int H, int I,
 /* A whole step of T tokens on device data, no host synchronisation: pairs sorted by expert, tile plan, rotation, gate|up, SwiGLU,
  * down, combine -- the chain of the entry points above (reference moe.prefill, sm120/moe.py:282-326) with the casts of its caller
  * (x.half(), ids.long(), w.half(), out.to(dtype), sm120/serve/nq_vllm.py:522,573) at the loads and the final store. Ids outside
- * [0, E) contribute nothing. Steps with at most 32 pairs per expert on average or pairs * H * I <= 2^34 run on `stream` alone, longer
- * ones fork onto the side streams, where there are some, and join again, also when a launch between fails. The bits do not depend on it. Calls that share scratch must be ordered on one
+ * [0, E) contribute nothing. Steps of few pairs per expert or little work run on `stream` alone, longer ones
+ * fork onto the side streams, where there are some, and join again, also when a launch between fails. The bits do not depend on it. Calls that share scratch must be ordered on one
  * stream; side streams and events belong to the calls of one stream. */
 typedef struct NqPfArgs
 {

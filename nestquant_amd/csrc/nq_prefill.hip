@@ -952,7 +952,7 @@ int launch_pf_step(const NqPfArgs& a, hipStream_t st)
         for (int i = 1; fork && i < CHAINS; ++i) if (int rc = hip_ok(hipStreamWaitEvent(streams[i], (hipEvent_t)a.events[0], 0))) return rc;
         auto gemms = [&](int mode) {
             const int32_t* lists[CHAINS] = {m.dense + 8 * (size_t)E, m.dense + 4 * (size_t)E, m.dense};
-            const int counts[CHAINS] = {n / 129, std::min(E, n / 65), std::min(E, n)};      // the most tiles that n rows make
+            const int counts[CHAINS] = {std::min(m.cap, n / 129), std::min(E, n / 65), std::min(E, n)};   // the most tiles that n rows make, all inside the list
             for (int i = 0; i < CHAINS; ++i)
             {
                 static const int bm[CHAINS] = {256, 128, SHORT_LIST};

@@ -408,6 +408,30 @@ def test_tiles_of_every_list_of_a_tall_step(R):
     assert rel_err(got.cpu().numpy(), want.cpu().numpy()) < 5e-5 and not got[sel.flatten() == 8].any()
 
 
+@pytest.mark.parametrize("E,T,R", [(3, 1000, None), (3, 1000, 900), (2, 1600, None), (16, 520, None)])
+def test_tile_lists_are_read_to_their_end_only(E, T, R):
+    """steps whose rows could make more tiles than their lists hold (few experts, no remainders to speak of), in memory that is full of valid
+    tiles of expert 0 and of nothing finite: every row is computed, none by an entry that is not the step's"""
+    H, I, K = 2048, 1024, min(E, 8)
+    ex = to_dev(experts_on_gpu(H, I, 2, 87, nested_ids=(1,)))
+    L = M.MoELayer(E, H, I, Bmax=8, topk=K)
+    for e in range(E):
+        L.set(e, ex[e % 2], 4 if e % 2 else 2)
+    g = torch.Generator().manual_seed(88)
+    sel = torch.stack([torch.randperm(E, generator=g)[:K] for _ in range(T)]).to(DEV)
+    rw = (torch.rand(T, K, generator=g) + 0.1).half().to(DEV)
+    x = (torch.randn(T, H, generator=g) * 0.3).half().to(DEV)
+    want = sliced_decode(L, x, sel, rw)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    n = 4 * T * K * (2 * H + 3 * I) + (1 << 22)                   # beyond the step's scratch
+    for junk in ([0, 0, 256, 0], [-1, -1, -1, -1]):              # as floats, 0xffffffff is NaN
+        torch.tensor(junk, dtype=torch.int32, device=DEV).repeat(n // 2)
+        got = L.prefill(x, sel, rw, R=R)
+        torch.cuda.synchronize()
+        assert rel_err(got.cpu().numpy(), want.cpu().numpy()) < 5e-5, junk
+
+
 @pytest.mark.parametrize("H,I,n", [(128, 128, 1), (640, 384, 37), (2176, 512, 2050), (256, 768, 4100)])
 def test_row_kernels_against_a_float64_hadamard(H, I, n):
     """nq_pf_pre and nq_pf_mid where chunks do not fill a wavefront's four and where a workgroup takes one, two, more rows"""
