@@ -240,10 +240,9 @@ static __device__ __constant__ const RcpTable c_rcp = make_rcp();
 // level-2 constants with the ring's sign (sgm = 0x80008000 negates exactly)
 __device__ __forceinline__ FoldK consts_l2(uint32_t sgm) { return FoldK{0u, 0u, MUL1_A2 ^ sgm, MUL1_B2 ^ sgm}; }
 // fold constants, fp32 operations in the spec's order without contraction (reference sm120/ref15_spec.py:79-84)
-__device__ __forceinline__ uint32_t fold_ac(uint32_t dw)         // A' | C << 16
+__device__ __forceinline__ uint32_t fold_ac(uint32_t dw, float rc)                   // A' | C << 16; rc = 1 / Mb, c_rcp's
 {
-    const uint32_t Mb = dw & 0xFFu, N = (dw >> 8) & 0xFFu;
-    const float rc = c_rcp.v[Mb];
+    const uint32_t N = (dw >> 8) & 0xFFu;
     const _Float16 Ah = (_Float16)__fmul_rn(1.732421875f, rc);
     const float t = __fadd_rn(__fmul_rn(__fmul_rn((float)N, rc), -3.453125f), -3.453125f);
     const _Float16 Ch = (_Float16)__fsub_rn(t, __fmul_rn(1024.f, (float)Ah));
@@ -255,7 +254,7 @@ __device__ __forceinline__ FoldK fold_k(uint32_t dw, uint32_t ac, uint32_t sgm)
     return FoldK{__builtin_amdgcn_perm(dw, dw, 0x00000000u), __builtin_amdgcn_perm(dw, dw, 0x01010101u),
                  __builtin_amdgcn_perm(ac, ac, 0x01000100u) ^ sgm, __builtin_amdgcn_perm(ac, ac, 0x03020302u) ^ sgm};
 }
-__device__ __forceinline__ FoldK consts_fold(uint32_t dw, uint32_t sgm) { return fold_k(dw, fold_ac(dw), sgm); }
+__device__ __forceinline__ FoldK consts_fold(uint32_t dw, uint32_t sgm) { return fold_k(dw, fold_ac(dw, c_rcp.v[dw & 0xFFu]), sgm); }
 
 __device__ __forceinline__ uint32_t pk_fma(uint32_t h, uint32_t a, uint32_t c)
 {

@@ -653,11 +653,13 @@ __device__ __forceinline__ void finish_dn_all(const MoeArgs& a, const PickInfo& 
 // +1.5 us), so the register allocator is told to aim at exactly that. The common down launch gains from five (90 registers): its
 // 1536 workgroups then need 1.2 rounds instead of 1.5 (-0.4 us per layer at one token, -2.5 us at four).
 // OWN (gate|up of the common rows only): no routing launch comes before, see launch_moe; the last plane of blocks does that launch's other
-// work. A kernel of its own: carried along in the other one, unused, it cost 0.5 to 1.5 % of a call.
-template <int MODE, bool ANYROW, bool OWN = false>
+// work. A kernel of its own: carried along in the other one, unused, it cost 0.5 to 1.5 % of a call. The down launch behind it (SMALL too) differs by
+// gemv_chunks' FEW alone.
+template <int MODE, bool ANYROW, bool SMALL = false>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == 1 && !ANYROW ? 5 : 4, MODE == 1 && !ANYROW ? 5 : 4)))
 nq_gemv_k(MoeArgs a, int NC)
 {
+    constexpr bool OWN = SMALL && MODE == 0;
     extern __shared__ __align__(16) char smem[];
     // Exactly four gate|up workgroups per CU: at one token the launch has four for every CU, and with room for a fifth the
     // dispatcher fills some CUs with five and leaves others with three. The body needs 90 registers; naming v100 claims 104.
@@ -826,11 +828,11 @@ nq_gemv_k(MoeArgs a, int NC)
     }
     else if (R.level == 2)
     {
-        if (a.hoist && P.var == nullptr) gemv_chunks<false, 0, 0, false, true>(P, L, NC, acc, nb0);   // block-uniform: the caller's option
-        else gemv_chunks<false, 0, 0, false>(P, L, NC, acc, nb0);
+        if (a.hoist && P.var == nullptr) gemv_chunks<false, 0, 0, false, true, SMALL>(P, L, NC, acc, nb0);   // block-uniform: the caller's option
+        else gemv_chunks<false, 0, 0, false, false, SMALL>(P, L, NC, acc, nb0);
     }
-    else if (a.hoist && P.var == nullptr) dispatch_code(P.code, [&](auto tag) { gemv_chunks<true, decltype(tag)::value, 0, false, true>(P, L, NC, acc, nb0); });
-    else dispatch_code(P.code, [&](auto tag) { gemv_chunks<true, decltype(tag)::value, 0, false>(P, L, NC, acc, nb0); });
+    else if (a.hoist && P.var == nullptr) dispatch_code(P.code, [&](auto tag) { gemv_chunks<true, decltype(tag)::value, 0, false, true, SMALL>(P, L, NC, acc, nb0); });
+    else dispatch_code(P.code, [&](auto tag) { gemv_chunks<true, decltype(tag)::value, 0, false, false, SMALL>(P, L, NC, acc, nb0); });
 
     __builtin_amdgcn_s_setprio(3);                               // the tail is a chain of latencies: nothing should wait behind decoders
     PickLanes picks = {};
@@ -929,7 +931,7 @@ int launch_moe(const MoeArgs& a, const int* cfg_gu, const int* cfg_dn, int which
         b.fuse = which == 3 || defer;                             // both launches belong to this call (or the caller says the other one follows)
         b.mb_apply = a.mb_table != nullptr && mode == last_mode;  // the call's last projection launch carries the mailbox block
         const bool self = own && mode == 0;
-        auto kern = self ? nq_gemv_k<0, false, true> : mode == 0 ? (any ? nq_gemv_k<0, true> : nq_gemv_k<0, false>) : (any ? nq_gemv_k<1, true> : nq_gemv_k<1, false>);
+        auto kern = self ? nq_gemv_k<0, false, true> : mode == 0 ? (any ? nq_gemv_k<0, true> : nq_gemv_k<0, false>) : (any ? nq_gemv_k<1, true> : own ? nq_gemv_k<1, false, true> : nq_gemv_k<1, false>);
         if (shm > 48 * 1024)
         {
             hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, shm);

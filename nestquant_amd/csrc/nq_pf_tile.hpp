@@ -105,7 +105,7 @@ __device__ __forceinline__ void pf_chunks(const Planes& P, const LaneCtx& L, int
     const uint64_t mflags = masked ? (P.flags ? P.flags[L.strip] : (C >= 64 ? ~0ull : (1ull << C) - 1ull)) : 0ull;
     if constexpr (RES && !masked) load_record<CODE>(nr, P.res, L.rec0, L.nrec);
     UnitConsts<RES> consts;                                      // mask mode works a chunk's constants out itself
-    if constexpr (!masked) consts.start(P, L, C);
+    if constexpr (!masked) consts.start(unit_words(P, L, 0, C, RES));
     else if (P.var) nvar = at_offset<uint8_t>(P.var, L.unit0);
     const int lane = threadIdx.x & 63, warp = threadIdx.x >> 6, t4 = lane >> 4, n = lane & 15;
     const TokenSource tokens = token_source(A, K, row0, nrows, smem, warp, lane);
@@ -144,6 +144,7 @@ __device__ __forceinline__ void pf_chunks(const Planes& P, const LaneCtx& L, int
             if constexpr (RES && !masked) load_record<CODE>(nr, P.res, L.rec0 + (uint32_t)(c + 1) * 32, L.nrec);
             if (masked && P.var) nvar = at_offset<uint8_t>(P.var, L.unit0 + c + 1);
         }
+        if constexpr (!masked) consts.begin(P, L, c, C);
         ext_base<BK>(wb, __shfl(wb[0], L.src));
         const uint32_t sgm = masked ? ((var >> L.g) & 1u) * 0x80008000u : 0u;
         half8_t aop[4][2];
@@ -153,7 +154,7 @@ __device__ __forceinline__ void pf_chunks(const Planes& P, const LaneCtx& L, int
             {
                 prepare_record<CODE>(wr);
                 ext_words<Rec<CODE>::BITS, Rec<CODE>::NW>(wr, __shfl(wr[0], L.src));
-                if constexpr (masked) consts.k = consts_fold(dw, sgm); else consts.take(P, L, c, C);
+                if constexpr (masked) consts.k = consts_fold(dw, sgm); else consts.take(P, L, c);
                 const FoldK& k = consts.k;
                 static_for<4>([&](auto mm) {
                     constexpr int MM = decltype(mm)::value;
@@ -165,7 +166,7 @@ __device__ __forceinline__ void pf_chunks(const Planes& P, const LaneCtx& L, int
         }
         else
         {
-            if constexpr (masked) consts.k = consts_l2(sgm); else consts.take(P, L, c, C);
+            if constexpr (masked) consts.k = consts_l2(sgm); else consts.take(P, L, c);
             const FoldK& k = consts.k;
             static_for<4>([&](auto mm) {
                 constexpr int MM = decltype(mm)::value;

@@ -280,38 +280,50 @@ struct LaneCtx
     uint32_t half0;       // unit index of strip lane / 32 of the wavefront's two, first chunk (UnitConsts)
 };
 
+// Block word and sign byte of chunk c + lane % 32 (the last one's beyond it) of strip lane / 32 of the wavefront's two; res: the level has block words
+struct UnitWords { uint32_t word, var; };
+__device__ __forceinline__ UnitWords unit_words(const Planes& P, const LaneCtx& L, int c, int NC, bool res)
+{
+    const uint32_t unit = L.half0 + (uint32_t)min(c + (int)(threadIdx.x & 31), NC - 1);
+    UnitWords w = {0u, 0u};
+    if (res) w.word = at_offset<uint32_t>((gp_u8)P.dw, unit * 4u);
+    if (P.var) w.var = at_offset<uint8_t>(P.var, unit);
+    return w;
+}
+
 // What a chunk's decode needs beside the records, fold constants and ring signs, for 32 chunks of the wavefront's two strips at a time: lane 32 s + i
 // reads the block word and sign byte of strip s, chunk c0 + i, and works out its constants; a chunk's come from there by one
 // lane permute (two at levels 3 / 4). Worked out by every lane in every chunk they were some 25 of the 600 vector instructions of a refined chunk
-// and, with no sign plane, 5 of the 275 of a chunk at level 2, beside one or two loads.
+// and, with no sign plane, 5 of the 275 of a chunk at level 2, beside one or two loads. us anew in every chunk / as now: 4 tokens of 6144 x 2048 203 / 198,
+// one 63.3 / 62.0, a lone gate|up projection of 8 tokens at level 3 13.8 / 13.5, 48 and 201 tokens 1144 / 1127 and 1335 / 1307.
 template <bool RES>
 struct UnitConsts
 {
     uint32_t word, ac, next_word, next_var;       // block word | sign byte << 16; fold_ac of it; as loaded, 32 chunks on
     int from;                                     // 4 * the lane that holds this lane's strip, chunk 0
     FoldK k;
-    __device__ __forceinline__ void request(const Planes& P, const LaneCtx& L, int c, int NC)
+    __device__ __forceinline__ void start(const UnitWords& first)
     {
-        const uint32_t unit = L.half0 + (uint32_t)min(c + (int)(threadIdx.x & 31), NC - 1);
-        if constexpr (RES) next_word = at_offset<uint32_t>((gp_u8)P.dw, unit * 4u);
-        if (P.var) next_var = at_offset<uint8_t>(P.var, unit);
-    }
-    __device__ __forceinline__ void start(const Planes& P, const LaneCtx& L, int NC)
-    {
-        word = ac = next_word = next_var = 0u;
+        word = ac = 0u; next_word = first.word; next_var = first.var;
         from = (int)(threadIdx.x & 8u) << 4;
         k = consts_l2(0u);
-        request(P, L, 0, NC);
     }
-    // the constants of chunk c, in k
-    __device__ __forceinline__ void take(const Planes& P, const LaneCtx& L, int c, int NC)
+    // at chunk c's beginning, ahead of the next chunk's requests: behind them, with a branch in between, the wait for the block words was one for those
+    // requests too. The reciprocal is divided out (IEEE, the table's bits): its entry would be another latency before a slice's first product.
+    __device__ __forceinline__ void begin(const Planes& P, const LaneCtx& L, int c, int NC)
     {
         if ((RES || P.var) && (c & 31) == 0)
         {
-            if constexpr (RES) ac = fold_ac(next_word);
+            const uint32_t Mb = next_word & 0xFFu;
+            if constexpr (RES) ac = fold_ac(next_word, Mb ? 1.0f / (float)Mb : 0.f);
             word = (next_word & 0xFFFFu) | next_var << 16;
-            if (c + 32 < NC) request(P, L, c + 32, NC);
+            const UnitWords next = unit_words(P, L, c + 32, NC, RES);      // the last chunk's once more, where there are none: no branch
+            next_word = next.word; next_var = next.var;
         }
+    }
+    // the constants of chunk c, in k
+    __device__ __forceinline__ void take(const Planes& P, const LaneCtx& L, int c)
+    {
         const int lane = from + 4 * (c & 31);
         if constexpr (RES) k = fold_k((uint32_t)__builtin_amdgcn_ds_bpermute(lane, (int)word), (uint32_t)__builtin_amdgcn_ds_bpermute(lane, (int)ac), 0u);
         if (P.var)
@@ -381,7 +393,9 @@ __device__ __forceinline__ void gemv_chunks_masked(const Planes& P, const LaneCt
 // loop's ~276 vector instructions per chunk) and, with it, the rounding of each weight to fp16: the result is that of the
 // UNROUNDED weights, ~2e-4 (relative, l2) from the product with the exact fp16 weights that the other form and the reference
 // compute -- inside the layer's 1e-3, outside the 5e-5 that the exact form holds, hence an option the caller has to ask for.
-template <bool RES, int CODE, int BK = 0, bool MASKOK = true, bool RAW = false>
+// FEW (slices of few chunks that nothing runs beside): every lane works out its own unit's constants chunk by chunk instead. UnitConsts' permutes and its
+// work at a slice's beginning are latency there: a layer of 512 x 256, two tokens, 14.1 us / 14.3 with them.
+template <bool RES, int CODE, int BK = 0, bool MASKOK = true, bool RAW = false, bool FEW = false>
 __device__ __forceinline__ void gemv_chunks(const Planes& P, const LaneCtx& L, int NC, float4_t* acc, u32x4 nb)
 {
     static_assert(!RAW || BK == 0, "the hoisted value map is built for base window code 0");
@@ -396,10 +410,15 @@ __device__ __forceinline__ void gemv_chunks(const Planes& P, const LaneCtx& L, i
     if constexpr (RES && MASKOK)
         if (P.flags) { gemv_chunks_masked<CODE, BK>(P, L, NC, acc, nb); return; }     // block-uniform
     constexpr int NW = RES ? Rec<CODE>::NW : 1;
-    uint32_t nr[NW + 2] = {0};
-    if constexpr (RES) load_record<CODE>(nr, P.res, L.rec0, L.nrec);
+    uint32_t nr[NW + 2] = {0}, ndw = 0, nvar = 0;
     UnitConsts<RES> consts;
-    consts.start(P, L, NC);
+    if constexpr (!FEW) consts.start(unit_words(P, L, 0, NC, RES));              // before the records: they are waited for first
+    if constexpr (RES) load_record<CODE>(nr, P.res, L.rec0, L.nrec);
+    auto own_words = [&](int c) {                                // FEW
+        if constexpr (RES) ndw = at_offset<uint32_t>((gp_u8)P.dw, (L.unit0 + c) * 4u);
+        if (P.var) nvar = at_offset<uint8_t>(P.var, L.unit0 + c);
+    };
+    if constexpr (FEW) own_words(0);
     for (int c = 0; c < NC; ++c)
     {
         progress_priority(c, NC);
@@ -407,10 +426,13 @@ __device__ __forceinline__ void gemv_chunks(const Planes& P, const LaneCtx& L, i
         wb[0] = nb.x; wb[1] = nb.y; wb[2] = nb.z; wb[3] = nb.w;
 #pragma unroll
         for (int i = 0; i < NW; ++i) wr[i] = nr[i];
+        const uint32_t dw = ndw, sgm = ((nvar >> L.g) & 1u) * 0x80008000u;
+        if constexpr (!FEW) consts.begin(P, L, c, NC);
         if (c + 1 < NC)                                         // prefetch the next chunk's records
         {
             nb = load_base<BK>(P, L.rec0 + (uint32_t)(c + 1) * 32, L.nrec);
             if constexpr (RES) load_record<CODE>(nr, P.res, L.rec0 + (uint32_t)(c + 1) * 32, L.nrec);
+            if constexpr (FEW) own_words(c + 1);
         }
         ext_base<BK>(wb, __shfl(wb[0], L.src));
         if constexpr (RES)
@@ -418,7 +440,8 @@ __device__ __forceinline__ void gemv_chunks(const Planes& P, const LaneCtx& L, i
             prepare_record<CODE>(wr);
             ext_words<Rec<CODE>::BITS, Rec<CODE>::NW>(wr, __shfl(wr[0], L.src));
         }
-        consts.take(P, L, c, NC);
+        if constexpr (!FEW) consts.take(P, L, c);
+        else consts.k = RES ? consts_fold(dw, sgm) : consts_l2(sgm);
         const FoldK& k = consts.k;
         const char* xp = L.xs + c * L.xstep;
         if constexpr (RAW && RES)
