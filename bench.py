@@ -267,7 +267,7 @@ def prefill_leg(L, ex, dev, T=4096, reps=3):
     rel = float(np.linalg.norm(y[toks].cpu().numpy() - want) / np.linalg.norm(want))
     assert rel < 1e-3, f"prefill output of tokens {toks} is {rel:.2e} from the oracle"
     parts = prefill_parts(L, x, sel, dev)
-    # the same call with the operand scratch for experts of several tiles switched on (32 slots; off by default)
+    # the same call with decoded weights for every expert of several tiles (32 slots), in place of the library's own choice
     M.PF_HOT_SLOTS = 32
     try:
         yh = L.prefill(x, sel, rw)

@@ -1,5 +1,5 @@
 // Prefill path (steps of more tokens than a decode call takes): every routed expert's weights are decoded once per 16..256-row tile of its tokens, inside
-// the grouped GEMM itself, never written to HBM (reference: pf_decode to fp16 in HBM + Triton/cuBLAS grouped GEMM,
+// the grouped GEMM itself, not by way of HBM but for experts of many rows (reference: pf_decode to fp16 in HBM + Triton/cuBLAS grouped GEMM,
 // sm120/nqmoe.cu:942-1240, sm120/pf_gemm.py:7-34, sm120/moe.py:282-326).
 //
 //   nq_pf_sort_k  pairs sorted by expert, per-expert counts, hits; the tile list of a step without tall tiles
