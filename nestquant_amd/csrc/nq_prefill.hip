@@ -884,13 +884,14 @@ static bool pf_is_short(int64_t P, int E, int H, int I, bool fork)
     return P <= (fork ? 8 : 32) * (int64_t)E || work <= (int64_t)1 << 32 || (P <= 96 * (int64_t)E && work <= (int64_t)1 << (fork ? 34 : 35));
 }
 
-// Which experts take decoded weights: at least WIDE_MIN rows (three tiles), above level 2, if their tiles make WIDE_UNITS units of gate|up
-// together (two per CU; the plan counts them). us a step without / from 512 / 768 / 1024 rows on (6144 x 2048, top-8, level 4): 4096 tokens, 256
-// experts, Zipf 5743 / 5679 / 5609 / 5688; 32 experts, evenly 3976 / 3776 / 3735 / 3869; 16 experts, Zipf 3910 / 3459 / 3481 / 3647;
-// 2000 tokens, 16 experts, evenly 1997 / 1830 / 1847 / 2048. At level 2, where a tile's decode is half as long, 16 experts of 2048 rows lose: 3173 / 3281.
+// Which experts take decoded weights: at least WIDE_MIN rows (two and a half tiles), above level 2, if their tiles make WIDE_UNITS units of gate|up
+// together (two per CU; the plan counts them). us a step from 512 / 640 / 768 / 1024 rows on (6144 x 2048, top-8, level 4): 4096 tokens, 256
+// experts, Zipf 5198 / 5260 / 5300 / 5222; 64 experts, Zipf 4002 / 3890 / 3962 / 3896; 32, evenly 3656 / 3665 / 3666 / 3850; 16, Zipf 3270 / 3275 / 3268 / 3484;
+// 2000 tokens, 64 experts, Zipf 2190 / 2210 / 2225 / 2220; 16, evenly 1791 / 1792 / 1793 / 1892. On another box without /
+// from 768 on 5335 / 5325, 4030 / 3985, 3840 / 3678, 3763 / 3288, 2175 / 2181, 1888 / 1774. At level 2, where a tile's decode is half as long, 16 experts of 2048 rows lose: 3173 / 3281.
 // Fewer units leave CUs idle for the 0.2 ms of one: 1000 tokens, 16 experts, Zipf (a single expert of 993 rows) 1070 / 1173.
 // A block of 128 weight rows costs what one of 256 does: 2304 + 4096 rows, 11 % of them padding in gate|up, 1922 / 1961. Scratch: 2 GB at most.
-constexpr int WIDE_MIN = 768, WIDE_UNITS = 512;
+constexpr int WIDE_MIN = 640, WIDE_UNITS = 512;
 constexpr int64_t WIDE_BYTES = (int64_t)1 << 31;
 static int wide_tiles(int I) { const int ncol = 2 * ((I + 255) / 256); return (WIDE_UNITS + ncol - 1) / ncol; }
 

@@ -155,10 +155,10 @@ def test_which_steps_are_given_decoded_weights():
 
     def slots(T, topk, E, H, I, rows=32768, side=1):
         return L.nq_pf_wide_slots(T, topk, rows, E, H, I, side, C.byref(m))
-    assert slots(4096, 8, 256, 6144, 2048) == 2**31 // (6 * 6144 * 2048) and m.value == 768
+    assert slots(4096, 8, 256, 6144, 2048) == 2**31 // (6 * 6144 * 2048) and m.value == 640
     assert slots(1100, 8, 8, 2048, 2048) == 8
     assert slots(1024, 8, 8, 2048, 2048) == 8 and slots(1023, 8, 8, 2048, 2048) == 0          # 32 tiles of 256 rows
-    assert slots(767, 64, 8, 6144, 2048) == 0
+    assert slots(639, 64, 8, 6144, 2048) == 0
     assert slots(1000, 8, 256, 6144, 2048) == 0                  # at most 32 rows per expert on average
     assert slots(4096, 8, 16, 256, 512) == 0                     # little work
     assert slots(1100, 8, 280, 6144, 2048, side=0) == 0 and slots(1100, 8, 280, 6144, 2048) > 0    # without side streams short tiles go further
