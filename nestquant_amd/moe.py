@@ -334,14 +334,19 @@ def _pf_slots(R):
 
 
 def pf_bytes(H, I, R, G=0):
-    """bytes of prefill scratch for R pair rows (G is accepted for signature compatibility: the decoded-weight scratch is sized
-    by the rows, not by a group of experts)"""
-    return _pf_offsets(H, I, R)[1] + _pf_slots(R) * 6 * H * I
+    """bytes of scratch that a step of up to R pair rows at a time takes beside its lists (nq_pf_meta_bytes): the regions of pf_scratch and the decoded
+    weights. With PF_HOT_SLOTS = 0 the most that the library gives any step of such chunks, whatever its tokens, picks and experts. (G is accepted for
+    signature compatibility: the decoded-weight scratch is sized by the rows, not by a group of experts)"""
+    slots = _pf_slots(R)
+    if PF_HOT_SLOTS == 0 and R > 0:                  # a step of one pair more than a chunk holds, over more experts than could take a slot
+        slots = _lib.lib().nq_pf_wide_slots(min(R + 1, 2**31 - 1), 1, R, R, H, I, 1, C.byref(C.c_int32()))
+    return _pf_offsets(H, I, R)[1] + slots * 6 * H * I
 
 
 def pf_scratch(dev, H, I, R, G=0):
     """Prefill scratch for R pair rows on `dev`, not initialised: xg | xu fp16 [R, H], acc fp32 [R, 2I], h fp16 [R, I], y fp32
-    [R, H], the low-rank plane's zg | zd fp32 [R, 4], and wop: decoded weights of up to PF_HOT_SLOTS hot experts (None without).
+    [R, H], the low-rank plane's zg | zd fp32 [R, 4], and wop: decoded weights of up to PF_HOT_SLOTS hot experts (None without; what a step takes by the
+    library's own choice is not in it, see pf_bytes).
     A set belongs to whoever asks for it, and every step takes one of its own from torch's allocator: what another layer, stream
     or thread has in flight, or a captured graph holds, is never shared. Unlike the reference (sm120/moe.py:262-274), which
     keeps one set per device and decodes every expert of a group into it, only experts with several tiles go through

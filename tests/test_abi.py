@@ -169,6 +169,20 @@ def test_which_steps_are_given_decoded_weights():
     assert L.nq_pf_wide_slots(4096, 8, 32768, 256, 6144, 2048, 1, None) == 0
 
 
+def test_pf_bytes_covers_the_decoded_weights_of_every_step():
+    """pf_bytes knows the rows of a chunk only: it holds what nq_pf_wide_slots gives any step of such chunks, and is no larger than the largest of them"""
+    from nestquant_amd import moe as M
+    assert M.PF_HOT_SLOTS == 0
+    L, m = _lib.lib(), C.c_int32()
+    for H, I in ((6144, 2048), (2048, 2048), (4096, 1024), (4096, 1152), (512, 256)):
+        for R in (1, 640, 4096, 8191, 8192, 8800, 16384, 32768):
+            plain = M._pf_offsets(H, I, R)[1]
+            given = [L.nq_pf_wide_slots(T, k, R, E, H, I, side, C.byref(m)) for k in (1, 2, 8) for T in (R // k, R // k + 1, 4096, 40000)
+                     for E in (2, 16, 64, 256, 4096) for side in (0, 1) if min(T * k, R) == R]
+            assert M.pf_bytes(H, I, R) == plain + max(given) * 6 * H * I, (H, I, R)
+    assert M.pf_bytes(6144, 2048, 32768) - M._pf_offsets(6144, 2048, 32768)[1] == 28 * 6 * 6144 * 2048
+
+
 def test_counters_apart_are_asked_for_and_checked():
     """which bit 4 needs NQ_CNT_STEP * H / 128 counters and the down launch; without it H / 128 are enough, and no capacity changes what they mean"""
     L = _lib.lib()

@@ -526,6 +526,25 @@ def test_scratch_is_as_large_as_pf_bytes_says():
         assert S["wop"] is None and M.pf_scratch(torch.device(DEV), H, I, R)["xg"].data_ptr() != S["xg"].data_ptr()
 
 
+def test_a_step_takes_no_more_than_pf_bytes_says():
+    """the most that a step holds of the allocator's memory while it runs: pf_bytes and its lists, decoded weights among them"""
+    H = I = 2048
+    E, T = 8, 1100
+    L = M.MoELayer(E, H, I, Bmax=8, topk=8)
+    x, out = torch.zeros(T, H, dtype=torch.float16, device=DEV), torch.empty(T, H, device=DEV)
+    sel, rw = torch.arange(E, device=DEV).repeat(T, 1), torch.ones(T, E, dtype=torch.float16, device=DEV)
+    slots = M._lib.lib().nq_pf_wide_slots(T, 8, 8 * T, E, H, I, 1, M.C.byref(M.C.c_int32()))
+    L.prefill(x, sel, rw, out)                                   # side streams and the like are there
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    L.prefill(x, sel, rw, out)
+    took, lists = torch.cuda.max_memory_allocated() - before, M._lib.lib().nq_pf_meta_bytes(T, 8, 8 * T, E)
+    assert slots == E and took >= M._pf_offsets(H, I, 8 * T)[1] + slots * 6 * H * I
+    # the bound is for any number of experts: five slots more than this layer's eight; 2 MB of the allocator's rounding
+    assert took <= M.pf_bytes(H, I, 8 * T) + lists + (2 << 20) and M.pf_bytes(H, I, 8 * T) - took < 6 * 6 * H * I
+
+
 @pytest.mark.parametrize("H,I,T,E,K", [(256, 256, 13, 40, 3), (2560, 2304, 383, 8, 8)])      # the one-launch plan, and the tall tiles on side streams
 def test_a_captured_grouped_step_equals_the_eager_one(H, I, T, E, K):
     """the same kernels under capture: equal bits on every replay, with new inputs in the graph's buffers, longer and shorter eager
