@@ -394,6 +394,30 @@ def _pf_side(dev, stream):
     return S
 
 
+# Device index -> free bytes of the driver from which on a step there asks for decoded weights again, after it could not have them
+_PF_SHORT = {}
+
+
+def _pf_block(dev, need, extra, capturing=False):
+    """(a block of need + extra bytes, extra), or a block of `need` bytes and 0 where the device has no more. The refusal costs the allocator its cached
+    blocks and the host a wait for the device, so it is paid once and not by every step: the next steps do not ask before the driver has as much
+    more to give as was refused (3 us a step to find out; a step that is being captured neither asks then nor leaves word)."""
+    short = _PF_SHORT.get(dev.index) if extra else None
+    if extra and (short is None or (not capturing and torch.cuda.mem_get_info(dev)[0] >= short)):
+        try:
+            block = torch.empty(need + extra, dtype=torch.uint8, device=dev)
+            _PF_SHORT.pop(dev.index, None)
+            return block, extra
+        except torch.OutOfMemoryError:
+            refused = not capturing
+    else:
+        refused = False
+    block = torch.empty(need, dtype=torch.uint8, device=dev)
+    if refused:
+        _PF_SHORT[dev.index] = torch.cuda.mem_get_info(dev)[0] + need + extra
+    return block, 0
+
+
 def _pf_step(s, x, sel, rw, out, R=None, table=None):
     """one nq_pf_step call: x [T, H], sel and rw [T, k], out [T, H] in any of the types the decode kernels take and write"""
     T, k = sel.shape
@@ -419,19 +443,14 @@ def _pf_step(s, x, sel, rw, out, R=None, table=None):
         elif P >= PF_HOT_MIN:
             slots = _pf_slots(R)
     # one block per call, the step's own: it goes back to the allocator in the order of the caller's stream, which the side streams join
-    try:
-        block = torch.empty(wop_at + slots * 6 * H * I, dtype=torch.uint8, device=dev)
-    except torch.OutOfMemoryError:
-        if slots == 0:
-            raise
-        slots, block = 0, torch.empty(wop_at, dtype=torch.uint8, device=dev)
+    block, wop_bytes = _pf_block(dev, wop_at, slots * 6 * H * I, held is None)
     whole = out if out.dtype == torch.float32 or R == P else torch.empty(T, H, dtype=torch.float32, device=dev)   # chunks add up in fp32
     a, at = _lib.NqPfArgs(), block.data_ptr()
     a.x, a.sel, a.rw, a.table, a.out, a.hits = x.data_ptr(), sel.data_ptr(), rw.data_ptr(), tb.data_ptr(), whole.data_ptr(), s.hits_ptr or None
     a.meta, a.meta_bytes = at + meta_at, nb
     a.xg, a.xu, a.acc, a.h, a.y, a.zg, a.zd = (at + o for o in off)
-    if slots:
-        a.wop, a.wop_bytes, a.wop_slots, a.hot_min = at + wop_at, slots * 6 * H * I, slots, hot_min.value
+    if wop_bytes:
+        a.wop, a.wop_bytes, a.wop_slots, a.hot_min = at + wop_at, wop_bytes, slots, hot_min.value
     if held is not None:
         a.side, a.events = held[2], held[3]
     a.T, a.topk, a.E, a.H, a.I, a.rows = T, k, E, H, I, R
@@ -447,7 +466,7 @@ def prefill(s, x, sel, rw, out=None, R=None, G=None, table=None):
     """T > Bmax tokens (reference sm120/moe.py:282-326): pairs sorted by expert, each routed expert decoded inside the
     grouped GEMMs at the level of its live table row, same math as the decode path (fp32 accumulation order differs).
     No host synchronisation (the reference's prefill reads the expert counts back; here the sort and the tile lists are
-    built on the device). Exports routing hits like the decode kernel. A call's scratch is its own (pf_scratch; the reference's calls
+    built on the device), but for what torch's allocator does when the device runs out of memory. Exports routing hits like the decode kernel. A call's scratch is its own (pf_scratch; the reference's calls
     share one set per device, sm120/moe.py:262-274) and its side streams belong to the caller's stream."""
     if s.G != 4:
         raise NotImplementedError("prefill decodes rings of G = 4 lanes only (as the reference's pf_decode)")

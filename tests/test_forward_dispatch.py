@@ -44,3 +44,40 @@ def test_which_steps_are_grouped(monkeypatch):
     # under capture: the same route below pf_min, slices from there on
     assert route(monkeypatch, Stub(), 13, capturing=True) == ["grouped"]
     assert route(monkeypatch, Stub(), 384, capturing=True) == [4] * 96
+
+
+def test_memory_that_was_refused_is_not_asked_for_by_every_step(monkeypatch):
+    """the block of a step with decoded weights: a refusal is met once, the steps after it take the smaller block at once until the driver has
+    as much more to give; a captured step neither asks the driver nor leaves word; other devices are not concerned"""
+    dev, other = torch.device("cuda", 3), torch.device("cuda", 4)
+    asked, driver, have = [], [], {3: 150, 4: 1000}
+
+    def empty(n, dtype, device):
+        assert dtype == torch.uint8
+        asked.append((device.index, n))
+        if n > have[device.index]:
+            raise torch.OutOfMemoryError("no")
+        return ("block", n)
+
+    def info(d):
+        driver.append(d.index)
+        return have[d.index], 10**6
+    monkeypatch.setattr(torch, "empty", empty)
+    monkeypatch.setattr(torch.cuda, "mem_get_info", info)
+    monkeypatch.setattr(M, "_PF_SHORT", {})
+    block = lambda *a: (M._pf_block(*a), asked.copy(), driver.copy(), asked.clear(), driver.clear())[:3]
+    assert block(dev, 100, 0) == ((("block", 100), 0), [(3, 100)], [])
+    assert block(dev, 100, 80, True) == ((("block", 100), 0), [(3, 180), (3, 100)], [])            # captured: refused, no word left
+    assert block(dev, 100, 80) == ((("block", 100), 0), [(3, 180), (3, 100)], [3])
+    assert block(dev, 100, 80) == ((("block", 100), 0), [(3, 100)], [3])                           # not asked again
+    assert block(dev, 100, 80, True) == ((("block", 100), 0), [(3, 100)], [])
+    assert block(other, 100, 80) == ((("block", 180), 80), [(4, 180)], [])
+    have[3] = 329                                                # 150 + 180 - 1
+    assert block(dev, 100, 80)[1] == [(3, 100)]
+    have[3] = 330
+    assert block(dev, 100, 80) == ((("block", 180), 80), [(3, 180)], [3])
+    assert block(dev, 100, 80) == ((("block", 180), 80), [(3, 180)], [])
+    have[3] = 50
+    with pytest.raises(torch.OutOfMemoryError):                  # not even the smaller one
+        M._pf_block(dev, 100, 80)
+    assert not M._PF_SHORT

@@ -545,6 +545,35 @@ def test_a_step_takes_no_more_than_pf_bytes_says():
     assert took <= M.pf_bytes(H, I, 8 * T) + lists + (2 << 20) and M.pf_bytes(H, I, 8 * T) - took < 6 * 6 * H * I
 
 
+def test_a_step_that_cannot_have_decoded_weights_runs_without(monkeypatch):
+    """the first allocation of a step refused: the same bits in the smaller block, and the next step asks for that one only"""
+    H = I = 2048
+    E, T = 8, 1100
+    ex = to_dev(experts_on_gpu(H, I, 2, 79, nested_ids=(1,)))
+    L = M.MoELayer(E, H, I, Bmax=8, topk=8)
+    for e in range(E):
+        L.set(e, ex[e % 2], 4)
+    g = torch.Generator().manual_seed(81)
+    x = (torch.randn(T, H, generator=g) * 0.05).half().to(DEV)
+    sel, rw = torch.arange(E, device=DEV).repeat(T, 1), (torch.rand(T, E, generator=g) + 0.1).half().to(DEV)
+    want, asked, empty = L.prefill(x, sel, rw), [], torch.empty
+    limit = M._pf_offsets(H, I, 8 * T)[1] + 6 * H * I            # one expert's decoded weights
+
+    def short(*a, **kw):
+        if kw.get("dtype") == torch.uint8 and len(a) == 1:
+            asked.append(a[0])
+            if a[0] > limit:
+                raise torch.OutOfMemoryError("refused")
+        return empty(*a, **kw)
+    monkeypatch.setattr(M, "_PF_SHORT", {})
+    monkeypatch.setattr(M.torch, "empty", short)
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda d: (1 << 20, 1 << 38))
+    got = [L.prefill(x, sel, rw) for _ in range(2)]
+    torch.cuda.synchronize()
+    assert len(asked) == 3 and asked[0] - asked[1] == E * 6 * H * I and asked[2] == asked[1] <= limit
+    assert all(torch.equal(y, want) for y in got) and want.isfinite().all()
+
+
 @pytest.mark.parametrize("H,I,T,E,K", [(256, 256, 13, 40, 3), (2560, 2304, 383, 8, 8)])      # the one-launch plan, and the tall tiles on side streams
 def test_a_captured_grouped_step_equals_the_eager_one(H, I, T, E, K):
     """the same kernels under capture: equal bits on every replay, with new inputs in the graph's buffers, longer and shorter eager
