@@ -653,13 +653,12 @@ __device__ __forceinline__ void finish_dn_all(const MoeArgs& a, const PickInfo& 
 // +1.5 us), so the register allocator is told to aim at exactly that. The common down launch gains from five (90 registers): its
 // 1536 workgroups then need 1.2 rounds instead of 1.5 (-0.4 us per layer at one token, -2.5 us at four).
 // OWN (gate|up of the common rows only): no routing launch comes before, see launch_moe; the last plane of blocks does that launch's other
-// work. A kernel of its own: carried along in the other one, unused, it cost 0.5 to 1.5 % of a call. The down launch behind it (SMALL too) differs by
-// gemv_chunks' FEW alone.
-template <int MODE, bool ANYROW, bool SMALL = false>
+// work. A kernel of its own: carried along in the other one, unused, it cost 0.5 to 1.5 % of a call. FEW: gemv_chunks', see launch_moe.
+template <int MODE, bool ANYROW, bool OWN = false, bool FEW = false>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == 1 && !ANYROW ? 5 : 4, MODE == 1 && !ANYROW ? 5 : 4)))
 nq_gemv_k(MoeArgs a, int NC)
 {
-    constexpr bool OWN = SMALL && MODE == 0;
+    static_assert(!OWN || MODE == 0, "the gate|up launch takes over the routing");
     extern __shared__ __align__(16) char smem[];
     // Exactly four gate|up workgroups per CU: at one token the launch has four for every CU, and with room for a fifth the
     // dispatcher fills some CUs with five and leaves others with three. The body needs 90 registers; naming v100 claims 104.
@@ -828,11 +827,11 @@ nq_gemv_k(MoeArgs a, int NC)
     }
     else if (R.level == 2)
     {
-        if (a.hoist && P.var == nullptr) gemv_chunks<false, 0, 0, false, true, SMALL>(P, L, NC, acc, nb0);   // block-uniform: the caller's option
-        else gemv_chunks<false, 0, 0, false, false, SMALL>(P, L, NC, acc, nb0);
+        if (a.hoist && P.var == nullptr) gemv_chunks<false, 0, 0, false, true, FEW>(P, L, NC, acc, nb0);   // block-uniform: the caller's option
+        else gemv_chunks<false, 0, 0, false, false, FEW>(P, L, NC, acc, nb0);
     }
-    else if (a.hoist && P.var == nullptr) dispatch_code(P.code, [&](auto tag) { gemv_chunks<true, decltype(tag)::value, 0, false, true, SMALL>(P, L, NC, acc, nb0); });
-    else dispatch_code(P.code, [&](auto tag) { gemv_chunks<true, decltype(tag)::value, 0, false, false, SMALL>(P, L, NC, acc, nb0); });
+    else if (a.hoist && P.var == nullptr) dispatch_code(P.code, [&](auto tag) { gemv_chunks<true, decltype(tag)::value, 0, false, true, FEW>(P, L, NC, acc, nb0); });
+    else dispatch_code(P.code, [&](auto tag) { gemv_chunks<true, decltype(tag)::value, 0, false, false, FEW>(P, L, NC, acc, nb0); });
 
     __builtin_amdgcn_s_setprio(3);                               // the tail is a chain of latencies: nothing should wait behind decoders
     PickLanes picks = {};
@@ -902,6 +901,13 @@ __global__ void nq_mailbox_k(int64_t* table, const int64_t* stage, const int32_t
 // With a layer and inputs met for the first time, nothing of them in any cache, the heads cost more and the gain is smaller. us of the two
 // projection kernels, and of the routing launch before them: 512 x 256, 2 tokens 4.4 + 17.4 / 20.1; repeated 3.4 + 14.0 / 14.2.
 constexpr int OWN_ROUTE_WGS = 512;
+// Slices of fewer chunks work a unit's constants out where they are needed (gemv_chunks' FEW). us a call of mixed levels in a graph, UnitConsts
+// in both projections / in gate|up alone / in down alone / in neither; chunks of a gate|up and a down slice. One chunk, where there is nothing to share:
+//   1152 x 640, 8 picks (1, 1) 19.30 / 19.23 / 19.33 / 19.17; 1536 x 768, 8 (1, 1) 21.24 / 21.14 / 21.08 / 20.91; 2176 x 896, 24 (1, 1) 48.47 / 48.13 / 48.20 / 47.95;
+//   2048 x 1024, 6 (1, 1) 23.29 / 23.28 / 22.99 / 23.08, 16 (4, 1) 41.19 / 40.56 / 42.35 / 41.79; 6144 x 2048, 2 (3, 1) 33.19 / 33.04 / 33.25 / 33.32.
+// Two and more: 3072 x 1536, 16 (8, 3) 47.65 / 48.08 / 48.37 / 48.65; 4096 x 2048, 8 (8, 2) 46.92 / 47.01 / 47.46 / 47.59; 6144 x 2048, 8 (12, 4)
+//   60.81 / 61.14 / 61.21 / 61.77, 32 (24, 4) 201.2 / 202.1 / 204.4 / 205.4.
+constexpr int FEW_CHUNKS = 2;
 int launch_moe(const MoeArgs& a, const int* cfg_gu, const int* cfg_dn, int which, hipStream_t st)
 {
     const int S = a.B * a.topk;
@@ -931,7 +937,10 @@ int launch_moe(const MoeArgs& a, const int* cfg_gu, const int* cfg_dn, int which
         b.fuse = which == 3 || defer;                             // both launches belong to this call (or the caller says the other one follows)
         b.mb_apply = a.mb_table != nullptr && mode == last_mode;  // the call's last projection launch carries the mailbox block
         const bool self = own && mode == 0;
-        auto kern = self ? nq_gemv_k<0, false, true> : mode == 0 ? (any ? nq_gemv_k<0, true> : nq_gemv_k<0, false>) : (any ? nq_gemv_k<1, true> : own ? nq_gemv_k<1, false, true> : nq_gemv_k<1, false>);
+        const bool few = own || NC < FEW_CHUNKS;
+        auto kern = self ? nq_gemv_k<0, false, true, true>
+                  : mode == 0 ? (any ? nq_gemv_k<0, true> : few ? nq_gemv_k<0, false, false, true> : nq_gemv_k<0, false>)
+                              : (any ? nq_gemv_k<1, true> : few ? nq_gemv_k<1, false, false, true> : nq_gemv_k<1, false>);
         if (shm > 48 * 1024)
         {
             hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, shm);

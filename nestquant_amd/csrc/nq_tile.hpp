@@ -393,8 +393,8 @@ __device__ __forceinline__ void gemv_chunks_masked(const Planes& P, const LaneCt
 // loop's ~276 vector instructions per chunk) and, with it, the rounding of each weight to fp16: the result is that of the
 // UNROUNDED weights, ~2e-4 (relative, l2) from the product with the exact fp16 weights that the other form and the reference
 // compute -- inside the layer's 1e-3, outside the 5e-5 that the exact form holds, hence an option the caller has to ask for.
-// FEW (slices of few chunks that nothing runs beside): every lane works out its own unit's constants chunk by chunk instead. UnitConsts' permutes and its
-// work at a slice's beginning are latency there: a layer of 512 x 256, two tokens, 14.1 us / 14.3 with them.
+// FEW: every lane works out its own unit's constants chunk by chunk instead. In a slice of one chunk there is nothing for UnitConsts to share, and its
+// permutes and its work at the slice's beginning are latency: a layer of 512 x 256, two tokens, 14.1 us / 14.3 with them. Which call takes which: launch_moe.
 template <bool RES, int CODE, int BK = 0, bool MASKOK = true, bool RAW = false, bool FEW = false>
 __device__ __forceinline__ void gemv_chunks(const Planes& P, const LaneCtx& L, int NC, float4_t* acc, u32x4 nb)
 {

@@ -774,3 +774,28 @@ def test_calls_without_a_routing_launch(H, I, B, topk, force):
     L(x, sel, rw, which=1 | 8, cfg_gu=cg, cfg_dn=cd, sal=sal[1])
     torch.cuda.synchronize()
     assert torch.equal(sal[0].acc, sal[1].acc)
+
+
+@pytest.mark.parametrize("H,I,gu,dn,topk", [(256, 512, 1, 1, 8), (512, 512, 2, 1, 8), (384, 256, 1, 2, 8), (2048, 512, 2, 4, 3), (512, 256, 1, 1, 2)])
+@pytest.mark.parametrize("hoist", [False, True])
+def test_short_slices_give_the_bits_of_the_complete_kernel(H, I, gu, dn, topk, hoist):
+    """k-slices of one chunk and of several, with and without a routing launch (the last shape), at every level, over all window codes and with sign planes:
+    the kernels of common rows against the one for rows of any kind, which a caller's own table takes"""
+    rk = [(0, 0), (3, 7), (6, 9), (8, 3), (0, 0), (1, 2), (4, 5), (0, 0), (7, 6), (0, 0)]
+    ex = to_dev(experts_on_gpu(H, I, 10, 500, nested_ids=(4, 7, 9), rk=rk, var_ids=(1, 4, 5, 9)))
+    L = M.MoELayer(10, H, I, Bmax=8, topk=topk)
+    for e, lv in enumerate([2, 4, 4, 4, 3, 2, 4, 4, 2, 4]):
+        L.set(e, ex[e], lv)
+    g = torch.Generator().manual_seed(H + topk)
+    B = 8 if topk > 2 else 2
+    x = (torch.randn(B, H, generator=g) * 0.3).half().to(DEV)
+    sel = torch.stack([torch.randperm(10, generator=g)[:topk] for _ in range(B)]).to(DEV)
+    rw = (torch.rand(B, topk, generator=g) + 0.1).half().to(DEV)
+    assert (2 * I // 128 * (H // 128 // gu) * B * topk <= 512) == (topk == 2)
+    cfg = dict(cfg_gu=[1, 4, gu], cfg_dn=[1, 4, dn])
+    got = L(x, sel, rw, hoist=hoist, **cfg).clone()
+    want = L(x, sel, rw, hoist=hoist, table=L.table.clone(), **cfg).clone()
+    assert want.isfinite().all() and want.abs().max() > 0
+    if not hoist:                                                # the complete kernel has no hoisted form
+        assert torch.equal(got, want)
+    assert rel_err(got.cpu().numpy(), want.cpu().numpy()) < 1e-3
