@@ -254,6 +254,27 @@ def test_prepared_weights_equal_the_torch_form(N, K):
             assert torch.equal(rings[: N * K // 256], EN.to_rings(got[2]).nan_to_num()) and (n == 1 or torch.equal(rings[N * K // 256:], EN.to_rings(-got[2]).nan_to_num()))
 
 
+def test_transformed_weights_take_the_torch_form():
+    """a weight with a tangent keeps it, vmap and jvp go through prepare as on the CPU, a gradient comes back: against the same on a float64 weight, which
+    no kernel takes; 4 ulp of fp32 for the sums' other order"""
+    fw = torch.autograd.forward_ad
+    g = torch.Generator().manual_seed(31)
+    W, V = torch.randn(2, 128, 256, generator=g).cuda(), torch.randn(2, 128, 256, generator=g).cuda()
+    close = lambda a, b: float((a.double() - b.double()).norm() / b.double().norm()) < 2.0**-21
+    with fw.dual_level():
+        got, want = (EN.prepare(fw.make_dual(W[0].to(t), V[0].to(t)), 3) for t in (torch.float32, torch.float64))
+        for a, b in zip(got, want):
+            assert torch.equal(fw.unpack_dual(a).primal, fw.unpack_dual(b).primal)
+        assert close(fw.unpack_dual(got[2]).tangent, fw.unpack_dual(want[2]).tangent)
+        assert fw.unpack_dual(EN.encode_level2(fw.make_dual(W[0], V[0]), 3)["target"]).tangent is not None
+    target = lambda w: EN.prepare(w, 3)[2]
+    assert close(torch.func.jvp(target, (W[0],), (V[0],))[1], torch.func.jvp(target, (W[0].double(),), (V[0].double(),))[1])
+    for a, *b in zip(torch.func.vmap(lambda w: EN.prepare(w, 3), randomness="same")(W), *(EN.prepare(w, 3) for w in W)):
+        assert torch.equal(a, torch.stack(b))
+    a, b = (torch.func.grad(lambda w: (target(w) * V[1]).sum())(w) for w in (W[0], W[0].double()))
+    assert close(a, b)
+
+
 def test_orientation_of_rings_equals_the_torch_form():
     """each ring fitted as it is and negated: the better of the two, the first where they are equal (a ring of zeros, whose two searches give one path)"""
     g = torch.Generator().manual_seed(12)
