@@ -341,3 +341,17 @@ def test_hessian_aware_fit_equals_the_torch_form(N, K, var):
         for w in (W, W.double()):
             with pytest.raises(torch.linalg.LinAlgError):
                 EN.encode_ldlq(w, bad)
+
+
+def test_a_metric_that_is_not_positive_definite_is_reported_after_the_first_search(monkeypatch):
+    """not after a whole fit: one search here, and the one under which the torch form factorises"""
+    g = torch.Generator().manual_seed(41)
+    W, searches, search = torch.randn(128, 512, generator=g).cuda(), [], EN._viterbi_gpu
+    monkeypatch.setattr(EN, "_viterbi_gpu", lambda *a: (searches.append(a[0].shape[0]), search(*a))[1])
+    bad = torch.eye(512, device="cuda")
+    bad[200, 200] = -1e4                                         # below zero after the damping too
+    with pytest.raises(torch.linalg.LinAlgError):
+        EN.encode_ldlq(W, bad)
+    assert len(searches) <= 2
+    EN.encode_ldlq(W, torch.eye(512, device="cuda"))
+    assert len(searches) > 8
