@@ -385,11 +385,12 @@ extern "C" int nq_fit_pack(const int64_t* states, int K, const float* values, co
     return launch_fit_pack(states, K, values, sign, lut, Mb, N, strips * chunks, chunks, words, dw, var, Q, bad, (hipStream_t)stream);
 }
 
-static bool enc_shape_ok(int N, int K) { return N >= 128 && N % 128 == 0 && K >= 128 && K % 128 == 0 && N <= (1 << 23); }
+// rows: one 128-row block per place of a grid's second dimension
+static bool enc_shape_ok(int N, int K) { return N >= 128 && N % 128 == 0 && K >= 128 && K % 128 == 0 && N / 128 <= 65535; }
 
 extern "C" int nq_enc_prepare(const float* W, int N, int K, const int64_t* signs, double* ws, void* su, void* sv, float* target, float* rings, int negated, void* stream)
 {
-    NQ_REQUIRE(enc_shape_ok(N, K), "nq_enc_prepare: N=%d K=%d (positive multiples of 128)", N, K);
+    NQ_REQUIRE(enc_shape_ok(N, K), "nq_enc_prepare: N=%d K=%d (positive multiples of 128, at most 65535 * 128 rows)", N, K);
     NQ_REQUIRE(W && signs && ws && su && sv && target, "nq_enc_prepare: null pointer");
     return launch_enc_prepare(W, N, K, signs, ws, su, sv, target, rings, negated, (hipStream_t)stream);
 }

@@ -137,6 +137,7 @@ def test_encoder_entry_points_refuse_bad_arguments():
     err = lambda: L.nq_last_error().decode()
     b = 64
     assert L.nq_enc_prepare(b, 100, 128, b, b, b, b, b, None, 0, None) != 0 and "multiples of 128" in err()
+    assert L.nq_enc_prepare(b, 65536 * 128, 128, b, b, b, b, b, None, 0, None) != 0 and "65535" in err()        # more blocks of rows than a grid holds
     assert L.nq_enc_prepare(b, 128, 128, None, b, b, b, b, None, 0, None) != 0 and "null" in err()
     assert L.nq_enc_hessian(b, 64, b, b, None) != 0 and "multiple of 128" in err()
     assert L.nq_enc_inverse(b, 127, b, b, 0, None) != 0 and "lda" in err()

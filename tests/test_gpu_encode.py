@@ -254,6 +254,12 @@ def test_prepared_weights_equal_the_torch_form(N, K):
             assert torch.equal(rings[: N * K // 256], EN.to_rings(got[2]).nan_to_num()) and (n == 1 or torch.equal(rings[N * K // 256:], EN.to_rings(-got[2]).nan_to_num()))
 
 
+def test_weights_of_more_rows_than_a_launch_takes_have_the_torch_form():
+    """8.4 million rows; a view, nothing of it is read"""
+    W = torch.zeros(1, 128, device="cuda")
+    assert EN._plain_weight(W.expand(65535 * 128, 128)) and not EN._plain_weight(W.expand(65536 * 128, 128))
+
+
 def test_transformed_weights_take_the_torch_form():
     """a weight with a tangent keeps it, vmap and jvp go through prepare as on the CPU, a gradient comes back: against the same on a float64 weight, which
     no kernel takes; 4 ulp of fp32 for the sums' other order"""
