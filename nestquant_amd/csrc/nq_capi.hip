@@ -286,7 +286,7 @@ extern "C" int nq_pf_post(const float* y, const int32_t* pos, const int64_t* sel
 extern "C" int nq_pf_wdecode(const int64_t* table, const int32_t* hot, int E, int mode, void* Wop, int64_t wop_bytes, int slots, int H, int I, void* stream)
 {
     NQ_REQUIRE(table && hot && Wop, "nq_pf_wdecode: null pointer");
-    NQ_REQUIRE(E >= 1 && E <= 65535 && (mode == 0 || mode == 1) && slots >= 1 && slots <= 65535, "nq_pf_wdecode: E=%d (1..65535) mode=%d slots=%d", E, mode, slots);
+    NQ_REQUIRE(E >= 1 && E <= 65535 && (mode == 0 || mode == 1) && slots >= 1, "nq_pf_wdecode: E=%d (1..65535) mode=%d slots=%d", E, mode, slots);
     NQ_REQUIRE(shape_ok(H, I), "nq_pf_wdecode: H=%d I=%d (positive multiples of 128)", H, I);
     NQ_REQUIRE(aligned16(Wop) && wop_bytes >= (int64_t)slots * 3 * H * I * 2, "nq_pf_wdecode: the scratch needs %d slots of 3 * H * I halfs, 16-byte aligned", slots);
     return launch_pf_wdecode(table, hot, E, nullptr, mode, Wop, slots, H, I, (hipStream_t)stream);

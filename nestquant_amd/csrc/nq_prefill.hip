@@ -517,14 +517,14 @@ __device__ __forceinline__ void wdecode_chunks(const Planes& P, const LaneCtx& L
     }
 }
 
-// grid (N / 128, k-slices, slots), block 256: 128 weight rows x WDEC_CHUNKS chunks of the expert with scratch slot blockIdx.z, if its row is
+// grid (N / 128, k-slices, slots), block 256: 128 weight rows x WDEC_CHUNKS chunks of the expert with scratch slot slot0 + blockIdx.z, if its row is
 // of the common kind (K = 2 base plane, no mask-mode flags; others keep decoding inside the GEMM, whatever hot[] says). Bound by its writes:
 // 16 experts' down projections 89 us = 4.5 TB/s (a whole row of chunks per wavefront: 126 us, too few in flight); gate|up beside other launches 3.5 TB/s.
 // tiles (may be null): the number of tiles of decoded weights.
 constexpr int WDEC_CHUNKS = 8;
-__global__ void __launch_bounds__(256) nq_pf_wdecode_k(const int64_t* table, const int32_t* hot, int E, const int32_t* tiles, int mode, u32x4* Wop, int H, int I)
+__global__ void __launch_bounds__(256) nq_pf_wdecode_k(const int64_t* table, const int32_t* hot, int E, const int32_t* tiles, int mode, u32x4* Wop, int slot0, int H, int I)
 {
-    const int slot = blockIdx.z;
+    const int slot = slot0 + blockIdx.z;
     if (tiles && *tiles == 0) return;                            // no tile of decoded weights
     int e = -1;
     for (int i0 = 0; i0 < E && e < 0; i0 += 64)                  // every wavefront looks for itself
@@ -556,8 +556,11 @@ __global__ void __launch_bounds__(256) nq_pf_wdecode_k(const int64_t* table, con
 int launch_pf_wdecode(const int64_t* table, const int32_t* hot, int E, const int32_t* tiles, int mode, void* Wop, int slots, int H, int I, hipStream_t st)
 {
     const int N = mode == 0 ? 2 * I : H, C = (mode == 0 ? H : I) / 128;
-    nq_pf_wdecode_k<<<dim3(N / 128, (C + WDEC_CHUNKS - 1) / WDEC_CHUNKS, slots), 256, 0, st>>>(table, hot, E, tiles, mode, (u32x4*)Wop, H, I);
-    NQ_LAUNCH_CHECK("nq_pf_wdecode");
+    for (int s0 = 0; s0 < slots; s0 += 65535)                    // what a grid's third dimension holds
+    {
+        nq_pf_wdecode_k<<<dim3(N / 128, (C + WDEC_CHUNKS - 1) / WDEC_CHUNKS, std::min(slots - s0, 65535)), 256, 0, st>>>(table, hot, E, tiles, mode, (u32x4*)Wop, s0, H, I);
+        NQ_LAUNCH_CHECK("nq_pf_wdecode");
+    }
     return 0;
 }
 
@@ -962,7 +965,7 @@ int launch_pf_step(const NqPfArgs& a, hipStream_t st)
                 if (variants & 1) if (int rc = launch_tiles<false>(g, bm[i], counts[i], streams[i])) return rc;
                 if (variants & 2) if (int rc = launch_tiles<true>(g, bm[i], counts[i], streams[i])) return rc;
             }
-            if (wop) if (int rc = launch_pf_wdecode(a.table, m.hot, E, m.wide, mode, a.wop, a.wop_slots, H, I, st)) return rc;
+            if (wop) if (int rc = launch_pf_wdecode(a.table, m.hot, E, m.wide, mode, a.wop, std::min(a.wop_slots, E), H, I, st)) return rc;
             if (wop)
                 if (int rc = launch_wide(PfWide{a.table, m.wide + 4, m.wide, (const _Float16*)(mode ? a.h : a.xg), (const _Float16*)(mode ? nullptr : a.xu), mode ? y : acc, (const u32x4*)a.wop,
                                                 mode, E, H, I, 0}, most, st)) return rc;

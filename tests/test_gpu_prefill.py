@@ -148,6 +148,25 @@ def test_tiles_of_decoded_weights_give_the_bits_of_decode_fused_tiles(H, I):
     assert want.isfinite().all()
 
 
+def test_slots_beyond_a_grid_are_decoded():
+    """an expert with a slot of decoded weights beyond the 65535 of one launch (6.4 GB of the smallest shape's): the bytes of slot 0"""
+    from nestquant_amd import _lib
+    H = I = 128
+    slots = 65540
+    ex = to_dev(experts_on_gpu(H, I, 2, 89))
+    L = M.MoELayer(2, H, I, Bmax=2, topk=1)
+    for e in range(2):
+        L.set(e, ex[e], 4)
+    wop = torch.zeros(slots, 3 * H * I, dtype=torch.float16, device=DEV)
+    for hot in ((0, 1), (slots - 1, 65534)):
+        h = torch.tensor(hot, dtype=torch.int32, device=DEV)
+        for mode in (0, 1):
+            _lib.check(_lib.lib().nq_pf_wdecode(L.table.data_ptr(), h.data_ptr(), 2, mode, wop.data_ptr(), wop.numel() * 2, slots, H, I, _lib.stream_ptr()))
+    torch.cuda.synchronize()
+    assert wop[0].any() and wop[1].any() and not wop[2].any() and not wop[65535].any()
+    assert torch.equal(wop[slots - 1], wop[0]) and torch.equal(wop[65534], wop[1])
+
+
 @pytest.mark.parametrize("bm,rows", [(64, (33, 48, 49, 64)), (128, (1, 65, 80, 81, 96, 97, 112, 113, 128)), (256, (40, 129, 144, 145, 160, 161, 176, 177, 192, 193, 208, 209, 224, 225, 240, 241, 256))])
 def test_bodies_of_tall_tiles_give_the_bits_of_16_row_tiles(bm, rows):
     """nq_pf_gemm picks a body by a tile's rows: at the edges of each body the rows come out as in tiles of 16 (which are held against the oracle
