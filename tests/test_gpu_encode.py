@@ -324,6 +324,18 @@ def test_block_factors_on_the_gpu(m):
     assert factors(H * float("nan"))[2] == 1
 
 
+@pytest.mark.parametrize("var", [False, True])
+def test_nested_fit_equals_the_torch_form(var):
+    """encode_nested of a weight whose rings, with `var` the negated ones too, come from nq_enc_prepare, and of the same in float64, which takes the
+    torch form: the same bytes"""
+    W = torch.randn(128, 256, generator=torch.Generator().manual_seed(51)).cuda()
+    got, want = (EN.encode_nested(w, seed=6, var=var) for w in (W, W.double()))
+    assert got.keys() == want.keys() and (got["var"] is not None) == var
+    for k, w in want.items():
+        assert (w is None and got[k] is None) or (got[k].dtype == w.dtype and torch.equal(got[k], w)), k
+    assert not var or 0 < int((got["var"] != 0).sum())
+
+
 @pytest.mark.parametrize("N,K,var", [(128, 128, True), (128, 384, False), (256, 256, True)])
 def test_hessian_aware_fit_equals_the_torch_form(N, K, var):
     """encode_ldlq with its glue in kernels and level 3 at its own pace against the torch form (which a float64 weight takes): the same bytes, errors to
