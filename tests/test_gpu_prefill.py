@@ -89,8 +89,33 @@ def test_full_shape_prefill_vs_decode_slices():
     assert rel_err(y[idx].cpu().numpy(), want) < 5e-5
 
 
-def test_hot_expert_scratch_gives_the_same_bits():
-    """experts with more than one 256-row tile decoded once into the operand scratch (nq_pf_wdecode, off by default): the
+@pytest.fixture
+def decoded_slots(monkeypatch):
+    """how many slots of decoded weights each step since the last call has written, both projections of each: () -> [slots of a step, ...]. (Where slots are
+    written, their experts' tiles are nq_pf_wide_k's: both hang on the planner's one decision, and the decode-fused kernel leaves them out.)"""
+    steps, block = [], M._pf_block
+
+    def kept(dev, need, extra, capturing=False):
+        b, extra = block(dev, need, extra, capturing)
+        b[need:].zero_()
+        steps.append(b[need:])
+        return b, extra
+    monkeypatch.setattr(M, "_pf_block", kept)
+
+    def written(H, I):
+        torch.cuda.synchronize()
+        out = []
+        for b in steps:
+            gu, dn = b.view(-1, 6 * H * I).split([4 * H * I, 2 * H * I], 1)
+            assert torch.equal(gu.any(1), dn.any(1))
+            out.append(int(gu.any(1).sum()))
+        steps.clear()
+        return out
+    return written
+
+
+def test_hot_expert_scratch_gives_the_same_bits(decoded_slots):
+    """experts with more than one 256-row tile decoded once into the operand scratch (nq_pf_wdecode; the library itself gives a step this small none): the
     grouped GEMM multiplies the same operands in the same order, so the result is bitwise the one of the decode-fused tiles"""
     H, I, NE, T = 1024, 512, 6, 700
     levels = [4, 2, 3, 4, 2, 4]
@@ -114,6 +139,7 @@ def test_hot_expert_scratch_gives_the_same_bits():
         torch.cuda.synchronize()
     finally:
         M.PF_HOT_SLOTS = 0
+    assert decoded_slots(H, I) == [0, 1, min(4, int((cnt >= M.PF_HOT_MIN).sum()))]
     assert torch.equal(y0, y1) and torch.equal(y0, y2)
     ys = sliced_decode(L, x, sel, rw)
     torch.cuda.synchronize()
@@ -121,7 +147,7 @@ def test_hot_expert_scratch_gives_the_same_bits():
 
 
 @pytest.mark.parametrize("H,I", [(128, 128), (384, 256), (256, 640), (1024, 512)])        # one chunk; blocks of 128 weight rows; K = 128 .. 1024
-def test_tiles_of_decoded_weights_give_the_bits_of_decode_fused_tiles(H, I):
+def test_tiles_of_decoded_weights_give_the_bits_of_decode_fused_tiles(H, I, decoded_slots):
     """nq_pf_wdecode_k and nq_pf_wide_k at the edges of their tiles: one row more than a remainder that decodes in its GEMM, full tiles, a
     row beyond, several tiles; every level, window codes of several record lengths, sign planes; and the same in chunks of pair rows"""
     rows = [129, 255, 256, 257, 385, 512, 130, 700, 0, 1]
@@ -137,11 +163,14 @@ def test_tiles_of_decoded_weights_give_the_bits_of_decode_fused_tiles(H, I):
     try:
         M.PF_HOT_SLOTS = -1
         want = L.prefill(x, sel, rw)
+        assert decoded_slots(H, I) == [0]
         for M.PF_HOT_SLOTS, hot_min in ((10, 1), (3, 200)):
             hot, M.PF_HOT_MIN = M.PF_HOT_MIN, hot_min
             got = [L.prefill(x, sel, rw, R=R) for R in (None, 600)]
             M.PF_HOT_MIN = hot
             torch.cuda.synchronize()
+            whole, cut = decoded_slots(H, I)                     # nine experts have rows, six of them 200 or more; of a chunk of 600 rows fewer
+            assert whole == min(M.PF_HOT_SLOTS, 9 if hot_min == 1 else 6) and 0 < cut <= whole
             assert all(torch.equal(want, y) for y in got), (M.PF_HOT_SLOTS, hot_min)
     finally:
         M.PF_HOT_SLOTS, M.PF_HOT_MIN = 0, 257
@@ -198,7 +227,7 @@ def test_bodies_of_tall_tiles_give_the_bits_of_16_row_tiles(bm, rows):
                 assert want[8:8 + n].isfinite().all() and bool((want[:8] == 7).all() and (want[8 + n:] == 7).all() and (want[8:8 + n] != 7).any(1).all())
 
 
-def test_a_step_takes_decoded_weights_where_they_pay():
+def test_a_step_takes_decoded_weights_where_they_pay(decoded_slots):
     """the rule's first step (eight experts of 1100 rows: 32 tiles of a shape whose units are then 512): equal bits with all experts above
     level 2, and with one below, which leaves too few tiles"""
     H = I = 2048
@@ -220,6 +249,7 @@ def test_a_step_takes_decoded_weights_where_they_pay():
         finally:
             M.PF_HOT_SLOTS = 0
         torch.cuda.synchronize()
+        assert decoded_slots(H, I) == [0 if 2 in levels else E, 0]
         assert torch.equal(got, want) and got.isfinite().all()
 
 
