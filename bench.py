@@ -294,15 +294,16 @@ def prefill_leg(L, ex, dev, T=4096, reps=3):
                 launches_alone=parts,
                 with_hot_scratch=dict(ms=round(hot_ms, 3), result="bitwise equal", hot_experts=hot_parts["hot_experts"],
                                       wdecode_us=hot_parts["wdecode_us"], height_256=hot_parts["height_256"], sum_us=hot_parts["sum_us"]),
-                note="whole prefill() call: sort, plan, hot-expert decode, then per tile height pre, gate|up GEMM, mid, down GEMM on "
-                     "concurrent streams, post; the GEMMs decode their weights in the kernel and are bound by the issue rate of the "
-                     "decode's vector instructions")
+                note="whole prefill() call: sort, plan, rotation of all rows, then three chains (tiles of up to 64 rows, of up to 128, the taller ones "
+                     "with those of experts decoded once) of gate|up GEMM, mid, down GEMM on three streams, post; the other GEMMs decode their "
+                     "weights in the kernel and are bound by the issue rate of the decode's vector instructions. launches_alone takes nq_pf_gemm "
+                     "through the five heights of nq_pf_plan's lists, which the call itself launches as three")
 
 
 def prefill_parts(L, x, sel, dev):
-    """the grouped-GEMM launches of one prefill() call timed one at a time on one stream (inside the call they overlap on four
-    streams and their durations stretch): per tile height the tiles, pair rows, us of the gate|up and the down launch, and
-    the MFMA fraction of that height alone; plus the two launches that decode the hot experts into the operand scratch"""
+    """what the tiles of each height cost: nq_pf_gemm over the five lists of nq_pf_plan, one at a time on one stream (prefill() itself launches them as
+    three gapless lists, up to 64 rows, 128 and 256, on three streams that overlap): per height the tiles, pair rows, us of the gate|up and the down
+    launch, and the MFMA fraction of that height alone; plus the two launches that decode the hot experts into the operand scratch"""
     from nestquant_amd import _lib
     T = x.shape[0]
     Lb, tb, P = L.M, L.table, T * TOPK
@@ -345,8 +346,8 @@ def prefill_parts(L, x, sel, dev):
         rec[f"height_{bm}"] = dict(tiles=int(valid.sum()), hot_tiles=int((tl[i, :nt, 3][valid] > 0).sum()), rows=rows, gate_up_us=round(gu, 0),
                                    down_us=round(dn, 0), mfma_frac=round(rows * 6 * H * I / (gu + dn) / 1e6 / MFMA_PEAK_TFLOPS, 3))
     rec["sum_us"] = round(tot, 0)
-    # the two memory-bound kernels either side of the gate|up GEMM, over all pair rows at once (inside the call they run per
-    # tile height under the GEMMs of other heights): rotation of the tokens, and SwiGLU between the projections
+    # the two memory-bound kernels either side of the gate|up GEMM, over all pair rows at once: rotation of the tokens (as inside the call), and
+    # SwiGLU between the projections (there each chain's rows under the GEMMs of the others)
     pre = us(lambda: _lib.check(Lb.nq_pf_pre(x.data_ptr(), pt.data_ptr(), pe.data_ptr(), P, tb.data_ptr(), S["xg"].data_ptr(), S["xu"].data_ptr(),
                                              S["zg"].data_ptr(), E, H, I, st)))
     mid = us(lambda: _lib.check(Lb.nq_pf_mid(S["acc"].data_ptr(), pe.data_ptr(), P, tb.data_ptr(), S["h"].data_ptr(), S["zg"].data_ptr(),

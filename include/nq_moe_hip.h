@@ -222,7 +222,7 @@ int nq_pf_pre_rows(const void* x_f16, const int32_t* pt, const int32_t* pe, int 
  * the table row set): it handles only their tiles, the plain variant only the others, so a layer with such experts makes
  * both calls; mode | 4: this is the only call for these tiles (the host knows every row to be of one kind), so a tile of the
  * other kind, which nothing would compute, gets NaN results instead of stale scratch. Replaces pf_decode + the Triton grouped GEMM / aten.mm
- * (reference sm120/pf_gemm.py:7-34, sm120/moe.py:303-324); decoded weights never touch HBM. */
+ * (reference sm120/pf_gemm.py:7-34, sm120/moe.py:303-324); without Wop decoded weights never touch HBM. */
 int nq_pf_gemm(const int64_t* table, const int32_t* tiles, int ntiles, int bm, int mode, const void* A0_f16,
                const void* A1_f16, float* C, int E, int H, int I, const void* Wop, void* stream);
 

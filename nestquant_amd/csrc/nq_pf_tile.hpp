@@ -191,9 +191,9 @@ __device__ __forceinline__ void pf_chunks(const Planes& P, const LaneCtx& L, int
 // MASKED = true takes only those: the rarely used paths keep their extra registers out of the common kernel
 // Workgroups go to the eight XCDs in turn, and each XCD has an L2 of its own. Sixteen workgroups of neighbouring column blocks, which
 // read the same token rows, are therefore taken from one XCD's share of the grid (what does not fill 128 keeps its place): a
-// tile's rows come into two L2s instead of eight. For the one gapless list of the short tiles only: the lists by height have their
-// tiles scattered among unused entries, which sixteen workgroups at a time spread less evenly over the XCDs (a 4096-token step
-// lost 3 to 7 %; with the 256-row list alone, which has no gaps, it lost 0 to 1). Prompt of 1003 tokens 2038 -> 2000 us, step of 201 1361 -> 1347.
+// tile's rows come into two L2s instead of eight: prompt of 1003 tokens 2038 -> 2000 us, step of 201 1361 -> 1347. nq_pf_short_k only: nq_pf_gemm_k
+// was timed with it when its lists had unused entries between the tiles, which sixteen workgroups at a time spread less evenly over the
+// XCDs (a 4096-token step lost 3 to 7 %; with the 256-row list alone, which had none, 0 to 1), and not since they have no gaps.
 struct Block { int x, y; };
 __device__ __forceinline__ Block xcd_block()
 {
@@ -286,7 +286,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) n
 }
 
 // Tiles of up to 64 rows of any height in one launch (the plan of nq_pf_sort_k). Steps of a few hundred tokens over many experts
-// have nothing taller, so a projection is one launch on the caller's stream instead of five on four; with at most 64 rows a tile
+// have nothing taller, so a projection is one launch on the caller's stream instead of three on three; with at most 64 rows a tile
 // costs little more than decoding its expert, and the registers of the 64-row body (127) still let four wavefronts share a SIMD. The body of 48 rows
 // takes a prompt of 1003 tokens (24 to 47 rows an expert) from 1930 to 1865 us. Bound by
 // instruction issue: one vector instruction per 4.0 to 4.2 clocks and SIMD at 200 and 1000 tokens (profiles/grouped_steps.txt).

@@ -665,9 +665,11 @@ __device__ __forceinline__ void wide_unit(const PfWide& a, int unit, int nt, int
 // requested three stages ahead. Wavefronts w and w + 4 share a SIMD and work half a stage apart: one multiplies while the other reads its
 // operands and requests the next stage, so the matrix pipe always has a wavefront with its operands at hand (without that, all eight reading ahead
 // in step: 126 instead of 110 us for 64 units of 6144 columns on an otherwise idle GPU). Products and their order are those of the decode-fused
-// tiles, so are the bits. With all CUs at work it is bound by the power limit: 16 experts of 2048 rows, 6144 x 2048, gate|up 1.54 ms and down 0.88 =
-// 1070 / 940 TFLOP/s at 1.4 GHz, whatever the order of products, the number of stages or of wavefronts, as 32 x 32 products 6 % slower (the same
-// bits); 18.9 us per 256 rows, where a decode-fused tile takes 29.5 at level 4 and 23 at level 2. Its weights have to be decoded first: 17 us an expert.
+// tiles, so are the bits. 16 experts of 2048 rows, 6144 x 2048, in a row of steps: gate|up 1.54 ms and down 0.88 = 1070 / 940 TFLOP/s at the 1.4 GHz that the
+// power limit leaves; launches apart from one another (profiles/prefill_gemm_counters.txt) 1.39 and 0.83 ms at 1.9 to 2.0 GHz, the matrix pipe busy
+// 57 and 49 % of the clocks. A clock 40 % higher gives 10 %, so what bounds it is not the clock alone; the order of products and the number of stages
+// or of wavefronts made no difference, 32 x 32 products were 6 % slower (the same bits). 18.9 us per 256 rows, where a decode-fused tile takes
+// 29.5 at level 4 and 23 at level 2. Its weights have to be decoded first: 17 us an expert.
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) nq_pf_wide_k(PfWide a)
 {
     extern __shared__ __align__(16) char smem[];
@@ -890,8 +892,11 @@ static bool pf_is_short(int64_t P, int E, int H, int I, bool fork)
 // Which experts take decoded weights: at least WIDE_MIN rows (two and a half tiles), above level 2, if their tiles make WIDE_UNITS units of gate|up
 // together (two per CU; the plan counts them). us a step from 512 / 640 / 768 / 1024 rows on (6144 x 2048, top-8, level 4): 4096 tokens, 256
 // experts, Zipf 5198 / 5260 / 5300 / 5222; 64 experts, Zipf 4002 / 3890 / 3962 / 3896; 32, evenly 3656 / 3665 / 3666 / 3850; 16, Zipf 3270 / 3275 / 3268 / 3484;
-// 2000 tokens, 64 experts, Zipf 2190 / 2210 / 2225 / 2220; 16, evenly 1791 / 1792 / 1793 / 1892. On another box without /
-// from 768 on 5335 / 5325, 4030 / 3985, 3840 / 3678, 3763 / 3288, 2175 / 2181, 1888 / 1774. At level 2, where a tile's decode is half as long, 16 experts of 2048 rows lose: 3173 / 3281.
+// 2000 tokens, 64 experts, Zipf 2190 / 2210 / 2225 / 2220; 16, evenly 1791 / 1792 / 1793 / 1892: 640 and 768 cannot be told apart. Without decoded
+// weights / by this rule, in turn on one box, two routings: 4096 tokens, 256 experts, Zipf 5503 / 5378 and 5433 / 5304; 64 4091 / 3935, 4100 / 4028; 32,
+// evenly 3891 / 3698, 3923 / 3739; 16, Zipf 3833 / 3311, 3858 / 3634; 2000 tokens, 16, evenly 1902 / 1788, 1923 / 1800; of 2048 x 2048, 4096 tokens
+// 1439 / 1285, 1454 / 1294. Where the sizes allow it but the planner then finds too few tiles, the four launches that do nothing cost up to 25 us, most in
+// small steps: 256 experts of mixed levels, Zipf 4286 / 4326; 2000 tokens, 64 experts, Zipf 2211 / 2240; 4096, 16 experts, 2 picks 1085 / 1099. At level 2, where a tile's decode is half as long, 16 experts of 2048 rows lose: 3173 / 3281.
 // Fewer units leave CUs idle for the 0.2 ms of one: 1000 tokens, 16 experts, Zipf (a single expert of 993 rows) 1070 / 1173.
 // A block of 128 weight rows costs what one of 256 does: 2304 + 4096 rows, 11 % of them padding in gate|up, 1922 / 1961. Scratch: 2 GB at most.
 constexpr int WIDE_MIN = 640, WIDE_UNITS = 512;

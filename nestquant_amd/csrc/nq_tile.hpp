@@ -294,8 +294,10 @@ __device__ __forceinline__ UnitWords unit_words(const Planes& P, const LaneCtx& 
 // What a chunk's decode needs beside the records, fold constants and ring signs, for 32 chunks of the wavefront's two strips at a time: lane 32 s + i
 // reads the block word and sign byte of strip s, chunk c0 + i, and works out its constants; a chunk's come from there by one
 // lane permute (two at levels 3 / 4). Worked out by every lane in every chunk they were some 25 of the 600 vector instructions of a refined chunk
-// and, with no sign plane, 5 of the 275 of a chunk at level 2, beside one or two loads. us anew in every chunk / as now: 4 tokens of 6144 x 2048 203 / 198,
-// one 63.3 / 62.0, a lone gate|up projection of 8 tokens at level 3 13.8 / 13.5, 48 and 201 tokens 1144 / 1127 and 1335 / 1307.
+// and, with no sign plane, 5 of the 275 of a chunk at level 2, beside one or two loads. A tile of the grouped GEMMs has all chunks of its projection
+// (48 of gate|up at 6144 columns), a slice of a decode call at most 24 of gate|up and 4 of down; slices of one: gemv_chunks' FEW. us anew in every chunk /
+// as now: 4 tokens of 6144 x 2048 204 / 199, all at level 4 305 / 286, one token 61.1 / 60.5; a lone gate|up projection of 8 tokens at level 3 13.65 / 13.37;
+// 48 and 201 tokens, with the scalar token addresses, 1157 / 1136 and 1340 / 1313.
 template <bool RES>
 struct UnitConsts
 {
@@ -308,8 +310,8 @@ struct UnitConsts
         from = (int)(threadIdx.x & 8u) << 4;
         k = consts_l2(0u);
     }
-    // at chunk c's beginning, ahead of the next chunk's requests: behind them, with a branch in between, the wait for the block words was one for those
-    // requests too. The reciprocal is divided out (IEEE, the table's bits): its entry would be another latency before a slice's first product.
+    // at chunk c's beginning. gemv_chunks has it ahead of the next chunk's requests: behind them, with a branch in between, the wait for the block words
+    // was one for those requests too. In pf_chunks, whose chunks take ten times as long, it is behind them. The reciprocal is divided out (IEEE, the table's bits): its entry would be another latency before a slice's first product.
     __device__ __forceinline__ void begin(const Planes& P, const LaneCtx& L, int c, int NC)
     {
         if ((RES || P.var) && (c & 31) == 0)
