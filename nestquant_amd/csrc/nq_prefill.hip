@@ -674,8 +674,15 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
 {
     extern __shared__ __align__(16) char smem[];
     const int nb = (a.I + 255) / 256, ncol = a.mode == 0 ? 2 * nb : (a.H + 255) / 256;
+    const int nt = a.count ? *a.count : a.ntiles, units = nt * ncol;
+    if (!a.count)
+    {   // a list of the caller's, nq_pf_plan's with its gaps: units dealt out one by one, or a few XCDs have all tiles. gate|up of 98 tiles in 385
+        // places, 78 of them of decoded weights, 3226 us in runs, 1514 so
+        for (int unit = blockIdx.x; unit < units; unit += gridDim.x) wide_unit(a, unit, nt, ncol, nb, smem);
+        return;
+    }
     // An XCD works through a run of neighbouring units: WIDE_GROUP tiles by one column block after the other
-    const int nt = a.count ? *a.count : a.ntiles, units = nt * ncol, per = (units + 7) / 8, first = (int)(blockIdx.x & 7) * per;
+    const int per = (units + 7) / 8, first = (int)(blockIdx.x & 7) * per;
     for (int unit = first + (int)(blockIdx.x >> 3); unit < min(units, first + per); unit += (int)gridDim.x >> 3)
         wide_unit(a, unit, nt, ncol, nb, smem);
 }

@@ -177,6 +177,38 @@ def test_tiles_of_decoded_weights_give_the_bits_of_decode_fused_tiles(H, I, deco
     assert want.isfinite().all()
 
 
+@pytest.mark.parametrize("H,I", [(256, 128), (384, 640)])
+def test_decoded_weights_over_the_lists_of_the_plan(H, I):
+    """nq_pf_plan, nq_pf_wdecode and nq_pf_gemm one by one, as a caller of the single entry points has them: list 4 with its gaps, decoded weights for some of its
+    experts, the same bits as without, rows of other lists left alone"""
+    from nestquant_amd import _lib
+    Lb, rows, E = _lib.lib(), [300, 0, 129, 90, 1100, 40, 256, 770, 3], 9
+    ex = to_dev(experts_on_gpu(H, I, 3, 90, nested_ids=(1,)))
+    L = M.MoELayer(E, H, I, Bmax=2, topk=1)
+    for e in range(E):
+        L.set(e, ex[e % 3], 4 if e % 2 else 2)
+    P, cnt = sum(rows), torch.tensor(rows, dtype=torch.int32, device=DEV)
+    cap = E + P // 256 + 1
+    tiles, hot = torch.empty(5, cap, 4, dtype=torch.int32, device=DEV), torch.empty(E, dtype=torch.int32, device=DEV)
+    _lib.check(Lb.nq_pf_plan(cnt.data_ptr(), E, 0, P, tiles.data_ptr(), cap, hot.data_ptr(), 200, 3, _lib.stream_ptr()))
+    torch.cuda.synchronize()
+    assert hot.tolist() == [0, -1, -1, -1, 1, -1, 2, -1, -1]     # three slots for four experts of 200 rows
+    g = torch.Generator().manual_seed(91)
+    A0, A1 = [(torch.randn(P, max(H, I), generator=g) * 0.05).half().to(DEV) for _ in range(2)]
+    wop = torch.zeros(3, 3 * H * I, dtype=torch.float16, device=DEV)
+    for mode in (0, 1):
+        _lib.check(Lb.nq_pf_wdecode(L.table.data_ptr(), hot.data_ptr(), E, mode, wop.data_ptr(), wop.numel() * 2, 3, H, I, _lib.stream_ptr()))
+        C = [torch.full((P, 2 * I if mode == 0 else H), 7.0, device=DEV) for _ in range(2)]
+        for c, w in zip(C, (None, wop.data_ptr())):
+            _lib.check(Lb.nq_pf_gemm(L.table.data_ptr(), tiles[4].data_ptr(), cap, 256, mode | 4, A0.data_ptr(), A1.data_ptr(), c.data_ptr(), E, H, I, w, _lib.stream_ptr()))
+        torch.cuda.synchronize()
+        assert torch.equal(*C)
+        tall = torch.zeros(P, dtype=torch.bool)
+        for e, r0, n, _ in tiles[4].tolist():
+            tall[r0:r0 + n] |= e >= 0
+        assert torch.equal((C[1] != 7).any(1).cpu(), tall) and 0 < int(tall.sum()) < P
+
+
 def test_slots_beyond_a_grid_are_decoded():
     """an expert with a slot of decoded weights beyond the 65535 of one launch (6.4 GB of the smallest shape's): the bytes of slot 0"""
     from nestquant_amd import _lib
