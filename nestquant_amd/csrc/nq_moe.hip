@@ -817,8 +817,8 @@ nq_gemv_k(MoeArgs a, int NC)
     if constexpr (ANYROW)
         dispatch_base(P.bcode, [&](auto bk) {
             constexpr int BK = decltype(bk)::value;
-            if (R.level == 2) gemv_chunks<false, 0, BK>(P, L, NC, acc, nb0);
-            else dispatch_code(P.code, [&](auto tag) { gemv_chunks<true, decltype(tag)::value, BK>(P, L, NC, acc, nb0); });
+            if (R.level == 2) gemv_chunks<false, 0, BK, true, false, FEW>(P, L, NC, acc, nb0);
+            else dispatch_code(P.code, [&](auto tag) { gemv_chunks<true, decltype(tag)::value, BK, true, false, FEW>(P, L, NC, acc, nb0); });
         });
     else if (foreign)
     {
@@ -939,8 +939,8 @@ int launch_moe(const MoeArgs& a, const int* cfg_gu, const int* cfg_dn, int which
         const bool self = own && mode == 0;
         const bool few = own || NC < FEW_CHUNKS;
         auto kern = self ? nq_gemv_k<0, false, true, true>
-                  : mode == 0 ? (any ? nq_gemv_k<0, true> : few ? nq_gemv_k<0, false, false, true> : nq_gemv_k<0, false>)
-                              : (any ? nq_gemv_k<1, true> : few ? nq_gemv_k<1, false, false, true> : nq_gemv_k<1, false>);
+                  : mode == 0 ? (any ? few ? nq_gemv_k<0, true, false, true> : nq_gemv_k<0, true> : few ? nq_gemv_k<0, false, false, true> : nq_gemv_k<0, false>)
+                              : (any ? few ? nq_gemv_k<1, true, false, true> : nq_gemv_k<1, true> : few ? nq_gemv_k<1, false, false, true> : nq_gemv_k<1, false>);
         if (shm > 48 * 1024)
         {
             hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
