@@ -907,6 +907,8 @@ constexpr int OWN_ROUTE_WGS = 512;
 //   2048 x 1024, 6 (1, 1) 23.29 / 23.28 / 22.99 / 23.08, 16 (4, 1) 41.19 / 40.56 / 42.35 / 41.79; 6144 x 2048, 2 (3, 1) 33.19 / 33.04 / 33.25 / 33.32.
 // Two and more: 3072 x 1536, 16 (8, 3) 47.65 / 48.08 / 48.37 / 48.65; 4096 x 2048, 8 (8, 2) 46.92 / 47.01 / 47.46 / 47.59; 6144 x 2048, 8 (12, 4)
 //   60.81 / 61.14 / 61.21 / 61.77, 32 (24, 4) 201.2 / 202.1 / 204.4 / 205.4.
+// A lone projection's slices likewise (launch_proj), UnitConsts / without, its weights in no cache: 6144 x 4096, 8 tokens, level 3, three chunks 14.63 / 15.18.
+// In slices of one, weights at hand, 2048 x 2048, 8 tokens, level 4 7.38 / 7.22; 1024 x 1024, one 5.97 / 5.79; 512 x 512, 8, level 3 6.28 / 6.08.
 constexpr int FEW_CHUNKS = 2;
 int launch_moe(const MoeArgs& a, const int* cfg_gu, const int* cfg_dn, int which, hipStream_t st)
 {
@@ -1024,6 +1026,7 @@ __device__ __forceinline__ float4_t ld_dev4_issue(const float* p)
     asm volatile("global_load_dwordx4 %0, %1, off sc0 sc1" : "=v"(v) : "v"(p) : "memory");
     return v;
 }
+template <bool FEW>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) nq_proj_k(ProjArgs a, int NC)
 {
     extern __shared__ __align__(16) char smem[];
@@ -1072,8 +1075,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))
 
     float4_t acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
     if (foreign) { const float nan = __builtin_nanf(""); acc[0] = float4_t{nan, nan, nan, nan}; acc[1] = acc[0]; }
-    else if (level == 2) gemv_chunks<false, 0, 0, false>(P, L, NC, acc, nb0);
-    else if (live) dispatch_code(P.code, [&](auto tag) { gemv_chunks<true, decltype(tag)::value, 0, false>(P, L, NC, acc, nb0); });
+    else if (level == 2) gemv_chunks<false, 0, 0, false, false, FEW>(P, L, NC, acc, nb0);
+    else if (live) dispatch_code(P.code, [&](auto tag) { gemv_chunks<true, decltype(tag)::value, 0, false, false, FEW>(P, L, NC, acc, nb0); });
     __builtin_amdgcn_s_setprio(3);
 
     const int row = 16 * (2 * (blockIdx.x * SB + warp) + (t4 >> 1)) + 4 * (t4 & 1);
@@ -1116,12 +1119,13 @@ int launch_proj(const void* x, int x_dtype, int B, const int64_t* row, int H, in
 {
     const ProjArgs a{x, row, part, cnt, out, x_dtype, B, H, I, G, cnt_step};
     const int shm = B * (NC * 256 + 16) + 256;
+    auto kern = NC < FEW_CHUNKS ? nq_proj_k<true> : nq_proj_k<false>;
     if (shm > 48 * 1024)
     {
-        const hipError_t e = hipFuncSetAttribute((const void*)nq_proj_k, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
+        const hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
         if (e != hipSuccess) return set_error("nq_proj: LDS %d bytes: %s", shm, hipGetErrorString(e));
     }
-    nq_proj_k<<<dim3(2 * I / 32 / SB, H / 128 / NC), 64 * SB, shm, st>>>(a, NC);
+    kern<<<dim3(2 * I / 32 / SB, H / 128 / NC), 64 * SB, shm, st>>>(a, NC);
     NQ_LAUNCH_CHECK("nq_proj");
     return 0;
 }

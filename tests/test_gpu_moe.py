@@ -799,3 +799,7 @@ def test_short_slices_give_the_bits_of_the_complete_kernel(H, I, gu, dn, topk, h
     if not hoist:                                                # the complete kernel has no hoisted form
         assert torch.equal(got, want)
     assert rel_err(got.cpu().numpy(), want.cpu().numpy()) < 1e-3
+    if not hoist:                                                # and a lone projection against the layer call that stands for it with such rows
+        one = [M.proj_gemv(L, x, e, [1, 4, gu]) for e in range(10)]
+        L.rare_rows = True
+        assert all(torch.equal(y, M.proj_gemv(L, x, e, [1, 4, gu])) and y.any() for e, y in enumerate(one))
